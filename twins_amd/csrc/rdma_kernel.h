@@ -14,6 +14,7 @@ struct TeamState
     unsigned act;
     int stop;
     unsigned long long wake;
+    unsigned long long prof[2]; // (profiling builds: the slot's longest host and switch items)
 };
 // one launch: teams of T workgroups take worlds queue[0 .. nq) in order (qnext: the next index);
 // an entry is sim << QSHIFT | world: world `world` of the batch whose Sim is sims[sim] (a launch can
@@ -23,6 +24,7 @@ constexpr int LAUNCH_WAVES = 4; // waves of a launch's 256-thread workgroups
 struct LaunchCfg
 {
     int T, nq, hpw; // hpw: hosts of a host item (side by side on a wave's lanes, at most 64)
+    int by_group;   // a switch runs on a whole workgroup where a world has at most this many workgroup items per workgroup (0: never)
     const int *queue;
     unsigned *qnext;
     TeamState *teams;

@@ -17,16 +17,54 @@ constexpr long long LAUNCH_TICKS = 100000000;          // a launch's time: 1 s o
 constexpr unsigned long long WAIT_TICKS = 2000000000ull; // a barrier wait gives up after 20 s
 constexpr int WAVES = LAUNCH_WAVES;                    // waves of a 256-thread workgroup
 
-// (its LDS holds one workgroup per CU: one wave per SIMD, so all registers may be used)
+// (Four waves' workspaces of LDS: one workgroup per CU, one wave per SIMD, so all registers may be used.)
+// A host item: `hpw` hosts side by side, lane i's events are host e0 + i's. The lanes share out the
+// copying of the hosts' arrivals into their workspaces and of the frames sent out of them, 64 / hpw
+// lanes a host: one round of loads and one of stores a slot, off the hosts' chains of events (24
+// FatTree k=8 worlds as one batch 181 -> 156 ms of kernel; worlds alone, whose items have a host or
+// two, within 3%: there the events' own instructions bound the item).
+__device__ __forceinline__ bool host_item(SimRef s, int e0, int n, int hpw, int64_t slot, unsigned *flows_done, uint32_t *pend, int pend_n,
+                                          int64_t *wake, char *mem, int lane)
+{
+    const int per = WAVE_LDS / hpw & ~15, group = 64 / hpw, mine = lane / group, words = (int)(sizeof(LFrame) / 8);
+    HostSlot x = {false, 0, 0};
+    if (lane < n)
+        x = host_open(s, e0 + lane, slot, wake);
+    const HostWork w = host_work(mem + (size_t)(lane < hpw ? lane : 0) * per, per);
+    const int in_n = x.an < w.in_cap ? x.an : w.in_cap;
+    {
+        const HostWork g = host_work(mem + (size_t)(mine < hpw ? mine : 0) * per, per);
+        const int k = __shfl(in_n, mine < hpw ? mine : 0) * (mine < hpw ? words : 0);
+        const uint64_t at = __shfl(x.abase, mine < hpw ? mine : 0);
+        for (int i = lane % group; i < k; i += group)
+            in_word(g.in[i / words], i % words, in_load(s, at + i / words, i % words));
+    }
+    RD_WAVE_SYNC();
+    bool act = false;
+    int out_n = 0;
+    if (x.runs)
+        act = host_events(s, e0 + lane, slot, flows_done, pend, pend_n, wake, x.an, x.abase, w, in_n, &out_n);
+    RD_WAVE_SYNC();
+    {
+        const HostWork g = host_work(mem + (size_t)(mine < hpw ? mine : 0) * per, per);
+        const int k = __shfl(out_n, mine < hpw ? mine : 0) * (mine < hpw ? words : 0);
+        for (int i = lane % group; i < k; i += group)
+            out_store(g.out[i / words], i % words);
+    }
+    RD_WAVE_SYNC(); // (the workspace is reused by the next item)
+    return act;
+}
+
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) rdma_team_kernel(const LaunchCfg *__restrict__ lp)
 {
     const LaunchCfg L = *lp;
-    __shared__ SwWork work[WAVES];
+    __shared__ __attribute__((aligned(16))) char work[WAVES][WAVE_LDS];
     __shared__ int64_t s_slot;
     __shared__ int s_w, s_stop, s_err;
     __shared__ unsigned s_act;
     __shared__ unsigned long long s_wake;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    // (the wave's number made a scalar: what a wave's item indexes is then loaded by scalar loads)
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int T = L.T;
     // a team's workgroups have consecutive ids, so they spread over the 8 XCDs (workgroups reach
     // the XCDs round-robin by id). Teams kept on one XCD each were measured slower: the reference's
@@ -98,12 +136,26 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
         __syncthreads();
         if (s_w >= L.nq)
             return;
-        const int qe = L.queue[s_w], w = qe & ((1 << QSHIFT) - 1);
-        const Sim &s = *L.sims[qe >> QSHIFT];
+        const int qe = __builtin_amdgcn_readfirstlane(L.queue[s_w]), w = qe & ((1 << QSHIFT) - 1);
+        const uint64_t sp = (uint64_t)L.sims[qe >> QSHIFT];
+        // (the Sim record through a scalar pointer in the constant address space: its fields are
+        // scalar loads; through a generic one every use of a field was a flat load, which waits for
+        // the stores before it)
+        SimRef s = *(const Sim RD_C *)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(sp >> 32)) << 32 |
+                                       (uint32_t)__builtin_amdgcn_readfirstlane((int)sp));
         const World wd = s.wd[w];
         WorldRun &r = s.run[w];
         uint32_t *pend = s.pend + wd.pend_off;
-        const int hpw = L.hpw, nhw = (wd.nh + hpw - 1) / hpw, items = nhw + wd.ns, TW = T * WAVES, gw = rank * WAVES + wv;
+        const int hpw = L.hpw, nhw = (wd.nh + hpw - 1) / hpw;
+        // Work items: a wave each, or, where the team has about a workgroup per switch, a switch for a
+        // whole workgroup (its ports over four waves: a wave's lanes run unlike events one after
+        // another, so fewer ports a wave is a shorter slot: FatTree k=8 a2a, HPCC, the longest switch of
+        // a slot 191 us on a wave, 134 us on four) and a host item for each of its waves. With more
+        // switches than that, a wave each runs more of them side by side.
+        const bool by_group = L.by_group && wd.ns + (nhw + WAVES - 1) / WAVES <= L.by_group * T;
+        const int ngh = (nhw + WAVES - 1) / WAVES;
+        const int first = by_group ? rank : rank * WAVES + wv, step = by_group ? T : T * WAVES;
+        const int host_items = by_group ? ngh : nhw, items = host_items + wd.ns;
         const long long t_world = wall_clock64();
         for (;;)
         {
@@ -124,31 +176,39 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
 #ifdef RD_PROF
             long long p0 = wall_clock64(), ph = 0, psw = 0;
 #endif
-            for (int it = gw; it < items; it += TW)
+            for (int it = first; it < items; it += step)
             {
 #ifdef RD_PROF
                 const long long q0 = wall_clock64();
 #endif
-                if (it < nhw)
+                if (it < host_items)
                 {
-                    const int e = it * hpw + lane;
-                    if (lane < hpw && e < wd.nh)
-                    {
-                        int64_t hw = INT64_MAX;
-                        a |= host_step(s, wd.h0 + e, sl, &r.flows_done, pend, wd.pend_n, &hw) ? 1u : 0u;
-                        if (hw != INT64_MAX && (unsigned long long)hw < wk)
-                            wk = (unsigned long long)hw;
-                    }
+                    const int hi = by_group ? it * WAVES + wv : it;
+                    const int e0 = hi * hpw, n = wd.nh - e0 < hpw ? wd.nh - e0 : hpw;
+                    int64_t hw = INT64_MAX;
+                    if (n > 0)
+                        a |= host_item(s, wd.h0 + e0, n, hpw, sl, &r.flows_done, pend, wd.pend_n, &hw, work[wv], lane) ? 1u : 0u;
+                    if (hw != INT64_MAX && (unsigned long long)hw < wk)
+                        wk = (unsigned long long)hw;
                 }
                 else
                 {
-                    const int x = wd.s0 + (it - nhw);
+                    const int x = wd.s0 + (it - host_items);
                     const int deg = s.si[x].deg;
                     bool busy = false;
-                    if (s.sw_busy[x] || switch_has_input(s, x, sl))
+                    const bool run = s.sw_busy[x] || __any(switch_has_input(s, x, sl, lane, 64));
+                    if (by_group)
+                    {
+                        // (every wave has looked before the first sync, and the switch is this workgroup's alone)
+                        __syncthreads();
+                        if (run)
+                            busy = switch_slot_by(s, x, sl, pend, wd.pend_n, &work[0][0], WAVES * WAVE_LDS, lane * WAVES + wv, 64 * WAVES,
+                                                  [] { __syncthreads(); });
+                    }
+                    else if (run)
                     {
                         if (deg <= KS)
-                            busy = switch_slot(s, x, sl, pend, wd.pend_n, work[wv], lane, 64);
+                            busy = switch_slot(s, x, sl, pend, wd.pend_n, *reinterpret_cast<SwWork *>(work[wv]), lane, 64);
                         else if (deg <= KW && L.wide)
                             busy = switch_slot(s, x, sl, pend, wd.pend_n, L.wide[(size_t)blockIdx.x * WAVES + wv], lane, 64);
                         else
@@ -159,20 +219,22 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
                             busy = __shfl(b, 0) != 0;
                         }
                     }
-                    if (lane == 0)
+                    if (lane == 0 && (!by_group || wv == 0))
                     {
                         s.sw_busy[x] = busy ? 1 : 0;
                         a |= busy ? 1u : 0u;
                     }
                 }
 #ifdef RD_PROF
-                (it < nhw ? ph : psw) += wall_clock64() - q0;
+                (it < host_items ? ph : psw) += wall_clock64() - q0;
 #endif
             }
 #ifdef RD_PROF
             // (profiling builds: the waves' host and switch item time, and the time to the slot's end)
             if (lane == 0)
             {
+                atomicMax(&ts->prof[0], (unsigned long long)ph);
+                atomicMax(&ts->prof[1], (unsigned long long)psw);
                 if (ph)
                     atomicAdd(&s.ev[33], (unsigned long long)ph);
                 if (psw)
@@ -195,6 +257,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
                     atomicMin(&ts->wake, s_wake);
             }
             if (barrier([&] {
+#ifdef RD_PROF
+                    atomicAdd(&s.ev[22], atomicExch(&ts->prof[0], 0ull));
+                    atomicAdd(&s.ev[23], atomicExch(&ts->prof[1], 0ull));
+#endif
                     slot_end(s, wd, r, pend, atomicOr(&ts->act, 0u), atomicMin(&ts->wake, ~0ull));
                     coh_store(&ts->act, 0u);
                     coh_store(&ts->wake, ~0ull);

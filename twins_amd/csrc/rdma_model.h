@@ -21,8 +21,13 @@
 // them (a flat access waits on LDS traffic too)
 #if defined(__HIP_DEVICE_COMPILE__)
 #define RD_G __attribute__((address_space(1)))
+// What the host wrote before the launch and nothing writes during it (the Sim record, the worlds'
+// tables) carries the constant address space: its loads are scalar where the address is the same on
+// every lane, and never wait for the stores before them.
+#define RD_C __attribute__((address_space(4)))
 #else
 #define RD_G
+#define RD_C
 #endif
 #if defined(__HIPCC__)
 #include <hip/hip_runtime.h>
@@ -108,7 +113,7 @@ struct Chain
 };
 struct TailNode
 {
-    uint32_t code, cnt;
+    uint64_t run; // the run's code, its count above
     uint64_t next, pos;
 };
 
@@ -260,10 +265,11 @@ struct FlowInfo
 // a queue pair, sender side (RdmaQueuePair; src/rdma/rdma.h:174-229)
 struct SndQP
 {
-    uint64_t size, snd_nxt, snd_una;
-    uint64_t rate, max_rate;
+    uint64_t size, snd_nxt, snd_una; // (what the scheduler looks at, in one cache line)
     int64_t next_avail;
-    uint32_t last_pkt, win;
+    uint64_t lim; // the window's limit at this rate (qp_new_rate; while win)
+    uint32_t win, last_pkt;
+    uint64_t rate, max_rate;
     uint64_t base_rtt;
     uint8_t done, alpha_cnp, dec_cnp, first_cnp;
     uint32_t rp_stage;
@@ -375,7 +381,9 @@ struct Link
 // a sender's place in its out link's ring (src/rdma/rstep.cuh:45-66)
 struct OutBucket
 {
-    int64_t lo, hi; // its slot's times (hi 0: none open)
+    int64_t hi;     // the open bucket's end (0: none open)
+    int64_t a, end; // the arrival slot reached (the open bucket's, or before any the running slot) and its end
+    uint32_t b, pb; // its places in the link's ring and in the world's pending-slot ring
     uint64_t base;
     uint32_t cnt, n;
     int link;
@@ -454,18 +462,18 @@ struct Sim
     int H, S, F, W, L, R;
     int serial; // every switch slot on the serial path (--serial)
     int64_t D; // the slot (ns)
-    const Params RD_G *Pw;
-    const World RD_G *wd;
+    const Params RD_C *Pw;
+    const World RD_C *wd;
     WorldRun RD_G *run;
-    const int RD_G *h_world, *h_link_in, *h_link_out;
-    const SwInfo RD_G *si;
-    const int RD_G *s_world;
-    const PortCfg RD_G *pc;
-    const Route RD_G *rt;
-    const uint8_t RD_G *rtp;
-    const FlowInfo RD_G *fi;
-    const uint32_t RD_G *root_rank;
-    const int RD_G *start_list;
+    const int RD_C *h_world, *h_link_in, *h_link_out;
+    const SwInfo RD_C *si;
+    const int RD_C *s_world;
+    const PortCfg RD_C *pc;
+    const Route RD_C *rt;
+    const uint8_t RD_C *rtp;
+    const FlowInfo RD_C *fi;
+    const uint32_t RD_C *root_rank;
+    const int RD_C *start_list;
     SndQP RD_G *qp;
     QPChains RD_G *qc;
     RcvQP RD_G *rx;
@@ -482,21 +490,45 @@ struct Sim
     PortRun RD_G *pr;
     Pkt RD_G *q0, *q3;
     int q0_cap, q3_cap;
-    const Link RD_G *li;
+    const Link RD_C *li;
     LFrame RD_G *msg;
     uint32_t msg_bytes; // the link rings' size when below 2^31 (frames written 16 bytes a store), else 0
     int64_t RD_G *msg_cnt;
-    const int32_t RD_G *txt; // [R][TXT_N]
+    const int32_t RD_C *txt; // [R][TXT_N]
     uint32_t RD_G *pend;
     TailNode RD_G *tail;
     unsigned long long RD_G *tail_cnt; // [W]
-    const TailRing RD_G *rings;        // [W]
+    const TailRing RD_C *rings;        // [W]
     unsigned long long RD_G *memo;
     uint64_t memo_mask;
     int64_t RD_G *fct;
     unsigned long long RD_G *ev;
     TxTrace txt_rec; // the transmission trace (off unless asked for)
 };
+
+// a value that every active lane of the wave holds alike, in a scalar register
+#if defined(__HIP_DEVICE_COMPILE__)
+#define RD_UNIFORM(x) __builtin_amdgcn_readfirstlane(x)
+#else
+#define RD_UNIFORM(x) (x)
+#endif
+// the lanes of a wave wait for each other's LDS (and their own memory) accesses
+#if defined(__HIP_DEVICE_COMPILE__)
+#define RD_WAVE_SYNC()                                                                                                            \
+    do                                                                                                                            \
+    {                                                                                                                             \
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");                                                                    \
+        __builtin_amdgcn_wave_barrier();                                                                                          \
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");                                                                    \
+    } while (0)
+#else
+#define RD_WAVE_SYNC() \
+    do                 \
+    {                  \
+    } while (0)
+#endif
+typedef const Sim RD_C &SimRef;
+typedef const Params RD_C &ParamsRef;
 
 // ------------------------------------------------------------------ atomics (device) / plain (CPU build)
 RD_HD unsigned long long at_add64(unsigned long long *p, unsigned long long v)
@@ -540,7 +572,7 @@ RD_HD unsigned long long at_cas64(unsigned long long *p, unsigned long long cmp,
     return o;
 #endif
 }
-RD_HD void count(const Sim &s, int i) { at_add64(&s.ev[i], 1ull); }
+RD_HD void count(SimRef s, int i) { at_add64(&s.ev[i], 1ull); }
 RD_HD uint64_t mulhi64(uint64_t a, uint64_t b)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -560,21 +592,21 @@ RD_HD int64_t ns_seconds(double x)
 }
 // DataRate(bps).CalculateTxTime(bytes) in ns
 RD_HD int64_t tx_ns(uint64_t bps, uint32_t bytes) { return ns_seconds((double)bytes * 8 / (double)bps); }
-RD_HD int64_t rc_tx(const Sim &s, uint32_t rc, uint64_t bps, uint32_t bytes)
+RD_HD int64_t rc_tx(SimRef s, uint32_t rc, uint64_t bps, uint32_t bytes)
 {
     if (bytes < (uint32_t)TXT_N)
         return s.txt[(size_t)rc * TXT_N + bytes];
     return tx_ns(bps, bytes);
 }
-RD_HD int64_t link_tx(const Sim &s, int link, uint32_t bytes)
+RD_HD int64_t link_tx(SimRef s, int link, uint32_t bytes)
 {
-    const Link &l = s.li[link];
+    const Link RD_C &l = s.li[link];
     if (bytes < (uint32_t)TXT_N)
         return s.txt[(size_t)l.rc * TXT_N + bytes];
     return tx_ns(l.bps, bytes);
 }
 // link_tx for a sender's out link, remembering its last two sizes (a sender sends few sizes)
-RD_HD int64_t link_txo(const Sim &s, struct OutBucket &o, uint32_t bytes);
+RD_HD int64_t link_txo(SimRef s, struct OutBucket &o, uint32_t bytes);
 RD_HD uint64_t rate_of(double d) { return (uint64_t)d; }
 RD_HD int ring_add(int a, int b, int n)
 {
@@ -584,18 +616,27 @@ RD_HD int ring_add(int a, int b, int n)
 
 // ------------------------------------------------------------------ link rings (src/rdma/rstep.cuh:67-133; rdma.h:635-642)
 // frames of `link` arriving in `slot`: their count, first one at *base
-RD_HD int bucket(const Sim &s, int link, int64_t slot, uint64_t *base)
+// slot % n (a 64-bit division only for slots beyond 32 bits)
+RD_HD uint32_t ring_place(int64_t slot, uint32_t n)
 {
-    const Link &l = s.li[link];
-    int b = (int)(slot % (int64_t)l.nb);
+    return (uint64_t)slot >> 32 ? (uint32_t)(slot % (int64_t)n) : (uint32_t)slot % n;
+}
+RD_HD int bucket(SimRef s, int link, int64_t slot, uint64_t *base)
+{
+    const Link RD_C &l = s.li[link];
+    const uint32_t b = ring_place(slot, l.nb);
     const int64_t v = coh_load(s.msg_cnt + l.coff + b);
     *base = l.moff + (uint64_t)b * l.cap;
     return (v >> 16) == slot ? (int)(v & 0xFFFF) : 0;
 }
-RD_HD void ob_open(const Sim &s, OutBucket &o, int link, int64_t last)
+RD_HD void ob_open(SimRef s, OutBucket &o, int link, int64_t last, int64_t slot, int pend_n)
 {
     const Link l = s.li[link];
     o.hi = 0;
+    o.a = slot;
+    o.end = (slot + 1) * s.D;
+    o.b = ring_place(slot, l.nb);
+    o.pb = ring_place(slot, (uint32_t)pend_n);
     o.link = link;
     o.last = last;
     o.txs[0] = o.txs[1] = 0;
@@ -605,7 +646,7 @@ RD_HD void ob_open(const Sim &s, OutBucket &o, int link, int64_t last)
     o.cap = l.cap;
     o.delay = l.delay;
 }
-RD_HD int64_t link_txo(const Sim &s, OutBucket &o, uint32_t bytes)
+RD_HD int64_t link_txo(SimRef s, OutBucket &o, uint32_t bytes)
 {
     if (bytes == o.txs[0])
         return o.txv[0];
@@ -616,28 +657,35 @@ RD_HD int64_t link_txo(const Sim &s, OutBucket &o, uint32_t bytes)
     o.txs[0] = bytes, o.txv[0] = t;
     return t;
 }
-RD_HD void ob_flush(const Sim &s, OutBucket &o)
+RD_HD void ob_flush(SimRef s, OutBucket &o)
 {
     if (o.hi == 0)
         return;
-    o.last = (o.lo / s.D) << 16 | o.n;
+    o.last = o.a << 16 | o.n;
     coh_store(s.msg_cnt + o.cnt, o.last);
     o.hi = 0;
 }
-// a place in the bucket of the frame's arrival slot (null: full, counted)
-RD_HD LFrame RD_G *ob_push(const Sim &s, uint32_t *pend, int pend_n, int64_t ts, OutBucket &o)
+// a place in the bucket of the frame's arrival slot (null: full, counted). A link's frames arrive one
+// after another, so the arrival slot is found by stepping on from the last one's: one or two steps,
+// where the quotient and the ring places took three 64-bit divisions (some 500 instructions that
+// every lane of the wave waited for)
+RD_HD LFrame RD_G *ob_push(SimRef s, uint32_t *pend, int pend_n, int64_t ts, OutBucket &o)
 {
     if (ts >= o.hi)
     {
         ob_flush(s, o);
-        int64_t a = ts / s.D;
-        int b = (int)(a % (int64_t)o.nb);
-        o.cnt = o.coff + b;
-        o.lo = a * s.D;
-        o.hi = o.lo + s.D;
-        o.base = o.moff + (uint64_t)b * o.cap;
-        o.n = (o.last >> 16) == a ? (uint32_t)(o.last & 0xFFFF) : 0;
-        coh_store(pend + a % pend_n, 1u);
+        while (ts >= o.end)
+        {
+            o.a++;
+            o.end += s.D;
+            o.b = o.b + 1 < o.nb ? o.b + 1 : 0;
+            o.pb = o.pb + 1 < (uint32_t)pend_n ? o.pb + 1 : 0;
+        }
+        o.hi = o.end;
+        o.cnt = o.coff + o.b;
+        o.base = o.moff + (uint64_t)o.b * o.cap;
+        o.n = (o.last >> 16) == o.a ? (uint32_t)(o.last & 0xFFFF) : 0;
+        coh_store(pend + o.pb, 1u);
     }
     if (o.n >= o.cap)
     {
@@ -649,7 +697,7 @@ RD_HD LFrame RD_G *ob_push(const Sim &s, uint32_t *pend, int pend_n, int64_t ts,
 
 // A frame's packet and chain, written coherently: 16 bytes a store (sc1 buffer stores) where the
 // link rings fit a 32-bit offset, else 8-byte atomic stores; plain stores in the CPU build.
-RD_HD void frame_put_pkt(const Sim &s, LFrame RD_G *fr, const Pkt &q)
+RD_HD void frame_put_pkt(SimRef s, LFrame RD_G *fr, const Pkt &q)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
     if (s.msg_bytes)
@@ -665,7 +713,7 @@ RD_HD void frame_put_pkt(const Sim &s, LFrame RD_G *fr, const Pkt &q)
 #endif
     pkt_put(&fr->p, q);
 }
-RD_HD void frame_put_chain(const Sim &s, LFrame RD_G *fr, const Chain &c)
+RD_HD void frame_put_chain(SimRef s, LFrame RD_G *fr, const Chain &c)
 {
 #if defined(__HIP_DEVICE_COMPILE__)
     if (s.msg_bytes)
@@ -708,14 +756,13 @@ RD_HD uint64_t chash(uint64_t h, uint32_t code)
     return z ^ (z >> 31);
 }
 // a tail position's node in the rings
-RD_HD uint64_t tail_slot(const Sim &s, uint64_t pos)
+RD_HD uint64_t tail_slot(const TailRing &r, uint64_t pos)
 {
-    const TailRing r = s.rings[pos >> TAIL_WSHIFT];
     return r.off + (((pos & ((1ull << TAIL_WSHIFT) - 1)) - 1) & r.mask);
 }
 // the chain of an event scheduled with `code` by the event of chain par; the oldest run spills to
 // its world's tail ring when the inline runs are full
-RD_HD void cpush(const Sim &s, TailAlloc &ta, Chain *dst, uint32_t code, const Chain &par)
+RD_HD void cpush(SimRef s, TailAlloc &ta, Chain *dst, uint32_t code, const Chain &par)
 {
     Chain c;
     if (par.r[0].code == code)
@@ -741,9 +788,9 @@ RD_HD void cpush(const Sim &s, TailAlloc &ta, Chain *dst, uint32_t code, const C
                 ta.end = ta.next + TAIL_CHUNK;
             }
             const uint64_t pos = ta.next++;
-            TailNode RD_G *n = s.tail + tail_slot(s, pos);
-            coh_store(&n->code, par.r[RUNS - 1].code);
-            coh_store(&n->cnt, par.r[RUNS - 1].cnt);
+            // (its own world's ring, the same for every lane: a scalar load, not one that waits for stores)
+            TailNode RD_G *n = s.tail + tail_slot(s.rings[RD_UNIFORM((int)(ta.wbits >> TAIL_WSHIFT))], pos);
+            coh_store(&n->run, (uint64_t)par.r[RUNS - 1].code | (uint64_t)par.r[RUNS - 1].cnt << 32);
             coh_store(&n->next, par.tail);
             coh_store(&n->pos, pos);
             c.tail = pos;
@@ -769,7 +816,7 @@ struct RunReader
     uint32_t left;  // repetitions left of the current run
     bool lost;
 };
-RD_HD void rr_fetch(const Sim &s, RunReader &r)
+RD_HD void rr_fetch(SimRef s, RunReader &r)
 {
     if (r.at < RUNS)
     {
@@ -786,19 +833,19 @@ RD_HD void rr_fetch(const Sim &s, RunReader &r)
         r.code = 0;
         return;
     }
-    const TailNode RD_G *tn = s.tail + tail_slot(s, r.node);
-    const TailNode n = {coh_load(&tn->code), coh_load(&tn->cnt), coh_load(&tn->next), coh_load(&tn->pos)};
+    const TailNode RD_G *tn = s.tail + tail_slot(s.rings[r.node >> TAIL_WSHIFT], r.node);
+    const TailNode n = {coh_load(&tn->run), coh_load(&tn->next), coh_load(&tn->pos)};
     if (n.pos != r.node)
     {
         r.lost = true; // the ring has wrapped over it
         r.code = 0;
         return;
     }
-    r.code = n.code;
-    r.left = n.cnt;
+    r.code = (uint32_t)n.run;
+    r.left = (uint32_t)(n.run >> 32);
     r.after = n.next;
 }
-RD_HD void rr_open(const Sim &s, RunReader &r, const Chain &ch, uint32_t code0)
+RD_HD void rr_open(SimRef s, RunReader &r, const Chain &ch, uint32_t code0)
 {
     r.c = &ch;
     r.node = r.after = 0;
@@ -815,7 +862,7 @@ RD_HD void rr_open(const Sim &s, RunReader &r, const Chain &ch, uint32_t code0)
     r.at = joins ? 0 : -1;
     r.left = joins ? r0.cnt + 1 : 1;
 }
-RD_HD void rr_step(const Sim &s, RunReader &r)
+RD_HD void rr_step(SimRef s, RunReader &r)
 {
     if (r.at > RUNS)
         r.node = r.after;
@@ -836,7 +883,7 @@ RD_HD uint64_t memo_key(uint64_t ha, uint64_t hb)
     const uint64_t k = chash(ha * 0x9e3779b97f4a7c15ull ^ hb, 0x5bd1e995u) & ~3ull;
     return k ? k : 4;
 }
-RD_HD int memo_find(const Sim &s, uint64_t ha, uint64_t hb)
+RD_HD int memo_find(SimRef s, uint64_t ha, uint64_t hb)
 {
     const uint64_t k = memo_key(ha, hb);
     for (uint64_t i = 0; i < 4; i++)
@@ -850,7 +897,7 @@ RD_HD int memo_find(const Sim &s, uint64_t ha, uint64_t hb)
     }
     return 0;
 }
-RD_HD void memo_record(const Sim &s, uint64_t ha, uint64_t hb, int r)
+RD_HD void memo_record(SimRef s, uint64_t ha, uint64_t hb, int r)
 {
     const uint64_t k = memo_key(ha, hb);
     for (uint64_t i = 0; i < 4; i++)
@@ -867,7 +914,7 @@ RD_HD void memo_record(const Sim &s, uint64_t ha, uint64_t hb, int r)
 // first; with all leads equal the deepest differing ordinal decides, and distinct roots by their
 // start order. *by_lead: decided by a lead or an end, i.e. by the leads alone; *inexact: a chain
 // ended on an overwritten tail node.
-RD_COLD int order_walk(const Sim &s, uint32_t pa, const Chain &a, uint32_t pb, const Chain &b, bool *inexact, bool *by_lead)
+RD_COLD int order_walk(SimRef s, uint32_t pa, const Chain &a, uint32_t pb, const Chain &b, bool *inexact, bool *by_lead)
 {
     RunReader A, B;
     rr_open(s, A, a, pa);
@@ -917,7 +964,7 @@ RD_HD void lead_hashes(uint64_t *h, uint32_t code0, const Chain &c)
 // order_walk behind two shortcuts (src/rdma/rstep.cuh:504-575): lineages in lockstep (equal lead
 // hashes, distinct roots) run in their roots' rank order; and the memo, probed at each depth
 // while the leads agree. A walk decided by leads fills the memo at the depths it passed.
-RD_COLD int order_events(const Sim &s, uint32_t pa, const Chain &a, uint32_t pb, const Chain &b, bool *inexact)
+RD_COLD int order_events(SimRef s, uint32_t pa, const Chain &a, uint32_t pb, const Chain &b, bool *inexact)
 {
     uint64_t ha[NANC + 1], hb[NANC + 1];
     lead_hashes(ha, pa, a);
@@ -952,11 +999,8 @@ RD_COLD int order_events(const Sim &s, uint32_t pa, const Chain &a, uint32_t pb,
 // A quick test on the chains' first runs (src/rdma/rstep.cuh:577-624): the newest HEAD runs of the
 // chain code0 would make, compared by leads; 0 when they do not decide
 constexpr int HEAD = 3;
-RD_HD void head_runs(Run *out, uint32_t code0, const Chain &c)
+RD_HD void head_runs(Run *out, uint32_t code0, const Run *h)
 {
-    Run h[HEAD];
-    for (int i = 0; i < HEAD; i++)
-        h[i] = coh_get(&c.r[i]);
     const bool joins = code0 && h[0].code == code0;
     const int shift = code0 && !joins ? 1 : 0;
     for (int i = shift; i < HEAD; i++)
@@ -967,32 +1011,39 @@ RD_HD void head_runs(Run *out, uint32_t code0, const Chain &c)
         out[0].cnt = joins ? h[0].cnt + 1 : 1;
     }
 }
+// (run i of three by selects: an array indexed at run time would be kept in scratch memory)
+static_assert(HEAD == 3, "head_at selects of three");
+RD_HD Run head_at(const Run *h, int i) { return i == 0 ? h[0] : i == 1 ? h[1] : h[2]; }
 RD_HD int heads_cmp(const Run *a, const Run *b)
 {
     int i = 0, j = 0;
-    uint32_t la = a[0].cnt, lb = b[0].cnt;
-    while (i < HEAD && j < HEAD)
+    Run x = a[0], y = b[0];
+    for (;;)
     {
-        const uint32_t ca = a[i].code, cb = b[j].code;
-        if (!ca || !cb)
-            break;
-        if ((ca >> ORD_BITS) != (cb >> ORD_BITS))
-            return ca > cb ? -1 : 1;
-        const uint32_t m = la < lb ? la : lb;
-        la -= m;
-        lb -= m;
-        if (!la && ++i < HEAD)
-            la = a[i].cnt;
-        if (!lb && ++j < HEAD)
-            lb = b[j].cnt;
+        if (!x.code || !y.code)
+            return 0;
+        if ((x.code >> ORD_BITS) != (y.code >> ORD_BITS))
+            return x.code > y.code ? -1 : 1;
+        const uint32_t m = x.cnt < y.cnt ? x.cnt : y.cnt;
+        x.cnt -= m;
+        y.cnt -= m;
+        if (!x.cnt)
+        {
+            if (++i == HEAD)
+                return 0;
+            x = head_at(a, i);
+        }
+        if (!y.cnt)
+        {
+            if (++j == HEAD)
+                return 0;
+            y = head_at(b, j);
+        }
     }
-    return 0;
 }
 // does (ta, the event code pa pushes on a) run before (tb, the one pb pushes on b)? Times first,
 // then the chains; an undecided tie keeps b (src/rdma/rstep.cuh:635-657)
-// does (ta, the event code pa pushes on a) run before (tb, the one pb pushes on b)? Times first,
-// then the chains; an undecided tie keeps b (src/rdma/rstep.cuh:635-657)
-RD_COLD bool before(const Sim &s, int64_t ta, uint32_t pa, const Chain &a, int64_t tb, uint32_t pb, const Chain &b)
+RD_COLD bool before(SimRef s, int64_t ta, uint32_t pa, const Chain &a, int64_t tb, uint32_t pb, const Chain &b)
 {
     if (ta != tb)
         return ta < tb;
@@ -1005,29 +1056,51 @@ RD_COLD bool before(const Sim &s, int64_t ta, uint32_t pa, const Chain &a, int64
     return r < 0;
 }
 // at one time: the root rule on the events' own lead hashes, then the head runs, then before()
-// (the quick test src/rdma/rstep.cuh:626-633 applies to arrivals, TransmitCompletes and sends)
-RD_COLD bool before_q(const Sim &s, int64_t t, uint32_t pa, const Chain &a, uint32_t pb, const Chain &b)
+// (the quick test src/rdma/rstep.cuh:626-633 applies to arrivals, TransmitCompletes and sends).
+// quick_order: the part without the walk (0: undecided), on what it needs of the two chains
+struct Head
 {
-    const uint64_t a_hash = coh_load(&a.hash), b_hash = coh_load(&b.hash);
-    const uint32_t a_root = coh_load(&a.root), b_root = coh_load(&b.root);
-    const uint64_t ha = pa ? chash(a_hash, pa) : a_hash, hb = pb ? chash(b_hash, pb) : b_hash;
-    int r;
-    if (a_root && b_root && a_root != b_root && ha == hb)
-        r = s.root_rank[a_root - 1] < s.root_rank[b_root - 1] ? -1 : 1;
-    else
+    uint64_t hash;
+    uint32_t root;
+    Run r[HEAD];
+};
+RD_HD Head head_of(const Chain &c) // a chain at hand (registers, the workspace)
+{
+    Head h = {c.hash, c.root, {}};
+    for (int i = 0; i < HEAD; i++)
+        h.r[i] = c.r[i];
+    return h;
+}
+RD_HD Head head_load(const Chain &c) // a chain in memory
+{
+    Head h = {coh_load(&c.hash), coh_load(&c.root), {}};
+    for (int i = 0; i < HEAD; i++)
+        h.r[i] = coh_get(&c.r[i]);
+    return h;
+}
+RD_HD int quick_order(SimRef s, uint32_t pa, const Head &a, uint32_t pb, const Head &b)
+{
+    if (a.root && b.root && a.root != b.root)
     {
-        Run xa[HEAD], xb[HEAD];
-        head_runs(xa, pa, a);
-        head_runs(xb, pb, b);
-        r = heads_cmp(xa, xb);
+        const uint64_t ha = pa ? chash(a.hash, pa) : a.hash, hb = pb ? chash(b.hash, pb) : b.hash;
+        if (ha == hb)
+            return s.root_rank[a.root - 1] < s.root_rank[b.root - 1] ? -1 : 1;
     }
+    Run xa[HEAD], xb[HEAD];
+    head_runs(xa, pa, a.r);
+    head_runs(xb, pb, b.r);
+    return heads_cmp(xa, xb);
+}
+RD_COLD bool before_q(SimRef s, int64_t t, uint32_t pa, const Chain &a, uint32_t pb, const Chain &b)
+{
+    const int r = quick_order(s, pa, head_load(a), pb, head_load(b));
     return r ? r < 0 : before(s, t, pa, a, t, pb, b);
 }
 
 // ------------------------------------------------------------------ frames (src/rdma/rstep.cuh:855-913)
 RD_HD uint32_t node_ip(int id) { return 0x0b000001u + (id / 256) * 0x00010000u + (id % 256) * 0x00000100u; }
-RD_HD uint32_t data_hdr(const Params &P) { return 48 + P.int_size; }
-RD_HD uint32_t ack_size(const Params &P)
+RD_HD uint32_t data_hdr(ParamsRef P) { return 48 + P.int_size; }
+RD_HD uint32_t ack_size(ParamsRef P)
 {
     int base = 12 + P.int_size, pad = 60 - 14 - 20 - base;
     return (pad > 0 ? pad : 0) + base + 20 + 14;
@@ -1107,16 +1180,53 @@ RD_HD double rand_u01(double *x)
     return (p1 > p2) ? (p1 - p2) * norm : (p1 - p2 + m1) * norm;
 }
 
+#if defined(RD_PROF) && defined(__HIP_DEVICE_COMPILE__)
+// (profiling builds: the time a lane's event loop spends in its parts and its rounds, summed in
+// registers and counted at the loop's end)
+#define RD_PROF_SUMS unsigned long long prof_sum[4] = {0, 0, 0, 0}
+#define RD_PROF_T(v) const long long v = wall_clock64()
+#define RD_PROF_ADD(i, d) prof_sum[i] += (unsigned long long)(d)
+#define RD_PROF_OUT(a, b, c, d)                                                                                                   \
+    do                                                                                                                            \
+    {                                                                                                                             \
+        at_add64(&s.ev[a], prof_sum[0]);                                                                                          \
+        at_add64(&s.ev[b], prof_sum[1]);                                                                                          \
+        at_add64(&s.ev[c], prof_sum[2]);                                                                                          \
+        at_add64(&s.ev[d], prof_sum[3]);                                                                                          \
+    } while (0)
+#else
+#define RD_PROF_SUMS
+#define RD_PROF_T(v)
+#define RD_PROF_ADD(i, d)
+#define RD_PROF_OUT(a, b, c, d)
+#endif
+
 // ------------------------------------------------------------------ host: the NIC
 // A host's slot works on a NicSlot: the host record in registers, its out link's open bucket and
 // the chain of the event that runs. The NIC's behaviour is the HPCC simulator's QbbNetDevice +
 // RdmaHw (src/rdma/rstep.cuh:986-1647 restate it); here it is organised by concern: the egress
 // pump (what the NIC sends next and when), the receive side (ACK / NACK replies), the queue pairs'
 // lifecycle, and one rate controller per CC mode, each a small set of functions over the QP.
+// a frame of the slot's arrivals, copied to the workspace
+struct InFrame
+{
+    Chain c;
+    Pkt p;
+    int64_t ts;
+};
+// a frame sent, kept in the workspace until the slot's end: the frame, then its place in the link's ring
+struct OutFrame
+{
+    LFrame f;
+    LFrame RD_G *to;
+};
+static_assert(offsetof(LFrame, c) == 8 && offsetof(LFrame, p) == 8 + sizeof(Chain) && sizeof(LFrame) == 8 + sizeof(Chain) + sizeof(Pkt) &&
+                  sizeof(LFrame) % 8 == 0 && offsetof(InFrame, p) == sizeof(Chain) && offsetof(InFrame, ts) == sizeof(Chain) + sizeof(Pkt),
+              "frame words");
 struct NicSlot
 {
-    const Sim *s;
-    const Params *P;
+    const Sim RD_C *s;
+    const Params RD_C *P;
     uint32_t *pend;
     int pend_n;
     int h;
@@ -1128,6 +1238,11 @@ struct NicSlot
     int link;  // out link
     int64_t ldelay;
     OutBucket ob;
+    // the host's workspace (LDS on the GPU): the pending TransmitComplete's and m_nextSend's chains,
+    // and the frames it sends, until the slot's end (out_n of them, the rest went straight out)
+    Chain *tc, *ns;
+    OutFrame *out;
+    int out_n, out_cap;
 };
 
 // the chain of an event the running one schedules `lead` ns ahead (each takes the next ordinal)
@@ -1146,26 +1261,27 @@ RD_HD int64_t qp_serial(SndQP &q, uint64_t rate, uint32_t bytes)
     }
     return q.tx_val;
 }
-// the window: bytes in flight may not reach it (VAR_WIN scales it with the rate)
-RD_HD bool qp_window_full(const Params &P, const SndQP &q)
+// the window: bytes in flight may not reach it (VAR_WIN scales it with the rate). Its limit is
+// worked out when the rate changes, not at each look of the scheduler: the 64-bit division is some
+// 150 instructions, and a pump looks at several queue pairs.
+RD_HD bool qp_window_full(const SndQP &q) { return q.win && q.snd_nxt - q.snd_una >= q.lim; }
+RD_HD void qp_new_rate(ParamsRef P, SndQP &q, uint64_t rate)
 {
-    if (!q.win)
-        return false;
-    uint64_t lim = q.win;
-    if (P.var_win)
+    q.rate = rate;
+    q.lim = q.win;
+    if (P.var_win && q.win)
     {
-        lim = (uint64_t)q.win * q.rate / q.max_rate; // (q.win * rate stays below 2^64)
-        lim = lim ? lim : 1;
+        q.lim = (uint64_t)q.win * rate / q.max_rate; // (q.win * rate stays below 2^64)
+        q.lim = q.lim ? q.lim : 1;
     }
-    return q.snd_nxt - q.snd_una >= lim;
 }
 
 // a transmission-trace record (src/rdma/rstep.cuh:915-942): out of line, off the path when tracing is off
 // (the packet by value, as its words 6 and 7 and its sequence number: a packet passed by reference
 // to this out-of-line function would be kept in scratch memory on the transmit path)
-RD_COLD void trace_tx(const Sim &s, int64_t now, int node, int dev, uint32_t seq, uint64_t w6, uint64_t w7)
+RD_COLD void trace_tx(SimRef s, int64_t now, int node, int dev, uint32_t seq, uint64_t w6, uint64_t w7)
 {
-    const TxTrace &t = s.txt_rec;
+    const TxTrace RD_C &t = s.txt_rec;
     if (now < t.from || now > t.until)
         return;
     const unsigned long long i = at_add64(t.cnt, 1ull);
@@ -1190,29 +1306,37 @@ RD_COLD void trace_tx(const Sim &s, int64_t now, int node, int dev, uint32_t seq
 }
 
 // a frame onto the out link (TransmitStart): filed in its arrival bucket, the NIC busy until its
-// last bit is out (the frame is written before the chain work, so a packet in a ring is copied
-// straight into it)
-RD_HD void nic_emit(NicSlot &n, const Pkt &p)
+// last bit is out. It waits in the workspace for the slot's end when there is room: vector memory
+// counts in order, so every load of the next events would wait for its coherent stores (0.3 us and more).
+RD_HD void nic_emit(NicSlot &n, Pkt p)
 {
-    const Sim &s = *n.s;
+    SimRef s = *n.s;
     const int64_t busy = link_txo(s, n.ob, p.size), lands = n.now + busy + n.ldelay;
     n.st.tc_at = n.now + busy;
     const int done_ord = n.ord; // the TransmitComplete's ordinal; the arrival's is the next
     n.ord += 2;
     n.nout++;
     LFrame RD_G *fr = ob_push(s, n.pend, n.pend_n, lands, n.ob);
-    if (fr)
+    cpush(s, n.st.ta, n.tc, ccode(busy, done_ord), n.cur);
+    if (!fr)
+        return;
+    p.ord = (uint8_t)(done_ord < 254 ? done_ord + 1 : 255);
+    if (n.out_n < n.out_cap)
     {
-        Pkt q = p;
-        q.ord = (uint8_t)(done_ord < 254 ? done_ord + 1 : 255);
-        coh_store(&fr->ts, lands);
-        frame_put_pkt(s, fr, q);
-        if (s.txt_rec.rec)
-            trace_tx(s, n.now, n.h, 1, q.seq, pkt_w6(q), pkt_w7(q));
+        OutFrame &o = n.out[n.out_n++];
+        o.f.ts = lands;
+        o.f.c = n.cur;
+        o.f.p = p;
+        o.to = fr;
     }
-    cpush(s, n.st.ta, &s.h_tc[n.h], ccode(busy, done_ord), n.cur);
-    if (fr)
+    else
+    {
+        coh_store(&fr->ts, lands);
+        frame_put_pkt(s, fr, p);
         frame_put_chain(s, fr, n.cur);
+    }
+    if (s.txt_rec.rec)
+        trace_tx(s, n.now, n.h, 1, p.seq, pkt_w6(p), pkt_w7(p));
 }
 
 // The egress pump (DequeueAndTransmit + RdmaEgressQueue): when the link is free, the ACK queue
@@ -1229,7 +1353,7 @@ enum
 // place of list index `keep` (PICK_NONE stays)
 RD_HD int qp_list_prune(NicSlot &n, int *list, int from, int keep)
 {
-    const Sim &s = *n.s;
+    SimRef s = *n.s;
     int w = from;
     for (int i = from + 1; i < n.st.qp_n; i++)
     {
@@ -1244,7 +1368,7 @@ RD_HD int qp_list_prune(NicSlot &n, int *list, int from, int keep)
 }
 RD_HD int nic_pick(NicSlot &n)
 {
-    const Sim &s = *n.s;
+    SimRef s = *n.s;
     const int ack_class = n.P->ack_high_prio ? 0 : PG;
     if (n.st.ackq_n > 0 && !(n.st.paused >> ack_class & 1))
         return PICK_ACK;
@@ -1256,7 +1380,7 @@ RD_HD int nic_pick(NicSlot &n)
     {
         i = i + 1 < cnt ? i + 1 : 0;
         const SndQP &q = s.qp[list[i]];
-        const bool ready = !data_paused && qp_unsent(q) > 0 && !qp_window_full(*n.P, q);
+        const bool ready = !data_paused && qp_unsent(q) > 0 && !qp_window_full(q);
         if (!ready)
         {
             if (qp_finished(q) && (first_done < 0 || i < first_done))
@@ -1271,13 +1395,12 @@ RD_HD int nic_pick(NicSlot &n)
     }
     return first_done >= 0 ? qp_list_prune(n, list, first_done, pick) : pick;
 }
-// the next data segment of QP f (GetNxtPacket), then its pacing (PktSent, UpdateNextAvail)
-RD_HD void nic_send_segment(NicSlot &n, int f)
+// the next data segment of QP f (GetNxtPacket)
+RD_HD Pkt nic_next_segment(NicSlot &n, SndQP &q, int f)
 {
-    const Sim &s = *n.s;
-    const Params &P = *n.P;
-    SndQP &q = s.qp[f];
-    const FlowInfo &fi = s.fi[f];
+    SimRef s = *n.s;
+    ParamsRef P = *n.P;
+    const FlowInfo RD_C &fi = s.fi[f];
     const uint64_t left = qp_unsent(q);
     const uint32_t body = left < P.mtu ? (uint32_t)left : P.mtu;
     Pkt p = {};
@@ -1289,14 +1412,12 @@ RD_HD void nic_send_segment(NicSlot &n, int f)
     p.seq = (uint32_t)q.snd_nxt;
     p.size = (uint16_t)(body + data_hdr(P));
     q.snd_nxt += body;
-    nic_emit(n, p);
-    q.last_pkt = p.size;
-    q.next_avail = n.now + qp_serial(q, P.rate_bound ? q.rate : q.max_rate, p.size);
+    return p;
 }
 // nothing to send now: m_nextSend at the earliest pacing time of a QP with bytes left
 RD_HD void nic_arm_next_send(NicSlot &n)
 {
-    const Sim &s = *n.s;
+    SimRef s = *n.s;
     const int *list = s.qps + (size_t)n.h * s.qps_cap;
     int64_t at = INT64_MAX;
     for (int i = 0; i < n.st.qp_n; i++)
@@ -1308,29 +1429,57 @@ RD_HD void nic_arm_next_send(NicSlot &n)
     if (n.st.ns_at < 0 && at != INT64_MAX && at > n.now)
     {
         n.st.ns_at = at;
-        nic_schedule(n, &s.h_ns[n.h], at - n.now);
+        nic_schedule(n, n.ns, at - n.now);
     }
 }
-RD_HD void nic_pump(NicSlot &n)
+// (reply: an ACK or NACK made by the running event when the ACK queue was empty, not yet queued:
+// sent from the registers if the NIC may send it now, else it takes its place in the queue)
+RD_HD void nic_pump(NicSlot &n, const Pkt *reply)
 {
+    SimRef s = *n.s;
+    Pkt RD_G *ackq = s.ackq + (size_t)n.h * ACKQ_CAP;
+    const int ack_class = n.P->ack_high_prio ? 0 : PG;
+    if (reply)
+    {
+        if (n.st.tc_at < 0 && !(n.st.paused >> ack_class & 1))
+        {
+            n.st.ackq_head = ring_add(n.st.ackq_head, 1, ACKQ_CAP);
+            nic_emit(n, *reply);
+            return;
+        }
+        ackq[n.st.ackq_head] = *reply;
+        n.st.ackq_n = 1;
+    }
     if (n.st.tc_at >= 0)
         return; // a transmission is in progress
     const int pick = nic_pick(n);
-    const Sim &s = *n.s;
+    if (pick == PICK_NONE)
+    {
+        nic_arm_next_send(n);
+        return;
+    }
+    int f = 0;
+    Pkt p;
     if (pick == PICK_ACK)
     {
-        const Pkt &a = s.ackq[(size_t)n.h * ACKQ_CAP + n.st.ackq_head]; // (the slot outlives the copy into the frame)
+        p = ackq[n.st.ackq_head];
         n.st.ackq_head = ring_add(n.st.ackq_head, 1, ACKQ_CAP);
         n.st.ackq_n--;
-        nic_emit(n, a);
-    }
-    else if (pick != PICK_NONE)
-    {
-        n.st.rr = pick;
-        nic_send_segment(n, s.qps[(size_t)n.h * s.qps_cap + pick]);
     }
     else
-        nic_arm_next_send(n);
+    {
+        n.st.rr = pick;
+        f = s.qps[(size_t)n.h * s.qps_cap + pick];
+        p = nic_next_segment(n, s.qp[f], f);
+    }
+    nic_emit(n, p);
+    if (pick != PICK_ACK)
+    {
+        // its pacing (PktSent, UpdateNextAvail)
+        SndQP &q = s.qp[f];
+        q.last_pkt = p.size;
+        q.next_avail = n.now + qp_serial(q, n.P->rate_bound ? q.rate : q.max_rate, p.size);
+    }
 }
 
 // a QP's sending rate changes (ChangeRate): its pacing time moves by the difference of the last
@@ -1343,16 +1492,16 @@ RD_HD void qp_set_rate(NicSlot &n, SndQP &q, uint64_t rate)
     {
         const int64_t at = q.next_avail > n.now ? q.next_avail : n.now;
         n.st.ns_at = at;
-        nic_schedule(n, &n.s->h_ns[n.h], at - n.now);
+        nic_schedule(n, n.ns, at - n.now);
     }
-    q.rate = rate;
+    qp_new_rate(*n.P, q, rate);
 }
 
 // ---- HPCC (UpdateRateHp, one rate for the path): the path's utilization from the INT hops of
 // the ACK against those of the last update, then a multiplicative or additive step
 // the largest normalized utilization over the hops the ACK reports, and its hop's time delta; the
 // QP's stored hops become the ACK's. false: no hop took part (all skipped by sample feedback).
-RD_HD bool hpcc_path_load(const Params &P, SndQP &q, const Pkt &p, bool fast, double *U, uint64_t *tau_max)
+RD_HD bool hpcc_path_load(ParamsRef P, SndQP &q, const Pkt &p, bool fast, double *U, uint64_t *tau_max)
 {
     bool any = false;
     *U = 0;
@@ -1382,7 +1531,7 @@ RD_HD bool hpcc_path_load(const Params &P, SndQP &q, const Pkt &p, bool fast, do
 }
 RD_HD void hpcc_react(NicSlot &n, SndQP &q, double U, uint64_t tau, bool fast)
 {
-    const Params &P = *n.P;
+    ParamsRef P = *n.P;
     if (tau > q.base_rtt)
         tau = q.base_rtt;
     // the EWMA of U over a base RTT (the fork's build contracts u (B - tau) + U tau into one fma)
@@ -1427,14 +1576,14 @@ RD_HD void dcqcn_arm(NicSlot &n, int64_t *deadline, Chain *chain, int64_t lead)
         n.st.due_min = *deadline;
     nic_schedule(n, chain, lead);
 }
-RD_HD uint64_t dcqcn_cut(const Params &P, const SndQP &q)
+RD_HD uint64_t dcqcn_cut(ParamsRef P, const SndQP &q)
 {
     const uint64_t r = rate_of((double)q.rate * (1 - q.alpha / 2));
     return r > P.min_rate ? r : P.min_rate;
 }
 RD_HD void dcqcn_on_cnp(NicSlot &n, int f, SndQP &q)
 {
-    const Params &P = *n.P;
+    ParamsRef P = *n.P;
     q.alpha_cnp = q.dec_cnp = 1;
     if (!q.first_cnp)
         return;
@@ -1443,46 +1592,46 @@ RD_HD void dcqcn_on_cnp(NicSlot &n, int f, SndQP &q)
     q.alpha_cnp = 0;
     dcqcn_arm(n, &q.t_alpha, &n.s->qc[f].alpha, P.alpha_int);
     dcqcn_arm(n, &q.t_dec, &n.s->qc[f].dec, P.dec_int + 1);
-    q.rate = rate_of((double)q.rate * P.rate_first_cnp);
+    qp_new_rate(P, q, rate_of((double)q.rate * P.rate_first_cnp));
     q.target = q.rate;
 }
 RD_HD void dcqcn_alpha_tick(NicSlot &n, int f, SndQP &q)
 {
-    const Params &P = *n.P;
+    ParamsRef P = *n.P;
     q.alpha = q.alpha_cnp ? fma(1 - P.g, q.alpha, P.g) : (1 - P.g) * q.alpha;
     q.alpha_cnp = 0;
     dcqcn_arm(n, &q.t_alpha, &n.s->qc[f].alpha, P.alpha_int);
 }
 RD_HD void dcqcn_decrease_tick(NicSlot &n, int f, SndQP &q)
 {
-    const Params &P = *n.P;
+    ParamsRef P = *n.P;
     dcqcn_arm(n, &q.t_dec, &n.s->qc[f].dec, P.dec_int);
     if (!q.dec_cnp)
         return;
     if (q.rp_stage || P.clamp)
         q.target = q.rate;
-    q.rate = dcqcn_cut(P, q);
+    qp_new_rate(P, q, dcqcn_cut(P, q));
     q.rp_stage = 0;
     q.dec_cnp = 0;
     dcqcn_arm(n, &q.t_rp, &n.s->qc[f].rp, P.rp_int);
 }
 RD_HD void dcqcn_increase_tick(NicSlot &n, int f, SndQP &q)
 {
-    const Params &P = *n.P;
+    ParamsRef P = *n.P;
     dcqcn_arm(n, &q.t_rp, &n.s->qc[f].rp, P.rp_int);
     if (q.rp_stage >= P.rpg_threshold)
     {
         const uint64_t t = q.target + (q.rp_stage == P.rpg_threshold ? P.rai : P.rhai);
         q.target = t > q.max_rate ? q.max_rate : t;
     }
-    q.rate = rate_of((double)q.rate / 2) + rate_of((double)q.target / 2);
+    qp_new_rate(P, q, rate_of((double)q.rate / 2) + rate_of((double)q.target / 2));
     q.rp_stage++;
 }
 
 // ---- DCTCP over RDMA (HandleAckDctcp): alpha per window of segments, one cut per window with a
 // mark, an additive step per window without
 // closes the window of ACKs when one passes its end: alpha from its marked share; true if so
-RD_HD bool dctcp_window(const Params &P, SndQP &q, const Pkt &p)
+RD_HD bool dctcp_window(ParamsRef P, SndQP &q, const Pkt &p)
 {
     if (p.seq <= q.last_update_seq)
         return false;
@@ -1498,7 +1647,7 @@ RD_HD bool dctcp_window(const Params &P, SndQP &q, const Pkt &p)
     q.last_update_seq = (uint32_t)q.snd_nxt;
     return true;
 }
-RD_HD void dctcp_on_ack(const Params &P, SndQP &q, const Pkt &p)
+RD_HD void dctcp_on_ack(ParamsRef P, SndQP &q, const Pkt &p)
 {
     if (p.cnp)
         q.ecn_cnt++;
@@ -1507,31 +1656,31 @@ RD_HD void dctcp_on_ack(const Params &P, SndQP &q, const Pkt &p)
         q.ca_state = 0; // the reduced window is acknowledged
     if (q.ca_state == 0 && p.cnp)
     {
-        q.rate = dcqcn_cut(P, q); // (the same rate cut: rate (1 - alpha/2), at least the minimum)
+        qp_new_rate(P, q, dcqcn_cut(P, q)); // (the same rate cut: rate (1 - alpha/2), at least the minimum)
         q.ca_state = 1;
         q.high_seq = (uint32_t)q.snd_nxt;
     }
     if (q.ca_state == 0 && window_end)
     {
         const uint64_t r = q.rate + P.dctcp_rai;
-        q.rate = r > q.max_rate ? q.max_rate : r;
+        qp_new_rate(P, q, r > q.max_rate ? q.max_rate : r);
     }
 }
 
 // ---- the queue pairs' lifecycle
 // an ACK or NACK (ReceiveAck): the QP's acknowledged point moves; the last byte completes it (its
 // flow completion time is recorded, its timers end); a NACK rewinds sending to it (go-back-N);
-// then the CC mode's reaction and the pump
-RD_HD void nic_on_ack(NicSlot &n, const Pkt &p, unsigned *flows_done)
+// then the CC mode's reaction. (These return whether the pump follows.)
+RD_HD bool nic_on_ack(NicSlot &n, const Pkt &p, unsigned *flows_done)
 {
-    const Sim &s = *n.s;
-    const Params &P = *n.P;
+    SimRef s = *n.s;
+    ParamsRef P = *n.P;
     const int f = (int)p.flow;
     SndQP &q = s.qp[f];
     if (q.done)
     {
         count(s, EV_ACK_DONE);
-        return;
+        return false;
     }
     q.snd_una = p.seq > q.snd_una ? p.seq : q.snd_una;
     const bool completes = qp_finished(q);
@@ -1559,7 +1708,7 @@ RD_HD void nic_on_ack(NicSlot &n, const Pkt &p, unsigned *flows_done)
             dctcp_on_ack(P, q, p);
         break;
     }
-    nic_pump(n);
+    return true;
 }
 // a data frame at the receiver (ReceiveUdp, ReceiverCheckSeq): in order, it advances the
 // expected byte and is acknowledged at the ACK interval or a chunk's end; ahead of it, a NACK
@@ -1570,7 +1719,7 @@ enum
     RX_NACK,
     RX_QUIET
 };
-RD_HD int rx_check(const Params &P, RcvQP &r, const Pkt &p, int64_t now)
+RD_HD int rx_check(ParamsRef P, RcvQP &r, const Pkt &p, int64_t now)
 {
     const uint32_t body = p.size - data_hdr(P);
     if (p.seq == r.expected)
@@ -1584,44 +1733,52 @@ RD_HD int rx_check(const Params &P, RcvQP &r, const Pkt &p, int64_t now)
     r.last_nack = r.expected;
     return RX_NACK;
 }
-RD_HD void nic_on_data(NicSlot &n, const Pkt &p)
+// (*reply, *fresh: the reply, not yet queued, when the ACK queue is empty)
+RD_HD bool nic_on_data(NicSlot &n, const Pkt &p, Pkt *reply, bool *fresh)
 {
-    const Sim &s = *n.s;
+    SimRef s = *n.s;
     RcvQP &r = s.rx[p.flow];
     if (r.expected >= s.fi[p.flow].size)
         count(s, EV_DATA_DONE);
     const int v = rx_check(*n.P, r, p, n.now);
     if (v == RX_QUIET)
-        return;
+        return false;
     if (v == RX_NACK)
         count(s, EV_NACK);
     if (n.st.ackq_n >= ACKQ_CAP)
     {
         count(s, EV_ACKQ_OVF);
-        return;
+        return false;
     }
     // the reply carries the data frame's addresses and hops, the expected byte and the CE mark as CNP
-    Pkt &a = s.ackq[(size_t)n.h * ACKQ_CAP + ring_add(n.st.ackq_head, n.st.ackq_n, ACKQ_CAP)];
-    a = p;
+    Pkt a = p;
     a.kind = v == RX_ACK ? K_ACK : K_NACK;
     a.seq = r.expected;
     a.cnp = p.ecn ? 1 : 0;
     a.ecn = 0;
     a.size = (uint16_t)ack_size(*n.P);
+    if (n.st.ackq_n == 0)
+    {
+        *reply = a;
+        *fresh = true;
+        return true;
+    }
+    s.ackq[(size_t)n.h * ACKQ_CAP + ring_add(n.st.ackq_head, n.st.ackq_n, ACKQ_CAP)] = a;
     n.st.ackq_n++;
-    nic_pump(n);
+    return true;
 }
 // a flow starts (StartApplication, AddQueuePair): a fresh QP at line rate joins the host's list
-RD_HD void nic_add_qp(NicSlot &n, int f)
+RD_HD bool nic_add_qp(NicSlot &n, int f)
 {
-    const Sim &s = *n.s;
-    const FlowInfo &fi = s.fi[f];
+    SimRef s = *n.s;
+    const FlowInfo RD_C &fi = s.fi[f];
     const uint64_t line = s.li[n.link].bps;
     SndQP q = {};
     q.size = fi.size;
     q.win = fi.win;
     q.base_rtt = fi.base_rtt;
-    q.rate = q.max_rate = q.target = line;
+    q.max_rate = q.target = line;
+    qp_new_rate(*n.P, q, line);
     q.alpha = 1;
     q.first_cnp = 1;
     q.t_alpha = q.t_dec = q.t_rp = -1;
@@ -1635,23 +1792,23 @@ RD_HD void nic_add_qp(NicSlot &n, int f)
     if (n.st.qp_n >= s.qps_cap)
     {
         count(s, EV_QPS_OVF);
-        return;
+        return false;
     }
     s.qps[(size_t)n.h * s.qps_cap + n.st.qp_n++] = f;
-    nic_pump(n);
+    return true;
 }
 
-RD_HD const Chain &due_chain(const Sim &s, const Due &d)
+RD_HD const Chain &due_chain(SimRef s, const Due &d)
 {
     const QPChains &qc = s.qc[d.flow];
     return d.kind == 0 ? qc.alpha : d.kind == 1 ? qc.dec : qc.rp;
 }
-RD_HD int64_t due_now(const Sim &s, const Due &d)
+RD_HD int64_t due_now(SimRef s, const Due &d)
 {
     const SndQP &q = s.qp[d.flow];
     return d.kind == 0 ? q.t_alpha : d.kind == 1 ? q.t_dec : q.t_rp;
 }
-RD_HD int64_t qp_timer_min(const Sim &s, int h, int n)
+RD_HD int64_t qp_timer_min(SimRef s, int h, int n)
 {
     const int *list = s.qps + (size_t)h * s.qps_cap;
     int64_t mn = INT64_MAX;
@@ -1669,19 +1826,62 @@ RD_HD int64_t qp_timer_min(const Sim &s, int h, int n)
 // order - the candidates are its next arrival, its TransmitComplete, its m_nextSend, its next DCQCN
 // timer and its next flow start; the earliest runs, simultaneous ones by their chains. Returns
 // whether the host is active (sent, or holds frames); *wake: its earliest event without input.
-RD_HD bool host_step(const Sim &s, int h, int64_t slot, unsigned *flows_done, uint32_t *pend, int pend_n, int64_t *wake)
+//
+// In three parts: host_open (does it run? its arrivals), the events, and its frames out. On the GPU
+// the wave copies its hosts' arrivals into their workspaces in between and writes the frames out
+// afterwards, all lanes at it, so that a host's chain of events waits neither for a frame's loads
+// nor for a frame's stores (rdma_kernel.hip).
+struct HostSlot
+{
+    bool runs;
+    int an;         // arrivals
+    uint64_t abase; // the first one's place in the rings
+};
+RD_HD HostSlot host_open(SimRef s, int h, int64_t slot, int64_t *wake)
+{
+    HostSlot x;
+    x.an = bucket(s, s.h_link_in[h], slot, &x.abase);
+    const int64_t w = s.hs[h].wake;
+    x.runs = x.an || w < (slot + 1) * s.D;
+    if (!x.runs)
+        *wake = w;
+    return x;
+}
+// a host's workspace in `bytes` of memory: its two chains, then as many arrivals as frames to send
+struct HostWork
+{
+    Chain *tc, *ns;
+    InFrame *in;
+    OutFrame *out;
+    int in_cap, out_cap;
+};
+RD_HD HostWork host_work(char *mem, int bytes)
+{
+    HostWork w;
+    w.tc = reinterpret_cast<Chain *>(mem);
+    w.ns = w.tc + 1;
+    const int n = (bytes - 2 * (int)sizeof(Chain)) / (int)(sizeof(InFrame) + sizeof(OutFrame));
+    w.in = reinterpret_cast<InFrame *>(w.ns + 1);
+    w.out = reinterpret_cast<OutFrame *>(w.in + n);
+    w.in_cap = w.out_cap = n;
+    return w;
+}
+// the events; arrivals 0 .. in_n - 1 are in the workspace; returns the host's activity, *out_n the
+// frames left in the workspace
+RD_HD bool host_events(SimRef s, int h, int64_t slot, unsigned *flows_done, uint32_t *pend, int pend_n, int64_t *wake, int an, uint64_t abase,
+                       const HostWork &hw, int in_n, int *out_n)
 {
     const int64_t D = s.D, t0 = slot * D, t1 = t0 + D;
-    const Params &P = s.Pw[s.h_world[h]];
+    ParamsRef P = s.Pw[RD_UNIFORM(s.h_world[h])]; // (a wave's hosts are of one world)
     const int lin = s.h_link_in[h];
-    uint64_t abase;
-    const int an = bucket(s, lin, slot, &abase);
-    if (an == 0 && s.hs[h].wake >= t1)
-    {
-        *wake = s.hs[h].wake;
-        return false;
-    }
     NicSlot c;
+    c.tc = hw.tc;
+    c.ns = hw.ns;
+    *c.tc = s.h_tc[h];
+    *c.ns = s.h_ns[h];
+    c.out = hw.out;
+    c.out_n = 0;
+    c.out_cap = hw.out_cap;
     c.s = &s;
     c.P = &P;
     c.pend = pend;
@@ -1694,10 +1894,11 @@ RD_HD bool host_step(const Sim &s, int h, int64_t slot, unsigned *flows_done, ui
     c.st = s.hs[h];
     c.link = s.h_link_out[h];
     c.ldelay = s.li[c.link].delay;
-    ob_open(s, c.ob, c.link, c.st.ob_last);
+    ob_open(s, c.ob, c.link, c.st.ob_last, slot, pend_n);
     const int64_t in_delay = s.li[lin].delay;
-    uint32_t in_sz = 0; // the in-link's last frame size and its tx time
-    int64_t in_tx = 0;
+    // the in-link's tx times of full data frames and of ACKs
+    const uint32_t in_sz[2] = {P.mtu + data_hdr(P), ack_size(P)};
+    const int64_t in_tx[2] = {link_tx(s, lin, in_sz[0]), link_tx(s, lin, in_sz[1])};
     // the DCQCN timers due in this slot, in event order (their intervals are at least a slot: none
     // set in it falls due in it)
     Due *due = s.due + (size_t)h * MAX_DUE;
@@ -1735,32 +1936,37 @@ RD_HD bool host_step(const Sim &s, int h, int64_t slot, unsigned *flows_done, ui
     int di = 0, ai = 0;
     int sf = -1, sf_at = -1;
     int64_t sf_t = INT64_MAX;
-    // the next arrival's frame (written by the link's sender in an earlier slot: coherent reads):
-    // its time and packet read once, together (its chain when it runs)
-    const LFrame RD_G *af = nullptr;
-    FrameHead ah = {INT64_MAX, 0, 0};
+    // the next arrival: its time, code and packet (its chain when it runs), from the workspace or, for
+    // those it had no room for, from the link's ring (written in an earlier slot: coherent reads)
+    int64_t a_ts = INT64_MAX;
+    uint32_t acode = 0;
     Pkt apk;
     int a_at = -1;
+    RD_PROF_SUMS;
     for (;;)
     {
+        RD_PROF_T(prof_h0);
         if (a_at != ai)
         {
             a_at = ai;
-            af = ai < an ? s.msg + abase + ai : nullptr;
-            if (af)
+            a_ts = INT64_MAX;
+            if (ai < an)
             {
-                apk = pkt_get(&af->p);
-                ah = FrameHead{coh_load(&af->ts), apk.size, apk.ord};
+                if (ai < in_n)
+                {
+                    a_ts = hw.in[ai].ts;
+                    apk = hw.in[ai].p;
+                }
+                else
+                {
+                    const LFrame RD_G *af = s.msg + abase + ai;
+                    a_ts = coh_load(&af->ts);
+                    apk = pkt_get(&af->p);
+                }
+                const int64_t tx = apk.size == in_sz[0] ? in_tx[0] : apk.size == in_sz[1] ? in_tx[1] : link_tx(s, lin, apk.size);
+                acode = ccode(tx + in_delay, apk.ord);
             }
-            else
-                ah = FrameHead{INT64_MAX, 0, 0};
         }
-        if (af && ah.size != in_sz)
-        {
-            in_sz = ah.size;
-            in_tx = link_tx(s, lin, in_sz);
-        }
-        const uint32_t acode = af ? ccode(in_tx + in_delay, ah.ord) : 0;
         while (di < ndue && due_now(s, due[di]) != due[di].at)
             di++; // cancelled or moved
         if (sf_at != c.st.next_start)
@@ -1771,7 +1977,7 @@ RD_HD bool host_step(const Sim &s, int h, int64_t slot, unsigned *flows_done, ui
         }
         // candidate times: 0 arrival, 1 TransmitComplete, 2 m_nextSend, 3 DCQCN timer, 4 flow start
         int64_t tt[5];
-        tt[0] = ah.ts;
+        tt[0] = a_ts;
         tt[1] = c.st.tc_at >= 0 && c.st.tc_at < t1 ? c.st.tc_at : INT64_MAX;
         tt[2] = c.st.ns_at >= 0 && c.st.ns_at < t1 ? c.st.ns_at : INT64_MAX;
         tt[3] = di < ndue ? due[di].at : INT64_MAX;
@@ -1791,50 +1997,59 @@ RD_HD bool host_step(const Sim &s, int h, int64_t slot, unsigned *flows_done, ui
                 bk = k;
                 continue;
             }
-            // a tie: the quick prefixes where both are arrivals, TransmitCompletes or sends, else the chains
+            // a tie: the quick test where both are arrivals, TransmitCompletes or sends, else the chains
+            auto chain = [&](int q) -> const Chain & {
+                return q == 0   ? (ai < in_n ? hw.in[ai].c : (const Chain &)s.msg[abase + ai].c)
+                       : q == 1 ? *c.tc
+                       : q == 2 ? *c.ns
+                       : q == 3 ? due_chain(s, due[di])
+                                : (const Chain &)s.fi[sf].start_chain;
+            };
             const uint32_t pk = k == 0 ? acode : 0, pb = bk == 0 ? acode : 0;
-            const Chain &ck = k == 0 ? af->c : k == 1 ? s.h_tc[h] : k == 2 ? s.h_ns[h] : k == 3 ? due_chain(s, due[di]) : s.fi[sf].start_chain;
-            const Chain &cb = bk == 0 ? af->c : bk == 1 ? s.h_tc[h] : bk == 2 ? s.h_ns[h] : bk == 3 ? due_chain(s, due[di]) : s.fi[sf].start_chain;
-            const bool b4 = (k <= 2 && bk <= 2) ? before_q(s, t, pk, ck, pb, cb) : before(s, t, pk, ck, bt, pb, cb);
-            if (b4)
+            const int quick = k <= 2 && bk <= 2 ? quick_order(s, pk, head_load(chain(k)), pb, head_load(chain(bk))) : 0;
+            if (quick ? quick < 0 : before(s, t, pk, chain(k), bt, pb, chain(bk)))
                 bk = k;
         }
+        RD_PROF_T(prof_h1);
+        RD_PROF_ADD(0, prof_h1 - prof_h0);
+        RD_PROF_ADD(3, 1);
         if (bk < 0)
             break;
         if (bt < t0)
             count(s, EV_LATE);
         c.now = bt;
-        if (bk == 0)
-            cpush(s, c.st.ta, &c.cur, acode, chain_get(&af->c));
+        if (bk == 0 && ai < in_n)
+            cpush(s, c.st.ta, &c.cur, acode, hw.in[ai].c);
+        else if (bk == 0)
+            cpush(s, c.st.ta, &c.cur, acode, chain_get(&s.msg[abase + ai].c));
+        else if (bk <= 2)
+            c.cur = bk == 1 ? *c.tc : *c.ns;
         else
-            c.cur = bk == 1 ? s.h_tc[h] : bk == 2 ? s.h_ns[h] : bk == 3 ? due_chain(s, due[di]) : s.fi[sf].start_chain;
+            c.cur = bk == 3 ? due_chain(s, due[di]) : (const Chain &)s.fi[sf].start_chain;
         c.ord = 0;
+        // each event says whether the pump follows; the pump is here once, so that the hosts of a wave
+        // share it whatever their events are
+        bool pump = true, fresh = false;
+        Pkt reply;
         if (bk == 0)
         {
-            const Pkt p = apk;
             ai++;
-            if (p.kind == K_DATA)
-                nic_on_data(c, p);
-            else if (p.kind == K_ACK || p.kind == K_NACK)
-                nic_on_ack(c, p, flows_done);
-            else if (p.kind == K_PAUSE)
-                c.st.paused |= 1u << p.q;
-            else
+            if (apk.kind == K_DATA)
+                pump = nic_on_data(c, apk, &reply, &fresh);
+            else if (apk.kind == K_ACK || apk.kind == K_NACK)
+                pump = nic_on_ack(c, apk, flows_done);
+            else if (apk.kind == K_PAUSE)
             {
-                c.st.paused &= ~(1u << p.q);
-                nic_pump(c);
+                c.st.paused |= 1u << apk.q;
+                pump = false;
             }
+            else
+                c.st.paused &= ~(1u << apk.q);
         }
         else if (bk == 1)
-        {
             c.st.tc_at = -1;
-            nic_pump(c);
-        }
         else if (bk == 2)
-        {
             c.st.ns_at = -1;
-            nic_pump(c);
-        }
         else if (bk == 3)
         {
             // a DCQCN timer: 0 alpha update, 1 rate-decrease check, 2 rate increase
@@ -1846,13 +2061,24 @@ RD_HD bool host_step(const Sim &s, int h, int64_t slot, unsigned *flows_done, ui
                 dcqcn_decrease_tick(c, x.flow, q);
             else
                 dcqcn_increase_tick(c, x.flow, q);
+            pump = false;
         }
         else
         {
             c.st.next_start++;
-            nic_add_qp(c, sf);
+            pump = nic_add_qp(c, sf);
         }
+        RD_PROF_T(prof_h2);
+        RD_PROF_ADD(1, prof_h2 - prof_h1);
+        if (pump)
+            nic_pump(c, fresh ? &reply : nullptr);
+        RD_PROF_T(prof_h3);
+        RD_PROF_ADD(2, prof_h3 - prof_h2);
     }
+    RD_PROF_OUT(14, 15, 16, 17);
+    s.h_tc[h] = *c.tc;
+    s.h_ns[h] = *c.ns;
+    *out_n = c.out_n;
     bool act = c.nout > 0;
     int64_t w = INT64_MAX;
     if (c.st.next_start < c.st.start_end)
@@ -1879,6 +2105,35 @@ RD_HD bool host_step(const Sim &s, int h, int64_t slot, unsigned *flows_done, ui
     *wake = w;
     return act;
 }
+// word i of a frame of the link rings into the workspace (InFrame has the time last)
+RD_HD void in_word(InFrame &f, int i, uint64_t v)
+{
+    reinterpret_cast<uint64_t *>(&f)[i ? i - 1 : (int)(sizeof(LFrame) / 8) - 1] = v;
+}
+RD_HD uint64_t in_load(SimRef s, uint64_t at, int i) { return coh_load(reinterpret_cast<const uint64_t RD_G *>(s.msg + at) + i); }
+RD_HD void out_store(const OutFrame &f, int i)
+{
+    coh_store(reinterpret_cast<uint64_t RD_G *>(f.to) + i, reinterpret_cast<const uint64_t *>(&f.f)[i]);
+}
+#if !defined(__HIP_DEVICE_COMPILE__)
+// a host's whole slot on one thread (CPU builds; a small workspace, so that frames take both ways)
+inline bool host_step(SimRef s, int h, int64_t slot, unsigned *flows_done, uint32_t *pend, int pend_n, int64_t *wake)
+{
+    alignas(16) char mem[2 * sizeof(Chain) + 5 * (sizeof(InFrame) + sizeof(OutFrame))];
+    const HostSlot x = host_open(s, h, slot, wake);
+    if (!x.runs)
+        return false;
+    const HostWork w = host_work(mem, (int)sizeof mem);
+    const int in_n = x.an < w.in_cap ? x.an : w.in_cap, words = (int)(sizeof(LFrame) / 8);
+    for (int i = 0; i < in_n * words; i++)
+        in_word(w.in[i / words], i % words, in_load(s, x.abase + i / words, i % words));
+    int out_n = 0;
+    const bool act = host_events(s, h, slot, flows_done, pend, pend_n, wake, x.an, x.abase, w, in_n, &out_n);
+    for (int i = 0; i < out_n * words; i++)
+        out_store(w.out[i / words], i % words);
+    return act;
+}
+#endif
 
 // ------------------------------------------------------------------ switch: ports and the MMU
 // A switch's slot works on a SwSlot: its ports (in device memory, or LDS in a safe slot), the
@@ -1888,8 +2143,8 @@ RD_HD bool host_step(const Sim &s, int h, int64_t slot, unsigned *flows_done, ui
 // the egress port's queues and transmitter, and the ingress path that ties them together.
 struct SwSlot
 {
-    const Sim *s;
-    const Params *P;
+    const Sim RD_C *s;
+    const Params RD_C *P;
     uint32_t *pend;
     int pend_n;
     int x, node;
@@ -1904,7 +2159,6 @@ struct SwSlot
     uint32_t cur_code;
     bool cur_ok;
     int pbase; // its first port in the per-port arrays
-    bool safe; // a safe slot: this context runs one egress port's events (see switch_slot)
     int ep;    // the running event's port (its tail positions: one writer per port and slot)
     int ord;
 };
@@ -1978,7 +2232,7 @@ RD_HD bool mmu_ecn_mark(SwSlot &c, int port)
 // a frame onto the port's link (TransmitStart): as a NIC's, the frame first, then the chains
 RD_HD void port_emit(SwSlot &c, int port, const Pkt &p)
 {
-    const Sim &s = *c.s;
+    SimRef s = *c.s;
     PortRun &r = c.w[port];
     const int64_t busy = link_txo(s, r.ob, p.size), lands = c.now + busy + r.ob.delay;
     c.pt[port].tc_at = c.now + busy;
@@ -2004,7 +2258,7 @@ RD_HD void port_emit(SwSlot &c, int port, const Pkt &p)
 // in the port's slot state
 RD_HD void port_push(SwSlot &c, int port, int queue, const Pkt &p)
 {
-    const Sim &s = *c.s;
+    SimRef s = *c.s;
     Port &pt = c.pt[port];
     const size_t pi = (size_t)c.pbase + port;
     const bool ctrl = queue == 0;
@@ -2031,7 +2285,7 @@ RD_HD void port_push(SwSlot &c, int port, int queue, const Pkt &p)
 // the control queue's head onto an idle link
 RD_HD void port_send_ctrl(SwSlot &c, int port)
 {
-    const Sim &s = *c.s;
+    SimRef s = *c.s;
     Port &pt = c.pt[port];
     if (pt.tc_at >= 0)
         return;
@@ -2054,18 +2308,14 @@ RD_HD void port_pfc(SwSlot &c, int port, bool pause)
     if (c.pt[port].q0_n > 0)
         port_send_ctrl(c, port);
 }
-// a data-queue frame leaves through `port`: the MMU lets go of it (in a safe slot only its ingress
-// counter moves), it may be ECN-marked, its ingress port may RESUME, an HPCC frame gets this hop's
+// a data-queue frame leaves through `port`: the MMU lets go of it, it may be ECN-marked, its ingress port may RESUME, an HPCC frame gets this hop's
 // INT record, then it is sent
 RD_HD void port_send_data(SwSlot &c, int port, Pkt p)
 {
-    const Sim &s = *c.s;
-    const Params &P = *c.P;
+    SimRef s = *c.s;
+    ParamsRef P = *c.P;
     Port &pt = c.pt[port];
-    if (c.safe)
-        at_sub32(&c.pt[p.inport].ing, (uint32_t)p.size); // (no headroom, no pause anywhere in a safe slot)
-    else
-        mmu_release(c, p.inport, p.size);
+    mmu_release(c, p.inport, p.size);
     pt.egr -= p.size;
     if (P.ecn && mmu_ecn_mark(c, port))
     {
@@ -2073,7 +2323,7 @@ RD_HD void port_send_data(SwSlot &c, int port, Pkt p)
         count(s, EV_MARK);
     }
     Port &in = c.pt[p.inport];
-    if (!c.safe && in.mmu_paused && in.hdrm == 0)
+    if (in.mmu_paused && in.hdrm == 0)
     {
         const uint32_t sh = mmu_shared_of(in);
         if (sh == 0 || sh + RESUME_OFFSET <= mmu_pfc_limit(c, p.inport))
@@ -2098,7 +2348,7 @@ RD_HD void port_send_data(SwSlot &c, int port, Pkt p)
 // the data class is paused
 RD_HD void port_pump(SwSlot &c, int port)
 {
-    const Sim &s = *c.s;
+    SimRef s = *c.s;
     Port &pt = c.pt[port];
     if (pt.tc_at >= 0)
         return;
@@ -2122,9 +2372,9 @@ RD_HD void port_pump(SwSlot &c, int port)
 // ---- the ingress path
 // the egress port of a data frame or an ACK (-1: no route) and its queue: equal-cost routes to
 // the destination host, chosen by the 5-tuple's hash with the switch's seed
-RD_HD int sw_route(const Sim &s, const Params &P, int x, const Pkt &p, int *q)
+RD_HD int sw_route(SimRef s, ParamsRef P, int x, const Pkt &p, int *q)
 {
-    const SwInfo &si = s.si[x];
+    const SwInfo RD_C &si = s.si[x];
     const bool fwd = p.kind == K_DATA;
     const int a = (fwd ? p.src : p.dst) - si.hbase, b = (fwd ? p.dst : p.src) - si.hbase;
     *q = !fwd && P.ack_high_prio ? 0 : PG;
@@ -2141,12 +2391,7 @@ RD_HD void sw_ingress(SwSlot &c, int inport, Pkt p, int out, int q)
 {
     if (out < 0)
         return;
-    if (q && c.safe)
-    {
-        at_add32(&c.pt[inport].ing, (uint32_t)p.size); // (below every limit all slot: shared_used follows at its end)
-        c.pt[out].egr += p.size;
-    }
-    else if (q)
+    if (q)
     {
         if (!mmu_admit(c, inport, p.size))
         {
@@ -2174,12 +2419,12 @@ RD_HD void sw_ingress(SwSlot &c, int inport, Pkt p, int out, int q)
 }
 
 // a frame's tx time on a port's in-link
-RD_HD int64_t port_in_tx(const Sim &s, const PortRun &r, uint32_t bytes)
+RD_HD int64_t port_in_tx(SimRef s, const PortRun &r, uint32_t bytes)
 {
     return bytes == r.isz[0] ? r.itx[0] : bytes == r.isz[1] ? r.itx[1] : rc_tx(s, r.irc, r.ibps, bytes);
 }
 // a port's next arrival of the slot
-RD_HD void sw_peek(const Sim &s, const SwSlot &c, int p)
+RD_HD void sw_peek(SimRef s, const SwSlot &c, int p)
 {
     PortRun &w = c.w[p];
     w.ats = INT64_MAX;
@@ -2191,9 +2436,9 @@ RD_HD void sw_peek(const Sim &s, const SwSlot &c, int p)
     }
 }
 
-RD_HD void sw_ctx(SwSlot &c, const Sim &s, int x, int64_t slot, uint32_t *pend, int pend_n, Port *pt, PortRun *w)
+RD_HD void sw_ctx(SwSlot &c, SimRef s, int x, int64_t slot, uint32_t *pend, int pend_n, Port *pt, PortRun *w)
 {
-    const SwInfo &si = s.si[x];
+    const SwInfo RD_C &si = s.si[x];
     c.s = &s;
     c.P = &s.Pw[s.s_world[x]];
     c.pend = pend;
@@ -2206,21 +2451,20 @@ RD_HD void sw_ctx(SwSlot &c, const Sim &s, int x, int64_t slot, uint32_t *pend, 
     c.pc = s.pc + si.pbase;
     c.pbase = si.pbase;
     c.sw = s.sw[x];
-    c.safe = false;
     c.cur_ok = false;
     c.ord = 0;
     c.ep = 0;
     c.now = slot * s.D;
 }
 // a port's slot set-up: its arrivals' cursor and its out bucket
-RD_HD void sw_port_open(const Sim &s, SwSlot &c, int p, int64_t slot)
+RD_HD void sw_port_open(SimRef s, SwSlot &c, int p, int64_t slot)
 {
     PortRun &r = c.w[p];
     r.ai = 0;
     r.nout = 0;
     r.an = bucket(s, c.pc[p].link_in, slot, &r.abase);
     {
-        const Link &li = s.li[c.pc[p].link_in];
+        const Link RD_C &li = s.li[c.pc[p].link_in];
         r.idelay = li.delay;
         r.irc = li.rc;
         r.ibps = li.bps;
@@ -2231,10 +2475,10 @@ RD_HD void sw_port_open(const Sim &s, SwSlot &c, int p, int64_t slot)
     }
     if (c.pt[p].q3_n > 0)
         r.qhead = s.q3[((size_t)c.pbase + p) * s.q3_cap + c.pt[p].q3_head];
-    ob_open(s, r.ob, c.pc[p].link_out, c.pt[p].ob_last);
+    ob_open(s, r.ob, c.pc[p].link_out, c.pt[p].ob_last, slot, c.pend_n);
 }
 // a port's slot end: its bucket's count out; busy (sent, or holds frames)?
-RD_HD bool sw_port_close(const Sim &s, SwSlot &c, int p, unsigned long long *nout)
+RD_HD bool sw_port_close(SimRef s, SwSlot &c, int p, unsigned long long *nout)
 {
     ob_flush(s, c.w[p].ob);
     c.pt[p].ob_last = c.w[p].ob.last;
@@ -2245,7 +2489,7 @@ RD_HD bool sw_port_close(const Sim &s, SwSlot &c, int p, unsigned long long *nou
 // All of a switch's events of the slot in order on one lane (the reference's serial path,
 // src/rdma/rstep.cuh:3032-3189): candidates are each port's next arrival and its TransmitComplete,
 // in port order, arrival first; ties by the chains; undecided ties keep the earlier candidate.
-RD_HD void sw_serial_events(const Sim &s, SwSlot &c, int deg, int64_t t1)
+RD_HD void sw_serial_events(SimRef s, SwSlot &c, int deg, int64_t t1)
 {
     for (int p = 0; p < deg; p++)
         sw_peek(s, c, p);
@@ -2316,9 +2560,9 @@ RD_HD void sw_serial_events(const Sim &s, SwSlot &c, int deg, int64_t t1)
 
 // One switch's slot on one lane, its ports in HBM: the serial path for any number of ports.
 // Returns whether the switch is busy.
-RD_HD bool switch_step(const Sim &s, int x, int64_t slot, uint32_t *pend, int pend_n)
+RD_HD bool switch_step(SimRef s, int x, int64_t slot, uint32_t *pend, int pend_n)
 {
-    const SwInfo &si = s.si[x];
+    const SwInfo RD_C &si = s.si[x];
     SwSlot c;
     sw_ctx(c, s, x, slot, pend, pend_n, s.ps + si.pbase, s.pr + si.pbase);
     for (int p = 0; p < si.deg; p++)
@@ -2347,156 +2591,300 @@ RD_HD bool switch_step(const Sim &s, int x, int64_t slot, uint32_t *pend, int pe
 constexpr int KS = 32;  // ports of a switch whose slot runs from the LDS workspace
 constexpr int KW = 64;  // ports of a switch whose slot runs from a device-memory workspace (a lane per port of wave64)
 constexpr int LK = 512; // arrivals of a slot a safe slot takes
-template <int K>
-struct SwWorkT
+// The workspace's parts for a switch of deg ports, laid out in its bytes: what the ports need, the
+// arrivals' places, then as many of the arrivals' frames as there is room for (copied when they are
+// routed: a lane's chain of events then reads no frame from memory, where each read waited for the
+// coherent stores of the event before it).
+struct SwWs
 {
-    static constexpr int ports = K;
-    Port pt[K];
-    PortRun w[K];
-    PortCfg pc[K]; // (a copy: no load of a port's configuration per event)
-    Chain tc[K];   // the ports' pending TransmitCompletes' chains (copies, written back at the slot's end)
-    int cnt[K], first[K];
-    uint32_t abytes[K], ing0[K];
-    int16_t mc[K][K]; // [egress][ingress]: the ingress's next arrival for the egress (-1: none)
-    int16_t onext[LK];  // an arrival's next one of the same ingress and egress (-1: none)
-    int64_t ats[LK];
-    uint32_t acode[LK]; // its event code (the in-link's tx time and delay, its ordinal)
-    int8_t own[LK];     // the egress port it belongs to in a safe slot (-1: none)
-    uint8_t q[LK];
-    int total, safe;
-    unsigned act;
-    unsigned nout;
+    Port *pt;
+    PortRun *w;
+    PortCfg *pc; // (a copy: no load of a port's configuration per event)
+    Chain *tc;   // the ports' pending TransmitCompletes' chains (copies, written back at the slot's end)
+    int *cnt, *first;
+    uint32_t *abytes, *ing0;
+    int64_t *ats;    // [LK] the arrivals' times
+    uint32_t *acode; // [LK] their event codes (the in-link's tx time and delay, the ordinal)
+    int16_t *mc;     // [egress][ingress]: the ingress's next arrival for the egress (-1: none)
+    int16_t *onext;  // [LK] an arrival's next one of the same ingress and egress (-1: none)
+    int8_t *own;     // [LK] the egress port it belongs to in a safe slot (-1: none)
+    uint8_t *q;      // [LK]
+    unsigned *act, *nout; // busy ports, frames sent
+    uint32_t *sum, *bad, *moved; // arrived bytes; ports that make the slot unsafe; shared_used's change
+    InFrame *fr; // the first fr_n arrivals' frames
+    int fr_n, deg;
 };
-typedef SwWorkT<KS> SwWork;     // in LDS, a wave's
-typedef SwWorkT<KW> SwWorkWide; // in device memory, a wave's (switches of KS + 1 to KW ports)
-
-#if defined(__HIP_DEVICE_COMPILE__)
-#define RD_WAVE_SYNC()                                                                                                            \
-    do                                                                                                                            \
-    {                                                                                                                             \
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");                                                                    \
-        __builtin_amdgcn_wave_barrier();                                                                                          \
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");                                                                    \
-    } while (0)
-#else
-#define RD_WAVE_SYNC() \
-    do                 \
-    {                  \
-    } while (0)
-#endif
+constexpr int sw_work_bytes(int deg)
+{
+    return deg * (int)(sizeof(Port) + sizeof(PortRun) + sizeof(PortCfg) + sizeof(Chain) + 16) + LK * 16 + 24 + (deg * deg * 2 + 7 & ~7);
+}
+RD_HD SwWs sw_work(char *mem, int bytes, int deg)
+{
+    static_assert(sizeof(Port) % 8 == 0 && sizeof(PortRun) % 8 == 0 && sizeof(PortCfg) % 8 == 0 && sizeof(Chain) % 8 == 0, "8-byte parts");
+    SwWs k;
+    k.ats = reinterpret_cast<int64_t *>(mem);
+    k.acode = reinterpret_cast<uint32_t *>(k.ats + LK);
+    k.onext = reinterpret_cast<int16_t *>(k.acode + LK);
+    k.own = reinterpret_cast<int8_t *>(k.onext + LK);
+    k.q = reinterpret_cast<uint8_t *>(k.own + LK);
+    k.act = reinterpret_cast<unsigned *>(k.q + LK);
+    k.nout = k.act + 1;
+    k.sum = reinterpret_cast<uint32_t *>(k.nout + 1);
+    k.bad = k.sum + 1;
+    k.moved = k.sum + 2;
+    k.pt = reinterpret_cast<Port *>(k.sum + 4);
+    k.w = reinterpret_cast<PortRun *>(k.pt + deg);
+    k.pc = reinterpret_cast<PortCfg *>(k.w + deg);
+    k.tc = reinterpret_cast<Chain *>(k.pc + deg);
+    k.cnt = reinterpret_cast<int *>(k.tc + deg);
+    k.first = k.cnt + deg;
+    k.abytes = reinterpret_cast<uint32_t *>(k.first + deg);
+    k.ing0 = k.abytes + deg;
+    k.mc = reinterpret_cast<int16_t *>(k.ing0 + deg);
+    k.fr = reinterpret_cast<InFrame *>(mem + sw_work_bytes(deg));
+    k.fr_n = (bytes - sw_work_bytes(deg)) / (int)sizeof(InFrame);
+    k.deg = deg;
+    return k;
+}
+template <int K, int BYTES>
+struct alignas(16) SwWorkT
+{
+    static constexpr int ports = K, size = BYTES;
+    static_assert(BYTES >= sw_work_bytes(K), "the workspace holds the ports");
+    char mem[BYTES];
+};
+// a wave's workspace in LDS: a quarter of the CU's 160 KB less the workgroup's own words
+constexpr int WAVE_LDS = 40704;
+typedef SwWorkT<KS, WAVE_LDS> SwWork;              // in LDS, a wave's
+typedef SwWorkT<KW, sw_work_bytes(KW)> SwWorkWide; // in device memory, a wave's (switches of KS + 1 to KW ports)
 
 // arrival j's frame (of ingress p) in its link's ring (its code is in the workspace: k.acode[j])
-template <typename WK>
-RD_HD const LFrame RD_G *sw_arr(const Sim &s, const WK &k, int p, int j) { return s.msg + k.w[p].abase + (uint64_t)(j - k.first[p]); }
+RD_HD const LFrame RD_G *sw_arr(SimRef s, const SwWs &k, int p, int j) { return s.msg + k.w[p].abase + (uint64_t)(j - k.first[p]); }
 
-// egress port o's events of a safe slot (src/rdma/rstep.cuh:2806-3005)
-#if defined(RD_PROF) && defined(__HIP_DEVICE_COMPILE__)
-// (profiling builds: a wave's time in a part of the egress loop, counted once per wave)
-#define RD_PROF_T(v) const long long v = wall_clock64()
-#define RD_PROF_ADD(i, d)                                                                                                         \
-    do                                                                                                                            \
-    {                                                                                                                             \
-        if ((int)(__builtin_ffsll((long long)__ballot(1)) - 1) == (int)__lane_id())                                               \
-            at_add64(&s.ev[i], (unsigned long long)(d));                                                                          \
-    } while (0)
-#else
-#define RD_PROF_T(v)
-#define RD_PROF_ADD(i, d)
-#endif
-template <typename WK>
-RD_HD void sw_egress_events(const Sim &s, SwSlot &c, WK &k, int o, int deg, int64_t t1)
+// arrival j's chain: in the workspace, or in its frame
+RD_HD const Chain &sw_arr_chain(SimRef s, const SwWs &k, int p, int j) { return j < k.fr_n ? k.fr[j].c : (const Chain &)sw_arr(s, k, p, j)->c; }
+
+// Egress port o's events of a safe slot (src/rdma/rstep.cuh:2806-3005).
+// A lane runs these as one chain, so what bounds it is the chain's length, and the chain's slowest
+// links are loads: vector memory counts in order, so a load waits for the coherent stores issued
+// before it (measured: an L2 hit after the eight 8-byte stores of a packet takes 0.40 us, 0.09 us
+// without them). So the port's state is in registers for the slot (in the workspace it was some 40
+// LDS reads an event), the next arrival's packet and chain are read when it becomes the next (a
+// TransmitComplete before it hides them), the next queued frame when its predecessor leaves, and a
+// transmission's stores are followed by no load. One transmission site serves cut-through,
+// dequeue and control frames, so that the lanes of a wave share it whatever their events are.
+// (FatTree k=8 a2a under HPCC: 5.2 us a round of the loop before, 2.1 us now; what is left is the
+// round's instructions, some 900 on one wave of a SIMD, and the LDS reads of its merge.)
+RD_HD void sw_egress_events(SimRef s, SwSlot &c, const SwWs &k, int o, int deg, int64_t t1)
 {
+    ParamsRef P = *c.P;
+    const size_t pi = (size_t)c.pbase + o;
+    Pkt RD_G *q0 = s.q0 + pi * s.q0_cap, *q3 = s.q3 + pi * s.q3_cap;
+    Port &pm = k.pt[o]; // (its ingress counter stays there: every egress lane moves it)
+    int64_t tc_at = pm.tc_at;
+    uint32_t paused = pm.paused, bytes_total = pm.bytes_total, egr = pm.egr;
+    uint64_t tx_bytes = pm.tx_bytes;
+    int q0_head = pm.q0_head, q0_n = pm.q0_n, q3_head = pm.q3_head, q3_n = pm.q3_n, nout = k.w[o].nout;
+    TailAlloc ta = pm.ta;
+    OutBucket ob = k.w[o].ob;
+    Pkt qhead = k.w[o].qhead; // the data queue's head (while q3_n > 0)
+    const uint64_t bps = k.pc[o].bps;
     // the ingress ports with arrivals left for o (bit p: port p)
     uint64_t live = 0;
     for (int p = 0; p < deg; p++)
-        if (k.mc[o][p] >= 0)
+        if (k.mc[o * deg + p] >= 0)
             live |= 1ull << p;
+    // the next arrival: its ingress port, place and time, its packet and chain
+    bool look = true;
+    int bp = -1, kb = -1;
+    int64_t at = INT64_MAX;
+    uint32_t acode = 0;
+    Pkt apk = {};
+    Chain ach = {};
+    RD_PROF_SUMS;
     for (;;)
     {
-        RD_PROF_T(q0);
-        // the next arrival for o: the ingress heads in port order, the earlier (time, chains) kept
-        int bp = -1, kb = -1;
-        for (uint64_t m = live; m; m &= m - 1)
+        RD_PROF_T(prof_q0);
+        if (look)
         {
-            const int p = __builtin_ctzll(m);
-            const int j = k.mc[o][p];
-            if (bp < 0)
+            // the ingress heads in port order, the earlier (time, chains) kept
+            look = false;
+            bp = kb = -1;
+            at = INT64_MAX;
+            for (uint64_t m = live; m; m &= m - 1)
             {
-                bp = p, kb = j;
-                continue;
+                const int p = __builtin_ctzll(m);
+                const int j = k.mc[o * deg + p];
+                const int64_t t = k.ats[j];
+                if (bp >= 0 && (t > at || (t == at && !before_q(s, t, k.acode[j], sw_arr_chain(s, k, p, j), k.acode[kb], sw_arr_chain(s, k, bp, kb)))))
+                    continue;
+                bp = p, kb = j, at = t;
             }
-            bool b4;
-            if (k.ats[j] != k.ats[kb])
-                b4 = k.ats[j] < k.ats[kb];
-            else
+            if (kb >= 0)
             {
-                const LFrame RD_G *fa = sw_arr(s, k, p, j), *fb = sw_arr(s, k, bp, kb);
-                b4 = before_q(s, k.ats[j], k.acode[j], fa->c, k.acode[kb], fb->c);
+                acode = k.acode[kb];
+                if (kb < k.fr_n)
+                {
+                    apk = k.fr[kb].p;
+                    ach = k.fr[kb].c;
+                }
+                else
+                {
+                    const LFrame RD_G *fa = sw_arr(s, k, bp, kb);
+                    apk = pkt_get(&fa->p);
+                    ach = chain_get(&fa->c);
+                }
             }
-            if (b4)
-                bp = p, kb = j;
         }
-        const int64_t ta = kb >= 0 ? k.ats[kb] : INT64_MAX, tc = k.pt[o].tc_at;
-        const bool htc = tc >= 0 && tc < t1;
-        RD_PROF_T(q1);
-        RD_PROF_ADD(29, q1 - q0);
-        if (ta == INT64_MAX && !htc)
+        RD_PROF_T(prof_q1);
+        RD_PROF_ADD(0, prof_q1 - prof_q0);
+        RD_PROF_ADD(3, 1);
+        const bool htc = tc_at >= 0 && tc_at < t1;
+        if (kb < 0 && !htc)
             break;
-        bool arr;
-        const LFrame RD_G *fa = kb >= 0 ? sw_arr(s, k, bp, kb) : nullptr;
-        const uint32_t acode = fa ? k.acode[kb] : 0;
-        if (!htc || ta == INT64_MAX)
-            arr = !htc;
-        else if (ta != tc)
-            arr = ta < tc;
-        else
-            arr = before_q(s, ta, acode, fa->c, 0, c.tc[o]);
-        c.ord = 0;
-        c.ep = o;
-        c.cur_ok = false;
-        if (!arr)
+        // (a frame's arrival often meets the TransmitComplete of the one before it: back to back at one
+        // rate; the first leads decide, from the chains at hand)
+        bool arr = !htc || (kb >= 0 && at < tc_at);
+        if (htc && kb >= 0 && at == tc_at)
         {
-            c.now = tc;
-            c.cur_src = &c.tc[o];
-            c.cur_code = 0;
-            sw_event_chain(c);
-            k.pt[o].tc_at = -1;
-            port_pump(c, o);
-            RD_PROF_T(q2);
-            RD_PROF_ADD(30, q2 - q1);
-            continue;
+            const int r = quick_order(s, acode, head_of(ach), 0, head_of(k.tc[o]));
+            arr = r ? r < 0 : before(s, at, acode, sw_arr_chain(s, k, bp, kb), at, 0, k.tc[o]);
         }
-        k.mc[o][bp] = k.onext[kb];
-        if (k.onext[kb] < 0)
-            live &= ~(1ull << bp);
-        c.now = ta;
-        c.cur_src = &fa->c;
-        c.cur_code = acode;
-        const Pkt pk = pkt_get(&fa->p);
-        if (pk.kind == K_PAUSE || pk.kind == K_RESUME)
+        // the event: a frame to send at once (cut-through), or one queued, then the pump
+        bool send = false, pump = true, ctrl = false, took = false;
+        Pkt p = apk;
+        const int64_t now = arr ? at : tc_at;
+        if (!arr)
+            tc_at = -1;
+        else
         {
-            if (pk.kind == K_PAUSE)
-                k.pt[o].paused |= 1u << pk.q;
+            const int nx = k.onext[kb], q = k.q[kb];
+            k.mc[o * deg + bp] = (int16_t)nx;
+            if (nx < 0)
+                live &= ~(1ull << bp);
+            look = true;
+            if (p.kind == K_PAUSE)
+            {
+                paused |= 1u << p.q;
+                pump = false;
+            }
+            else if (p.kind == K_RESUME)
+                paused &= ~(1u << p.q);
             else
             {
-                k.pt[o].paused &= ~(1u << pk.q);
-                port_pump(c, o);
+                p.inport = (uint8_t)bp;
+                if (q)
+                {
+                    at_add32(&k.pt[bp].ing, (uint32_t)p.size); // (below every limit all slot: shared_used follows at its end)
+                    egr += p.size;
+                }
+                send = q && tc_at < 0 && q0_n == 0 && q3_n == 0 && !(paused >> PG & 1);
+                const int n = q ? q3_n : q0_n, cap = q ? s.q3_cap : s.q0_cap;
+                if (!send && n >= cap)
+                    count(s, EV_QUEUE_OVF);
+                else if (!send)
+                {
+                    (q ? q3 : q0)[ring_add(q ? q3_head : q0_head, n, cap)] = p;
+                    bytes_total += p.size;
+                    if (!q)
+                        q0_n++;
+                    else if (!q3_n++)
+                        qhead = p;
+                }
             }
         }
-        else
-            sw_ingress(c, bp, pk, o, k.q[kb]);
-        RD_PROF_T(q3);
-        RD_PROF_ADD(31, q3 - q1);
+        if (!send && pump && tc_at < 0)
+        {
+            if (q0_n > 0)
+            {
+                p = q0[q0_head];
+                q0_head = ring_add(q0_head, 1, s.q0_cap);
+                q0_n--;
+                bytes_total -= p.size;
+                send = ctrl = true;
+            }
+            else if (q3_n > 0 && !(paused >> PG & 1))
+            {
+                p = qhead;
+                q3_head = ring_add(q3_head, 1, s.q3_cap);
+                q3_n--;
+                bytes_total -= p.size;
+                send = took = true;
+            }
+        }
+        RD_PROF_T(prof_q2);
+        RD_PROF_ADD(1, prof_q2 - prof_q1);
+        if (!send)
+            continue;
+        if (!ctrl)
+        {
+            // a data-queue frame leaves (port_send_data in a safe slot: no headroom, no pause)
+            at_sub32(&k.pt[p.inport].ing, (uint32_t)p.size);
+            egr -= p.size;
+            const PortCfg &pc = k.pc[o];
+            if (P.ecn && (egr > pc.kmax || (egr > pc.kmin && rand_u01(pm.rng) < pc.pmax * (double)(egr - pc.kmin) / (double)(pc.kmax - pc.kmin))))
+            {
+                p.ecn = 3;
+                count(s, EV_MARK);
+            }
+            if (p.kind == K_DATA && P.cc == 3 && p.nhop < 0xFFFF)
+            {
+                const uint64_t rec = hop_make((uint64_t)now, tx_bytes, bytes_total, bps, P.int_multi);
+                const int slot_i = p.nhop % MAX_HOP;
+                for (int i = 0; i < MAX_HOP; i++)
+                    p.hop[i] = i == slot_i ? rec : p.hop[i];
+                p.nhop++;
+            }
+        }
+        tx_bytes += p.size;
+        // the transmission (port_emit): the frame, then the chains
+        const int64_t busy = link_txo(s, ob, p.size), lands = now + busy + ob.delay;
+        tc_at = now + busy;
+        nout++;
+        LFrame RD_G *fr = ob_push(s, c.pend, c.pend_n, lands, ob);
+        p.ord = 1; // (the event's first scheduled event is the TransmitComplete, its second the arrival)
+        Chain cur = k.tc[o];
+        if (arr)
+            cpush(s, ta, &cur, acode, ach);
+        cpush(s, ta, &k.tc[o], ccode(busy, 0), cur);
+        if (fr)
+        {
+            coh_store(&fr->ts, lands);
+            frame_put_pkt(s, fr, p);
+            frame_put_chain(s, fr, cur);
+            if (s.txt_rec.rec)
+                trace_tx(s, now, c.node, o + 1, p.seq, pkt_w6(p), pkt_w7(p));
+        }
+        // (the next head last: its load then has until the next dequeue)
+        if (took && q3_n > 0)
+            qhead = q3[q3_head];
+        RD_PROF_T(prof_q3);
+        RD_PROF_ADD(2, prof_q3 - prof_q2);
     }
+    RD_PROF_OUT(29, 30, 31, 39);
+    pm.tc_at = tc_at;
+    pm.paused = paused;
+    pm.bytes_total = bytes_total;
+    pm.egr = egr;
+    pm.tx_bytes = tx_bytes;
+    pm.q0_head = q0_head;
+    pm.q0_n = q0_n;
+    pm.q3_head = q3_head;
+    pm.q3_n = q3_n;
+    pm.ta = ta;
+    k.w[o].nout = nout;
+    k.w[o].ob = ob;
 }
 
-// One switch's slot by lane `lane` of `nlanes` (a wave on the GPU, one lane on the CPU); ports
-// p = lane, lane + nlanes, ... are this lane's. Returns (on every lane) whether the switch is busy.
-template <typename WK>
-RD_HD bool switch_slot(const Sim &s, int x, int64_t slot, uint32_t *pend, int pend_n, WK &k, int lane, int nlanes)
+// One switch's slot by lane `lane` of `nlanes` (on the GPU a wave, or a workgroup with sync() its
+// barrier; one lane on the CPU); ports p = lane, lane + nlanes, ... are this lane's. Returns (on
+// every lane) whether the switch is busy.
+template <typename SYNC>
+RD_HD bool switch_slot_by(SimRef s, int x, int64_t slot, uint32_t *pend, int pend_n, char *mem, int bytes, int lane, int nlanes, SYNC sync)
 {
-    const SwInfo &si = s.si[x];
+    const SwInfo RD_C &si = s.si[x];
     const int deg = si.deg;
+    const SwWs k = sw_work(mem, bytes, deg);
     const int64_t t1 = (slot + 1) * s.D;
     SwSlot c;
     sw_ctx(c, s, x, slot, pend, pend_n, k.pt, k.w);
@@ -2518,17 +2906,18 @@ RD_HD bool switch_slot(const Sim &s, int x, int64_t slot, uint32_t *pend, int pe
     }
     if (lane == 0)
     {
-        k.act = 0;
-        k.nout = 0;
+        *k.act = *k.nout = 0;
+        *k.sum = *k.bad = *k.moved = 0;
     }
-    RD_WAVE_SYNC();
+    sync();
 #if defined(RD_PROF) && defined(__HIP_DEVICE_COMPILE__)
     long long pt1 = wall_clock64();
 #endif
     int total = 0;
     for (int p = 0; p < deg; p++)
         total += k.cnt[p];
-    // routes and times of the arrivals (a safe slot's candidates), per ingress port
+    // routes, times and event codes of the arrivals (a safe slot's candidates), an arrival per lane:
+    // each is three loads one after another, which the lanes then wait for together
     if (total <= LK)
         for (int p = lane; p < deg; p += nlanes)
         {
@@ -2536,58 +2925,72 @@ RD_HD bool switch_slot(const Sim &s, int x, int64_t slot, uint32_t *pend, int pe
             for (int r = 0; r < p; r++)
                 f0 += k.cnt[r];
             k.first[p] = f0;
-            for (int i = 0; i < k.cnt[p]; i++)
+        }
+    sync();
+    if (total <= LK)
+        for (int j = lane; j < total; j += nlanes)
+        {
+            // arrival j's ingress port: the last one whose arrivals start at or before j
+            int p = 0;
+            for (int step = KW / 2; step; step /= 2)
+                if (p + step < deg && k.first[p + step] <= j)
+                    p += step;
+            const LFrame RD_G *f = sw_arr(s, k, p, j);
+            const int64_t at = coh_load(&f->ts);
+            const Pkt pk = pkt_get(&f->p);
+            if (j < k.fr_n)
             {
-                const int j = f0 + i;
-                const LFrame RD_G *f = s.msg + k.w[p].abase + i;
-                k.ats[j] = coh_load(&f->ts);
-                const Pkt pk = pkt_get(&f->p);
-                k.acode[j] = ccode(port_in_tx(s, k.w[p], pk.size) + k.w[p].idelay, pk.ord);
-                int q = 0;
-                if (pk.kind == K_PAUSE || pk.kind == K_RESUME)
-                    k.own[j] = (int8_t)p;
-                else
-                {
-                    const int out = sw_route(s, *c.P, x, pk, &q);
-                    k.own[j] = (int8_t)out;
-                    if (out >= 0 && q != 0)
-                        k.abytes[p] += pk.size;
-                }
-                k.q[j] = (uint8_t)q;
+                k.fr[j].c = chain_get(&f->c);
+                k.fr[j].p = pk;
             }
+            k.ats[j] = at;
+            k.acode[j] = ccode(port_in_tx(s, k.w[p], pk.size) + k.w[p].idelay, pk.ord);
+            int q = 0, out = p;
+            if (pk.kind != K_PAUSE && pk.kind != K_RESUME)
+            {
+                out = sw_route(s, *c.P, x, pk, &q);
+                if (out >= 0 && q != 0)
+                {
+                    at_add32(&k.abytes[p], (uint32_t)pk.size);
+                    at_add32(k.sum, (uint32_t)pk.size);
+                }
+            }
+            k.own[j] = (int8_t)out;
+            k.q[j] = (uint8_t)q;
+        }
+    sync();
+    // is the slot safe? Each lane looks at its ports. (GetPfcThreshold is uint32_t: with less buffer than
+    // headroom and reserves the difference wraps to about 2^32 and stays there, so such a switch never
+    // pauses)
+    if (total <= LK)
+    {
+        const int64_t amax = (int64_t)c.sw.shared_used + (int64_t)*k.sum;
+        const int64_t room = (int64_t)(uint32_t)(c.P->buffer_size - c.sw.total_hdrm - c.sw.total_rsrv) - amax;
+        const int64_t th_min = room > 0 ? room >> c.sw.max_shift : -1;
+        for (int p = lane; p < deg; p += nlanes)
+        {
+            const int64_t su = (int64_t)k.pt[p].ing + k.abytes[p] - RESERVE;
+            if (k.pt[p].hdrm || k.pt[p].mmu_paused || (su > 0 ? su : 0) >= th_min)
+                at_add32(k.bad, 1u);
+        }
+    }
+    // per ingress port and egress port, the arrivals in order
+    if (total <= LK)
+        for (int p = lane; p < deg; p += nlanes)
+        {
             for (int o = 0; o < deg; o++)
-                k.mc[o][p] = -1;
-            for (int j = f0 + k.cnt[p] - 1; j >= f0; j--)
+                k.mc[o * deg + p] = -1;
+            for (int j = k.first[p] + k.cnt[p] - 1; j >= k.first[p]; j--)
             {
                 const int o = k.own[j];
                 if (o < 0)
                     continue;
-                k.onext[j] = k.mc[o][p];
-                k.mc[o][p] = (int16_t)j;
+                k.onext[j] = k.mc[o * deg + p];
+                k.mc[o * deg + p] = (int16_t)j;
             }
         }
-    RD_WAVE_SYNC();
-    // is the slot safe? (every lane decides alike)
-    bool safe = !s.serial && total <= LK;
-    if (safe)
-    {
-        uint64_t sum = 0;
-        for (int p = 0; p < deg && safe; p++)
-        {
-            sum += k.abytes[p];
-            safe = !k.pt[p].hdrm && !k.pt[p].mmu_paused;
-        }
-        // (GetPfcThreshold is uint32_t: with less buffer than headroom and reserves the difference
-        // wraps to about 2^32 and stays there, so such a switch never pauses)
-        const int64_t amax = (int64_t)c.sw.shared_used + (int64_t)sum;
-        const int64_t room = (int64_t)(uint32_t)(c.P->buffer_size - c.sw.total_hdrm - c.sw.total_rsrv) - amax;
-        const int64_t th_min = room > 0 ? room >> c.sw.max_shift : -1;
-        for (int p = 0; p < deg && safe; p++)
-        {
-            const int64_t su = (int64_t)k.pt[p].ing + k.abytes[p] - RESERVE;
-            safe = (su > 0 ? su : 0) < th_min;
-        }
-    }
+    sync();
+    const bool safe = !s.serial && total <= LK && !*k.bad;
 #ifdef RD_PROF
     if (lane == 0)
         at_add64(&s.ev[safe ? 36 : 37], 1ull); // (profiling builds: safe and serial switch slots)
@@ -2597,7 +3000,6 @@ RD_HD bool switch_slot(const Sim &s, int x, int64_t slot, uint32_t *pend, int pe
 #endif
     if (safe)
     {
-        c.safe = true;
         for (int o = lane; o < deg; o += nlanes)
             sw_egress_events(s, c, k, o, deg, t1);
     }
@@ -2606,7 +3008,7 @@ RD_HD bool switch_slot(const Sim &s, int x, int64_t slot, uint32_t *pend, int pe
         sw_serial_events(s, c, deg, t1);
         s.sw[x] = c.sw;
     }
-    RD_WAVE_SYNC();
+    sync();
 #if defined(RD_PROF) && defined(__HIP_DEVICE_COMPILE__)
     long long pt3 = wall_clock64();
 #endif
@@ -2618,33 +3020,33 @@ RD_HD bool switch_slot(const Sim &s, int x, int64_t slot, uint32_t *pend, int pe
         act |= sw_port_close(s, c, p, &nout);
         s.ps[si.pbase + p] = k.pt[p];
         s.p_tc[si.pbase + p] = k.tc[p];
+        // (a safe slot: shared_used, the sum over ports of max(0, ing - reserve), changed with ing only;
+        // modulo 2^32, as the counter)
+        if (safe)
+        {
+            const uint32_t a = k.ing0[p] > RESERVE ? k.ing0[p] - RESERVE : 0, b = k.pt[p].ing > RESERVE ? k.pt[p].ing - RESERVE : 0;
+            if (a != b)
+                at_add32(k.moved, b - a);
+        }
     }
     if (act)
-        at_add32(&k.act, 1u);
+        at_add32(k.act, 1u);
     if (nout)
-        at_add32(&k.nout, (unsigned)nout);
-    RD_WAVE_SYNC();
+        at_add32(k.nout, (unsigned)nout);
+    sync();
     if (lane == 0)
     {
         if (safe)
         {
-            // shared_used = sum over ports of max(0, ing - reserve), which changed with ing only
-            // (modulo 2^32, as the counter)
-            uint32_t d = 0;
-            for (int p = 0; p < deg; p++)
-            {
-                const uint32_t a = k.ing0[p] > RESERVE ? k.ing0[p] - RESERVE : 0, b = k.pt[p].ing > RESERVE ? k.pt[p].ing - RESERVE : 0;
-                d += b - a;
-            }
             Switch sw = s.sw[x];
-            sw.shared_used += d;
+            sw.shared_used += *k.moved;
             s.sw[x] = sw;
         }
-        if (k.nout)
-            at_add64(&s.ev[EV_PKT], (unsigned long long)k.nout);
+        if (*k.nout)
+            at_add64(&s.ev[EV_PKT], (unsigned long long)*k.nout);
     }
-    const bool busy = k.act != 0;
-    RD_WAVE_SYNC(); // (the workspace is reused by the next switch)
+    const bool busy = *k.act != 0;
+    sync(); // (the workspace is reused by the next switch)
 #if defined(RD_PROF) && defined(__HIP_DEVICE_COMPILE__)
     // (profiling builds: the phases' time, summed over switch slots: ports in, routes, events, ports out;
     // and the arrivals)
@@ -2661,23 +3063,31 @@ RD_HD bool switch_slot(const Sim &s, int x, int64_t slot, uint32_t *pend, int pe
     return busy;
 }
 
-// does the switch have events in this slot? (busy last slot, or arrivals; src/rdma/rstep.cuh:3859-3881)
-RD_HD bool switch_has_input(const Sim &s, int x, int64_t slot)
+// a wave's (or the CPU's one lane's) switch slot in its workspace
+template <typename WK>
+RD_HD bool switch_slot(SimRef s, int x, int64_t slot, uint32_t *pend, int pend_n, WK &mem, int lane, int nlanes)
 {
-    const SwInfo &si = s.si[x];
-    for (int p = 0; p < si.deg; p++)
+    return switch_slot_by(s, x, slot, pend, pend_n, mem.mem, WK::size, lane, nlanes, [] { RD_WAVE_SYNC(); });
+}
+
+// does the switch have events in this slot? (busy last slot, or arrivals; src/rdma/rstep.cuh:3859-3881)
+// (by lane `lane` of `nlanes`, each its ports: true if one of them has arrivals)
+RD_HD bool switch_has_input(SimRef s, int x, int64_t slot, int lane = 0, int nlanes = 1)
+{
+    const SwInfo RD_C &si = s.si[x];
+    bool in = false;
+    for (int p = lane; p < si.deg; p += nlanes)
     {
         uint64_t base;
-        if (bucket(s, s.pc[si.pbase + p].link_in, slot, &base) > 0)
-            return true;
+        in |= bucket(s, s.pc[si.pbase + p].link_in, slot, &base) > 0;
     }
-    return false;
+    return in;
 }
 
 // The end of a world's slot, after all its entities ran it (src/rdma/rstep.cuh:3451-3585 without
 // windows): finish when every flow is done or at the stop; with nothing sent or queued anywhere,
 // skip to the slot of the earliest host event or pending arrival; with none, the run is quiescent.
-RD_HD void slot_end(const Sim &s, const World &wd, WorldRun &r, uint32_t *pend, unsigned act, unsigned long long wake)
+RD_HD void slot_end(SimRef s, const World &wd, WorldRun &r, uint32_t *pend, unsigned act, unsigned long long wake)
 {
     // (the ticket and the pending-slot flags are read and written coherently: every workgroup of
     // the team reads the ticket after the barrier, and every entity sets flags)
@@ -2685,13 +3095,13 @@ RD_HD void slot_end(const Sim &s, const World &wd, WorldRun &r, uint32_t *pend, 
     // (an atomic read: the lanes' completions were counted by atomics, in L2)
     if (at_add32(&r.flows_done, 0u) >= (uint32_t)wd.nf || slot + 1 >= wd.max_slots)
         coh_store(&r.finished, 1);
-    coh_store(pend + slot % wd.pend_n, 0u);
+    coh_store(pend + ring_place(slot, (uint32_t)wd.pend_n), 0u);
     int64_t next = slot + 1;
     if (act == 0)
     {
         int64_t ws = wake != ~0ull ? (int64_t)(wake / (unsigned long long)s.D) : INT64_MAX;
         for (int i = 1; i < wd.pend_n; i++)
-            if (coh_load(pend + (slot + i) % wd.pend_n))
+            if (coh_load(pend + ring_place(slot + i, (uint32_t)wd.pend_n)))
             {
                 ws = slot + i < ws ? slot + i : ws;
                 break;

@@ -257,13 +257,15 @@ int main(int argc, char **argv)
             // (profiling builds: wave-time of host items and of switch items summed over the team, and
             // the first workgroup's wait at the barrier, per slot; constant clock of 100 MHz)
             const double k = 0.01 / (double)st.slots;
-            printf("prof: per slot: host items %.2f wave-us, switch items %.2f wave-us, barrier %.2f us (%lld slots)\n",
-                   ev[33] * k, ev[34] * k, ev[35] * k, (long long)st.slots);
+            printf("prof: per slot: host items %.2f wave-us, switch items %.2f wave-us, longest %.2f / %.2f us, barrier %.2f us (%lld slots)\n",
+                   ev[33] * k, ev[34] * k, ev[22] * k, ev[23] * k, ev[35] * k, (long long)st.slots);
+            printf("prof: host event loops per slot: rounds %.1f, selection %.2f, events %.2f, pump %.2f lane-us\n",
+                   ev[17] / (double)st.slots, ev[14] * k, ev[15] * k, ev[16] * k);
             // the switch slots' phases (ports in, routes, events, ports out), their arrivals, and in the
-            // events of safe slots the egress merge, TransmitCompletes and arrivals (a wave's time each)
+            // events of safe slots the egress loops' rounds and the lanes' time in their parts
             printf("prof: switch phases per slot (wave-us): in %.2f, routes %.2f, events %.2f, out %.2f; arrivals %.1f; "
-                   "merge %.2f, tx-complete %.2f, arrival events %.2f; safe slots %llu, serial %llu\n",
-                   ev[24] * k, ev[25] * k, ev[26] * k, ev[27] * k, ev[28] / (double)st.slots, ev[29] * k, ev[30] * k, ev[31] * k,
+                   "rounds %.1f, merge %.2f, events %.2f, transmissions %.2f; safe slots %llu, serial %llu\n",
+                   ev[24] * k, ev[25] * k, ev[26] * k, ev[27] * k, ev[28] / (double)st.slots, ev[39] / (double)st.slots, ev[29] * k, ev[30] * k, ev[31] * k,
                    (unsigned long long)ev[36], (unsigned long long)ev[37]);
         }
         if (!txtrace.empty())
