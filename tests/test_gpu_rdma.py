@@ -203,3 +203,20 @@ def test_gpu_serial_flag():
     assert not bad, bad
     assert rdma_util.sum_counters([b.summary_line()]) == rdma_util.sum_counters([j[5] for j in sel])
     b.close()
+
+
+@pytest.mark.parametrize("team,hosts", [(0, 0), (1, 1), (1, 64), (3, 5), (28, 2), (40, 1), (104, 1), (16, 33)])
+def test_gpu_launch_shapes(team, hosts):
+    """Worlds of 16 and 128 hosts on teams where a switch takes a wave or a whole workgroup and a host
+    item 1 to 64 hosts (from a workspace of 100 frames a host down to one): every flow as in the
+    reference, PFC (serial slots) included."""
+    from twins_amd import rdma
+    by = {j[0]: j for j in rdma_util.jobs()}
+    for name in ("inc1_b1_cc1", "k8_incast16_b2_cc1", "k8_incast16_b2_cc3"):
+        _, topo, fl, kv, _, counters = by[name]
+        b = rdma.Batch([rdma.World(rdma_util.CONFIG, f"{rdma_util.INPUTS}/{topo}", f"{rdma_util.INPUTS}/{fl}", kv)],
+                       team_blocks=team, hosts_per_wave=hosts)
+        b.run()
+        assert b.fct_text(0) == rdma_util.ref_fct(name), name
+        assert rdma_util.sum_counters([b.summary_line()]) == rdma_util.sum_counters([counters]), name
+        b.close()

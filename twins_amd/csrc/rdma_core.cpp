@@ -925,44 +925,40 @@ extern "C" int trd_batch_run(trd_batch *b, trd_run_stats *st)
     int launches = 0;
     double kernel_s = 0;
     int64_t prev = -1;
-    // the launch shape: hosts per host item (fewer: less divergence among a wave's hosts, more
-    // waves), and one team size. Batches of up to 8 worlds take the fewest hosts per item (2, 4, 8
-    // or 16) whose items still fit a wave each of the largest team - 128 workgroups for a world
-    // alone, the GPU's share of each of up to 8 worlds (at least 32) - and a workgroup per item of
-    // the largest world up to that team. Measured with the slot barrier without cache fences:
-    // FatTree k=8 a2a50s (HPCC) alone 1.14, 0.80 and 0.70 s on 24 workgroups at 8 hosts per item, 64
-    // at 4 and 128 at 2; k8_perm 0.196 and 0.132 s on 24 at 8 and 96 at 2; Jellyfish a2a30 1.44 and
-    // 1.20 s on 12 at 8 and 96 at 2; FatTree k=16 a2a30 (DCQCN) 1.51 s on 112 at 8 and on 192 or 256
-    // alike; the 512-host leaf-spine (HPCC + DCQCN side by side) 1.27 s of kernel on 22 at 8 (a wave
-    // per item), 1.15 s on 48 at 4 and on 128 at 2. Larger batches: 64 hosts per item, teams of 16
-    // workgroups with a wave per item. As many teams as the GPU holds at once.
+    // The launch shape: one team size and hosts per host item. Every world that fits runs at once, each
+    // on its share of the GPU (worlds queued behind others leave it idle when few are left). A slot
+    // lasts as long as its longest item, and a wave runs unlike hosts one after another, so the fewest
+    // hosts per item (a power of two) of these: a switch a workgroup and four host items a workgroup,
+    // all side by side; else every item on a wave of its own; else every host item. Measured (kernel
+    // time): 24 FatTree k=8 worlds of 128 hosts (DCQCN, HPCC and DCTCP) 145 ms on teams of 16 at 64
+    // hosts per item (16 worlds at once), 88, 84 and 90 ms on teams of 10 at 2, 4 and 8 hosts; FatTree
+    // k=8 (HPCC) alone 104, 85 and 85 ms on 128 workgroups at 2 and 112 and 208 at 1; two 512-host
+    // leaf-spines 124, 107 and 121 ms on 128 workgroups each at 1, 2 and 4.
     const int cap = b->max_teams;
-    const bool small = b->W <= 8;
-    const int most = b->W == 1 ? std::min(128, cap) : small ? std::max(32, cap / b->W) : 16;
-    int hpw = b->hpw;
-    if (hpw <= 0)
-    {
-        hpw = small ? 2 : 64;
-        for (bool fits = false; small && !fits && hpw < 16;)
+    const int share = std::max(1, cap / b->W);
+    auto by_group = [&](int i, int h) { return b->ss[i] + ((b->hs[i] + h - 1) / h + 3) / 4; };
+    auto by_wave = [&](int i, int h) { return (b->hs[i] + h - 1) / h + b->ss[i]; };
+    const bool grouped = b->kmax <= rd::KS;
+    int T = b->team_blocks > 0 ? std::min(b->team_blocks, cap) : share, hpw = b->hpw;
+    for (int rule = grouped ? 0 : 1; hpw <= 0 && rule < 3; rule++)
+        for (int h = 1; hpw <= 0 && h <= 64; h *= 2)
         {
-            fits = true;
+            bool fits = true;
             for (int i = 0; i < b->W; i++)
-                fits = fits && (b->hs[i] + hpw - 1) / hpw + b->ss[i] <= most * 4;
-            if (!fits)
-                hpw *= 2;
+                fits = fits && (rule == 0 ? by_group(i, h) <= T : rule == 1 ? by_wave(i, h) <= 4 * T : (b->hs[i] + h - 1) / h <= 4 * T);
+            if (fits)
+                hpw = h;
         }
-    }
+    hpw = hpw > 0 ? hpw : 64;
     vector<int> items(b->W);
+    int most = 1;
     for (int i = 0; i < b->W; i++)
-        items[i] = (b->hs[i] + hpw - 1) / hpw + b->ss[i];
-    int T = b->team_blocks;
-    if (T <= 0)
     {
-        int mx = 1;
-        for (int v : items)
-            mx = std::max(mx, v);
-        T = std::min(most, small ? mx : (mx + 3) / 4);
+        items[i] = by_wave(i, hpw);
+        most = std::max(most, grouped ? by_group(i, hpw) : items[i]);
     }
+    if (b->team_blocks <= 0)
+        T = std::min(T, most);
     T = std::max(1, std::min(T, cap));
     // worlds by work items, largest first
     vector<int> order(b->W);
@@ -979,6 +975,7 @@ extern "C" int trd_batch_run(trd_batch *b, trd_run_stats *st)
         rd::LaunchCfg L = {};
         L.T = T;
         L.hpw = hpw;
+        L.by_group = grouped ? 3 : 0;
         L.nq = (int)queue.size();
         L.queue = b->queue_d;
         L.qnext = b->qnext_d;
