@@ -63,3 +63,25 @@ def test_gpu_batch_equals_standalone(tmp_path):
         assert b.counters(j)[25] == 0, name
         assert [(str(e), str(d)) for e, d in zip(est, done)] == exp, name
     b.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("runs", [9, 25])
+@pytest.mark.parametrize("team,hosts", [(0, 0), (52, 1), (1, 1), (3, 5), (1, 64), (16, 33)])
+def test_gpu_launch_shapes(team, hosts, runs):
+    """One host to a wave (the kernel whose hosts' branches are wave-uniform) and 5 to 64 (a lane
+    each, 100 staged frames a host down to none), on teams of few and many waves: loss and its
+    repair, sprayed reordering, FIN and a torus give ns-3's stored times."""
+    import twins_amd
+    pick = [c for c in CASES if c[0] in ("k8_incast16-cubic-fin", "k8_a2a30-newreno-spray", "torus6_a2a30-dctcp-base")]
+    assert len(pick) == 3
+    for name, fl, ref, args in pick:
+        print(f"case {name}", flush=True)
+        w = twins_amd.World([a.replace("topo/", util.GOLDEN + "/topo/") for a in args] + [f"--flows={util.GOLDEN}/{fl}"])
+        b = twins_amd.Batch([w], chain_runs=runs, team_blocks=team, hosts_per_wave=hosts)
+        assert b.run().worlds_done == 1
+        est, done = b.fct(0)
+        exp = util.read_cols(os.path.join(util.GOLDEN, ref), (4, 5))
+        if not b.counters(0)[25]:  # (no tie left undecided by chains of 9)
+            assert [(str(e), str(d)) for e, d in zip(est, done)] == exp, name
+        b.close()

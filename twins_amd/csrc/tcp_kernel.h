@@ -10,10 +10,11 @@ namespace tw
 constexpr double SERVER_WAIT_S = 600.0;
 // a launch of the persistent world-queue kernel: `blocks` workgroups of `threads` (their teams,
 // sizes and queues are the batch's TeamPlan); `teams` when a team has several workgroups (the
-// grid must then fit the GPU at once); each world runs at most slot_budget slots per launch
+// grid must then fit the GPU at once); `one` when every world has a wave for each of its work items
+// at one host per item (the kernel built for that); each world runs at most slot_budget slots per launch
 struct LaunchShape
 {
-    int blocks, threads, teams, pad;
+    int blocks, threads, teams, one;
     int64_t slot_budget;
 };
 // per chain length (tcp_kernel.hip is built once for 9 runs, once for 25)

@@ -24,16 +24,13 @@
 namespace tw
 {
 
-// per wave, for the item it runs: a switch item's rows, in_win, base, cnt, sort and route slots;
-// a host item's slots for the connection records of an event, one SndState, one RcvState and one
-// ConnStatic per lane. A wave runs its items one after another, so the two share one region.
-constexpr int LDS_SWITCH = Model<9>::SW_LDS_TOTAL;
-constexpr int LDS_SND = 0, LDS_RCV = LDS_SND + 64 * (int)(sizeof(SndState) / 4);
-constexpr int LDS_CONN = LDS_RCV + 64 * (int)(sizeof(RcvState) / 4);
-constexpr int LDS_RECORDS = LDS_CONN + 64 * (int)(sizeof(ConnStatic) / 4);
-constexpr int LDS_PER_WAVE = LDS_RECORDS > LDS_SWITCH ? LDS_RECORDS : LDS_SWITCH;
-static_assert(sizeof(SndState) % 128 == 0 && sizeof(RcvState) % 128 == 0 && sizeof(ConnStatic) % 16 == 0, "LDS record alignment");
-static_assert(4 * (size_t)LDS_PER_WAVE * 4 + 1024 <= 160 * 1024, "a 256-thread workgroup's LDS");
+// A wave's LDS, for the item it runs (one after another, so the items share it): a switch item's
+// rows, in_win, base, cnt, sort and route slots; a host item's slots for its hosts' first frames out,
+// an equal share each. Four waves take the CU's 160 KB but for the workgroup's own words.
+constexpr int WAVE_LDS = 40704; // bytes
+constexpr int LDS_PER_WAVE = WAVE_LDS / 4;
+static_assert(Model<9>::SW_LDS_TOTAL * 4 <= WAVE_LDS, "a wave's LDS");
+static_assert(4 * (size_t)WAVE_LDS + 512 <= 160 * 1024, "a 256-thread workgroup's LDS");
 constexpr unsigned long long WAIT_TICKS = 2000000000ull;  // a team-barrier wait gives up after 20 s (100 MHz clock)
 constexpr unsigned long long SERVER_MAX_WAIT = (unsigned long long)(SERVER_WAIT_S * 100e6); // (100 MHz clock)
 
@@ -51,10 +48,12 @@ __device__ __forceinline__ T *uniform_ptr(T *p)
 // (tcp_worlds_kernel), SRV = true takes requests from the serving loop's queues
 // (tcp_server_kernel). One body, specialised at compile time, so the batch kernel carries nothing
 // of the server's.
-template <int RUNS, bool SRV>
+// ONE: every world's host items are of one host (Model::U).
+template <int RUNS, bool SRV, bool ONE>
 __device__ __forceinline__ void world_loop(const BatchT<RUNS> *__restrict__ Bp, const ServerCtl *__restrict__ Sp, int64_t slot_budget)
 {
-    typedef Model<RUNS> Md;
+    typedef Model<RUNS, SRV> Md;
+    typedef Model<RUNS, SRV, ONE> Mh; // the hosts'
     extern __shared__ __attribute__((aligned(128))) int lds[];
     __shared__ int s_w;
     __shared__ int64_t s_t;
@@ -62,7 +61,7 @@ __device__ __forceinline__ void world_loop(const BatchT<RUNS> *__restrict__ Bp, 
     __shared__ unsigned s_act;
     __shared__ unsigned long long s_wake;
     __shared__ const BatchT<RUNS> *s_b;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, nwaves = blockDim.x >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = blockDim.x >> 6;
     const int32_t *team_of = SRV ? Sp->team_of : Bp->team_of;
     const TeamPlan *plans = SRV ? Sp->plan : Bp->plan;
     const int team = team_of[blockIdx.x] >> 8;
@@ -186,11 +185,13 @@ __device__ __forceinline__ void world_loop(const BatchT<RUNS> *__restrict__ Bp, 
         }
         // (the request's batch pointer made wave-uniform, so its fields load into scalar registers
         // as a kernel argument's do)
-        const BatchT<RUNS> &B = SRV ? *uniform_ptr(s_b) : *Bp;
-        const WorldDesc &W = B.worlds[w];
+        typename Md::Batch &B = *(typename Md::Batch *)(uint64_t)(SRV ? uniform_ptr(s_b) : Bp);
+        typename Md::World &W = *(typename Md::World *)(uint64_t)(B.worlds + __builtin_amdgcn_readfirstlane(w));
         int hpw = P.hpw, spw = 64 / W.k;
         if (hpw <= 0)
             slot_items(W.H, W.S, W.k, T * nwaves, &hpw, &spw);
+        if constexpr (ONE)
+            hpw = 1; // (the launch's condition; a constant for the compiler)
         WorldRun *R = B.run + w;
         const int k = W.k;
         const int host_items = (W.H + hpw - 1) / hpw, items = host_items + (W.S + spw - 1) / spw;
@@ -239,17 +240,35 @@ __device__ __forceinline__ void world_loop(const BatchT<RUNS> *__restrict__ Bp, 
             {
                 if (item < host_items)
                 {
-                    const int hl = item * hpw + lane;
+                    const int h0 = item * hpw, hl = h0 + lane;
 #ifdef TW_PROF
                     const unsigned long long q0 = wall_clock64();
 #endif
-                    if (lane < hpw && hl < W.H)
-                    {
-                        int64_t x = INT64_MAX;
-                        act += Md::host_step(B, W, R, hl, t, &x, (SndState *)(wl + LDS_SND) + lane, (RcvState *)(wl + LDS_RCV) + lane,
-                                             (ConnStatic *)(wl + LDS_CONN) + lane);
-                        wk = (unsigned long long)x < wk ? (unsigned long long)x : wk;
-                    }
+                    char *ws = reinterpret_cast<char *>(wl);
+                    constexpr int FR = (int)sizeof(typename Md::Frame);
+                    typename Md::HostIn in = {0, 0, 0, 0};
+                    int64_t x = INT64_MAX;
+                    const bool runs = lane < hpw && hl < W.H && Md::host_open(B, W, hl, t, in, &x);
+                    // The frames out, from a host's workspace to its link's message, `group` lanes at it: one
+                    // round of coherent stores, off the host's chain of events (a load after a frame's eight
+                    // 8-byte stores waits 0.4 us for them, 0.09 us without).
+                    auto send = [&](int host, const char *from, int frames, int first, int group) {
+                        const uint64_t *f = reinterpret_cast<const uint64_t *>(from);
+                        uint64_t TW_G *to = reinterpret_cast<uint64_t TW_G *>(B.msg + ((size_t)(t % NRING) * B.nlinks + W.link0 + host) * MAX_TX);
+                        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // (a wave's LDS accesses are in order)
+                        for (int i = first; i < frames * (FR / 8); i += group)
+                            coh_store(to + i, f[i]);
+                        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    };
+                    const int per = WAVE_LDS / hpw & ~15, group = 64 / hpw, mine = lane / group, src = mine < hpw ? mine : 0;
+                    int out_n = 0;
+                    if (runs)
+                        act += Mh::host_run(B, W, R, hl, t, &x, typename Mh::HostIn{in.in, in.i2, in.n2, in.n1},
+                                            (typename Mh::Frame *)(ws + lane * per), per / FR, &out_n);
+                    const int n = __shfl(out_n, src);
+                    send(h0 + src, ws + src * per, mine < hpw ? n : 0, lane % group, group);
+                    if ((unsigned long long)x < wk)
+                        wk = (unsigned long long)x;
 #ifdef TW_PROF
                     p_h += wall_clock64() - q0;
 #endif
@@ -350,10 +369,10 @@ __device__ __forceinline__ void world_loop(const BatchT<RUNS> *__restrict__ Bp, 
     }
 }
 
-template <int RUNS>
+template <int RUNS, bool ONE>
 __global__ void __launch_bounds__(256) tcp_worlds_kernel(const BatchT<RUNS> *__restrict__ Bp, int64_t slot_budget)
 {
-    world_loop<RUNS, false>(Bp, nullptr, slot_budget);
+    world_loop<RUNS, false, ONE>(Bp, nullptr, slot_budget);
 }
 
 // The serving loop's persistent kernel. Requests are single-world batches already in device
@@ -366,7 +385,7 @@ __global__ void __launch_bounds__(256) tcp_worlds_kernel(const BatchT<RUNS> *__r
 template <int RUNS>
 __global__ void __launch_bounds__(256) tcp_server_kernel(const ServerCtl *__restrict__ Sp)
 {
-    world_loop<RUNS, true>(nullptr, Sp, INT64_MAX);
+    world_loop<RUNS, true, false>(nullptr, Sp, INT64_MAX);
 }
 
 // This file is compiled once per chain length (TW_RUNS = 9 or 25, two objects built in parallel:
@@ -385,7 +404,10 @@ hipError_t TW_NAME(tcp_launch_, TW_RUNS)(const void *batch_dev, const LaunchShap
     // resource that one process can hold while another waits for it.
     const size_t lds = (size_t)(s.threads / 64) * LDS_PER_WAVE * sizeof(int);
     const BatchT<TW_RUNS> *b = reinterpret_cast<const BatchT<TW_RUNS> *>(batch_dev);
-    hipLaunchKernelGGL(tcp_worlds_kernel<TW_RUNS>, dim3(s.blocks), dim3(s.threads), lds, stream, b, s.slot_budget);
+    if (s.one)
+        hipLaunchKernelGGL((tcp_worlds_kernel<TW_RUNS, true>), dim3(s.blocks), dim3(s.threads), lds, stream, b, s.slot_budget);
+    else
+        hipLaunchKernelGGL((tcp_worlds_kernel<TW_RUNS, false>), dim3(s.blocks), dim3(s.threads), lds, stream, b, s.slot_budget);
     return hipGetLastError();
 }
 
@@ -400,7 +422,12 @@ hipError_t TW_NAME(tcp_server_launch_, TW_RUNS)(const void *ctl_dev, int blocks,
 hipError_t TW_NAME(tcp_max_blocks_, TW_RUNS)(int threads, int *per_cu)
 {
     const size_t lds = (size_t)(threads / 64) * LDS_PER_WAVE * sizeof(int);
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, tcp_worlds_kernel<TW_RUNS>, threads, lds);
+    // (the fewer of the two kernels')
+    int one = 0;
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&one, tcp_worlds_kernel<TW_RUNS, true>, threads, lds);
+    const hipError_t f = hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, tcp_worlds_kernel<TW_RUNS, false>, threads, lds);
+    *per_cu = one < *per_cu ? one : *per_cu;
+    return e != hipSuccess ? e : f;
 }
 
 #if TW_RUNS == 9

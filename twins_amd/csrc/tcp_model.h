@@ -22,10 +22,23 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
-template <int RUNS>
+// ONE: the host code for a wave that runs one host at a time on one lane. Every branch is then the
+// wave's, and U() says so: the compiler branches on a scalar instead of masking lanes in and out and
+// merging the masks at every join (a third of the host code's instructions, and as many as its
+// registers could not hold).
+template <int RUNS, bool SRV = false, bool ONE = false>
 struct Model
 {
-    typedef BatchT<RUNS> Batch;
+    static __device__ __forceinline__ bool U(bool c)
+    {
+#if defined(__HIP_DEVICE_COMPILE__)
+        if constexpr (ONE)
+            return __builtin_amdgcn_ballot_w64(c) != 0;
+#endif
+        return c;
+    }
+    typedef typename ReadOnly<BatchT<RUNS>, SRV>::type Batch; // (const)
+    typedef typename ReadOnly<WorldDesc, SRV>::type World;    // (const)
     typedef FrameT<RUNS> Frame;
     static constexpr int CW = RUNS + 1; // a chain's words: RUNS runs (code | count << 16), the root
     struct Chain
@@ -74,10 +87,10 @@ struct Model
     static __device__ __forceinline__ void chain_child(Chain &dst, uint32_t code, const Chain &parent)
     {
         const Chain p = parent;
-        if ((p.r[0] & 0xFFFF) == code)
+        if (U((p.r[0] & 0xFFFF) == code))
         {
             dst = p;
-            if ((p.r[0] >> 16) < 0xFFFF)
+            if (U((p.r[0] >> 16) < 0xFFFF))
                 dst.r[0] += 1u << 16;
             return;
         }
@@ -99,32 +112,32 @@ struct Model
         for (;;)
         {
             uint32_t ca = a(ia) & 0xFFFF, cb = b(ib) & 0xFFFF;
-            if (ca == 0 && cb != 0 && (a(RUNS) & 0xFFFF) != 0)
+            if (U(ca == 0 && cb != 0 && (a(RUNS) & 0xFFFF) != 0))
                 return -1;
-            if (cb == 0 && ca != 0 && (b(RUNS) & 0xFFFF) != 0)
+            if (U(cb == 0 && ca != 0 && (b(RUNS) & 0xFFFF) != 0))
                 return 1;
-            if (ca == 0 || cb == 0)
+            if (U(ca == 0 || cb == 0))
                 break;
-            if (ca != cb)
+            if (U(ca != cb))
                 return ca > cb ? -1 : 1;
             uint32_t m = ra < rb ? ra : rb;
             ra -= m;
             rb -= m;
-            if (ra == 0)
+            if (U(ra == 0))
             {
-                if (++ia == RUNS)
+                if (U(++ia == RUNS))
                     break;
                 ra = a(ia) >> 16;
             }
-            if (rb == 0)
+            if (U(rb == 0))
             {
-                if (++ib == RUNS)
+                if (U(++ib == RUNS))
                     break;
                 rb = b(ib) >> 16;
             }
         }
         uint32_t xa = a(RUNS) << 16 | a(RUNS) >> 16, xb = b(RUNS) << 16 | b(RUNS) >> 16; // the root keys
-        if (xa == 0 || xb == 0 || xa == xb)
+        if (U(xa == 0 || xb == 0 || xa == xb))
             return 0;
         return xa < xb ? -1 : 1;
     }
@@ -158,21 +171,28 @@ struct Model
     // queue-disc length ns-3 would see (src/step.cuh:167-317 restates the same rules).
     struct Fifo
     {
-        const Batch *B;
+        Batch *B;
+        World *W;
         WorldRun *R;
-        int lid;
+        int lid, rt;
         Frame *ring;
         int cap, head, size, red_k, limit, sent, early;
         int64_t link_free, last_start, woke, idle_start, slot_end;
-        int64_t head_ts; // the first queued frame's enqueue time (while size > 0)
         Chain last; // the chain of the transmission in progress (kept in registers for the slot)
+        Frame hd;   // the first queued frame (while size > 0); not yet in the ring if hd_new
+        bool hd_new;
         Frame *out;
+        // the slot's first frames out wait in the workspace (LDS), if the entity has one
+        Frame *stage;
+        int stage_cap;
 
-        __device__ __forceinline__ void load(const Batch &b, WorldRun *r, int link, int64_t t, int ring_t)
+        __device__ __forceinline__ void load(Batch &b, World &w, WorldRun *r, int link, int64_t t, int ring_t, Frame *st = nullptr, int st_cap = 0)
         {
             B = &b;
+            W = &w;
             R = r;
             lid = link;
+            rt = ring_t;
             ring = b.qring + b.q_base[link];
             cap = b.q_cap[link];
             head = b.q_head[link];
@@ -185,40 +205,77 @@ struct Model
             woke = idle_start = -1;
             slot_end = (t + 1) * SLOT_PS;
             sent = early = 0;
-            head_ts = size > 0 ? ring[head].ts : 0;
+            hd_new = false;
+            if (U(size > 0))
+                hd = ring[head];
             out = b.msg + ((size_t)ring_t * b.nlinks + link) * MAX_TX;
+            stage = st;
+            stage_cap = st_cap;
         }
         // the slot's message count word (msg_word) and the queue back to memory
         __device__ __forceinline__ void store(int64_t t, int ring_t)
         {
             coh_store(B->msg_cnt + (size_t)ring_t * B->nlinks + lid, msg_word(t, early, sent));
+            if (U(size > 0 && hd_new))
+                ring[head] = hd;
             B->q_head[lid] = head;
             B->q_size[lid] = size;
             B->q_link_free[lid] = link_free;
             B->q_last_start[lid] = last_start;
             chain_store(B->q_last_chain + (size_t)lid * CW, last);
-            if (sent)
+            if (U(sent))
                 count(R, EV_PKT_EVENTS, (unsigned long long)sent);
+        }
+        // frame i of the slot's message: into the workspace, or out device-coherently, 16 bytes a store
+        // (the world's messages of a slot lie within the 2^31 bytes a buffer store reaches)
+        __device__ __forceinline__ void put(int i, const Frame &o)
+        {
+            if (U(i < stage_cap))
+            {
+                stage[i] = o;
+                return;
+            }
+#if defined(__HIP_DEVICE_COMPILE__)
+            const uint64_t bytes = (uint64_t)W->L * MAX_TX * sizeof(Frame);
+            if (U(bytes <= 0x7FFFFFF0ull))
+            {
+                const __amdgpu_buffer_rsrc_t r = twc::coh_buffer((const void *)(B->msg + ((size_t)rt * B->nlinks + W->link0) * MAX_TX), (uint32_t)bytes);
+                const uint32_t at = ((uint32_t)(lid - W->link0) * MAX_TX + (uint32_t)i) * (uint32_t)sizeof(Frame);
+                uint64_t w[sizeof(Frame) / 8];
+                __builtin_memcpy(w, &o, sizeof o);
+#pragma unroll
+                for (int k = 0; k < (int)(sizeof(Frame) / 16); k++)
+                    twc::coh_store16(r, at + 16 * k, w[2 * k], w[2 * k + 1]);
+                return;
+            }
+#endif
+            coh_put(out + i, o); // (read by the link's far end in a later slot)
         }
         // Starts, in order, the frames whose transmission begins by `until` within the slot. The
         // event that starts a frame is the previous frame's TransmitComplete when the frame had
         // to wait for the link (its chain: the last transmission's, one more run), else the
         // frame's own enqueue (a link that never sent counts as idle).
+        // (Vector memory counts in order: a load waits for the stores issued before it. So the first
+        // queued frame is in registers, a frame queued and sent while it was first passes through no
+        // memory, and the next one's load is issued before the sent one's stores.)
         __device__ void advance(int64_t until)
         {
-            while (size > 0)
+            while (U(size > 0))
             {
-                if (sent >= MAX_TX)
+                if (U(sent >= MAX_TX))
                 {
                     count(R, EV_TXCAP);
                     return;
                 }
-                // (the head's time is kept in a register, so a call that starts nothing reads no frame)
-                const int64_t start = head_ts > link_free ? head_ts : link_free;
-                if (start >= slot_end || start > until)
+                const int64_t start = hd.ts > link_free ? hd.ts : link_free;
+                if (U(start >= slot_end || start > until))
                     return;
-                Frame o = ring[head];
-                if (head_ts <= link_free && link_free > last_start)
+                Frame o = hd;
+                head = head + 1 < cap ? head + 1 : 0;
+                hd_new = false;
+                if (U(--size > 0))
+                    hd = ring[head];
+                if (U(o.ts <= link_free && link_free > last_start))
                 {
                     chain_child(last, (uint32_t)((link_free - last_start) / PS_PER_BYTE), last);
                     chain_store(o.chain, last);
@@ -232,18 +289,15 @@ struct Model
                 link_free = start + (int64_t)o.len * PS_PER_BYTE;
                 o.ts = link_free + PROP_PS; // its arrival at the far end
                 early += o.ts < slot_end + SLOT_PS;
-                coh_put(out + sent, o); // (read by the link's far end in a later slot)
+                put(sent, o);
                 sent++;
-                head = head + 1 < cap ? head + 1 : 0;
-                if (--size > 0)
-                    head_ts = ring[head].ts;
             }
         }
         // a queue-trace record (src/step.cuh:266-279), stored field by field (no record on the stack)
         __device__ __forceinline__ void trace(int64_t now, int qlen, uint32_t flow, uint32_t sa, uint16_t len, uint8_t flags, uint8_t to_sender)
         {
             const unsigned long long i = atomicAdd(B->qt.cnt, 1ull);
-            if (i < B->qt.cap)
+            if (U(i < B->qt.cap))
             {
                 QRec *r = B->qt.rec + i;
                 r->ts = now;
@@ -265,50 +319,74 @@ struct Model
             const bool pulled = last_start < now || (woke == now && idle_start == now);
             return size > 0 && link_free > now && pulled ? size - 1 : size;
         }
-        // a frame offered at `now`: RED marks (ECN-capable) or drops it at K, the queue limit
-        // drops it; false if dropped
+        // a frame offered at `now`, to which the queue has advanced: RED marks (ECN-capable) or drops it
+        // at K, the queue limit drops it; false if dropped
         __device__ bool enqueue(const Frame &f, int64_t now)
         {
-            advance(now);
             const int len = qdisc_len(now);
             Frame g = f;
             g.ts = now;
             const bool over_k = len >= red_k && len > 1;
-            if (over_k && !(g.flags & F_ECT))
+            if (U(over_k && !(g.flags & F_ECT)))
             {
                 count(R, EV_DROP);
                 return false;
             }
-            if (over_k)
+            if (U(over_k))
             {
                 g.flags |= F_CE;
                 count(R, EV_MARK);
             }
-            if (len >= limit)
+            if (U(len >= limit))
             {
                 count(R, EV_DROP);
                 return false;
             }
-            if (B->qt.rec && now >= B->qt.from && now < B->qt.until)
+            if (U(B->qt.rec && now >= B->qt.from && now < B->qt.until))
                 trace(now, len + 1, g.flow, g.sa, g.len, g.flags, g.to_sender);
-            if (size >= cap)
+            if (U(size >= cap))
             {
                 count(R, EV_RING_OVF);
                 return false;
             }
-            const int at = head + size < cap ? head + size : head + size - cap;
-            ring[at] = g;
-            if (size++ == 0)
-                head_ts = g.ts;
+            if (U(size == 0))
+            {
+                hd = g;
+                hd_new = true;
+            }
+            else
+                ring[head + size < cap ? head + size : head + size - cap] = g;
+            size++;
             return true;
         }
     };
 
     // -------------------------------------------------------------- host context
+    // a frame an event asks for: its sequence or acknowledgement number, length, flags and direction
+    struct Out
+    {
+        uint32_t sa;
+        uint16_t len;
+        uint8_t flags, to_sender;
+    };
+    // what the events of a connection's sending (receiving) side use of its static record; way: its
+    // frames' destination and equal-cost index
+    struct ConnSnd
+    {
+        uint64_t it_off;
+        uint32_t it_cap, way;
+        int32_t m_first, m_cnt;
+        bool fin_on;
+    };
+    struct ConnRcv
+    {
+        uint64_t oo_off;
+        uint32_t oo_cap, way;
+    };
     struct Host
     {
-        const Batch *B;
-        const WorldDesc *W;
+        Batch *B;
+        World *W;
         WorldRun *R;
         Fifo nic;
         int h, hl; // global, world-local
@@ -318,72 +396,109 @@ struct Model
         int nd, id;
         int64_t due_head; // due[id].at (INT64_MAX when none is left): the next timer of the slot
         int64_t slot_end;
-        // the records of the connection side an event works on, copied into this lane's LDS
-        // slots for the event (snd_open / rcv_open) and written back once at its end
-        SndState *ls;
-        RcvState *lr;
-        ConnStatic *lc; // the event's connection's static record, copied with its side's record
-#ifndef __HIP_DEVICE_COMPILE__
-        int lc_flow = -1; // (CPU builds: which connection lc holds, checked by conn())
-#endif
+        // The records of the connection sides that events work on, in registers: one sending side and one
+        // receiving side (sf, rf: whose; -1: none), each with its connection's static record. A record is
+        // read when its first event of the slot runs and written back when another connection's event
+        // or the slot's end comes. (In LDS an event made some 160 accesses to them, 28 ns each when the
+        // next waits for it.)
+        SndState S;
+        RcvState Q;
+        ConnSnd cs;
+        ConnRcv cr;
+        int sf, rf;
+        uint32_t max_it; // the longest sent ledger of the slot
+        // What the running event sends, queued after its handler by the one place that builds frames
+        // (host_step's loop): the frames asked for (at most 4: an ACK at a CE edge, one for the data,
+        // the close's; or one segment sent again), then, if fill, segments while the window has room,
+        // then one more asked for after that.
+        Out ask[4], post;
+        int n_ask, i_ask, fill_n;
+        int f;        // the running event's connection
+        uint32_t way; // where its frames go: the host (world-local) and, above it, the equal-cost index
+        bool fill, has_post;
     };
-    // an event on connection f's sending (receiving) side: its record from device memory into
-    // the lane's LDS slot, and back when the event ends (a record is 16 (8) independent 16-byte
-    // loads, issued together, instead of a dependent load per field use)
-    // (dst and src: one record type, in LDS and in device memory, either way round)
-    template <typename D, typename S>
-    static __device__ __forceinline__ void rec_move(D *dst, const S *src)
+    // A record between registers and device memory: words of 4 or 8 bytes as its fields lie (adjacent
+    // ones become 16-byte accesses, issued together)
+    typedef uint32_t __attribute__((may_alias)) word4;
+    typedef uint64_t __attribute__((may_alias)) word8;
+    template <typename W, int FROM, int TO, typename D, typename S>
+    static __device__ __forceinline__ void words(D *dst, const S *src)
     {
-        static_assert(sizeof(D) == sizeof(S) && sizeof(D) % 16 == 0, "records move in 16-byte pieces");
 #pragma unroll
-        for (int i = 0; i < (int)(sizeof(D) / 16); i++)
-            reinterpret_cast<uint4 *>(dst)[i] = reinterpret_cast<const uint4 *>(src)[i];
+        for (int i = FROM / (int)sizeof(W); i < TO / (int)sizeof(W); i++)
+            reinterpret_cast<W *>(dst)[i] = reinterpret_cast<const W *>(src)[i];
     }
-    // the static record comes along with either side's record (its loads issued with the record's)
-    static __device__ __forceinline__ void conn_open(Host &x, int f)
+    static_assert(offsetof(SndState, srtt) == 120 && offsetof(SndState, cub_cnt) == 192 && offsetof(SndState, cub_k) == 224 &&
+                      offsetof(RcvState, r_fin) == 32 && offsetof(RcvState, ecn_ce_seq) == 96,
+                  "the records' words");
+    // (a sender's Cubic state stays in memory: only Cubic's worlds look at it)
+    template <typename D, typename S>
+    static __device__ __forceinline__ void snd_move(D *dst, const S *src)
     {
-        rec_move(x.lc, &x.B->cs[f]);
-#ifndef __HIP_DEVICE_COMPILE__
-        x.lc_flow = f;
-#endif
+        words<word4, 0, 120>(dst, src);
+        words<word8, 120, 192>(dst, src);
     }
-    // the open connection's static record (connection f's: an event works on one connection)
-    static __device__ __forceinline__ const ConnStatic &conn(const Host &x, int f)
+    template <typename D, typename S>
+    static __device__ __forceinline__ void rcv_move(D *dst, const S *src)
     {
-#ifndef __HIP_DEVICE_COMPILE__
-        assert(x.lc_flow == f);
-#endif
-        return *x.lc;
+        words<word4, 0, 32>(dst, src);
+        words<word8, 32, 104>(dst, src);
     }
-    static __device__ __forceinline__ SndState &snd_open(Host &x, int f)
+    static __device__ __forceinline__ uint32_t way_to(const Host &x, int host, uint32_t hash)
     {
-        rec_move(x.ls, &x.B->snd[f]);
-        conn_open(x, f);
-        return *x.ls;
+        return (uint32_t)(uint16_t)(host - x.W->host0) | (hash % (uint32_t)x.W->ecmp_n & 0xFF) << 16;
     }
     // The receiver's host reads a sender's end state (compact_rcv): the 4-byte word holding
     // SndState::st goes out device-coherently once the sender is done.
     static constexpr size_t ST_WORD = offsetof(SndState, st) & ~(size_t)3;
     static constexpr int ST_SHIFT = (int)(offsetof(SndState, st) & 3) * 8;
-    static __device__ __forceinline__ void snd_close(Host &x, int f)
+    static __device__ __forceinline__ void snd_flush(Host &x)
     {
-        rec_move(&x.B->snd[f], x.ls);
-        if (x.ls->st == S_DONE)
-            coh_store(reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(&x.B->snd[f]) + ST_WORD),
-                      *reinterpret_cast<const uint32_t *>(reinterpret_cast<const char *>(x.ls) + ST_WORD));
+        if (U(x.sf < 0))
+            return;
+        snd_move(&x.B->snd[x.sf], &x.S);
+        if (U(x.S.st == S_DONE))
+            coh_store(reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(&x.B->snd[x.sf]) + ST_WORD),
+                      *reinterpret_cast<const word4 *>(reinterpret_cast<const char *>(&x.S) + ST_WORD));
     }
-    static __device__ __forceinline__ bool snd_done_seen(const Batch &B, int f)
+    static __device__ __forceinline__ void rcv_flush(Host &x)
+    {
+        if (U(x.rf >= 0))
+            rcv_move(&x.B->rcv[x.rf], &x.Q);
+    }
+    static __device__ __forceinline__ SndState &snd_open(Host &x, int f)
+    {
+        if (U(x.sf != f))
+        {
+            snd_flush(x);
+            snd_move(&x.S, &x.B->snd[f]);
+            const ConnStatic TW_G &c = x.B->cs[f];
+            x.cs = ConnSnd{c.it_off, c.it_cap, way_to(x, c.dst, c.hash_data), c.m_first, c.m_cnt, c.fin_on != 0};
+            x.sf = f;
+        }
+        x.f = f;
+        x.way = x.cs.way;
+        return x.S;
+    }
+    static __device__ __forceinline__ bool snd_done_seen(Batch &B, int f)
     {
         const uint32_t w = coh_load(reinterpret_cast<const uint32_t *>(reinterpret_cast<const char *>(&B.snd[f]) + ST_WORD));
         return (uint8_t)(w >> ST_SHIFT) == S_DONE;
     }
     static __device__ __forceinline__ RcvState &rcv_open(Host &x, int f)
     {
-        rec_move(x.lr, &x.B->rcv[f]);
-        conn_open(x, f);
-        return *x.lr;
+        if (U(x.rf != f))
+        {
+            rcv_flush(x);
+            rcv_move(&x.Q, &x.B->rcv[f]);
+            const ConnStatic TW_G &c = x.B->cs[f];
+            x.cr = ConnRcv{c.oo_off, c.oo_cap, way_to(x, c.src, c.hash_ack)};
+            x.rf = f;
+        }
+        x.f = f;
+        x.way = x.cr.way;
+        return x.Q;
     }
-    static __device__ __forceinline__ void rcv_close(Host &x, int f) { rec_move(&x.B->rcv[f], x.lr); }
 
     // Active lists: a host's sending and receiving connections. A connection leaves its list at
     // the end of a slot in which it is finished (sender: closed; receiver: the sender closed and
@@ -393,19 +508,19 @@ struct Model
     // (Both walk their list COMPACT_RUN entries at a time: the entries' records are all read
     // before any entry is written back, so the reads of a run are in flight together.)
     static constexpr int COMPACT_RUN = 4;
-    static __device__ __forceinline__ int64_t compact_snd(const Batch &B, int h)
+    static __device__ __forceinline__ int64_t compact_snd(Batch &B, int h)
     {
         int64_t next = INT64_MAX;
         int32_t *l = B.act_snd + (size_t)h * MAX_ACTIVE;
         int k = 0, n = B.n_snd[h];
-        for (int i0 = 0; i0 < n; i0 += COMPACT_RUN)
+        for (int i0 = 0; U(i0 < n); i0 += COMPACT_RUN)
         {
             int f[COMPACT_RUN];
             bool done[COMPACT_RUN];
             int64_t rto[COMPACT_RUN], syn[COMPACT_RUN];
 #pragma unroll
             for (int j = 0; j < COMPACT_RUN; j++)
-                if (i0 + j < n)
+                if (U(i0 + j < n))
                 {
                     f[j] = l[i0 + j];
                     const SndState &s = B.snd[f[j]];
@@ -415,31 +530,31 @@ struct Model
                 }
 #pragma unroll
             for (int j = 0; j < COMPACT_RUN; j++)
-                if (i0 + j < n && !done[j])
+                if (U(i0 + j < n && !done[j]))
                 {
                     l[k++] = f[j];
-                    if (rto[j] >= 0 && rto[j] < next)
+                    if (U(rto[j] >= 0 && rto[j] < next))
                         next = rto[j];
-                    if (syn[j] >= 0 && syn[j] < next)
+                    if (U(syn[j] >= 0 && syn[j] < next))
                         next = syn[j];
                 }
         }
         B.n_snd[h] = k;
         return next;
     }
-    static __device__ __forceinline__ int64_t compact_rcv(const Batch &B, int h)
+    static __device__ __forceinline__ int64_t compact_rcv(Batch &B, int h)
     {
         int64_t next = INT64_MAX;
         int32_t *l = B.act_rcv + (size_t)h * MAX_ACTIVE;
         int k = 0, n = B.n_rcv[h];
-        for (int i0 = 0; i0 < n; i0 += COMPACT_RUN)
+        for (int i0 = 0; U(i0 < n); i0 += COMPACT_RUN)
         {
             int f[COMPACT_RUN];
             bool gone[COMPACT_RUN];
             int64_t tmin[COMPACT_RUN];
 #pragma unroll
             for (int j = 0; j < COMPACT_RUN; j++)
-                if (i0 + j < n)
+                if (U(i0 + j < n))
                 {
                     f[j] = l[i0 + j];
                     const RcvState &r = B.rcv[f[j]];
@@ -448,12 +563,12 @@ struct Model
                     tmin[j] = INT64_MAX;
 #pragma unroll
                     for (int q = 0; q < 4; q++)
-                        if (v[q] >= 0 && v[q] < tmin[j])
+                        if (U(v[q] >= 0 && v[q] < tmin[j]))
                             tmin[j] = v[q];
                 }
 #pragma unroll
             for (int j = 0; j < COMPACT_RUN; j++)
-                if (i0 + j < n && !gone[j])
+                if (U(i0 + j < n && !gone[j]))
                 {
                     l[k++] = f[j];
                     next = tmin[j] < next ? tmin[j] : next;
@@ -465,22 +580,22 @@ struct Model
 
     static __device__ void due_insert(Host &x, int64_t at, int f, int kind)
     {
-        if (at >= x.slot_end)
+        if (U(at >= x.slot_end))
             return;
-        if (x.nd >= MAX_DUE)
+        if (U(x.nd >= MAX_DUE))
         {
             count(x.R, EV_DUE_OVF);
             return;
         }
         int j = x.nd;
-        while (j > x.id && x.due[j - 1].at > at)
+        while (U(j > x.id && x.due[j - 1].at > at))
         {
             x.due[j] = x.due[j - 1];
             j--;
         }
         x.due[j] = {at, f, kind};
         x.nd++;
-        if (j == x.id)
+        if (U(j == x.id))
             x.due_head = at;
     }
     static __device__ __forceinline__ void timer_chain(Host &x, uint32_t *base, int f, int64_t lead)
@@ -489,21 +604,61 @@ struct Model
         chain_child(c, code_lead(lead), x.echain);
         chain_store(base + (size_t)f * CW, c);
     }
-    static __device__ void emit(Host &x, int f, uint8_t flags, uint32_t seq, uint32_t ack, uint16_t len, bool to_sender, int64_t now)
+    static __device__ __forceinline__ Out out_of(uint8_t flags, uint32_t seq, uint32_t ack, uint16_t len, bool to_sender)
     {
-        const ConnStatic &cs = conn(x, f);
+        return Out{(flags & F_DATA) ? seq : ack, len, flags, (uint8_t)(to_sender ? 1 : 0)};
+    }
+    static __device__ __forceinline__ void emit(Host &x, int f, uint8_t flags, uint32_t seq, uint32_t ack, uint16_t len, bool to_sender, int64_t now)
+    {
+        const Out o = out_of(flags, seq, ack, len, to_sender);
+        if (U(x.fill))
+        {
+            x.post = o;
+            x.has_post = true;
+            return;
+        }
+        const int n = x.n_ask++;
+#pragma unroll
+        for (int i = 0; i < 4; i++) // (static places: registers)
+            if (i == n)
+                x.ask[i] = o;
+    }
+    // the frame of what the running event sends, with the event's chain
+    static __device__ __forceinline__ Frame frame_of(const Host &x, const Out &o, int64_t now)
+    {
         Frame fr;
         fr.ts = now;
-        fr.flow = (uint32_t)f;
-        fr.sa = (flags & F_DATA) ? seq : ack;
-        fr.len = len;
-        fr.dst = (uint16_t)((to_sender ? cs.src : cs.dst) - x.W->host0);
-        fr.flags = flags | (x.dctcp ? F_ECT : 0);
-        fr.to_sender = to_sender ? 1 : 0;
-        fr.up = (uint8_t)((to_sender ? cs.hash_ack : cs.hash_data) % (uint32_t)x.W->ecmp_n);
+        fr.flow = (uint32_t)x.f;
+        fr.sa = o.sa;
+        fr.len = o.len;
+        fr.dst = (uint16_t)x.way; // (a side's frames all go one way)
+        fr.flags = o.flags | (x.dctcp ? F_ECT : 0);
+        fr.to_sender = o.to_sender;
+        fr.up = (uint8_t)(x.way >> 16);
         fr.pad = 0;
         chain_store(fr.chain, x.echain);
-        x.nic.enqueue(fr, now);
+        return fr;
+    }
+    // the next of it; false: all is out
+    static __device__ __forceinline__ bool next_out(Host &x, int64_t now, Out *o)
+    {
+        if (U(x.i_ask < x.n_ask))
+        {
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                if (i == x.i_ask)
+                    *o = x.ask[i];
+            x.i_ask++;
+            return true;
+        }
+        if (U(x.fill && fill_next(x, x.f, now, o)))
+            return true;
+        x.fill = false;
+        if (U(!x.has_post))
+            return false;
+        *o = x.post;
+        x.has_post = false;
+        return true;
     }
 
     // -------------------------------------------------------------- the sent ledger
@@ -516,73 +671,70 @@ struct Model
     struct Ledger
     {
         SndState &s;
-        uint32_t TW_G *first;
-        uint8_t TW_G *marks;
+        SentEntry TW_G *ring;
         uint32_t cap;
-        __device__ Ledger(const Batch &B, SndState &rec, const ConnStatic &c) : s(rec)
+        __device__ __forceinline__ Ledger(Host &x) : s(x.S)
         {
-            first = B.it_start + c.it_off;
-            marks = B.it_fl + c.it_off;
-            cap = c.it_cap;
+            ring = x.B->it + x.cs.it_off;
+            cap = x.cs.it_cap;
         }
-        __device__ uint32_t pos(uint32_t i) const { return s.it_head + i < cap ? s.it_head + i : s.it_head + i - cap; }
-        __device__ uint32_t lo(uint32_t i) const { return first[pos(i)]; }
-        __device__ uint32_t hi(uint32_t i) const { return i + 1 < s.it_n ? first[pos(i + 1)] : s.high; }
-        __device__ uint8_t mk(uint32_t i) const { return marks[pos(i)]; }
+        __device__ __forceinline__ uint32_t pos(uint32_t i) const { return s.it_head + i < cap ? s.it_head + i : s.it_head + i - cap; }
+        __device__ __forceinline__ SentEntry at(uint32_t i) const { return ring[pos(i)]; }
+        __device__ __forceinline__ uint32_t lo(uint32_t i) const { return ring[pos(i)].first; }
+        __device__ __forceinline__ uint32_t hi(uint32_t i) const { return i + 1 < s.it_n ? ring[pos(i + 1)].first : s.high; }
+        __device__ __forceinline__ uint8_t mk(uint32_t i) const { return (uint8_t)ring[pos(i)].mark; }
     };
     static __device__ __forceinline__ bool lg_candidate(uint8_t m) { return (m & (IT_LOST | IT_RETX | IT_SACKED)) == IT_LOST; }
     // adds (sign 1) or removes (sign -1) an entry of `len` bytes with marks m from the totals
     static __device__ __forceinline__ void lg_count(SndState &s, uint8_t m, uint32_t len, int sign)
     {
         const uint32_t d = sign > 0 ? len : 0u - len, one = sign > 0 ? 1u : 0u - 1u;
-        if (m & IT_SACKED)
+        if (U(m & IT_SACKED))
         {
             s.sack_b += d;
             s.sacked_n += one;
         }
-        if (m & IT_LOST)
+        if (U(m & IT_LOST))
             s.lost_b += d;
-        if (m & IT_RETX)
+        if (U(m & IT_RETX))
             s.rtx_b += d;
-        if (lg_candidate(m))
+        if (U(lg_candidate(m)))
             s.cand_n += one;
     }
     // entry i's marks become m
     static __device__ void lg_remark(Ledger &L, uint32_t i, uint8_t m)
     {
         const uint32_t k = L.pos(i);
-        const uint8_t was = L.marks[k];
-        if (was == m)
+        const uint8_t was = (uint8_t)L.ring[k].mark;
+        if (U(was == m))
             return;
-        const uint32_t len = L.hi(i) - L.first[k];
+        const uint32_t len = L.hi(i) - L.ring[k].first;
         lg_count(L.s, was, len, -1);
         lg_count(L.s, m, len, 1);
-        if (lg_candidate(m) && !lg_candidate(was) && i < L.s.cand)
+        if (U(lg_candidate(m) && !lg_candidate(was) && i < L.s.cand))
             L.s.cand = i;
-        L.marks[k] = m;
+        L.ring[k].mark = m;
     }
     // a new entry at place i (the entries from i on move up one); its bytes were counted before
     // (a split) or are new (unmarked); false if the ring is full
     static __device__ bool lg_insert(Ledger &L, WorldRun *R, uint32_t i, uint32_t start, uint8_t m)
     {
         SndState &s = L.s;
-        if (s.it_n >= L.cap)
+        if (U(s.it_n >= L.cap))
         {
             count(R, EV_RTT_OVF);
             return false;
         }
-        for (uint32_t j = s.it_n; j > i; j--)
+        for (uint32_t j = s.it_n; U(j > i); j--)
         {
             const uint32_t to = L.pos(j), from = L.pos(j - 1);
-            L.first[to] = L.first[from];
-            L.marks[to] = L.marks[from];
+            L.ring[to] = L.ring[from];
         }
-        L.first[L.pos(i)] = start;
-        L.marks[L.pos(i)] = m;
+        L.ring[L.pos(i)] = SentEntry{start, m};
         s.it_n++;
-        if (s.cand > 0 && s.cand >= i)
+        if (U(s.cand > 0 && s.cand >= i))
             s.cand++;
-        if (lg_candidate(m))
+        if (U(lg_candidate(m)))
         {
             s.cand_n++;
             s.cand = i < s.cand ? i : s.cand;
@@ -593,24 +745,23 @@ struct Model
     static __device__ void lg_erase(Ledger &L, uint32_t i)
     {
         SndState &s = L.s;
-        for (uint32_t j = i + 1; j < s.it_n; j++)
+        for (uint32_t j = i + 1; U(j < s.it_n); j++)
         {
             const uint32_t to = L.pos(j - 1), from = L.pos(j);
-            L.first[to] = L.first[from];
-            L.marks[to] = L.marks[from];
+            L.ring[to] = L.ring[from];
         }
         s.it_n--;
-        if (s.cand > i)
+        if (U(s.cand > i))
             s.cand--;
     }
     // the first entry starting at or after seq
     static __device__ uint32_t lg_find(const Ledger &L, uint32_t seq)
     {
         uint32_t a = 0, b = L.s.it_n;
-        while (a < b)
+        while (U(a < b))
         {
             const uint32_t m = (a + b) / 2;
-            if (L.lo(m) < seq)
+            if (U(L.lo(m) < seq))
                 a = m + 1;
             else
                 b = m;
@@ -626,8 +777,8 @@ struct Model
     {
         SndState &s = L.s;
         uint32_t i = s.sacked_n + 1;
-        for (; i < s.it_n; i++)
-            if (!(L.mk(i) & IT_SACKED))
+        for (; U(i < s.it_n); i++)
+            if (U(!(L.mk(i) & IT_SACKED)))
             {
                 lg_remark(L, i, L.mk(i) | IT_SACKED);
                 s.sack_seen = 1;
@@ -638,15 +789,15 @@ struct Model
     // the oldest entry lost (and no longer sacked or retransmitted)
     static __device__ void lg_head_lost(Ledger &L)
     {
-        if (L.s.it_n)
+        if (U(L.s.it_n))
             lg_remark(L, 0, (uint8_t)(IT_LOST | (L.mk(0) & ~(IT_SACKED | IT_RETX))));
     }
     // a retransmission timeout: every entry lost, nothing sacked or retransmitted
     static __device__ void lg_all_lost(Ledger &L)
     {
         SndState &s = L.s;
-        for (uint32_t i = 0; i < s.it_n; i++)
-            L.marks[L.pos(i)] = IT_LOST;
+        for (uint32_t i = 0; U(i < s.it_n); i++)
+            L.ring[L.pos(i)].mark = IT_LOST;
         s.lost_b = lg_sent(s);
         s.sack_b = s.rtx_b = 0;
         s.sacked_n = 0;
@@ -657,44 +808,51 @@ struct Model
     }
     // the bytes up to ack are acknowledged (DiscardUpTo): entries wholly below it leave, one cut by
     // it starts there; returns the bytes of the entries that left
-    static __device__ uint32_t lg_release(Ledger &L, uint32_t ack)
+    // (pre: the first LG_PRE entries, read together before they are needed: one after another each was
+    // a wait of its own)
+    static constexpr int LG_PRE = 4;
+    static __device__ uint32_t lg_release(Ledger &L, uint32_t ack, const SentEntry *pre)
     {
         SndState &s = L.s;
         uint32_t freed = 0, gone = 0;
-        while (s.it_n)
+        SentEntry e = pre[0];
+        while (U(s.it_n))
         {
-            const uint32_t k = L.pos(0), a = L.first[k], b = L.hi(0);
-            if (b > ack)
+            SentEntry nx = gone == 0 ? pre[1] : gone == 1 ? pre[2] : pre[3];
+            if (U(gone + 1 >= LG_PRE && s.it_n > 1))
+                nx = L.at(1);
+            const uint32_t a = e.first, b = s.it_n > 1 ? nx.first : s.high;
+            if (U(b > ack))
             {
-                if (ack > a)
+                if (U(ack > a))
                 {
                     // the entry's acknowledged front leaves its mark totals
-                    const uint8_t m = L.marks[k];
                     const uint32_t cut = ack - a;
-                    s.sack_b -= m & IT_SACKED ? cut : 0u;
-                    s.lost_b -= m & IT_LOST ? cut : 0u;
-                    s.rtx_b -= m & IT_RETX ? cut : 0u;
-                    L.first[k] = ack;
+                    s.sack_b -= e.mark & IT_SACKED ? cut : 0u;
+                    s.lost_b -= e.mark & IT_LOST ? cut : 0u;
+                    s.rtx_b -= e.mark & IT_RETX ? cut : 0u;
+                    L.ring[L.pos(0)].first = ack;
                 }
                 break;
             }
-            if (L.marks[k])
+            if (U(e.mark))
                 lg_remark(L, 0, 0);
             s.it_head = L.pos(1);
             s.it_n--;
             gone++;
             freed += b - a;
+            e = nx;
         }
-        if (gone)
+        if (U(gone))
             s.cand = s.cand > gone ? s.cand - gone : 0;
         s.una = ack;
-        if (s.it_n && (L.mk(0) & IT_SACKED))
+        if (U(s.it_n && (e.mark & IT_SACKED)))
         {
             lg_remark(L, 0, (uint8_t)(L.mk(0) & ~IT_SACKED));
             lg_dup_sack(L);
             lg_head_lost(L);
         }
-        if (s.hisack <= ack)
+        if (U(s.hisack <= ack))
             s.sack_seen = 0, s.hisack = 0;
         return freed;
     }
@@ -703,17 +861,17 @@ struct Model
     static __device__ bool lg_next(Ledger &L, uint32_t *seq)
     {
         SndState &s = L.s;
-        for (uint32_t i = s.cand; s.cand_n && i < s.it_n; i++)
+        for (uint32_t i = s.cand; U(s.cand_n && i < s.it_n); i++)
         {
-            if (!lg_candidate(L.mk(i)))
+            if (U(!lg_candidate(L.mk(i))))
                 continue;
             s.cand = i;
-            if (s.sack_seen && L.lo(i) >= s.hisack)
+            if (U(s.sack_seen && L.lo(i) >= s.hisack))
                 break;
             *seq = L.lo(i);
             return true;
         }
-        if (s.high >= s.tail)
+        if (U(s.high >= s.tail))
             return false;
         *seq = s.high;
         return true;
@@ -728,10 +886,10 @@ struct Model
     static __device__ bool lg_retx_ends_at(const Ledger &L, uint32_t x)
     {
         const SndState &s = L.s;
-        if (!s.it_n || x <= s.una || x > s.high)
+        if (U(!s.it_n || x <= s.una || x > s.high))
             return false;
         const uint32_t n = lg_find(L, x);
-        if (!n || L.hi(n - 1) != x)
+        if (U(!n || L.hi(n - 1) != x))
             return false;
         const uint8_t m = L.mk(n - 1);
         return (m & IT_RETX) && !(m & IT_SACKED);
@@ -748,25 +906,25 @@ struct Model
         const bool mergeable = has_next && !(b & IT_SACKED) && (a & IT_LOST) == (b & IT_LOST);
         const uint32_t most = mergeable ? len + (L.hi(i + 1) - L.lo(i + 1)) : len;
         const uint32_t sz = num < most ? num : most;
-        if (sz > len)
+        if (U(sz > len))
         {
             // entry i + 1 joins entry i: only one of them may stay retransmitted-marked
             uint8_t nb = b;
-            if ((a ^ b) & IT_RETX)
+            if (U((a ^ b) & IT_RETX))
             {
-                if (a & IT_RETX)
+                if (U(a & IT_RETX))
                     lg_remark(L, i, (uint8_t)(a & ~IT_RETX));
                 else
                     lg_remark(L, i + 1, nb = (uint8_t)(b & ~IT_RETX));
             }
-            if (lg_candidate(nb))
+            if (U(lg_candidate(nb)))
                 s.cand_n--;
             lg_erase(L, i + 1);
             len = L.hi(i) - L.lo(i);
         }
-        if (sz < len)
+        if (U(sz < len))
             lg_insert(L, R, i + 1, L.lo(i) + sz, L.mk(i));
-        if (!(L.mk(i) & IT_RETX))
+        if (U(!(L.mk(i) & IT_RETX)))
             lg_remark(L, i, L.mk(i) | IT_RETX);
         return sz;
     }
@@ -779,20 +937,20 @@ struct Model
         for (;;)
         {
             const uint32_t sz = s.tail <= seq ? 0u : num < s.tail - seq ? num : s.tail - seq;
-            if (!sz)
+            if (U(!sz))
                 return 0;
-            if (s.high <= seq)
+            if (U(s.high <= seq))
             {
-                if (!lg_insert(L, R, s.it_n, seq, 0))
+                if (U(!lg_insert(L, R, s.it_n, seq, 0)))
                     return 0;
                 s.high = seq + sz;
                 *retx = false;
                 return sz;
             }
-            if (s.high >= seq + sz)
+            if (U(s.high >= seq + sz))
             {
                 const uint32_t i = lg_find(L, seq);
-                if (i >= s.it_n || L.lo(i) != seq)
+                if (U(i >= s.it_n || L.lo(i) != seq))
                 {
                     count(R, EV_RTT_OVF);
                     return 0;
@@ -815,38 +973,35 @@ struct Model
     }
     static __device__ void rtt_note(Host &x, int f, uint32_t seq, uint32_t sz, bool retx, int64_t now)
     {
-        const Batch &B = *x.B;
-        SndState &s = *x.ls;
-        const ConnStatic &c = conn(x, f);
-        uint32_t *hs = B.h_seq + c.it_off, *hc = B.h_cnt + c.it_off;
-        if (retx)
+        SndState &s = x.S;
+        const uint32_t cap = x.cs.it_cap;
+        SentNote TW_G *ht = x.B->ht + x.cs.it_off;
+        if (U(retx))
         {
             // the record holding seq: resent up to seq + sz
-            for (uint32_t j = 0; j < s.h_n; j++)
+            for (uint32_t j = 0; U(j < s.h_n); j++)
             {
-                const uint32_t k = rtt_pos(s, c.it_cap, j);
-                if (seq >= hs[k] && seq - hs[k] < (hc[k] & 0x7FFFFFFFu))
+                const uint32_t k = rtt_pos(s, cap, j);
+                const SentNote e = ht[k];
+                if (U(seq >= e.seq && seq - e.seq < (e.cnt & 0x7FFFFFFFu)))
                 {
-                    hc[k] = 0x80000000u | (seq + sz - hs[k]);
+                    ht[k].cnt = 0x80000000u | (seq + sz - e.seq);
                     return;
                 }
             }
             return;
         }
-        if (s.h_n >= c.it_cap)
+        if (U(s.h_n >= cap))
         {
             count(x.R, EV_RTT_OVF);
             return;
         }
-        const uint32_t k = rtt_pos(s, c.it_cap, s.h_n++);
-        hs[k] = seq;
-        hc[k] = sz;
-        B.h_t[c.it_off + k] = now;
+        ht[rtt_pos(s, cap, s.h_n++)] = SentNote{now, seq, sz};
     }
     // a measurement m: the smoothed RTT and its variation, then the timeout (at least MinRto)
     static __device__ void rtt_sample(SndState &s, int64_t m)
     {
-        if (s.srtt < 0)
+        if (U(s.srtt < 0))
         {
             s.srtt = m;
             s.rttvar = m / 2;
@@ -860,23 +1015,24 @@ struct Model
         const int64_t spread = 4 * s.rttvar > CLOCK_GRAN_PS ? 4 * s.rttvar : CLOCK_GRAN_PS;
         s.rto = s.srtt + spread > MIN_RTO_PS ? s.srtt + spread : MIN_RTO_PS;
     }
-    static __device__ void rtt_on_ack(Host &x, int f, uint32_t ack, int64_t now)
+    // (pre: the first RTT_PRE notes, read together with the ledger's first entries)
+    static constexpr int RTT_PRE = 3;
+    static __device__ void rtt_on_ack(Host &x, uint32_t ack, int64_t now, const SentNote *pre)
     {
-        const Batch &B = *x.B;
-        SndState &s = *x.ls;
-        if (!s.h_n)
+        SndState &s = x.S;
+        if (U(!s.h_n))
             return;
-        const ConnStatic &c = conn(x, f);
-        const uint32_t *hs = B.h_seq + c.it_off, *hc = B.h_cnt + c.it_off;
-        const uint32_t k0 = rtt_pos(s, c.it_cap, 0);
-        if (!(hc[k0] & 0x80000000u) && ack >= hs[k0] + hc[k0])
-            rtt_sample(s, now - B.h_t[c.it_off + k0]);
-        for (; s.h_n; s.h_n--)
+        const uint32_t cap = x.cs.it_cap;
+        if (U(!(pre[0].cnt & 0x80000000u) && ack >= pre[0].seq + pre[0].cnt))
+            rtt_sample(s, now - pre[0].t);
+        for (int i = 0; U(s.h_n); i++, s.h_n--)
         {
-            const uint32_t k = rtt_pos(s, c.it_cap, 0);
-            if (hs[k] + (hc[k] & 0x7FFFFFFFu) > ack)
+            SentNote e = i == 0 ? pre[0] : i == 1 ? pre[1] : pre[2];
+            if (U(i >= RTT_PRE))
+                e = x.B->ht[x.cs.it_off + rtt_pos(s, cap, 0)];
+            if (U(e.seq + (e.cnt & 0x7FFFFFFFu) > ack))
                 break;
-            s.h_head = rtt_pos(s, c.it_cap, 1);
+            s.h_head = rtt_pos(s, cap, 1);
         }
     }
 
@@ -886,139 +1042,151 @@ struct Model
     // growth (IncreaseWindow). Cubic follows ns-3's TcpCubic (with HyStart), DCTCP its alpha EWMA
     // per window of data, NewReno slow start and congestion avoidance.
     static __device__ __forceinline__ uint32_t to_u32(double d) { return (uint32_t)(uint64_t)(int64_t)d; }
-    static __device__ void cubic_round_start(SndState &s, int64_t now)
+    static __device__ void cubic_round_start(Host &x, int64_t now)
     {
-        s.cub_roundstart = now;
-        s.cub_lastack = now;
-        s.cub_endseq = s.st == S_EST ? s.high + 1 : 0;
-        s.cub_currrtt = INT64_MIN;
-        s.cub_samples = 0;
+        SndState &s = x.S;
+        SndRec TW_G &c = x.B->snd[x.sf];
+        c.cub_roundstart = now;
+        c.cub_lastack = now;
+        c.cub_endseq = s.st == S_EST ? s.high + 1 : 0;
+        c.cub_currrtt = INT64_MIN;
+        c.cub_samples = 0;
     }
     // ACKs per window increment in congestion avoidance (TcpCubic::Update): the cubic curve's
     // target at now + delay_min against the window, bounded by the TCP-friendly estimate
-    static __device__ uint32_t cubic_acks_per_inc(SndState &s, uint32_t segs, int64_t now)
+    static __device__ uint32_t cubic_acks_per_inc(Host &x, uint32_t segs, int64_t now)
     {
+        SndState &s = x.S;
+        SndRec TW_G &c = x.B->snd[x.sf];
         const double C = 0.4, BETA = 0.7;
         const uint32_t w = s.cwnd / MSS;
-        s.cub_ackcnt += segs;
-        if (s.cub_epoch == INT64_MIN)
+        c.cub_ackcnt += segs;
+        if (U(c.cub_epoch == INT64_MIN))
         {
             // a new epoch: the curve's origin and the time K to reach it
-            s.cub_epoch = now;
-            s.cub_ackcnt = segs;
-            s.cub_tcpcwnd = w;
-            const bool below = s.cub_lastmax > w;
-            s.cub_origin = below ? s.cub_lastmax : w;
-            s.cub_k = below ? tw_pow((double)(s.cub_lastmax - w) / C, 1 / 3.) : 0.0;
+            c.cub_epoch = now;
+            c.cub_ackcnt = segs;
+            c.cub_tcpcwnd = w;
+            const bool below = c.cub_lastmax > w;
+            c.cub_origin = below ? c.cub_lastmax : w;
+            c.cub_k = below ? tw_pow((double)(c.cub_lastmax - w) / C, 1 / 3.) : 0.0;
         }
-        const int64_t dt = (int64_t)((uint64_t)now + (uint64_t)s.cub_delaymin - (uint64_t)s.cub_epoch);
-        const double t = tw_seconds(dt), k = s.cub_k;
+        const int64_t dt = (int64_t)((uint64_t)now + (uint64_t)c.cub_delaymin - (uint64_t)c.cub_epoch);
+        const double t = tw_seconds(dt), k = c.cub_k;
         const uint32_t off = to_u32(C * tw_pow(t < k ? k - t : t - k, 3));
-        const uint32_t target = t < k ? s.cub_origin - off : s.cub_origin + off;
+        const uint32_t target = t < k ? c.cub_origin - off : c.cub_origin + off;
         uint32_t n = target > w ? w / (target - w) : 100 * w;
-        if (!s.cub_lastmax && n > 20)
+        if (U(!c.cub_lastmax && n > 20))
             n = 20;
         // the TCP-friendly window: one segment per `per` ACKs
         const uint32_t per = (w * to_u32(8 * (1024 + BETA * 1024) / 3 / (1024 - BETA * 1024))) >> 3;
-        for (; per > 0 && s.cub_ackcnt > per; s.cub_ackcnt -= per)
-            s.cub_tcpcwnd++;
-        if (s.cub_tcpcwnd > w)
+        for (; U(per > 0 && c.cub_ackcnt > per); c.cub_ackcnt -= per)
+            c.cub_tcpcwnd++;
+        if (U(c.cub_tcpcwnd > w))
         {
-            const uint32_t cap = w / (s.cub_tcpcwnd - w);
+            const uint32_t cap = w / (c.cub_tcpcwnd - w);
             n = n > cap ? cap : n;
         }
         return n < 2 ? 2 : n;
     }
     // HyStart's delay check and the minimum delay (TcpCubic::PktsAcked)
-    static __device__ void cubic_measure(SndState &s, int64_t now)
+    static __device__ void cubic_measure(Host &x, int64_t now)
     {
+        SndState &s = x.S;
+        SndRec TW_G &c = x.B->snd[x.sf];
         const int64_t ACK_DELTA = 2000000000, DELAY_MIN = 4000000000, DELAY_MAX = 1000000000000, CUBIC_DELTA = 10000000000;
-        if (s.cub_epoch != INT64_MIN && now - s.cub_epoch < CUBIC_DELTA)
+        if (U(c.cub_epoch != INT64_MIN && now - c.cub_epoch < CUBIC_DELTA))
             return;
         const int64_t rtt = s.srtt;
-        if (s.cub_delaymin == INT64_MIN || rtt < s.cub_delaymin)
-            s.cub_delaymin = rtt;
+        if (U(c.cub_delaymin == INT64_MIN || rtt < c.cub_delaymin))
+            c.cub_delaymin = rtt;
         const bool slow_start_window = s.cwnd <= s.ssthresh && s.cwnd >= 16 * MSS;
-        if (!slow_start_window || s.cub_found)
+        if (U(!slow_start_window || s.cub_found))
             return;
-        if (now - s.cub_lastack <= ACK_DELTA)
+        if (U(now - c.cub_lastack <= ACK_DELTA))
         {
             // the ACK train
-            s.cub_lastack = now;
-            if (now - s.cub_roundstart > s.cub_delaymin)
+            c.cub_lastack = now;
+            if (U(now - c.cub_roundstart > c.cub_delaymin))
                 s.cub_found = 1;
         }
-        if (s.cub_samples >= 8)
+        if (U(c.cub_samples >= 8))
         {
             // the delay increase
-            const int64_t dm = s.cub_delaymin, eta = dm < DELAY_MIN ? DELAY_MIN : dm > DELAY_MAX ? DELAY_MAX : dm;
-            if (s.cub_currrtt > dm + eta)
+            const int64_t dm = c.cub_delaymin, eta = dm < DELAY_MIN ? DELAY_MIN : dm > DELAY_MAX ? DELAY_MAX : dm;
+            if (U(c.cub_currrtt > dm + eta))
                 s.cub_found = 1;
         }
         else
         {
-            if (s.cub_currrtt == INT64_MIN || rtt < s.cub_currrtt)
-                s.cub_currrtt = rtt;
-            s.cub_samples++;
+            if (U(c.cub_currrtt == INT64_MIN || rtt < c.cub_currrtt))
+                c.cub_currrtt = rtt;
+            c.cub_samples++;
         }
-        if (s.cub_found)
+        if (U(s.cub_found))
             s.ssthresh = s.cwnd;
     }
-    static __device__ void cubic_grow(SndState &s, uint32_t segs, uint32_t ack, int64_t now)
+    static __device__ void cubic_grow(Host &x, uint32_t segs, uint32_t ack, int64_t now)
     {
-        if (!s.cwnd_limited)
+        SndState &s = x.S;
+        SndRec TW_G &c = x.B->snd[x.sf];
+        if (U(!s.cwnd_limited))
             return;
-        if (s.cwnd < s.ssthresh)
+        if (U(s.cwnd < s.ssthresh))
         {
-            if (ack + 1 > s.cub_endseq)
-                cubic_round_start(s, now);
+            if (U(ack + 1 > c.cub_endseq))
+                cubic_round_start(x, now);
             s.cwnd += segs * MSS;
             segs = 0;
         }
-        if (segs == 0 || s.cwnd < s.ssthresh)
+        if (U(segs == 0 || s.cwnd < s.ssthresh))
             return;
-        s.cub_cnt += segs;
-        const uint32_t n = cubic_acks_per_inc(s, segs, now);
-        if (s.cub_cnt >= n)
+        c.cub_cnt += segs;
+        const uint32_t n = cubic_acks_per_inc(x, segs, now);
+        if (U(c.cub_cnt >= n))
         {
-            s.cub_cnt -= n;
+            c.cub_cnt -= n;
             s.cwnd += MSS;
         }
     }
     // the threshold after a loss: beta times the window (fast convergence lowers the remembered
     // maximum when the window is below it); a new epoch starts
-    static __device__ uint32_t cubic_ssthresh(SndState &s)
+    static __device__ uint32_t cubic_ssthresh(Host &x)
     {
+        SndState &s = x.S;
+        SndRec TW_G &c = x.B->snd[x.sf];
         const double BETA = 0.7;
         const uint32_t w = s.cwnd / MSS;
-        s.cub_lastmax = w < s.cub_lastmax ? to_u32((w * (1 + BETA)) / 2) : w;
-        s.cub_epoch = INT64_MIN;
+        c.cub_lastmax = w < c.cub_lastmax ? to_u32((w * (1 + BETA)) / 2) : w;
+        c.cub_epoch = INT64_MIN;
         const uint32_t th = to_u32(w * BETA);
         return (th < 2 ? 2 : th) * MSS;
     }
-    static __device__ void cubic_timeout(SndState &s, int64_t now)
+    static __device__ void cubic_timeout(Host &x, int64_t now)
     {
-        s.cub_origin = 0;
-        s.cub_k = 0;
-        s.cub_ackcnt = 0;
-        s.cub_tcpcwnd = 0;
-        s.cub_delaymin = INT64_MIN;
+        SndState &s = x.S;
+        SndRec TW_G &c = x.B->snd[x.sf];
+        c.cub_origin = 0;
+        c.cub_k = 0;
+        c.cub_ackcnt = 0;
+        c.cub_tcpcwnd = 0;
+        c.cub_delaymin = INT64_MIN;
         s.cub_found = 0;
-        cubic_round_start(s, now);
+        cubic_round_start(x, now);
     }
     // DCTCP's alpha: the marked share of the bytes acknowledged over each window of data
     static __device__ void dctcp_measure(SndState &s, uint32_t segs, uint32_t ack)
     {
         const uint32_t bytes = segs * MSS;
         s.acked_total += bytes;
-        if (s.ecn_s == E_ECE_RCVD)
+        if (U(s.ecn_s == E_ECE_RCVD))
             s.acked_ecn += bytes;
-        if (!s.next_seq_flag)
+        if (U(!s.next_seq_flag))
         {
             s.next_seq_flag = 1;
             s.next_seq = s.nxt;
         }
-        if (ack < s.next_seq)
+        if (U(ack < s.next_seq))
             return;
         const double share = s.acked_total ? (double)s.acked_ecn / s.acked_total : 0.0;
         s.alpha = __builtin_fma(1.0 - DCTCP_G, s.alpha, DCTCP_G * share);
@@ -1028,9 +1196,9 @@ struct Model
     // DCTCP's growth: slow start up to the threshold, then a segment per window's worth of ACKs
     static __device__ void dctcp_grow(SndState &s, uint32_t segs)
     {
-        if (s.cwnd < s.ssthresh)
+        if (U(s.cwnd < s.ssthresh))
         {
-            if (segs)
+            if (U(segs))
             {
                 const uint64_t w = (uint64_t)s.cwnd + (uint64_t)segs * MSS;
                 s.cwnd = (uint32_t)(w < s.ssthresh ? w : s.ssthresh);
@@ -1039,13 +1207,13 @@ struct Model
         }
         const uint32_t per = s.cwnd / MSS ? s.cwnd / MSS : 1;
         uint32_t acc = s.cwnd_cnt;
-        if (acc >= per)
+        if (U(acc >= per))
         {
             acc = 0;
             s.cwnd += MSS;
         }
         acc += segs;
-        if (acc >= per)
+        if (U(acc >= per))
         {
             s.cwnd += acc / per * MSS;
             acc %= per;
@@ -1055,12 +1223,12 @@ struct Model
     // NewReno: one segment per ACK in slow start, then about MSS^2 / cwnd bytes (at least 1)
     static __device__ void newreno_grow(SndState &s, uint32_t segs)
     {
-        if (s.cwnd < s.ssthresh && segs)
+        if (U(s.cwnd < s.ssthresh && segs))
         {
             s.cwnd += MSS;
             segs--;
         }
-        if (s.cwnd >= s.ssthresh && segs)
+        if (U(s.cwnd >= s.ssthresh && segs))
         {
             const double add = (double)MSS * MSS / s.cwnd;
             s.cwnd += (uint32_t)(add < 1.0 ? 1.0 : add);
@@ -1068,24 +1236,24 @@ struct Model
     }
     static __device__ uint32_t cc_ssthresh(Host &x, SndState &s, uint32_t in_flight)
     {
-        if (x.cubic)
-            return cubic_ssthresh(s);
-        if (x.dctcp)
+        if (U(x.cubic))
+            return cubic_ssthresh(x);
+        if (U(x.dctcp))
             return (uint32_t)((1.0 - s.alpha / 2.0) * s.cwnd);
         return in_flight / 2 > 2 * MSS ? in_flight / 2 : 2 * MSS;
     }
     static __device__ void cc_acked(Host &x, SndState &s, uint32_t segs, uint32_t ack, int64_t now)
     {
-        if (x.cubic)
-            cubic_measure(s, now);
-        else if (x.dctcp)
+        if (U(x.cubic))
+            cubic_measure(x, now);
+        else if (U(x.dctcp))
             dctcp_measure(s, segs, ack);
     }
     static __device__ void cc_grow(Host &x, SndState &s, uint32_t segs, uint32_t ack, int64_t now)
     {
-        if (x.cubic)
-            cubic_grow(s, segs, ack, now);
-        else if (x.dctcp)
+        if (U(x.cubic))
+            cubic_grow(x, segs, ack, now);
+        else if (U(x.dctcp))
             dctcp_grow(s, segs);
         else
             newreno_grow(s, segs);
@@ -1098,35 +1266,35 @@ struct Model
     // recovery, loss). Every function works on the record of the event's connection in LDS.
     // one segment of up to max_size bytes at seq (SendDataPacket): CWR on the first new segment
     // after an echo, FIN on the last byte once the application closed; the timer is armed if
-    // idle; returns its bytes
-    static __device__ uint32_t tx_segment(Host &x, int f, uint32_t seq, uint32_t max_size, int64_t now)
+    // idle; *o: the frame; returns its bytes
+    static __device__ uint32_t tx_segment(Host &x, int f, uint32_t seq, uint32_t max_size, int64_t now, Out *o)
     {
-        const Batch &B = *x.B;
-        SndState &s = *x.ls;
-        Ledger L(B, s, conn(x, f));
+        Batch &B = *x.B;
+        SndState &s = x.S;
+        Ledger L(x);
         bool retx = false;
         const uint32_t len = lg_take(L, x.R, max_size, seq, &retx);
-        if (!len)
+        if (U(!len))
             return 0;
         uint8_t flags = F_DATA;
-        if (!retx && s.ecn_s == E_ECE_RCVD && s.ecn_echo_seq > s.ecn_cwr_seq)
+        if (U(!retx && s.ecn_s == E_ECE_RCVD && s.ecn_echo_seq > s.ecn_cwr_seq))
         {
             flags |= F_CWR;
             s.ecn_s = E_CWR_SENT;
             s.ecn_cwr_seq = seq;
         }
-        if ((s.fin & FIN_CLOSE) && seq + len == s.tail)
+        if (U((s.fin & FIN_CLOSE) && seq + len == s.tail))
         {
             flags |= F_FIN;
             s.fin |= FIN_SENT;
         }
-        emit(x, f, flags, seq, 0, (uint16_t)(len + 42), false, now);
-        if (retx)
+        *o = out_of(flags, seq, 0, (uint16_t)(len + 42), false);
+        if (U(retx))
         {
             count(x.R, EV_RETX);
             count(x.R, EV_RETX_BY_STATE + s.cong);
         }
-        if (s.rto_at < 0)
+        if (U(s.rto_at < 0))
         {
             s.rto_at = now + s.rto;
             timer_chain(x, B.rchain, f, s.rto);
@@ -1134,61 +1302,73 @@ struct Model
         s.cwnd_limited = s.cwnd < inflight(s) + MSS;
         rtt_note(x, f, seq, len, retx, now);
         s.high = seq + len > s.high ? seq + len : s.high;
-        atomicMax(&x.R->ev[EV_MAX_INFLIGHT], (unsigned long long)s.it_n);
+        x.max_it = s.it_n > x.max_it ? s.it_n : x.max_it;
         return len;
     }
-    // sends while the window has room (SendPendingData): whole segments only, unless the rest of
-    // the data is smaller; nothing more once a FIN is out in the open state
-    static __device__ void tx_fill(Host &x, int f, int64_t now)
+    // a segment asked for by the handler itself
+    static __device__ void tx_now(Host &x, int f, uint32_t seq, int64_t now)
     {
-        SndState &s = *x.ls;
-        if (s.st != S_EST)
-            return;
-        Ledger L(*x.B, s, conn(x, f));
-        for (int n = 0; n < 4096; n++)
-        {
-            const bool fin_out = (s.fin & (FIN_SENT | FIN_ACKED)) == FIN_SENT;
-            if (s.cong == C_OPEN && fin_out)
-                return;
-            const uint32_t pipe = inflight(s), room = s.cwnd > pipe ? s.cwnd - pipe : 0;
-            uint32_t seq;
-            if (!room || !lg_next(L, &seq))
-                return;
-            if (room < MSS && s.tail - seq > room)
-                return; // (no runt segment while more data waits)
-            s.nxt = seq;
-            const uint32_t len = tx_segment(x, f, seq, room < MSS ? room : MSS, now);
-            if (!len)
-                return;
-            s.nxt = seq + len;
-        }
+        Out o;
+        if (U(tx_segment(x, f, seq, MSS, now, &o)))
+            emit(x, f, o.flags, o.sa, 0, o.len, false, now);
+    }
+    // sending while the window has room (SendPendingData), a segment at a time (fill_next) once the
+    // handler is through: whole segments only, unless the rest of the data is smaller; nothing more
+    // once a FIN is out in the open state
+    static __device__ __forceinline__ void tx_fill(Host &x)
+    {
+        x.fill = true;
+        x.fill_n = 0;
+    }
+    static __device__ bool fill_next(Host &x, int f, int64_t now, Out *o)
+    {
+        SndState &s = x.S;
+        if (U(s.st != S_EST || x.fill_n >= 4096))
+            return false;
+        x.fill_n++;
+        Ledger L(x);
+        const bool fin_out = (s.fin & (FIN_SENT | FIN_ACKED)) == FIN_SENT;
+        if (U(s.cong == C_OPEN && fin_out))
+            return false;
+        const uint32_t pipe = inflight(s), room = s.cwnd > pipe ? s.cwnd - pipe : 0;
+        uint32_t seq;
+        if (U(!room || !lg_next(L, &seq)))
+            return false;
+        if (U(room < MSS && s.tail - seq > room))
+            return false; // (no runt segment while more data waits)
+        s.nxt = seq;
+        const uint32_t len = tx_segment(x, f, seq, room < MSS ? room : MSS, now, o);
+        if (U(!len))
+            return false;
+        s.nxt = seq + len;
+        return true;
     }
     // one segment again from the first candidate (else the oldest byte)
     static __device__ void tx_resend_one(Host &x, int f, int64_t now)
     {
-        SndState &s = *x.ls;
-        Ledger L(*x.B, s, conn(x, f));
+        SndState &s = x.S;
+        Ledger L(x);
         uint32_t seq;
-        if (!lg_next(L, &seq))
+        if (U(!lg_next(L, &seq)))
             seq = s.una;
-        if (s.una >= s.tail)
+        if (U(s.una >= s.tail))
             return;
         s.nxt = seq;
-        tx_segment(x, f, seq, MSS, now);
+        tx_now(x, f, seq, now);
     }
     // the retransmission timer after new data is acknowledged (NewAck): restarted from the RTT
     // estimate when asked, stopped once all data (and no FIN) is acknowledged
     static __device__ void rto_after_ack(Host &x, int f, uint32_t ack, bool restart, int64_t now)
     {
-        SndState &s = *x.ls;
-        if (restart)
+        SndState &s = x.S;
+        if (U(restart))
         {
             const int64_t base = s.srtt >= 0 ? s.srtt : INIT_RTT_PS, spread = 4 * s.rttvar > CLOCK_GRAN_PS ? 4 * s.rttvar : CLOCK_GRAN_PS;
             s.rto = base + spread > MIN_RTO_PS ? base + spread : MIN_RTO_PS;
             s.rto_at = now + s.rto;
             timer_chain(x, x.B->rchain, f, s.rto);
         }
-        if (ack >= s.tail && !(s.fin & FIN_SENT))
+        if (U(ack >= s.tail && !(s.fin & FIN_SENT)))
             s.rto_at = -1;
         s.nxt = ack > s.nxt ? ack : s.nxt;
     }
@@ -1196,8 +1376,8 @@ struct Model
     // the segment sent again
     static __device__ void fast_retransmit(Host &x, int f, int64_t now)
     {
-        SndState &s = *x.ls;
-        Ledger L(*x.B, s, conn(x, f));
+        SndState &s = x.S;
+        Ledger L(x);
         lg_dup_sack(L);
         lg_head_lost(L);
         s.cong = C_RECOVERY;
@@ -1205,24 +1385,23 @@ struct Model
         s.recover_active = 1;
         s.ssthresh = cc_ssthresh(x, s, inflight(s) + MSS);
         s.cwnd = s.ssthresh;
-        tx_segment(x, f, s.una, MSS, now);
+        tx_now(x, f, s.una, now);
     }
     // messages wholly acknowledged complete (their completion time is the flow's); the connection
     // is done with its last message (and its FIN, if it sends one)
     static __device__ void msgs_complete(Host &x, int f, int64_t now)
     {
-        const Batch &B = *x.B;
-        SndState &s = *x.ls;
-        const ConnStatic &c = conn(x, f);
-        for (; s.m_dn < s.m_wr; s.m_dn++)
+        Batch &B = *x.B;
+        SndState &s = x.S;
+        for (; U(s.m_dn < s.m_wr); s.m_dn++)
         {
-            const int m = c.m_first + s.m_dn;
-            if (s.una < B.mg_end[m])
+            const int m = x.cs.m_first + s.m_dn;
+            if (U(s.una < (s.m_dn + 1 == s.m_wr ? s.tail : B.mg_end[m]))) // (the last one written ends at the tail)
                 break;
             B.mg_done[m] = now;
             atomicAdd(&x.R->flows_done, 1u);
         }
-        if (s.m_dn == c.m_cnt && (!c.fin_on || (s.fin & FIN_ACKED)))
+        if (U(s.m_dn == x.cs.m_cnt && (!x.cs.fin_on || (s.fin & FIN_ACKED))))
         {
             s.st = S_DONE;
             s.rto_at = -1;
@@ -1231,17 +1410,17 @@ struct Model
     // DCTCP's response to an echo (EnterCwr): a new echo beyond the last one cuts the window once
     static __device__ void ack_echo(Host &x, SndState &s, uint32_t ack, bool ece, bool advancing)
     {
-        if (!(advancing && x.dctcp && ece))
+        if (U(!(advancing && x.dctcp && ece)))
         {
-            if (!ece && s.ecn_s == E_ECE_RCVD)
+            if (U(!ece && s.ecn_s == E_ECE_RCVD))
                 s.ecn_s = E_IDLE;
             return;
         }
-        if ((int64_t)ack <= s.ecn_echo_seq)
+        if (U((int64_t)ack <= s.ecn_echo_seq))
             return;
         s.ecn_echo_seq = ack;
         s.ecn_s = E_ECE_RCVD;
-        if (s.cong == C_CWR)
+        if (U(s.cong == C_CWR))
             return;
         s.ssthresh = cc_ssthresh(x, s, inflight(s));
         s.cwnd = s.ssthresh;
@@ -1253,19 +1432,19 @@ struct Model
     static __device__ void ack_duplicate(Host &x, int f, SndState &s, uint32_t una_before, int64_t now)
     {
         uint8_t state = s.cong;
-        if (state == C_LOSS)
+        if (U(state == C_LOSS))
             return;
-        if (state != C_RECOVERY)
+        if (U(state != C_RECOVERY))
             s.dupacks++;
-        if (state == C_OPEN)
+        if (U(state == C_OPEN))
             s.cong = state = C_DISORDER;
-        Ledger L(*x.B, s, conn(x, f));
-        if (state == C_RECOVERY)
+        Ledger L(x);
+        if (U(state == C_RECOVERY))
             lg_dup_sack(L);
-        else if (state == C_DISORDER)
+        else if (U(state == C_DISORDER))
         {
             const bool third = s.dupacks == (uint32_t)DUPTHRESH && (!s.recover_active || una_before >= s.recover);
-            if (third || lg_head_is_lost(L))
+            if (U(third || lg_head_is_lost(L)))
                 fast_retransmit(x, f, now);
         }
     }
@@ -1273,11 +1452,11 @@ struct Model
     // the timer restarted on the first partial ACK only) or during loss (slow start again)
     static __device__ void ack_partial(Host &x, int f, SndState &s, uint32_t ack, uint32_t segs, int64_t now)
     {
-        if (s.cong == C_RECOVERY)
+        if (U(s.cong == C_RECOVERY))
         {
-            Ledger L(*x.B, s, conn(x, f));
+            Ledger L(x);
             lg_head_lost(L);
-            if (!lg_retx_ends_at(L, ack + MSS))
+            if (U(!lg_retx_ends_at(L, ack + MSS)))
                 tx_resend_one(x, f, now);
             cc_acked(x, s, 1, ack, now);
             rto_after_ack(x, f, ack, s.first_partial, now);
@@ -1293,7 +1472,7 @@ struct Model
     static __device__ void ack_advance(Host &x, int f, SndState &s, uint32_t ack, uint32_t una_before, uint32_t segs, uint32_t dups, int64_t now)
     {
         const uint8_t state = s.cong;
-        if (state == C_CWR)
+        if (U(state == C_CWR))
         {
             cc_acked(x, s, segs, ack, now);
             rto_after_ack(x, f, ack, true, now);
@@ -1305,7 +1484,7 @@ struct Model
             cc_acked(x, s, segs, ack, now);
             break;
         case C_DISORDER:
-            if (segs >= dups)
+            if (U(segs >= dups))
                 cc_acked(x, s, segs - dups, ack, now);
             break;
         case C_RECOVERY:
@@ -1321,9 +1500,9 @@ struct Model
             break;
         }
         s.cong = C_OPEN;
-        if (ack >= s.recover)
+        if (U(ack >= s.recover))
             s.recover_active = 0;
-        if (state == C_RECOVERY)
+        if (U(state == C_RECOVERY))
         {
             rto_after_ack(x, f, ack, true, now);
             s.cwnd = s.ssthresh;
@@ -1337,29 +1516,38 @@ struct Model
     // last the FIN's acknowledgment, the completed messages and more sending
     static __device__ void ack_in(Host &x, int f, uint32_t ack, bool ece, int64_t now)
     {
-        SndState &s = *x.ls;
-        if (s.st != S_EST || ack < s.una)
+        SndState &s = x.S;
+        if (U(s.st != S_EST || ack < s.una))
             return;
         const uint32_t una_before = s.una;
         const bool advancing = ack > una_before;
-        rtt_on_ack(x, f, ack, now);
-        Ledger L(*x.B, s, conn(x, f));
-        const uint32_t acked = advancing ? lg_release(L, ack) : 0;
-        if (s.cong == C_CWR && ack > s.recover)
+        Ledger L(x);
+        // (past the rings' ends their first entries again: read, not used)
+        SentNote notes[RTT_PRE];
+        SentEntry entries[LG_PRE];
+#pragma unroll
+        for (int i = 0; i < RTT_PRE; i++)
+            notes[i] = x.B->ht[x.cs.it_off + rtt_pos(s, L.cap, (uint32_t)i < s.h_n ? i : 0)];
+#pragma unroll
+        for (int i = 0; i < LG_PRE; i++)
+            entries[i] = L.at((uint32_t)i < s.it_n ? i : 0);
+        rtt_on_ack(x, ack, now, notes);
+        const uint32_t acked = advancing ? lg_release(L, ack, entries) : 0;
+        if (U(s.cong == C_CWR && ack > s.recover))
         {
             s.cong = C_OPEN;
             s.cwnd = s.ssthresh;
         }
         ack_echo(x, s, ack, ece, advancing);
         const uint32_t dups = s.dupacks;
-        if (!advancing)
+        if (U(!advancing))
         {
-            if (ack < s.high)
+            if (U(ack < s.high))
             {
                 ack_duplicate(x, f, s, una_before, now);
                 cc_acked(x, s, 1, ack, now);
             }
-            else if (ack > s.high)
+            else if (U(ack > s.high))
                 s.nxt = ack;
         }
         else
@@ -1367,44 +1555,44 @@ struct Model
             // whole segments acknowledged, the remainders carried over
             uint32_t segs = acked / MSS;
             s.ack_rem += acked % MSS;
-            if (s.ack_rem >= MSS)
+            if (U(s.ack_rem >= MSS))
             {
                 s.ack_rem -= MSS;
                 segs++;
             }
             s.dupacks = 0;
-            if (ack < s.recover && (s.cong == C_RECOVERY || s.cong == C_LOSS))
+            if (U(ack < s.recover && (s.cong == C_RECOVERY || s.cong == C_LOSS)))
                 ack_partial(x, f, s, ack, segs, now);
             else
                 ack_advance(x, f, s, ack, una_before, segs, dups, now);
         }
-        if ((s.fin & FIN_SENT) && !s.it_n && ack == s.high + 1)
+        if (U((s.fin & FIN_SENT) && !s.it_n && ack == s.high + 1))
             s.fin |= FIN_ACKED;
-        if (advancing)
+        if (U(advancing))
         {
             msgs_complete(x, f, now);
-            if (s.st == S_DONE)
+            if (U(s.st == S_DONE))
                 return;
         }
-        tx_fill(x, f, now);
+        tx_fill(x);
     }
     // the retransmission timeout: every outstanding segment lost, the timeout doubled (to 60 s at
     // most), one segment's window, then sending again
     static __device__ void rto_fire(Host &x, int f, int64_t now)
     {
-        SndState &s = *x.ls;
+        SndState &s = x.S;
         s.rto_at = -1;
-        if (s.st != S_EST)
+        if (U(s.st != S_EST))
             return;
-        if (s.una >= s.tail)
+        if (U(s.una >= s.tail))
         {
-            if ((s.fin & (FIN_SENT | FIN_ACKED)) == FIN_SENT)
+            if (U((s.fin & (FIN_SENT | FIN_ACKED)) == FIN_SENT))
                 count(x.R, EV_RTT_OVF);
             return;
         }
         count(x.R, EV_RTO);
         const uint32_t was_in_flight = inflight(s);
-        Ledger L(*x.B, s, conn(x, f));
+        Ledger L(x);
         lg_all_lost(L);
         s.dupacks = 0;
         s.recover = s.high;
@@ -1412,11 +1600,11 @@ struct Model
         s.rto = 2 * s.rto < 60000000000000ll ? 2 * s.rto : 60000000000000ll;
         s.h_n = 0;
         s.ssthresh = cc_ssthresh(x, s, was_in_flight);
-        if (x.cubic)
-            cubic_timeout(s, now);
+        if (U(x.cubic))
+            cubic_timeout(x, now);
         s.cong = C_LOSS;
         s.cwnd = MSS;
-        tx_fill(x, f, now);
+        tx_fill(x);
     }
 
     // -------------------------------------------------------------- the receiving endpoint
@@ -1427,10 +1615,10 @@ struct Model
     // always with force_ece
     static __device__ void rcv_ack(Host &x, int f, uint32_t ack, bool force_ece, bool no_ece, int64_t now)
     {
-        RcvState &r = *x.lr;
+        RcvState &r = x.Q;
         const bool echoing = r.ecn_r == E_CE_RCVD || r.ecn_r == E_SENDING_ECE;
         const bool ece = force_ece || (!no_ece && echoing);
-        if (!force_ece && ece)
+        if (U(!force_ece && ece))
             r.ecn_r = E_SENDING_ECE;
         r.delack_at = -1;
         r.delack_count = 0;
@@ -1438,19 +1626,19 @@ struct Model
     }
     static __device__ void rcv_synack(Host &x, int f, int64_t now)
     {
-        RcvState &r = *x.lr;
+        RcvState &r = x.Q;
         const int64_t backoff = CONN_TIMEOUT_PS << r.srv_syn_n++;
-        if (r.r_synack_t < 0)
+        if (U(r.r_synack_t < 0))
             r.r_synack_t = now;
         emit(x, f, F_SYN | F_ACK, 0, 0, SYN_FRAME, true, now);
-        if (r.srv_syn_at >= 0)
+        if (U(r.srv_syn_at >= 0))
             return;
         r.srv_syn_at = now + backoff;
         timer_chain(x, x.B->dchain, f, backoff);
     }
     static __device__ __forceinline__ void rcv_established(RcvState &r)
     {
-        if (r.r_est)
+        if (U(r.r_est))
             return;
         r.r_est = 1;
         r.srv_syn_at = -1;
@@ -1459,47 +1647,47 @@ struct Model
     // before it, with the previous state's ECE (set when leaving CE, cleared when entering it)
     static __device__ void rcv_ce_edge(Host &x, int f, bool ce, int64_t now)
     {
-        RcvState &r = *x.lr;
+        RcvState &r = x.Q;
         const bool flips = (bool)r.ce_state != ce;
-        if (flips && r.reserved && r.prior_flag)
+        if (U(flips && r.reserved && r.prior_flag))
             rcv_ack(x, f, r.prior_rcv_nxt, !ce, ce, now);
         r.ce_state = ce ? 1 : 0;
-        if (ce)
+        if (U(ce))
             r.ecn_r = E_CE_RCVD;
-        else if (r.ecn_r == E_CE_RCVD || r.ecn_r == E_SENDING_ECE)
+        else if (U(r.ecn_r == E_CE_RCVD || r.ecn_r == E_SENDING_ECE))
             r.ecn_r = E_IDLE;
         r.prior_flag = 1;
         r.prior_rcv_nxt = r.rcv_nxt;
     }
     static __device__ void rcv_ecn_in(Host &x, int f, const Frame &p, int64_t now)
     {
-        if (!x.dctcp)
+        if (U(!x.dctcp))
             return;
-        RcvState &r = *x.lr;
-        if ((p.flags & F_CE) && r.ecn_ce_seq < (int64_t)p.sa)
+        RcvState &r = x.Q;
+        if (U((p.flags & F_CE) && r.ecn_ce_seq < (int64_t)p.sa))
         {
             r.ecn_ce_seq = p.sa;
             r.ecn_r = E_CE_RCVD;
             rcv_ce_edge(x, f, true, now);
         }
-        else if (p.flags & F_ECT)
+        else if (U(p.flags & F_ECT))
             rcv_ce_edge(x, f, false, now);
     }
     // the CE state of the sending side's own ECN (ACKs carrying CE)
     static __device__ void snd_ecn_in(Host &x, SndState &s, const Frame &p)
     {
-        if (!x.dctcp)
+        if (U(!x.dctcp))
             return;
-        if ((p.flags & F_CE) && !(s.s_ce & 1))
+        if (U((p.flags & F_CE) && !(s.s_ce & 1)))
         {
             s.s_ce = 3;
             s.ecn_s = E_CE_RCVD;
             return;
         }
-        if (!(p.flags & F_ECT))
+        if (U(!(p.flags & F_ECT)))
             return;
         s.s_ce &= ~2;
-        if (s.ecn_s == E_CE_RCVD || s.ecn_s == E_SENDING_ECE)
+        if (U(s.ecn_s == E_CE_RCVD || s.ecn_s == E_SENDING_ECE))
             s.ecn_s = E_IDLE;
     }
     // The reassembly ring (TcpRxBuffer::Add): out-of-order blocks, disjoint and sorted, in a ring
@@ -1507,60 +1695,68 @@ struct Model
     // rcv_nxt is delivered. False if nothing was new (or the ring is full).
     static __device__ bool reasm_add(Host &x, int f, uint32_t seq, uint32_t end)
     {
-        const Batch &B = *x.B;
-        RcvState &r = *x.lr;
-        const ConnStatic &c = conn(x, f);
+        Batch &B = *x.B;
+        RcvState &r = x.Q;
         const uint32_t from = seq > r.rcv_nxt ? seq : r.rcv_nxt;
-        if (from >= end)
+        if (U(from >= end))
             return false;
-        uint32_t *lo = B.oo_s + c.oo_off, *hi = B.oo_e + c.oo_off;
-        const uint32_t cap = c.oo_cap, h0 = r.ooo_h;
+        uint32_t *lo = B.oo_s + x.cr.oo_off, *hi = B.oo_e + x.cr.oo_off;
+        const uint32_t cap = x.cr.oo_cap, h0 = r.ooo_h;
         uint32_t n = r.ooo_n;
+        if (U(n == 0 && from == r.rcv_nxt))
+        {
+            // in order, nothing held: delivered without a place in the ring
+            r.rcv_nxt = end;
+            r.ooo_h = 0;
+            if (U(r.r_fin >= 0 && r.rcv_nxt == (uint32_t)r.r_fin))
+                r.rcv_nxt++; // (the FIN's sequence number)
+            return true;
+        }
         auto at = [&](uint32_t i) { return h0 + i < cap ? h0 + i : h0 + i - cap; };
         // the first block ending at or after `from`
         uint32_t i = n;
-        if (n && hi[at(n - 1)] >= from)
+        if (U(n && hi[at(n - 1)] >= from))
         {
             uint32_t a = 0, b = n - 1;
-            while (a < b)
+            while (U(a < b))
             {
                 const uint32_t m = (a + b) / 2;
-                if (hi[at(m)] < from)
+                if (U(hi[at(m)] < from))
                     a = m + 1;
                 else
                     b = m;
             }
             i = a;
         }
-        if (i < n && lo[at(i)] <= from && hi[at(i)] >= end)
+        if (U(i < n && lo[at(i)] <= from && hi[at(i)] >= end))
             return false; // (all of it is held already)
         // blocks i .. j - 1 touch [from, end): they merge into one
         uint32_t j = i, nlo = from, nhi = end;
-        for (; j < n && lo[at(j)] <= nhi; j++)
+        for (; U(j < n && lo[at(j)] <= nhi); j++)
         {
             nlo = lo[at(j)] < nlo ? lo[at(j)] : nlo;
             nhi = hi[at(j)] > nhi ? hi[at(j)] : nhi;
         }
-        if (j == i)
+        if (U(j == i))
         {
             // a new block at i
-            if (n >= cap)
+            if (U(n >= cap))
             {
                 count(x.R, EV_OOO_OVF);
                 return false;
             }
-            for (uint32_t k = n; k > i; k--)
+            for (uint32_t k = n; U(k > i); k--)
             {
                 lo[at(k)] = lo[at(k - 1)];
                 hi[at(k)] = hi[at(k - 1)];
             }
             n++;
         }
-        else if (j - i > 1)
+        else if (U(j - i > 1))
         {
             // the merged blocks after the first close up
             const uint32_t gone = j - i - 1;
-            for (uint32_t k = j; k < n; k++)
+            for (uint32_t k = j; U(k < n); k++)
             {
                 lo[at(k - gone)] = lo[at(k)];
                 hi[at(k - gone)] = hi[at(k)];
@@ -1570,7 +1766,7 @@ struct Model
         lo[at(i)] = nlo;
         hi[at(i)] = nhi;
         uint32_t head = h0;
-        if (from == r.rcv_nxt)
+        if (U(from == r.rcv_nxt))
         {
             // the first block is in order now: delivered
             r.rcv_nxt = hi[at(0)];
@@ -1579,7 +1775,7 @@ struct Model
         }
         r.ooo_n = n;
         r.ooo_h = n ? head : 0;
-        if (r.r_fin >= 0 && r.rcv_nxt == (uint32_t)r.r_fin)
+        if (U(r.r_fin >= 0 && r.rcv_nxt == (uint32_t)r.r_fin))
             r.rcv_nxt++; // (the FIN's sequence number)
         return true;
     }
@@ -1592,11 +1788,11 @@ struct Model
     // FIN+ACK of the passive close, with its retransmission timer (at least MinRto) if none runs
     static __device__ void rcv_fin_ack(Host &x, int f, int64_t now)
     {
-        RcvState &r = *x.lr;
+        RcvState &r = x.Q;
         r.delack_at = -1;
         r.delack_count = 0;
         emit(x, f, F_ACK | F_FIN, 0, r.rcv_nxt, CTRL_FRAME, true, now);
-        if (r.r_frx_at >= 0)
+        if (U(r.r_frx_at >= 0))
             return;
         const int64_t t = rcv_rto(r) > MIN_RTO_PS ? rcv_rto(r) : MIN_RTO_PS;
         r.r_frx_at = now + t;
@@ -1605,7 +1801,7 @@ struct Model
     // the peer closed: LAST_ACK, our FIN+ACK, and the LastAck timer with its retries
     static __device__ void rcv_peer_closed(Host &x, int f, int64_t now)
     {
-        RcvState &r = *x.lr;
+        RcvState &r = x.Q;
         r.r_st = R_LAST_ACK;
         rcv_fin_ack(x, f, now);
         r.r_last_n = DATA_RETRIES;
@@ -1622,21 +1818,21 @@ struct Model
     // filled), for nothing new, or for every second segment; else the delayed ACK
     static __device__ void rcv_data(Host &x, int f, uint32_t seq, uint32_t len, bool fin, int64_t now)
     {
-        RcvState &r = *x.lr;
+        RcvState &r = x.Q;
         const uint32_t before = r.rcv_nxt;
-        if (!reasm_add(x, f, seq, seq + len))
+        if (U(!reasm_add(x, f, seq, seq + len)))
         {
             rcv_ack(x, f, r.rcv_nxt, false, false, now);
             return;
         }
-        if (!fin && before < r.rcv_nxt && rcv_fin_in(r))
+        if (U(!fin && before < r.rcv_nxt && rcv_fin_in(r)))
         {
             rcv_peer_closed(x, f, now);
             return;
         }
         const bool irregular = r.ooo_n > 0 || r.rcv_nxt > before + len;
         const uint32_t held = r.delack_count + 1u;
-        if (irregular || held >= DELACK_COUNT)
+        if (U(irregular || held >= DELACK_COUNT))
         {
             r.reserved = 0;
             rcv_ack(x, f, r.rcv_nxt, false, false, now);
@@ -1644,7 +1840,7 @@ struct Model
         }
         r.delack_count = (uint8_t)held;
         r.reserved = 1;
-        if (r.delack_at >= 0)
+        if (U(r.delack_at >= 0))
             return;
         r.delack_at = now + DELACK_PS;
         timer_chain(x, x.B->dchain, f, DELACK_PS);
@@ -1655,48 +1851,48 @@ struct Model
     // order, marks the end and closes passively once delivered
     static __device__ void rcv_segment(Host &x, int f, const Frame &p, int64_t now)
     {
-        RcvState &r = *x.lr;
-        if (!r.r_up || r.r_st == R_CLOSED)
+        RcvState &r = x.Q;
+        if (U(!r.r_up || r.r_st == R_CLOSED))
             return;
         const bool fin = p.flags & F_FIN;
         const uint32_t seq = p.sa, len = (p.flags & F_DATA) ? p.len - 42u : 0u, end = seq + len;
-        if (len && r.r_est)
+        if (U(len && r.r_est))
         {
             const bool stale = r.r_st == R_LAST_ACK ? seq != r.rcv_nxt : end < r.rcv_nxt;
-            if (stale)
+            if (U(stale))
             {
                 rcv_ack(x, f, r.rcv_nxt, false, true, now);
                 return;
             }
         }
         rcv_ecn_in(x, f, p, now);
-        if ((p.flags & F_CWR) && r.r_est && r.r_st == R_OPEN && r.ecn_r != E_CE_RCVD)
+        if (U((p.flags & F_CWR) && r.r_est && r.r_st == R_OPEN && r.ecn_r != E_CE_RCVD))
             r.ecn_r = E_IDLE;
-        if (!r.r_est)
+        if (U(!r.r_est))
         {
-            if (fin && seq != r.rcv_nxt)
+            if (U(fin && seq != r.rcv_nxt))
                 return;
             rcv_established(r);
         }
-        if (r.r_st == R_LAST_ACK)
+        if (U(r.r_st == R_LAST_ACK))
         {
-            if (fin || seq == r.rcv_nxt)
+            if (U(fin || seq == r.rcv_nxt))
                 rcv_closed(r);
             return;
         }
-        if (!fin)
+        if (U(!fin))
         {
             rcv_data(x, f, seq, len, false, now);
             return;
         }
-        if (seq < r.rcv_nxt)
+        if (U(seq < r.rcv_nxt))
             return;
         r.r_fin = end;
-        if (r.rcv_nxt == end)
+        if (U(r.rcv_nxt == end))
             r.rcv_nxt++;
-        if (len)
+        if (U(len))
             rcv_data(x, f, seq, len, true, now);
-        if (rcv_fin_in(r))
+        if (U(rcv_fin_in(r)))
             rcv_peer_closed(x, f, now);
     }
 
@@ -1705,7 +1901,7 @@ struct Model
     {
         int32_t *n = snd ? x.B->n_snd : x.B->n_rcv;
         const int k = n[x.h];
-        if (k >= MAX_ACTIVE)
+        if (U(k >= MAX_ACTIVE))
         {
             count(x.R, EV_ACTIVE_OVF);
             return;
@@ -1714,27 +1910,26 @@ struct Model
         n[x.h] = k + 1;
     }
     // the application writes its due messages (FlowSender::Write); Socket::Send defers
-    // SendPendingData by 1 ps when the window has room (src/step.cuh:2120-2145)
-    static __device__ void app_write(Host &x, int f, int64_t now)
+    // SendPendingData by 1 ps when the window has room (src/step.cuh:2120-2145); at: the write's chain
+    static __device__ void app_write(Host &x, int f, int64_t now, const Chain &at)
     {
-        const Batch &B = *x.B;
-        SndState &s = *x.ls;
-        const ConnStatic &c = conn(x, f);
-        if (s.m_wr >= s.m_due)
+        Batch &B = *x.B;
+        SndState &s = x.S;
+        if (U(s.m_wr >= s.m_due))
             return;
-        for (; s.m_wr < s.m_due; s.m_wr++)
+        for (; U(s.m_wr < s.m_due); s.m_wr++)
         {
-            const int m = c.m_first + s.m_wr;
+            const int m = x.cs.m_first + s.m_wr;
             B.mg_est[m] = now;
             s.tail = B.mg_end[m];
         }
-        if (c.fin_on && s.m_wr == c.m_cnt)
+        if (U(x.cs.fin_on && s.m_wr == x.cs.m_cnt))
             s.fin |= FIN_CLOSE;
-        if (s.cwnd <= inflight(s) || s.syn_at >= 0)
+        if (U(s.cwnd <= inflight(s) || s.syn_at >= 0))
             return;
         s.syn_at = now + 1;
         Chain ch;
-        chain_child(ch, 2, x.echain);
+        chain_child(ch, 2, at);
         chain_store(B.schain + (size_t)f * CW, ch);
         due_insert(x, now + 1, f, 2);
     }
@@ -1743,24 +1938,25 @@ struct Model
     // sender's close) is acknowledged once, any other ACK goes to ack_in
     static __device__ void on_frame_snd(Host &x, int f, const Frame &p, int64_t now)
     {
-        SndState &s = *x.ls;
-        if (p.flags & F_SYN)
+        SndState &s = x.S;
+        if (U(p.flags & F_SYN))
         {
-            if (s.st != S_SYN_SENT)
+            if (U(s.st != S_SYN_SENT))
                 return;
             s.st = S_EST;
             s.syn_at = -1;
             rtt_sample(s, now - s.timing_time);
             emit(x, f, F_ACK, 0, 0, CTRL_FRAME, false, now);
-            chain_child(x.echain, 1, x.echain);
-            app_write(x, f, now);
+            Chain w; // (the write is an event scheduled now; it sends nothing itself)
+            chain_child(w, 1, x.echain);
+            app_write(x, f, now, w);
             return;
         }
-        if (s.fin & FIN_TW)
+        if (U(s.fin & FIN_TW))
             return;
         snd_ecn_in(x, s, p);
         ack_in(x, f, p.sa, p.flags & F_ECE, now);
-        if (!(p.flags & F_FIN))
+        if (U(!(p.flags & F_FIN)))
             return;
         s.fin |= FIN_TW;
         emit(x, f, F_ACK, 0, 1, CTRL_FRAME, false, now);
@@ -1769,64 +1965,63 @@ struct Model
     // comes up; a SYN-ACK unless established), data, or an ACK (establishes; ends LAST_ACK)
     static __device__ void on_frame_rcv(Host &x, int f, const Frame &p, int64_t now)
     {
-        RcvState &r = *x.lr;
+        RcvState &r = x.Q;
         const bool syn = p.flags & F_SYN;
-        if (!syn && r.r_up && r.r_srtt < 0 && r.r_synack_t >= 0)
+        if (U(!syn && r.r_up && r.r_srtt < 0 && r.r_synack_t >= 0))
         {
             const int64_t m = now - r.r_synack_t;
             r.r_srtt = m;
             r.r_rttvar = m / 2;
         }
-        if (syn)
+        if (U(syn))
         {
-            if (!r.r_up)
+            if (U(!r.r_up))
             {
                 r.r_up = 1;
                 r.delack_count = DELACK_COUNT;
                 add_active(x, false, f);
             }
-            if (r.r_est)
+            if (U(r.r_est))
                 return;
             x.nic.woke = now;
             chain_child(x.echain, 1, x.echain);
             rcv_synack(x, f, now);
             return;
         }
-        if (p.flags & (F_DATA | F_FIN))
+        if (U(p.flags & (F_DATA | F_FIN)))
         {
             rcv_segment(x, f, p, now);
             return;
         }
-        if (!r.r_up || r.r_st == R_CLOSED)
+        if (U(!r.r_up || r.r_st == R_CLOSED))
             return;
         rcv_ecn_in(x, f, p, now);
         rcv_established(r);
-        if (r.r_st == R_LAST_ACK)
+        if (U(r.r_st == R_LAST_ACK))
             rcv_closed(r);
     }
     // one event per frame: the side's record in LDS for its duration
     static __device__ void on_frame(Host &x, const Frame &p, int64_t now)
     {
         const int f = (int)p.flow;
-        if (p.to_sender)
+        if (U(p.to_sender))
         {
             snd_open(x, f);
             on_frame_snd(x, f, p, now);
-            snd_close(x, f);
         }
         else
         {
             rcv_open(x, f);
             on_frame_rcv(x, f, p, now);
-            rcv_close(x, f);
         }
     }
-    static __device__ __forceinline__ const uint32_t *due_chain(const Batch &B, const Due &d)
+    static __device__ __forceinline__ const uint32_t *due_chain(const Host &x, const Due &d)
     {
+        Batch &B = *x.B;
         const uint32_t *base = d.kind == 1 || d.kind == 3 || d.kind == 4 ? B.dchain
                                : d.kind == 5                            ? B.fchain
-                               : (d.kind == 2 && B.snd[d.flow].st == S_EST) ? B.schain
-                                                                            : B.rchain;
+                               : (d.kind == 2 && (x.sf == d.flow ? x.S.st : B.snd[d.flow].st) == S_EST) ? B.schain
+                                                                                                           : B.rchain;
         return base + (size_t)d.flow * CW;
     }
     // a timer and an arrival at one instant: the one scheduled first runs first (undecided: the timer)
@@ -1835,16 +2030,54 @@ struct Model
         Chain arr, pc;
         msg_chain(pc, p);
         chain_child(arr, 2048u + msg_head(p).len, pc);
-        int r = chain_cmp(due_chain(*x.B, d), arr.r);
-        if (r == 0)
+        int r = chain_cmp(due_chain(x, d), arr.r);
+        if (U(r == 0))
             count(x.R, EV_UNDECIDED);
         return r <= 0;
     }
 
     // -------------------------------------------------------------- one slot of a host
+    // its arrivals: the later part of slot t-2's message of its in-link, the earlier of t-1's
+    struct HostIn
+    {
+        int in, i2, n2, n1;
+    };
+    // has the host events in this slot? If not, *wake: its next slot
+    static __device__ __forceinline__ bool host_open(Batch &B, World &W, int hl, int64_t t, HostIn &in, int64_t *wake)
+    {
+        const int h = W.host0 + hl, lid = W.link0 + hl;
+        in.in = B.in_link[lid];
+        in.i2 = in.n2 = in.n1 = 0;
+        const int64_t w = B.wake[h];
+        const int queued = B.q_size[lid];
+        if (t >= 2)
+        {
+            const long long v = coh_load(B.msg_cnt + (size_t)((t - 2) % NRING) * B.nlinks + in.in);
+            if (msg_slot(v) == t - 2)
+                in.i2 = msg_early(v), in.n2 = msg_sent(v);
+        }
+        if (t >= 1)
+        {
+            const long long v = coh_load(B.msg_cnt + (size_t)((t - 1) % NRING) * B.nlinks + in.in);
+            in.n1 = msg_slot(v) == t - 1 ? msg_early(v) : 0;
+        }
+        if (in.i2 < in.n2 || in.n1 > 0 || t >= w || queued != 0)
+            return true;
+        *wake = w;
+        return false;
+    }
     // (src/step.cuh:2263-2528): returns 1 if it sent or holds frames; *wake: its next slot
-    static __device__ int host_step(const Batch &B, const WorldDesc &W, WorldRun *R, int hl, int64_t t, int64_t *wake, SndState *ls,
-                                    RcvState *lr, ConnStatic *lc)
+    // (three arguments of callers that keep record slots are taken and not used)
+    static __device__ int host_step(Batch &B, World &W, WorldRun *R, int hl, int64_t t, int64_t *wake, SndState *, RcvState *, ConnStatic *)
+    {
+        HostIn in;
+        int staged;
+        return host_open(B, W, hl, t, in, wake) ? host_run(B, W, R, hl, t, wake, in, nullptr, 0, &staged) : 0;
+    }
+    // the slot of a host that has events; st: the lane's workspace for the first st_cap frames out,
+    // which the caller moves to the link's message (*staged of them)
+    static __device__ int host_run(Batch &B, World &W, WorldRun *R, int hl, int64_t t, int64_t *wake, const HostIn &hi, Frame *st, int st_cap,
+                                   int *staged)
     {
         const int64_t S0 = t * SLOT_PS, E0 = S0 + SLOT_PS;
         const int h = W.host0 + hl, lid = W.link0 + hl;
@@ -1852,34 +2085,13 @@ struct Model
         const unsigned long long pr0 = wall_clock64();
         unsigned long long pr_ev = 0, pr_n = 0;
 #endif
-        const int in = B.in_link[lid];
-        const Frame *m2 = nullptr, *m1 = nullptr;
-        int n2 = 0, n1 = 0, i2 = 0, i1 = 0;
-        // this slot's arrivals: the later part of slot t-2's message, the earlier of t-1's
-        if (t >= 2)
-        {
-            size_t r = (size_t)((t - 2) % NRING) * B.nlinks + in;
-            const long long v = coh_load(B.msg_cnt + r);
-            if (msg_slot(v) == t - 2)
-                i2 = msg_early(v), n2 = msg_sent(v);
-            m2 = B.msg + r * MAX_TX;
-        }
-        if (t >= 1)
-        {
-            size_t r = (size_t)((t - 1) % NRING) * B.nlinks + in;
-            const long long v = coh_load(B.msg_cnt + r);
-            n1 = msg_slot(v) == t - 1 ? msg_early(v) : 0;
-            m1 = B.msg + r * MAX_TX;
-        }
-        bool input = i2 < n2 || n1 > 0;
-        if (!input && t < B.wake[h] && B.q_size[lid] == 0)
-        {
-            *wake = B.wake[h];
-            return 0;
-        }
+        const Frame *m2 = B.msg + ((size_t)((t + NRING - 2) % NRING) * B.nlinks + hi.in) * MAX_TX;
+        const Frame *m1 = B.msg + ((size_t)((t + NRING - 1) % NRING) * B.nlinks + hi.in) * MAX_TX;
+        const int n2 = hi.n2, n1 = hi.n1;
+        int i2 = hi.i2, i1 = 0;
         const int rt = (int)(t % NRING);
         Host x;
-        x.nic.load(B, R, lid, t, rt);
+        x.nic.load(B, W, R, lid, t, rt, st, st_cap);
         x.B = &B;
         x.W = &W;
         x.R = R;
@@ -1889,9 +2101,12 @@ struct Model
         x.cubic = B.host_cc[h] == CC_CUBIC;
         x.due = B.due + (size_t)h * MAX_DUE;
         x.slot_end = E0;
-        x.ls = ls;
-        x.lr = lr;
-        x.lc = lc;
+        x.sf = x.rf = -1;
+        x.S = SndState{};
+        x.Q = RcvState{};
+        x.cs = ConnSnd{};
+        x.cr = ConnRcv{};
+        x.max_it = 0;
         Due *due = x.due;
         // timers due in this slot, by time. A list is scanned only when one of its timers falls in
         // the slot: tmin_s / tmin_r are its earliest, exact since the end of the host's last slot
@@ -1901,36 +2116,36 @@ struct Model
         const bool scan_s = bound_s < E0, scan_r = bound_r < E0;
         const int ns = scan_s ? B.n_snd[h] : 0, nr = scan_r ? B.n_rcv[h] : 0;
         const int32_t *as = B.act_snd + (size_t)h * MAX_ACTIVE, *ar = B.act_rcv + (size_t)h * MAX_ACTIVE;
-        for (int i = 0; i < ns; i++)
+        for (int i = 0; U(i < ns); i++)
         {
             int f = as[i];
             int64_t a = B.snd[f].rto_at, b = B.snd[f].syn_at;
-            if (a >= 0 && a < E0 && nd < MAX_DUE)
+            if (U(a >= 0 && a < E0 && nd < MAX_DUE))
                 due[nd++] = {a, f, 0};
-            if (b >= 0 && b < E0 && nd < MAX_DUE)
+            if (U(b >= 0 && b < E0 && nd < MAX_DUE))
                 due[nd++] = {b, f, 2};
         }
-        for (int i = 0; i < nr; i++)
+        for (int i = 0; U(i < nr); i++)
         {
             int f = ar[i];
             const RcvState &r = B.rcv[f];
             int64_t a = r.delack_at, b = r.srv_syn_at, l = r.r_last_at, xx = r.r_frx_at;
-            if (a >= 0 && a < E0 && nd < MAX_DUE)
+            if (U(a >= 0 && a < E0 && nd < MAX_DUE))
                 due[nd++] = {a, f, 1};
-            if (b >= 0 && b < E0 && nd < MAX_DUE)
+            if (U(b >= 0 && b < E0 && nd < MAX_DUE))
                 due[nd++] = {b, f, 3};
-            if (l >= 0 && l < E0 && nd < MAX_DUE)
+            if (U(l >= 0 && l < E0 && nd < MAX_DUE))
                 due[nd++] = {l, f, 4};
-            if (xx >= 0 && xx < E0 && nd < MAX_DUE)
+            if (U(xx >= 0 && xx < E0 && nd < MAX_DUE))
                 due[nd++] = {xx, f, 5};
         }
-        if (nd >= MAX_DUE)
+        if (U(nd >= MAX_DUE))
             count(R, EV_DUE_OVF);
-        for (int i = 1; i < nd; i++)
+        for (int i = 1; U(i < nd); i++)
         {
             Due v = due[i];
             int j = i - 1;
-            while (j >= 0 && due[j].at > v.at)
+            while (U(j >= 0 && due[j].at > v.at))
             {
                 due[j + 1] = due[j];
                 j--;
@@ -1949,17 +2164,17 @@ struct Model
         // (the next arrival's whole frame is read with its time, so taking it waits for no load)
         Frame fa;
         auto next_arrival = [&]() -> int64_t {
-            if (i2 >= n2 && i1 >= n1)
+            if (U(i2 >= n2 && i1 >= n1))
                 return INT64_MAX;
             fa = coh_get(i2 < n2 ? m2 + i2 : m1 + i1);
             return fa.ts;
         };
         auto next_start = [&](int &m) -> int64_t {
             m = pn < pe ? B.pend_msg[pn] : -1;
-            if (m >= 0)
+            if (U(m >= 0))
             {
                 const int64_t at = B.mg_start[m];
-                if (at < E0)
+                if (U(at < E0))
                     return at;
             }
             return INT64_MAX;
@@ -1969,21 +2184,23 @@ struct Model
 #ifdef TW_PROF
         const unsigned long long pr1 = wall_clock64();
 #endif
+        x.fill = x.has_post = false;
         for (;;)
         {
             const int64_t td = x.due_head;
             int64_t now = tr < td ? tr : td;
             now = now < tp ? now : tp;
-            if (now == INT64_MAX)
+            const bool last = now == INT64_MAX;
+            now = now < S0 ? S0 : now;
+            x.nic.advance(last ? E0 - 1 : now);
+            if (U(last))
                 break;
-            if (now < S0)
-                now = S0;
-            x.nic.advance(now);
+            x.n_ask = x.i_ask = 0;
 #ifdef TW_PROF
             const unsigned long long pq = wall_clock64();
             pr_n++;
 #endif
-            if (now == tp && B.cs[B.mg_conn[pm]].m_first != pm)
+            if (U(now == tp && B.cs[B.mg_conn[pm]].m_first != pm))
             {
                 // a later message of a connection (FlowSender::SendMessage)
                 const int m = pm;
@@ -1993,11 +2210,10 @@ struct Model
                 chain_root_msg(x.echain, m - W.msg0);
                 SndState &s = snd_open(x, f);
                 s.m_due++;
-                if (s.st == S_EST)
-                    app_write(x, f, now);
-                snd_close(x, f);
+                if (U(s.st == S_EST))
+                    app_write(x, f, now, x.echain);
             }
-            else if (now == tp)
+            else if (U(now == tp))
             {
                 // a connection's application starts: SYN
                 const int m = pm;
@@ -2009,39 +2225,37 @@ struct Model
                 s.m_due = 1;
                 add_active(x, true, f);
                 s.st = S_SYN_SENT;
-                if (x.cubic)
-                    cubic_round_start(s, now);
+                if (U(x.cubic))
+                    cubic_round_start(x, now);
                 s.rto = CONN_TIMEOUT_PS;
                 s.syn_at = now + CONN_TIMEOUT_PS;
                 timer_chain(x, B.rchain, f, CONN_TIMEOUT_PS);
                 s.timing_time = now;
                 emit(x, f, F_SYN, 0, 0, SYN_FRAME, false, now);
-                snd_close(x, f);
             }
-            else if (now == td && (now != tr || timer_before_arrival(x, due[x.id], i2 < n2 ? m2 + i2 : m1 + i1)))
+            else if (U(now == td && (now != tr || timer_before_arrival(x, due[x.id], i2 < n2 ? m2 + i2 : m1 + i1))))
             {
                 Due d = due[x.id++];
                 x.due_head = x.id < x.nd ? due[x.id].at : INT64_MAX;
-                chain_load(x.echain, due_chain(B, d));
+                chain_load(x.echain, due_chain(x, d));
                 const int f = d.flow;
-                if (d.kind == 0)
+                if (U(d.kind == 0))
                 {
-                    if (B.snd[f].rto_at == d.at)
+                    if (U((x.sf == f ? x.S.rto_at : B.snd[f].rto_at) == d.at))
                     {
                         snd_open(x, f);
                         rto_fire(x, f, now);
-                        snd_close(x, f);
                     }
                 }
-                else if (d.kind == 2)
+                else if (U(d.kind == 2))
                 {
                     SndState &s = snd_open(x, f);
-                    if (s.syn_at == d.at && s.st == S_EST)
+                    if (U(s.syn_at == d.at && s.st == S_EST))
                     {
                         s.syn_at = -1; // the deferred SendPendingData
-                        tx_fill(x, f, now);
+                        tx_fill(x);
                     }
-                    else if (s.syn_at == d.at && s.st == S_SYN_SENT)
+                    else if (U(s.syn_at == d.at && s.st == S_SYN_SENT))
                     {
                         int tries = ++s.syn_tries; // SYN retransmission, backed off
                         s.rto = CONN_TIMEOUT_PS << tries;
@@ -2049,21 +2263,20 @@ struct Model
                         timer_chain(x, B.rchain, f, s.rto);
                         emit(x, f, F_SYN, 0, 0, SYN_FRAME, false, now);
                     }
-                    snd_close(x, f);
                 }
                 else
                 {
                     RcvState &r = rcv_open(x, f);
-                    if (d.kind == 1 && r.delack_at == d.at)
+                    if (U(d.kind == 1 && r.delack_at == d.at))
                     {
                         r.delack_at = -1;
                         r.delack_count = 0;
                         r.reserved = 1;
                         rcv_ack(x, f, r.rcv_nxt, false, false, now);
                     }
-                    else if (d.kind == 4 && r.r_last_at == d.at && r.r_st == R_LAST_ACK)
+                    else if (U(d.kind == 4 && r.r_last_at == d.at && r.r_st == R_LAST_ACK))
                     {
-                        if (r.r_last_n == 0)
+                        if (U(r.r_last_n == 0))
                             rcv_closed(r);
                         else
                         {
@@ -2074,23 +2287,22 @@ struct Model
                             timer_chain(x, B.dchain, f, lr);
                         }
                     }
-                    else if (d.kind == 5 && r.r_frx_at == d.at && r.r_st == R_LAST_ACK)
+                    else if (U(d.kind == 5 && r.r_frx_at == d.at && r.r_st == R_LAST_ACK))
                     {
                         r.r_frx_at = -1;
                         rcv_fin_ack(x, f, now);
                     }
-                    else if (d.kind == 3 && r.srv_syn_at == d.at && !r.r_est)
+                    else if (U(d.kind == 3 && r.srv_syn_at == d.at && !r.r_est))
                     {
                         r.srv_syn_at = -1;
                         rcv_synack(x, f, now);
                     }
-                    rcv_close(x, f);
                 }
             }
             else
             {
                 const Frame p = fa;
-                if (i2 < n2)
+                if (U(i2 < n2))
                     i2++;
                 else
                     i1++;
@@ -2100,6 +2312,17 @@ struct Model
                 chain_child(x.echain, 2048u + p.len, pc);
                 on_frame(x, p, now);
             }
+            // what the event sends, into the queue in order (made here once for all events: inlined at
+            // every sender, the frame's making and the queue's advance were most of the code)
+            bool first = true;
+            Out o;
+            while (U(next_out(x, now, &o)))
+            {
+                if (U(!first))
+                    x.nic.advance(now); // (the event began with the queue advanced)
+                first = false;
+                x.nic.enqueue(frame_of(x, o, now), now);
+            }
 #ifdef TW_PROF
             pr_ev += wall_clock64() - pq;
 #endif
@@ -2107,15 +2330,19 @@ struct Model
 #ifdef TW_PROF
         const unsigned long long pr2 = wall_clock64();
 #endif
-        x.nic.advance(E0 - 1);
         x.nic.store(t, rt);
+        snd_flush(x);
+        rcv_flush(x);
+        if (U(x.max_it))
+            atomicMax(&R->ev[EV_MAX_INFLIGHT], (unsigned long long)x.max_it);
+        *staged = x.nic.sent < st_cap ? x.nic.sent : st_cap;
         B.pend_next[h] = pn;
         // drop finished connections from the active lists; their earliest timers; the next wake-up
         const int64_t nb_s = compact_snd(B, h), nb_r = compact_rcv(B, h);
         B.tmin_s[h] = nb_s;
         B.tmin_r[h] = nb_r;
         int64_t next = nb_s < nb_r ? nb_s : nb_r;
-        if (pn < pe && B.mg_start[B.pend_msg[pn]] < next)
+        if (U(pn < pe && B.mg_start[B.pend_msg[pn]] < next))
             next = B.mg_start[B.pend_msg[pn]];
         int64_t wk = x.nic.size > 0 ? t + 1 : (next == INT64_MAX ? INT64_MAX : next / SLOT_PS);
         B.wake[h] = wk;
@@ -2132,19 +2359,19 @@ struct Model
     }
 
     // -------------------------------------------------------------- routing (src/step.cuh:2541-2630)
-    static __device__ int epoch_of(const Batch &B, const WorldDesc &W, int64_t ts)
+    static __device__ int epoch_of(Batch &B, World &W, int64_t ts)
     {
         int e = 0;
         while (e < W.n_fail && ts >= B.g_fail_t[W.o_fail + e])
             e++;
         return e;
     }
-    static __device__ __forceinline__ size_t rt_index(const WorldDesc &W, int ep, int x, int e)
+    static __device__ __forceinline__ size_t rt_index(World &W, int ep, int x, int e)
     {
         return (size_t)W.o_rt + ((size_t)ep * W.S + x) * W.S + e;
     }
     // the output port at switch sw (world-local) towards host dst; up: the equal-cost index
-    static __device__ int route_up(const Batch &B, const WorldDesc &W, int sw, int dst, int up, int ep)
+    static __device__ int route_up(Batch &B, World &W, int sw, int dst, int up, int ep)
     {
         if (W.kind == TOPO_GRAPH)
         {
@@ -2167,7 +2394,7 @@ struct Model
             return dst_pod == (sw - E) / hk ? dst_edge : hk + up;
         return dst_pod;
     }
-    static __device__ int route(const Batch &B, const WorldDesc &W, int sw, const FrameHead &p, int ep)
+    static __device__ int route(Batch &B, World &W, int sw, const FrameHead &p, int ep)
     {
         if (W.kind == TOPO_GRAPH)
         {
@@ -2180,11 +2407,11 @@ struct Model
         }
         return route_up(B, W, sw, p.dst, p.up, ep);
     }
-    static __device__ __forceinline__ bool port_down(const Batch &B, const WorldDesc &W, int sw, int q, int ep)
+    static __device__ __forceinline__ bool port_down(Batch &B, World &W, int sw, int q, int ep)
     {
         return W.n_fail && B.g_port_dn[W.o_pdn + ((size_t)ep * W.S + sw) * W.k + q];
     }
-    static __device__ int routes_to(const Batch &B, const WorldDesc &W, int sw, int dst, int ep)
+    static __device__ int routes_to(Batch &B, World &W, int sw, int dst, int ep)
     {
         if (W.kind == TOPO_GRAPH)
         {
@@ -2220,13 +2447,16 @@ struct Model
     // cnt[k]; per-wave global scratch holds the arrivals sorted per egress.
     // a switch item's LDS: per lane rows (33 ints), in_win (3), base, cnt, then (after the
     // spray merge's 64) per lane SORT_LDS arrival times and refs for the egress sort, then per
-    // lane the egress ports of its first EGRESS_LDS arrivals (one byte each: the count phase
-    // routes them, the scatter phase reads the routes back), then per lane its port's in-link
-    static constexpr int SW_LDS_INTS = 64 * 33 + 64 * 3 + 64 + 64, SORT_LDS = 24, EGRESS_LDS = 64;
+    // lane its first EGRESS_LDS arrivals' times in the slot (20 bits) and egress ports (above: the
+    // count phase reads and routes them, the scatter phase reads no frame), then per lane its port's
+    // in-link
+    static constexpr int SW_LDS_INTS = 64 * 33 + 64 * 3 + 64 + 64, SORT_LDS = 24, EGRESS_LDS = 40;
     static constexpr int SW_LDS_EGRESS = SW_LDS_INTS + 64 * SORT_LDS * 3;
-    static constexpr int SW_LDS_INLINK = SW_LDS_EGRESS + 64 * EGRESS_LDS / 4;
+    static constexpr int SW_LDS_INLINK = SW_LDS_EGRESS + 64 * EGRESS_LDS;
     static constexpr int SW_LDS_TOTAL = SW_LDS_INLINK + 64;
-    static constexpr uint8_t NO_EGRESS = 0xFF;
+    static constexpr uint32_t NO_EGRESS = 0xFF;
+    static_assert(SLOT_PS < 1 << 20, "an arrival's time in its slot: 20 bits");
+    static constexpr int COUNT_RUN = 4; // arrivals' heads read together
     struct SwLds
     {
         int *rows, *in_win, *base, *cnt;
@@ -2241,7 +2471,7 @@ struct Model
         __device__ const Frame *at(int j) const { return j < n2 - i2 ? m2 + i2 + j : m1 + (j - (n2 - i2)); }
         __device__ FrameHead head(int j) const { return msg_head(at(j)); }
     };
-    static __device__ In input_of(const Batch &B, int link, int64_t t, const int *win)
+    static __device__ In input_of(Batch &B, int link, int64_t t, const int *win)
     {
         In in;
         in.i2 = win[0];
@@ -2266,7 +2496,7 @@ struct Model
         uint8_t *scr_up;
     };
     // port q's input of the slot (its in-link from LDS, where the window phase put it)
-    static __device__ In lane_input(const Batch &B, const WorldDesc &W, const SwLane &x, int64_t t, const SwLds &L, int q)
+    static __device__ In lane_input(Batch &B, World &W, const SwLane &x, int64_t t, const SwLds &L, int q)
     {
         return input_of(B, L.wave[SW_LDS_INLINK + sw_lane_of(L, x) - x.q + q], t, L.in_win + 3 * q);
     }
@@ -2275,11 +2505,11 @@ struct Model
     {
         return (int)(L.cnt - L.wave - (64 * 33 + 64 * 3 + 64)) + x.q;
     }
-    static __device__ __forceinline__ uint8_t *lane_egress_lds(const SwLds &L, const SwLane &x)
+    static __device__ __forceinline__ uint32_t *lane_egress_lds(const SwLds &L, const SwLane &x)
     {
-        return reinterpret_cast<uint8_t *>(L.wave + SW_LDS_EGRESS) + sw_lane_of(L, x) * EGRESS_LDS;
+        return reinterpret_cast<uint32_t *>(L.wave + SW_LDS_EGRESS) + sw_lane_of(L, x) * EGRESS_LDS;
     }
-    static __device__ int lane_egress(const Batch &B, const WorldDesc &W, const SwLane &x, int j, const FrameHead &p)
+    static __device__ int lane_egress(Batch &B, World &W, const SwLane &x, int j, const FrameHead &p)
     {
         int ep = W.n_fail ? epoch_of(B, W, p.ts) : 0;
         if (port_down(B, W, x.swl, x.q, ep))
@@ -2288,7 +2518,7 @@ struct Model
     }
     // 1: the ingress window of port q (tail of slot t-2's message from S0 on, head of t-1's
     // before E0) into LDS; the port's row of egress counts cleared
-    static __device__ void sw_window(const Batch &B, const WorldDesc &W, const SwLane &x, int64_t t, const SwLds &L)
+    static __device__ void sw_window(Batch &B, World &W, const SwLane &x, int64_t t, const SwLds &L)
     {
         if (!x.active)
             return;
@@ -2317,27 +2547,39 @@ struct Model
             row[i] = 0;
     }
     // 2: arrivals counted by egress (after the spray draws, if any)
-    static __device__ void sw_count(const Batch &B, const WorldDesc &W, WorldRun *R, const SwLane &x, int64_t t, const SwLds &L)
+    static __device__ void sw_count(Batch &B, World &W, WorldRun *R, const SwLane &x, int64_t t, const SwLds &L)
     {
         if (!x.active)
             return;
         In in = lane_input(B, W, x, t, L, x.q);
         int *row = L.rows + x.q * (W.k + 1);
-        uint8_t *eg = lane_egress_lds(L, x);
+        uint32_t *eg = lane_egress_lds(L, x);
         const int n = in.count();
-        for (int j = 0; j < n; j++)
+        // (COUNT_RUN heads at a time: one after another each was a wait of its own)
+        for (int j0 = 0; j0 < n; j0 += COUNT_RUN)
         {
-            int e = lane_egress(B, W, x, j, in.head(j));
-            if (j < EGRESS_LDS)
-                eg[j] = e >= 0 ? (uint8_t)e : NO_EGRESS;
-            if (e >= 0)
-                row[e]++;
-            else
-                count(R, EV_DROP);
+            FrameHead h[COUNT_RUN];
+#pragma unroll
+            for (int u = 0; u < COUNT_RUN; u++)
+                h[u] = in.head(j0 + u < n ? j0 + u : n - 1);
+#pragma unroll
+            for (int u = 0; u < COUNT_RUN; u++)
+            {
+                const int j = j0 + u;
+                if (j >= n)
+                    break;
+                const int e = lane_egress(B, W, x, j, h[u]);
+                if (j < EGRESS_LDS)
+                    eg[j] = (uint32_t)(h[u].ts - t * SLOT_PS) | (e >= 0 ? (uint32_t)e : NO_EGRESS) << 20;
+                if (e >= 0)
+                    row[e]++;
+                else
+                    count(R, EV_DROP);
+            }
         }
     }
     // 3: for egress q, each ingress's offset in its region and the region's size
-    static __device__ void sw_prefix(const WorldDesc &W, const SwLane &x, const SwLds &L)
+    static __device__ void sw_prefix(World &W, const SwLane &x, const SwLds &L)
     {
         if (!x.active)
             return;
@@ -2377,23 +2619,35 @@ struct Model
 #endif
     }
     // 5: every arrival of ingress q into its egress's region, in arrival order
-    static __device__ void sw_scatter(const Batch &B, const WorldDesc &W, const SwLane &x, int64_t t, const SwLds &L)
+    static __device__ void sw_scatter(Batch &B, World &W, const SwLane &x, int64_t t, const SwLds &L)
     {
         if (!x.active)
             return;
         In in = lane_input(B, W, x, t, L, x.q);
         int *row = L.rows + x.q * (W.k + 1);
-        const uint8_t *eg = lane_egress_lds(L, x);
+        const uint32_t *eg = lane_egress_lds(L, x);
         const int n = in.count();
         auto scatter = [&](auto *ts, auto *ref) {
             for (int j = 0; j < n; j++)
             {
-                const FrameHead p = in.head(j);
-                const int e = j < EGRESS_LDS ? (eg[j] == NO_EGRESS ? -1 : (int)eg[j]) : lane_egress(B, W, x, j, p);
+                int64_t at_ts;
+                int e;
+                if (j < EGRESS_LDS)
+                {
+                    const uint32_t v = eg[j];
+                    at_ts = t * SLOT_PS + (v & 0xFFFFF);
+                    e = v >> 20 == NO_EGRESS ? -1 : (int)(v >> 20);
+                }
+                else
+                {
+                    const FrameHead p = in.head(j);
+                    at_ts = p.ts;
+                    e = lane_egress(B, W, x, j, p);
+                }
                 if (e < 0)
                     continue;
                 int at = L.base[e] + row[e]++;
-                ts[at] = p.ts;
+                ts[at] = at_ts;
                 ref[at] = (uint32_t)(x.q << 16 | j);
             }
         };
@@ -2404,7 +2658,7 @@ struct Model
     }
     // the switch's egress lists go to LDS (its lanes' SORT_LDS slots each, laid out by L.base)
     // when all of them fit there, else to the wave's device scratch
-    static __device__ __forceinline__ bool sw_lists_in_lds(const WorldDesc &W, const SwLds &L)
+    static __device__ __forceinline__ bool sw_lists_in_lds(World &W, const SwLds &L)
     {
         return L.base[W.k - 1] + L.cnt[W.k - 1] <= W.k * SORT_LDS;
     }
@@ -2419,21 +2673,22 @@ struct Model
     }
     // 6: egress q's arrivals sorted by (time, frame_before), enqueued with the arrival event's
     // chain (RED), and the slot's transmissions; returns 1 if the port sent or holds frames
-    static __device__ int sw_egress(const Batch &B, const WorldDesc &W, WorldRun *R, const SwLane &x, int64_t t, const SwLds &L)
+    static __device__ int sw_egress(Batch &B, World &W, WorldRun *R, const SwLane &x, int64_t t, const SwLds &L)
     {
         if (!x.active)
             return 0;
         const int n = L.cnt[x.q], b0 = L.base[x.q];
+        if (n == 0 && B.q_size[x.lid] == 0)
+            return 0; // (nothing to send: the port's message of an older slot stands for an empty one)
         auto frame_at = [&](uint32_t r) -> const Frame * { return lane_input(B, W, x, t, L, (int)(r >> 16)).at((int)(r & 0xFFFF)); };
         Fifo eg;
         const int rt = (int)(t % NRING);
-        eg.load(B, R, x.lid, t, rt);
+        eg.load(B, W, R, x.lid, t, rt);
         // an insertion sort by (time, frame_before): chain comparison is no strict weak order
-        // when chains are truncated, and this gives the reference's order in every case; then the
-        // arrivals in that order into the queue. (Inlined at two calls, for the list in LDS and for
-        // the list in device scratch, so that each copy's accesses have one address space: LDS or
-        // global instructions, not flat ones that wait on both.)
-        auto sort_enqueue = [&](auto *ts, auto *ref) {
+        // when chains are truncated, and this gives the reference's order in every case. (Inlined at
+        // two calls, for a list in LDS and for one in device scratch, so that each copy's accesses have
+        // one address space: LDS or global instructions, not flat ones that wait on both.)
+        auto sort = [&](auto *ts, auto *ref) {
             for (int i = 1; i < n; i++)
             {
                 const int64_t xv = ts[i];
@@ -2448,40 +2703,51 @@ struct Model
                 ts[j + 1] = xv;
                 ref[j + 1] = r;
             }
-            for (int i = 0; i < n; i++)
-            {
-                Frame p = coh_get(frame_at(ref[i]));
-                Chain up, c;
-                chain_load(up, p.chain);
-                chain_child(c, 2048u + p.len, up);
-                chain_store(p.chain, c);
-                eg.enqueue(p, p.ts);
-            }
         };
-        if (sw_lists_in_lds(W, L))
-            sort_enqueue(sort_ts_lds(L, x) + b0, sort_ref_lds(L, x) + b0); // (the usual case: scattered into LDS)
-        else if (n <= SORT_LDS)
+        // where the sorted refs are: in LDS when all of the switch's lists were scattered there, or for a
+        // short list of a switch whose lists overflow LDS (copied to the lane's own slots: one round of
+        // loads instead of a device-memory round trip per comparison and move), else in device scratch
+        const bool all_lds = sw_lists_in_lds(W, L), in_lds = all_lds || n <= SORT_LDS;
+        const int lane = sw_lane_of(L, x);
+        int64_t *lts = all_lds ? sort_ts_lds(L, x) + b0 : reinterpret_cast<int64_t *>(L.wave + SW_LDS_INTS) + lane * SORT_LDS;
+        uint32_t *lref = all_lds ? sort_ref_lds(L, x) + b0 : reinterpret_cast<uint32_t *>(L.wave + SW_LDS_INTS + 2 * 64 * SORT_LDS) + lane * SORT_LDS;
+        if (in_lds)
         {
-            // a short list of a switch whose lists overflow LDS is sorted in the lane's own slots:
-            // one round of loads instead of a device-memory round trip per comparison and move
-            const int lane = sw_lane_of(L, x);
-            int64_t *lts = reinterpret_cast<int64_t *>(L.wave + SW_LDS_INTS) + lane * SORT_LDS;
-            uint32_t *lref = reinterpret_cast<uint32_t *>(L.wave + SW_LDS_INTS + 2 * 64 * SORT_LDS) + lane * SORT_LDS;
-            for (int i = 0; i < n; i++)
-            {
-                lts[i] = x.scr_ts[b0 + i];
-                lref[i] = x.scr_ref[b0 + i];
-            }
-            sort_enqueue(lts, lref);
+            if (!all_lds)
+                for (int i = 0; i < n; i++)
+                {
+                    lts[i] = x.scr_ts[b0 + i];
+                    lref[i] = x.scr_ref[b0 + i];
+                }
+            sort(lts, lref);
         }
         else
-            sort_enqueue(x.scr_ts + b0, x.scr_ref + b0);
-        eg.advance((t + 1) * SLOT_PS - 1);
+            sort(x.scr_ts + b0, x.scr_ref + b0);
+        // in that order into the queue, then the slot's transmissions; the next arrival is read while one
+        // is queued (before its transmissions' stores, which a later load would wait for)
+        auto ref_at = [&](int i) -> uint32_t { return in_lds ? lref[i] : x.scr_ref[b0 + i]; };
+        Frame nx;
+        if (n > 0)
+            nx = coh_get(frame_at(ref_at(0)));
+        for (int i = 0;; i++)
+        {
+            Frame p = nx;
+            if (i + 1 < n)
+                nx = coh_get(frame_at(ref_at(i + 1)));
+            eg.advance(i < n ? p.ts : (t + 1) * SLOT_PS - 1);
+            if (i >= n)
+                break;
+            Chain up, c;
+            chain_load(up, p.chain);
+            chain_child(c, 2048u + p.len, up);
+            chain_store(p.chain, c);
+            eg.enqueue(p, p.ts);
+        }
         eg.store(t, rt);
         return (eg.sent > 0 || eg.size > 0) ? 1 : 0;
     }
     // one slot of a switch on the GPU: the lanes of one wavefront, phases separated by wave_sync()
-    static __device__ int switch_step(const Batch &B, const WorldDesc &W, WorldRun *R, const SwLane &x, int64_t t, const SwLds &L)
+    static __device__ int switch_step(Batch &B, World &W, WorldRun *R, const SwLane &x, int64_t t, const SwLds &L)
     {
 #ifdef TW_PROF
         // profiler builds: the phases' wall-clock ticks, summed over switch items (counters 20-23)
@@ -2496,7 +2762,12 @@ struct Model
 #else
 #define TW_PHASE(i)
 #endif
+        // (a switch with no arrivals and nothing queued has no events)
+        const int queued = x.active ? B.q_size[x.lid] : 0;
         sw_window(B, W, x, t, L);
+        const int *win = L.in_win + 3 * x.q;
+        if (!__any(x.active && (queued || win[1] > win[0] || win[2])))
+            return 0;
         if (W.rng0 >= 0)
         {
             wave_sync();
@@ -2552,7 +2823,7 @@ struct Model
         bool done;
     };
     // the packed entry of arrival j: time offset (20 bits), route count or 255 (a down port)
-    static __device__ uint32_t spray_code(const Batch &B, const WorldDesc &W, const SwLane &x, int64_t S0, const FrameHead &f)
+    static __device__ uint32_t spray_code(Batch &B, World &W, const SwLane &x, int64_t S0, const FrameHead &f)
     {
         const int ep = W.n_fail ? epoch_of(B, W, f.ts) : 0;
         const uint32_t nr = port_down(B, W, x.swl, x.q, ep) ? 255u : (uint32_t)routes_to(B, W, x.swl, f.dst, ep);
@@ -2560,13 +2831,13 @@ struct Model
     }
     // this port's lane in the wavefront (its switch's first lane, base, plus the port)
     static __device__ int spray_lane(const SwLane &x, const SwLds &L) { return sw_lane_of(L, x); }
-    static __device__ uint32_t spray_entry(const Batch &B, const WorldDesc &W, const SwLane &x, const SwLds &L, const Spray &sp, int64_t S0, int j)
+    static __device__ uint32_t spray_entry(Batch &B, World &W, const SwLane &x, const SwLds &L, const Spray &sp, int64_t S0, int j)
     {
         if (j < SPRAY_CACHE)
             return (uint32_t)L.wave[spray_lane(x, L) * 33 + j];
         return spray_code(B, W, x, S0, sp.in.head(j));
     }
-    static __device__ void spray_init(const Batch &B, const WorldDesc &W, const SwLane &x, int64_t t, const SwLds &L, Spray &sp)
+    static __device__ void spray_init(Batch &B, World &W, const SwLane &x, int64_t t, const SwLds &L, Spray &sp)
     {
         sp.c = 0;
         sp.p = 0;
@@ -2596,7 +2867,7 @@ struct Model
         L.base[x.q] = sp.p;
     }
     // one step of the merge; true when the switch has no arrivals left
-    static __device__ bool spray_pick(const Batch &B, const WorldDesc &W, WorldRun *R, const SwLane &x, int64_t t, const SwLds &L, Spray &sp)
+    static __device__ bool spray_pick(Batch &B, World &W, WorldRun *R, const SwLane &x, int64_t t, const SwLds &L, Spray &sp)
     {
         if (!x.active || sp.done)
             return true;
@@ -2642,7 +2913,7 @@ struct Model
         }
         return false;
     }
-    static __device__ void spray_end(const Batch &B, const WorldDesc &W, const SwLane &x, const SwLds &L, Spray &sp)
+    static __device__ void spray_end(Batch &B, World &W, const SwLane &x, const SwLds &L, Spray &sp)
     {
         if (!x.active)
             return;

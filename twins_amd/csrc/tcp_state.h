@@ -32,6 +32,22 @@
 namespace tw
 {
 
+// The batch record and a world's description, which nothing writes while a launch runs: in the
+// constant address space their fields are scalar loads that wait for no store. The serving kernel
+// (SRV) reads them as global memory: it sees new ones in the same places while it runs.
+template <typename T, bool SRV>
+struct ReadOnly
+{
+    typedef const T type;
+};
+#if defined(__HIP_DEVICE_COMPILE__)
+template <typename T>
+struct ReadOnly<T, false>
+{
+    typedef const T __attribute__((address_space(4))) type;
+};
+#endif
+
 // Device-coherent accesses (coherent.h): what a team's workgroups hand each other from slot to slot
 using twc::coh_get;
 using twc::coh_load;
@@ -159,8 +175,9 @@ struct alignas(16) ConnStatic // (64 bytes: moved into LDS in 16-byte pieces wit
 };
 static_assert(sizeof(ConnStatic) == 64, "ConnStatic: 64 bytes");
 
-// the sending side (touched only by the sender's host)
-struct alignas(128) SndState
+// the sending side (touched only by the sender's host). In LDS as it is; in device memory each record
+// starts a cache line of its own (SndRec), since the two ends of a connection may run on two XCDs.
+struct alignas(16) SndState
 {
     uint32_t tail, una, nxt, high, cwnd, ssthresh, dupacks, recover;
     uint32_t it_head, it_n, sack_b, lost_b, rtx_b, sacked_n, cand_n, cand;
@@ -174,14 +191,34 @@ struct alignas(128) SndState
     double cub_k;
     int64_t cub_delaymin, cub_epoch, cub_roundstart, cub_lastack, cub_currrtt;
 };
+struct alignas(128) SndRec : SndState
+{
+};
+static_assert(sizeof(SndState) == 272 && sizeof(SndRec) == 384, "SndState: 17 pieces of 16 bytes");
 
 // the receiving side (touched only by the receiver's host)
-struct alignas(128) RcvState
+struct alignas(16) RcvState
 {
     uint32_t rcv_nxt, ooo_n, ooo_h, prior_rcv_nxt;
     uint8_t r_up, r_est, r_st, r_last_n, srv_syn_n, delack_count, ce_state, prior_flag;
     uint8_t reserved, ecn_r, pad[6];
     int64_t r_fin, r_synack_t, r_srtt, r_rttvar, r_last_at, r_frx_at, srv_syn_at, delack_at, ecn_ce_seq;
+};
+struct alignas(128) RcvRec : RcvState
+{
+};
+static_assert(sizeof(RcvState) == 112 && sizeof(RcvRec) == 128, "RcvState: 7 pieces of 16 bytes");
+
+// an entry of a sent ledger (its first byte, its marks) and an RTT note (when, from which byte, how
+// many): records, so that a look at one is one load
+struct alignas(8) SentEntry
+{
+    uint32_t first, mark;
+};
+struct alignas(16) SentNote
+{
+    int64_t t;
+    uint32_t seq, cnt;
 };
 
 // MRG32k3a state (the layout of TwMrg in exact_math.h)
@@ -307,12 +344,12 @@ struct BatchT
     WorldRun TW_G *run;
     // connections
     ConnStatic TW_G *cs;
-    SndState TW_G *snd;
-    RcvState TW_G *rcv;
+    SndRec TW_G *snd;
+    RcvRec TW_G *rcv;
     uint32_t TW_G *rchain, *schain, *dchain, *fchain; // [conn][CW] timer chains
-    uint32_t TW_G *it_start, *h_seq, *h_cnt, *oo_s, *oo_e;
-    uint8_t TW_G *it_fl;
-    int64_t TW_G *h_t;
+    SentEntry TW_G *it; // rings of the sent ledgers
+    SentNote TW_G *ht;  // and of the RTT notes
+    uint32_t TW_G *oo_s, *oo_e;
     // messages
     int32_t TW_G *mg_conn;
     uint32_t TW_G *mg_end;

@@ -583,7 +583,7 @@ static uint64_t world_bytes(const tw_world &w, int runs)
     uint64_t b = 0;
     b += (uint64_t)NRING * w.L * MAX_TX * F + (uint64_t)NRING * w.L * 8;          // link messages
     b += (uint64_t)w.L * (std::max(w.queue, 1) + 2) * F + (uint64_t)w.L * (40 + CHB); // queues
-    b += (uint64_t)w.NC * (sizeof(ConnStatic) + sizeof(SndState) + sizeof(RcvState) + 4 * CHB);
+    b += (uint64_t)w.NC * (sizeof(ConnStatic) + sizeof(SndRec) + sizeof(RcvRec) + 4 * CHB);
     b += w.it_total * 21 + w.oo_total * 8;
     b += (uint64_t)w.M * 40 + (uint64_t)w.H * (2 * MAX_ACTIVE * 4 + MAX_DUE * 16 + 40);
     b += w.rt_off.size() * 5 + w.rt_ports.size() + w.port_dn.size() + w.rng.size() * 48;
@@ -1003,8 +1003,8 @@ static int pack(tw_batch &b, const tw_pack_cfg &cfg)
     B.nworlds = W, B.nhosts = (int32_t)H, B.nswitches = (int32_t)S, B.nlinks = (int32_t)L, B.nconns = (int32_t)NC, B.nmsgs = (int32_t)M;
     // host-side images
     std::vector<ConnStatic> cs(NC);
-    std::vector<SndState> snd(NC);
-    std::vector<RcvState> rcv(NC);
+    std::vector<SndRec> snd(NC);
+    std::vector<RcvRec> rcv(NC);
     std::vector<int32_t> mg_conn(M), pend_msg(M), host_world(H), pend_next(H), pend_end(H), in_link(L, -1), sw_world(S);
     std::vector<uint32_t> mg_end(M), g_rt_off(RT);
     std::vector<int64_t> mg_start(M), neg(M, -1), g_fail(FT), wake(H, 0), neg_links(L, 0);
@@ -1014,14 +1014,14 @@ static int pack(tw_batch &b, const tw_pack_cfg &cfg)
     std::vector<int32_t> q_cap(L), q_red_k(L), q_limit(L);
     std::vector<TwMrgState> rng(RNG);
     std::vector<WorldRun> run(W);
-    SndState s0;
-    memset(&s0, 0, sizeof s0);
+    SndRec s0;
+    memset((void *)&s0, 0, sizeof s0);
     s0.cwnd = INIT_CWND, s0.ssthresh = 0xFFFFFFFFu, s0.first_partial = 1;
     s0.cub_delaymin = s0.cub_epoch = s0.cub_roundstart = s0.cub_lastack = s0.cub_currrtt = INT64_MIN;
     s0.ecn_echo_seq = s0.ecn_cwr_seq = -1, s0.ecn_s = E_IDLE, s0.alpha = 1.0;
     s0.srtt = -1, s0.rttvar = 0, s0.rto = MIN_RTO_PS, s0.rto_at = -1, s0.timing_time = 0, s0.syn_at = -1;
-    RcvState r0;
-    memset(&r0, 0, sizeof r0);
+    RcvRec r0;
+    memset((void *)&r0, 0, sizeof r0);
     r0.r_st = R_OPEN, r0.r_fin = r0.r_synack_t = r0.r_srtt = r0.r_last_at = r0.r_frx_at = r0.srv_syn_at = r0.delack_at = r0.ecn_ce_seq = -1;
     r0.ecn_r = E_IDLE;
     uint64_t qf = 0;
@@ -1106,11 +1106,8 @@ static int pack(tw_batch &b, const tw_pack_cfg &cfg)
     ZERO(schain, NC * CW);
     ZERO(dchain, NC * CW);
     ZERO(fchain, NC * CW);
-    ZERO(it_start, IT);
-    ZERO(h_seq, IT);
-    ZERO(h_cnt, IT);
-    ZERO(it_fl, IT);
-    ZERO(h_t, IT);
+    ZERO(it, IT);
+    ZERO(ht, IT);
     ZERO(oo_s, OO);
     ZERO(oo_e, OO);
     UP(mg_conn, mg_conn);
@@ -1285,6 +1282,18 @@ static int pack(tw_batch &b, const tw_pack_cfg &cfg)
         return fail(TW_EINVAL, "the plan's %d workgroups exceed the %d the GPU holds at once (a team's workgroups must all be resident)",
                     blocks, resident);
     sh.blocks = blocks;
+    // one host per item everywhere? (each world on every team that may take it)
+    sh.one = 1;
+    for (int j = 0; j < nteams; j++)
+        for (int i = 0; i < W; i++)
+            if (world_q[i] == plan[j].queue)
+            {
+                const tw_world &w = *b.worlds[i];
+                int hpw = plan[j].hpw, spw = 0;
+                if (hpw <= 0)
+                    slot_items(w.H, w.S, w.k, plan[j].T * (sh.threads / 64), &hpw, &spw);
+                sh.one &= hpw == 1;
+            }
     sh.slot_budget = cfg.slot_budget > 0 ? cfg.slot_budget : 200000;
     UP(world_order, worder);
     UP(wq_off, wq_off);
