@@ -57,8 +57,8 @@ __device__ __forceinline__ void world_loop(const BatchT<RUNS> *__restrict__ Bp, 
     extern __shared__ __attribute__((aligned(128))) int lds[];
     __shared__ int s_w;
     __shared__ int64_t s_t;
-    __shared__ int s_done, s_err;
-    __shared__ unsigned s_act;
+    __shared__ int s_err;
+    __shared__ unsigned s_act, s_flags;
     __shared__ unsigned long long s_wake;
     __shared__ const BatchT<RUNS> *s_b;
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = blockDim.x >> 6;
@@ -75,23 +75,23 @@ __device__ __forceinline__ void world_loop(const BatchT<RUNS> *__restrict__ Bp, 
     uint32_t *scr_ref = (SRV ? Sp->scr_ref : Bp->scr_ref) + (size_t)gwave * 64 * 2 * MAX_TX;
     uint8_t *scr_up = (SRV ? Sp->scr_up : Bp->scr_up) + (size_t)gwave * 64 * 2 * MAX_TX;
     unsigned gen = 0; // the team barrier's generation this block has passed
+    unsigned slot_count = 0; // slots run in this launch (thread 0)
     // a barrier wait's limit; the server's claim waits as long as a request may take to come
     unsigned long long wait_limit = WAIT_TICKS;
 
-    // The team barrier; the last workgroup to arrive runs `last` first. Fenced (a world's start
-    // and end): agent-scope release and acquire, so that the world's records, written with plain
-    // stores, are in memory when it ends and no stale copy is read when it starts. Unfenced (the
-    // barrier between slots): what workgroups hand each other from slot to slot goes through
-    // device-coherent accesses only (coh_load / coh_store, tcp_state.h), so it is enough that
-    // every wave's stores have completed (s_waitcnt) before its workgroup arrives; the caches,
-    // and each entity's records in them, stay warm from slot to slot.
-    auto team_barrier = [&](auto last, bool fenced) -> bool {
+    // The barrier at a world's start and end; the last workgroup to arrive runs `last` first.
+    // Agent-scope release and acquire, so that the world's records, written with plain stores, are
+    // in memory when it ends and no stale copy is read when it starts. The barrier between slots
+    // (the end of the slot loop) has no cache fence: what workgroups hand each other from slot to
+    // slot goes through device-coherent accesses only (coh_load / coh_store, tcp_state.h), so it is
+    // enough that every wave's stores have completed (s_waitcnt) before its workgroup arrives; the
+    // caches, and each entity's records in them, stay warm from slot to slot.
+    auto team_barrier = [&](auto last) -> bool {
         __builtin_amdgcn_s_waitcnt(0); // (this wave's stores have completed)
         __syncthreads();
         if (tid == 0)
         {
-            if (fenced)
-                __threadfence();
+            __threadfence();
             if (T == 1)
                 last();
             else
@@ -119,8 +119,7 @@ __device__ __forceinline__ void world_loop(const BatchT<RUNS> *__restrict__ Bp, 
                 }
                 gen = g + 1;
             }
-            if (fenced)
-                __threadfence();
+            __threadfence();
             s_err = T > 1 && __hip_atomic_load(&ts->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         __syncthreads();
@@ -133,7 +132,7 @@ __device__ __forceinline__ void world_loop(const BatchT<RUNS> *__restrict__ Bp, 
         if constexpr (!SRV)
         {
             // the team's next world, from its queue
-            if (team_barrier([&] { ts->world = atomicAdd(Bp->queue_next + P.queue, 1); }, true))
+            if (team_barrier([&] { ts->world = atomicAdd(Bp->queue_next + P.queue, 1); }))
                 return;
             if (tid == 0)
                 s_w = __hip_atomic_load(&ts->world, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -169,7 +168,7 @@ __device__ __forceinline__ void world_loop(const BatchT<RUNS> *__restrict__ Bp, 
                     __builtin_amdgcn_s_sleep(8);
                 }
                 ts->world = got;
-            }, true);
+            });
             wait_limit = WAIT_TICKS;
             if (err)
                 return;
@@ -196,24 +195,32 @@ __device__ __forceinline__ void world_loop(const BatchT<RUNS> *__restrict__ Bp, 
         const int k = W.k;
         const int host_items = (W.H + hpw - 1) / hpw, items = host_items + (W.S + spw - 1) / spw;
         const unsigned long long c_begin = wall_clock64();
+        if (tid == 0)
+        {
+            s_t = __hip_atomic_load(&R->slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            s_flags = (__hip_atomic_load(&R->finished, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ? SlotGo::FIN : 0) |
+                      (__hip_atomic_load(&R->act_prev, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ? 0 : SlotGo::IDLE);
+            s_act = __hip_atomic_load(&R->act_cur, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); // (a world's first slot)
+            s_wake = ~0ull;
+        }
+        __syncthreads();
         for (int64_t it = 0;; it++)
         {
-            if (tid == 0)
-            {
-                s_t = __hip_atomic_load(&R->slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                s_done = __hip_atomic_load(&R->finished, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) || it >= slot_budget;
-                s_act = 0;
-                s_wake = ~0ull;
-            }
-            __syncthreads();
-            if (s_done)
+            const int64_t t = s_t;
+            const unsigned flags = s_flags;
+            if ((flags & SlotGo::FIN) || it >= slot_budget)
             {
                 // every workgroup of the team leaves at the same slot, after a fenced barrier (the
-                // world's records in memory before its results are read); the first accounts the
-                // time (and, serving, tells the host)
-                (void)team_barrier([] {}, true);
+                // world's records in memory before its results are read); the first writes where
+                // the world stands, accounts the time (and, serving, tells the host)
+                (void)team_barrier([] {});
                 if (rank == 0 && tid == 0)
                 {
+                    R->slot = t;
+                    R->slots_run += it;
+                    R->act_cur = 0;
+                    R->act_prev = flags & SlotGo::IDLE ? 0 : 1;
+                    R->finished = flags & SlotGo::FIN ? 1 : 0;
                     R->ticks += wall_clock64() - c_begin;
                     R->team = T;
                     if constexpr (SRV)
@@ -225,7 +232,6 @@ __device__ __forceinline__ void world_loop(const BatchT<RUNS> *__restrict__ Bp, 
                 }
                 break;
             }
-            const int64_t t = s_t;
             unsigned act = 0;
             unsigned long long wk = ~0ull;
 #ifdef TW_PROF
@@ -302,37 +308,60 @@ __device__ __forceinline__ void world_loop(const BatchT<RUNS> *__restrict__ Bp, 
             atomicMax(&p_host, p_h);
             atomicMax(&p_sw, p_s);
 #endif
-            if (act)
-                atomicAdd(&s_act, act);
-            if (wk != ~0ull)
-                atomicMin(&s_wake, wk);
-            __syncthreads();
-            if (tid == 0 && T > 1)
+            // The slot's end. A wake-up counts in a slot without any activity only, so a workgroup
+            // with some brings one word, its arrival, and the others bring their wake-up before it.
+            if (__ballot(act != 0))
             {
-                if (s_act)
-                    atomicAdd(&ts->act, s_act);
-                if (s_wake != ~0ull)
-                    atomicMin(&ts->wake, s_wake);
+                if (lane == 0)
+                    atomicOr(&s_act, 1u);
             }
-#ifdef TW_PROF
+            else if (wk != ~0ull)
+                atomicMin(&s_wake, wk);
+            __builtin_amdgcn_s_waitcnt(0); // (this wave's stores have completed)
+            __syncthreads();
             if (tid == 0)
             {
+#ifdef TW_PROF
                 atomicMax(&ts->prof[0], p_host);
                 atomicMax(&ts->prof[1], p_sw);
                 atomicMax(&ts->prof[2], wall_clock64() - p0);
-            }
 #endif
-            const bool err = team_barrier([&] {
-                // the ticket (src/kernel.cuh:79-112): finish, or the next slot with the exact idle skip
-                unsigned a = T > 1 ? atomicExch(&ts->act, 0u) : s_act;
-                unsigned long long nw = T > 1 ? atomicExch(&ts->wake, ~0ull) : s_wake;
-                unsigned cur = a + coh_load(&R->act_cur), prev = coh_load(&R->act_prev);
-                bool fin = atomicAdd(&R->flows_done, 0u) >= (unsigned)W.M || t + 1 >= W.max_slots;
-                int64_t next = t + 1;
-                if (cur == 0 && prev == 0 && nw != ~0ull && (int64_t)nw > next)
-                    next = (int64_t)nw < W.max_slots ? (int64_t)nw : W.max_slots;
-#ifdef TW_PROF
+                const int par = slot_count++ & 1;
+                const unsigned active = s_act != 0;
+                unsigned arrived = 0; // before this workgroup
+                if (T > 1)
                 {
+                    if (!active && s_wake != ~0ull)
+                    {
+                        atomicMax(&ts->wake[par], ~s_wake);
+                        __builtin_amdgcn_s_waitcnt(0);
+                    }
+                    arrived = atomicAdd(&ts->slot_arrive[par], 1u | active << 16);
+                }
+                unsigned long long go;
+                if ((arrived & 0xFFFFu) == (unsigned)T - 1)
+                {
+                    // the ticket (src/kernel.cuh:79-112): finish, or the next slot with the exact idle skip
+                    const bool idle = (arrived >> 16) + active == 0;
+                    const unsigned done = coh_load(&R->flows_done);
+                    const int bad = T > 1 ? coh_load(&ts->err) : 0;
+                    const bool fin = done >= (unsigned)W.M || t + 1 >= W.max_slots;
+                    int64_t next = t + 1;
+                    if (idle && (flags & SlotGo::IDLE))
+                    {
+                        const unsigned long long nw = T > 1 ? ~coh_load(&ts->wake[par]) : s_wake;
+                        if (nw != ~0ull && (int64_t)nw > next)
+                            next = (int64_t)nw < W.max_slots ? (int64_t)nw : W.max_slots;
+                    }
+                    go = SlotGo::pack(next, (fin ? SlotGo::FIN : 0) | (idle ? SlotGo::IDLE : 0) | (bad ? SlotGo::ERR : 0), slot_count);
+                    if (T > 1)
+                    {
+                        coh_store(&ts->go, go);
+                        // (these words are next used two slots on, after this wave's next wait for its stores)
+                        coh_store(&ts->slot_arrive[par], 0u);
+                        coh_store(&ts->wake[par], 0ull);
+                    }
+#ifdef TW_PROF
                     const unsigned long long now = wall_clock64();
                     const unsigned long long before = atomicExch(&ts->prof[3], now);
                     if (before)
@@ -340,15 +369,29 @@ __device__ __forceinline__ void world_loop(const BatchT<RUNS> *__restrict__ Bp, 
                     atomicAdd(&R->ev[EV_PROF_HOSTS], atomicExch(&ts->prof[0], 0ull));
                     atomicAdd(&R->ev[EV_PROF_SWITCHES], atomicExch(&ts->prof[1], 0ull));
                     atomicAdd(&R->ev[EV_PROF_WORK], atomicExch(&ts->prof[2], 0ull));
-                }
 #endif
-                coh_store(&R->act_prev, cur);
-                coh_store(&R->act_cur, 0u);
-                coh_store(&R->slot, next);
-                coh_store(&R->slots_run, coh_load(&R->slots_run) + 1);
-                if (fin)
-                    coh_store(&R->finished, 1);
-            }, false);
+                }
+                else
+                {
+                    const unsigned long long w0 = wall_clock64();
+                    while (SlotGo::count(go = coh_load(&ts->go)) != (slot_count & 0xFFFFu))
+                    {
+                        __builtin_amdgcn_s_sleep(1);
+                        if (wall_clock64() - w0 > WAIT_TICKS)
+                        {
+                            atomicExch(&ts->err, 1);
+                            go = SlotGo::pack(t, SlotGo::ERR, slot_count);
+                            break;
+                        }
+                    }
+                }
+                s_t = SlotGo::next(go);
+                s_flags = SlotGo::flags(go);
+                s_act = 0;
+                s_wake = ~0ull;
+            }
+            __syncthreads();
+            const bool err = s_flags & SlotGo::ERR;
             if (err)
             {
                 if (tid == 0)

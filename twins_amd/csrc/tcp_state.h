@@ -292,19 +292,35 @@ struct TeamPlan
     int32_t first, T, hpw, queue;
 };
 
-// a team's barrier and reductions (teams of several workgroups run one world), each word on its
-// own cache line
+// a team's barriers (teams of several workgroups run one world), each polled word on its own cache
+// line. A world's start and end: arrive and gen. Between slots: slot_arrive and wake of the slot's
+// parity (the other parity's are cleared meanwhile), answered by go (SlotGo).
 struct alignas(128) TeamState
 {
     unsigned arrive;
     unsigned pad0[31];
     unsigned gen;
-    unsigned pad1[31];
+    unsigned pad1;
+    unsigned long long go; // (nobody waits for gen and go at the same time)
+    unsigned pad2[28];
     int32_t world, err;
-    unsigned act;
-    unsigned pad2;
-    unsigned long long wake;
+    unsigned slot_arrive[2];    // workgroups that have arrived, and << 16 those with activity
+    unsigned long long wake[2]; // ~ of the earliest wake-up of those without
     unsigned long long prof[4]; // TW_PROF: this slot's maxima (hosts, switches, work); last ticket time
+};
+
+// What the last workgroup of a slot tells the others, in one word: the next slot, how the world
+// goes on, and the count of slots run in this launch (its low bits), which they wait for.
+struct SlotGo
+{
+    static constexpr unsigned FIN = 1, IDLE = 2, ERR = 4;
+    TW_HD static unsigned long long pack(int64_t next, unsigned flags, unsigned count)
+    {
+        return (unsigned long long)(count & 0xFFFFu) << 48 | (unsigned long long)flags << 32 | (uint32_t)next;
+    }
+    TW_HD static unsigned count(unsigned long long g) { return (unsigned)(g >> 48); }
+    TW_HD static unsigned flags(unsigned long long g) { return (unsigned)(g >> 32) & 0xFFFFu; }
+    TW_HD static int64_t next(unsigned long long g) { return (int64_t)(uint32_t)g; }
 };
 
 // The serving loop (tcp_server_kernel): requests are single-world batches resident in device
