@@ -260,7 +260,7 @@ __device__ __forceinline__ void world_loop(const BatchT<RUNS> *__restrict__ Bp, 
                     // 8-byte stores waits 0.4 us for them, 0.09 us without).
                     auto send = [&](int host, const char *from, int frames, int first, int group) {
                         const uint64_t *f = reinterpret_cast<const uint64_t *>(from);
-                        uint64_t TW_G *to = reinterpret_cast<uint64_t TW_G *>(B.msg + ((size_t)(t % NRING) * B.nlinks + W.link0 + host) * MAX_TX);
+                        uint64_t TW_G *to = (uint64_t TW_G *)Md::msg_of(B, t, W.link0 + host);
                         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); // (a wave's LDS accesses are in order)
                         for (int i = first; i < frames * (FR / 8); i += group)
                             coh_store(to + i, f[i]);

@@ -22,6 +22,11 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
+// A condition that is seldom (usually) true where it stands: the code for the other case is laid out
+// next, so the usual way through an event takes few branches.
+#define TW_RARE(c) (ONE ? __builtin_expect((long)U(c), 0) : (long)U(c))
+#define TW_USUAL(c) (ONE ? __builtin_expect((long)U(c), 1) : (long)U(c))
+
 // ONE: the host code for a wave that runs one host at a time on one lane. Every branch is then the
 // wave's, and U() says so: the compiler branches on a scalar instead of masking lanes in and out and
 // merging the masks at every join (a third of the host code's instructions, and as many as its
@@ -52,8 +57,9 @@ struct Model
     // 2048 + len, timers 4096 + lead/16 ns (saturating)
     static __device__ __forceinline__ uint32_t code_lead(int64_t lead_ps)
     {
-        int64_t c = 4096 + lead_ps / 16000;
-        return (uint32_t)(c < 0xFFFE ? c : 0xFFFE);
+        // (a lead is not negative; in 32 bits where it does not saturate)
+        constexpr int64_t MOST = (int64_t)(0xFFFE - 4096) * 16000;
+        return lead_ps < MOST ? 4096 + (uint32_t)lead_ps / 16000 : 0xFFFE;
     }
     static __device__ __forceinline__ void chain_load(Chain &c, const uint32_t *p)
     {
@@ -145,6 +151,12 @@ struct Model
     {
         return chain_cmp_by([&](int i) { return a[i]; }, [&](int i) { return b[i]; });
     }
+    // the message of link `link` in slot t's ring place
+    static __device__ __forceinline__ auto msg_of(Batch &B, int64_t t, int link)
+    {
+        return B.msg + (uint64_t)(ring_of(t) * (uint32_t)B.nlinks + (uint32_t)link) * MAX_TX;
+    }
+    static __device__ __forceinline__ auto msg_cnt_of(Batch &B, int64_t t, int link) { return B.msg_cnt + (uint64_t)(ring_of(t) * (uint32_t)B.nlinks + (uint32_t)link); }
     // a link message's frame, read device-coherently: its head (all but the chain), its chain
     struct FrameHead
     {
@@ -216,7 +228,7 @@ struct Model
         __device__ __forceinline__ void store(int64_t t, int ring_t)
         {
             coh_store(B->msg_cnt + (size_t)ring_t * B->nlinks + lid, msg_word(t, early, sent));
-            if (U(size > 0 && hd_new))
+            if (TW_USUAL(size > 0 && hd_new))
                 ring[head] = hd;
             B->q_head[lid] = head;
             B->q_size[lid] = size;
@@ -230,7 +242,7 @@ struct Model
         // (the world's messages of a slot lie within the 2^31 bytes a buffer store reaches)
         __device__ __forceinline__ void put(int i, const Frame &o)
         {
-            if (U(i < stage_cap))
+            if (TW_USUAL(i < stage_cap))
             {
                 stage[i] = o;
                 return;
@@ -262,7 +274,7 @@ struct Model
         {
             while (U(size > 0))
             {
-                if (U(sent >= MAX_TX))
+                if (TW_RARE(sent >= MAX_TX))
                 {
                     count(R, EV_TXCAP);
                     return;
@@ -277,7 +289,7 @@ struct Model
                     hd = ring[head];
                 if (U(o.ts <= link_free && link_free > last_start))
                 {
-                    chain_child(last, (uint32_t)((link_free - last_start) / PS_PER_BYTE), last);
+                    chain_child(last, (uint32_t)(link_free - last_start) / (uint32_t)PS_PER_BYTE, last);
                     chain_store(o.chain, last);
                 }
                 else
@@ -327,24 +339,24 @@ struct Model
             Frame g = f;
             g.ts = now;
             const bool over_k = len >= red_k && len > 1;
-            if (U(over_k && !(g.flags & F_ECT)))
+            if (TW_RARE(over_k && !(g.flags & F_ECT)))
             {
                 count(R, EV_DROP);
                 return false;
             }
-            if (U(over_k))
+            if (TW_RARE(over_k))
             {
                 g.flags |= F_CE;
                 count(R, EV_MARK);
             }
-            if (U(len >= limit))
+            if (TW_RARE(len >= limit))
             {
                 count(R, EV_DROP);
                 return false;
             }
-            if (U(B->qt.rec && now >= B->qt.from && now < B->qt.until))
+            if (TW_RARE(B->qt.rec && now >= B->qt.from && now < B->qt.until))
                 trace(now, len + 1, g.flow, g.sa, g.len, g.flags, g.to_sender);
-            if (U(size >= cap))
+            if (TW_RARE(size >= cap))
             {
                 count(R, EV_RING_OVF);
                 return false;
@@ -468,7 +480,7 @@ struct Model
     }
     static __device__ __forceinline__ SndState &snd_open(Host &x, int f)
     {
-        if (U(x.sf != f))
+        if (TW_RARE(x.sf != f))
         {
             snd_flush(x);
             snd_move(&x.S, &x.B->snd[f]);
@@ -487,7 +499,7 @@ struct Model
     }
     static __device__ __forceinline__ RcvState &rcv_open(Host &x, int f)
     {
-        if (U(x.rf != f))
+        if (TW_RARE(x.rf != f))
         {
             rcv_flush(x);
             rcv_move(&x.Q, &x.B->rcv[f]);
@@ -582,7 +594,7 @@ struct Model
     {
         if (U(at >= x.slot_end))
             return;
-        if (U(x.nd >= MAX_DUE))
+        if (TW_RARE(x.nd >= MAX_DUE))
         {
             count(x.R, EV_DUE_OVF);
             return;
@@ -611,7 +623,7 @@ struct Model
     static __device__ __forceinline__ void emit(Host &x, int f, uint8_t flags, uint32_t seq, uint32_t ack, uint16_t len, bool to_sender, int64_t now)
     {
         const Out o = out_of(flags, seq, ack, len, to_sender);
-        if (U(x.fill))
+        if (TW_RARE(x.fill))
         {
             x.post = o;
             x.has_post = true;
@@ -654,7 +666,7 @@ struct Model
         if (U(x.fill && fill_next(x, x.f, now, o)))
             return true;
         x.fill = false;
-        if (U(!x.has_post))
+        if (TW_USUAL(!x.has_post))
             return false;
         *o = x.post;
         x.has_post = false;
@@ -698,7 +710,7 @@ struct Model
             s.lost_b += d;
         if (U(m & IT_RETX))
             s.rtx_b += d;
-        if (U(lg_candidate(m)))
+        if (TW_RARE(lg_candidate(m)))
             s.cand_n += one;
     }
     // entry i's marks become m
@@ -720,7 +732,7 @@ struct Model
     static __device__ bool lg_insert(Ledger &L, WorldRun *R, uint32_t i, uint32_t start, uint8_t m)
     {
         SndState &s = L.s;
-        if (U(s.it_n >= L.cap))
+        if (TW_RARE(s.it_n >= L.cap))
         {
             count(R, EV_RTT_OVF);
             return false;
@@ -732,9 +744,9 @@ struct Model
         }
         L.ring[L.pos(i)] = SentEntry{start, m};
         s.it_n++;
-        if (U(s.cand > 0 && s.cand >= i))
+        if (TW_RARE(s.cand > 0 && s.cand >= i))
             s.cand++;
-        if (U(lg_candidate(m)))
+        if (TW_RARE(lg_candidate(m)))
         {
             s.cand_n++;
             s.cand = i < s.cand ? i : s.cand;
@@ -819,12 +831,12 @@ struct Model
         while (U(s.it_n))
         {
             SentEntry nx = gone == 0 ? pre[1] : gone == 1 ? pre[2] : pre[3];
-            if (U(gone + 1 >= LG_PRE && s.it_n > 1))
+            if (TW_RARE(gone + 1 >= LG_PRE && s.it_n > 1))
                 nx = L.at(1);
             const uint32_t a = e.first, b = s.it_n > 1 ? nx.first : s.high;
             if (U(b > ack))
             {
-                if (U(ack > a))
+                if (TW_RARE(ack > a))
                 {
                     // the entry's acknowledged front leaves its mark totals
                     const uint32_t cut = ack - a;
@@ -835,7 +847,7 @@ struct Model
                 }
                 break;
             }
-            if (U(e.mark))
+            if (TW_RARE(e.mark))
                 lg_remark(L, 0, 0);
             s.it_head = L.pos(1);
             s.it_n--;
@@ -846,7 +858,7 @@ struct Model
         if (U(gone))
             s.cand = s.cand > gone ? s.cand - gone : 0;
         s.una = ack;
-        if (U(s.it_n && (e.mark & IT_SACKED)))
+        if (TW_RARE(s.it_n && (e.mark & IT_SACKED)))
         {
             lg_remark(L, 0, (uint8_t)(L.mk(0) & ~IT_SACKED));
             lg_dup_sack(L);
@@ -939,7 +951,7 @@ struct Model
             const uint32_t sz = s.tail <= seq ? 0u : num < s.tail - seq ? num : s.tail - seq;
             if (U(!sz))
                 return 0;
-            if (U(s.high <= seq))
+            if (TW_USUAL(s.high <= seq))
             {
                 if (U(!lg_insert(L, R, s.it_n, seq, 0)))
                     return 0;
@@ -947,7 +959,7 @@ struct Model
                 *retx = false;
                 return sz;
             }
-            if (U(s.high >= seq + sz))
+            if (TW_RARE(s.high >= seq + sz))
             {
                 const uint32_t i = lg_find(L, seq);
                 if (U(i >= s.it_n || L.lo(i) != seq))
@@ -976,7 +988,7 @@ struct Model
         SndState &s = x.S;
         const uint32_t cap = x.cs.it_cap;
         SentNote TW_G *ht = x.B->ht + x.cs.it_off;
-        if (U(retx))
+        if (TW_RARE(retx))
         {
             // the record holding seq: resent up to seq + sz
             for (uint32_t j = 0; U(j < s.h_n); j++)
@@ -991,7 +1003,7 @@ struct Model
             }
             return;
         }
-        if (U(s.h_n >= cap))
+        if (TW_RARE(s.h_n >= cap))
         {
             count(x.R, EV_RTT_OVF);
             return;
@@ -1001,7 +1013,7 @@ struct Model
     // a measurement m: the smoothed RTT and its variation, then the timeout (at least MinRto)
     static __device__ void rtt_sample(SndState &s, int64_t m)
     {
-        if (U(s.srtt < 0))
+        if (TW_RARE(s.srtt < 0))
         {
             s.srtt = m;
             s.rttvar = m / 2;
@@ -1020,7 +1032,7 @@ struct Model
     static __device__ void rtt_on_ack(Host &x, uint32_t ack, int64_t now, const SentNote *pre)
     {
         SndState &s = x.S;
-        if (U(!s.h_n))
+        if (TW_RARE(!s.h_n))
             return;
         const uint32_t cap = x.cs.it_cap;
         if (U(!(pre[0].cnt & 0x80000000u) && ack >= pre[0].seq + pre[0].cnt))
@@ -1028,7 +1040,7 @@ struct Model
         for (int i = 0; U(s.h_n); i++, s.h_n--)
         {
             SentNote e = i == 0 ? pre[0] : i == 1 ? pre[1] : pre[2];
-            if (U(i >= RTT_PRE))
+            if (TW_RARE(i >= RTT_PRE))
                 e = x.B->ht[x.cs.it_off + rtt_pos(s, cap, 0)];
             if (U(e.seq + (e.cnt & 0x7FFFFFFFu) > ack))
                 break;
@@ -1274,7 +1286,7 @@ struct Model
         Ledger L(x);
         bool retx = false;
         const uint32_t len = lg_take(L, x.R, max_size, seq, &retx);
-        if (U(!len))
+        if (TW_RARE(!len))
             return 0;
         uint8_t flags = F_DATA;
         if (U(!retx && s.ecn_s == E_ECE_RCVD && s.ecn_echo_seq > s.ecn_cwr_seq))
@@ -1283,18 +1295,18 @@ struct Model
             s.ecn_s = E_CWR_SENT;
             s.ecn_cwr_seq = seq;
         }
-        if (U((s.fin & FIN_CLOSE) && seq + len == s.tail))
+        if (TW_RARE((s.fin & FIN_CLOSE) && seq + len == s.tail))
         {
             flags |= F_FIN;
             s.fin |= FIN_SENT;
         }
         *o = out_of(flags, seq, 0, (uint16_t)(len + 42), false);
-        if (U(retx))
+        if (TW_RARE(retx))
         {
             count(x.R, EV_RETX);
             count(x.R, EV_RETX_BY_STATE + s.cong);
         }
-        if (U(s.rto_at < 0))
+        if (TW_RARE(s.rto_at < 0))
         {
             s.rto_at = now + s.rto;
             timer_chain(x, B.rchain, f, s.rto);
@@ -1323,22 +1335,22 @@ struct Model
     static __device__ bool fill_next(Host &x, int f, int64_t now, Out *o)
     {
         SndState &s = x.S;
-        if (U(s.st != S_EST || x.fill_n >= 4096))
+        if (TW_RARE(s.st != S_EST || x.fill_n >= 4096))
             return false;
         x.fill_n++;
         Ledger L(x);
         const bool fin_out = (s.fin & (FIN_SENT | FIN_ACKED)) == FIN_SENT;
-        if (U(s.cong == C_OPEN && fin_out))
+        if (TW_RARE(s.cong == C_OPEN && fin_out))
             return false;
         const uint32_t pipe = inflight(s), room = s.cwnd > pipe ? s.cwnd - pipe : 0;
         uint32_t seq;
         if (U(!room || !lg_next(L, &seq)))
             return false;
-        if (U(room < MSS && s.tail - seq > room))
+        if (TW_RARE(room < MSS && s.tail - seq > room))
             return false; // (no runt segment while more data waits)
         s.nxt = seq;
         const uint32_t len = tx_segment(x, f, seq, room < MSS ? room : MSS, now, o);
-        if (U(!len))
+        if (TW_RARE(!len))
             return false;
         s.nxt = seq + len;
         return true;
@@ -1361,14 +1373,14 @@ struct Model
     static __device__ void rto_after_ack(Host &x, int f, uint32_t ack, bool restart, int64_t now)
     {
         SndState &s = x.S;
-        if (U(restart))
+        if (TW_USUAL(restart))
         {
             const int64_t base = s.srtt >= 0 ? s.srtt : INIT_RTT_PS, spread = 4 * s.rttvar > CLOCK_GRAN_PS ? 4 * s.rttvar : CLOCK_GRAN_PS;
             s.rto = base + spread > MIN_RTO_PS ? base + spread : MIN_RTO_PS;
             s.rto_at = now + s.rto;
             timer_chain(x, x.B->rchain, f, s.rto);
         }
-        if (U(ack >= s.tail && !(s.fin & FIN_SENT)))
+        if (TW_RARE(ack >= s.tail && !(s.fin & FIN_SENT)))
             s.rto_at = -1;
         s.nxt = ack > s.nxt ? ack : s.nxt;
     }
@@ -1401,7 +1413,7 @@ struct Model
             B.mg_done[m] = now;
             atomicAdd(&x.R->flows_done, 1u);
         }
-        if (U(s.m_dn == x.cs.m_cnt && (!x.cs.fin_on || (s.fin & FIN_ACKED))))
+        if (TW_RARE(s.m_dn == x.cs.m_cnt && (!x.cs.fin_on || (s.fin & FIN_ACKED))))
         {
             s.st = S_DONE;
             s.rto_at = -1;
@@ -1416,7 +1428,7 @@ struct Model
                 s.ecn_s = E_IDLE;
             return;
         }
-        if (U((int64_t)ack <= s.ecn_echo_seq))
+        if (TW_RARE((int64_t)ack <= s.ecn_echo_seq))
             return;
         s.ecn_echo_seq = ack;
         s.ecn_s = E_ECE_RCVD;
@@ -1439,7 +1451,7 @@ struct Model
         if (U(state == C_OPEN))
             s.cong = state = C_DISORDER;
         Ledger L(x);
-        if (U(state == C_RECOVERY))
+        if (TW_RARE(state == C_RECOVERY))
             lg_dup_sack(L);
         else if (U(state == C_DISORDER))
         {
@@ -1502,7 +1514,7 @@ struct Model
         s.cong = C_OPEN;
         if (U(ack >= s.recover))
             s.recover_active = 0;
-        if (U(state == C_RECOVERY))
+        if (TW_RARE(state == C_RECOVERY))
         {
             rto_after_ack(x, f, ack, true, now);
             s.cwnd = s.ssthresh;
@@ -1517,7 +1529,7 @@ struct Model
     static __device__ void ack_in(Host &x, int f, uint32_t ack, bool ece, int64_t now)
     {
         SndState &s = x.S;
-        if (U(s.st != S_EST || ack < s.una))
+        if (TW_RARE(s.st != S_EST || ack < s.una))
             return;
         const uint32_t una_before = s.una;
         const bool advancing = ack > una_before;
@@ -1533,14 +1545,14 @@ struct Model
             entries[i] = L.at((uint32_t)i < s.it_n ? i : 0);
         rtt_on_ack(x, ack, now, notes);
         const uint32_t acked = advancing ? lg_release(L, ack, entries) : 0;
-        if (U(s.cong == C_CWR && ack > s.recover))
+        if (TW_RARE(s.cong == C_CWR && ack > s.recover))
         {
             s.cong = C_OPEN;
             s.cwnd = s.ssthresh;
         }
         ack_echo(x, s, ack, ece, advancing);
         const uint32_t dups = s.dupacks;
-        if (U(!advancing))
+        if (TW_RARE(!advancing))
         {
             if (U(ack < s.high))
             {
@@ -1555,23 +1567,23 @@ struct Model
             // whole segments acknowledged, the remainders carried over
             uint32_t segs = acked / MSS;
             s.ack_rem += acked % MSS;
-            if (U(s.ack_rem >= MSS))
+            if (TW_RARE(s.ack_rem >= MSS))
             {
                 s.ack_rem -= MSS;
                 segs++;
             }
             s.dupacks = 0;
-            if (U(ack < s.recover && (s.cong == C_RECOVERY || s.cong == C_LOSS)))
+            if (TW_RARE(ack < s.recover && (s.cong == C_RECOVERY || s.cong == C_LOSS)))
                 ack_partial(x, f, s, ack, segs, now);
             else
                 ack_advance(x, f, s, ack, una_before, segs, dups, now);
         }
-        if (U((s.fin & FIN_SENT) && !s.it_n && ack == s.high + 1))
+        if (TW_RARE((s.fin & FIN_SENT) && !s.it_n && ack == s.high + 1))
             s.fin |= FIN_ACKED;
         if (U(advancing))
         {
             msgs_complete(x, f, now);
-            if (U(s.st == S_DONE))
+            if (TW_RARE(s.st == S_DONE))
                 return;
         }
         tx_fill(x);
@@ -1618,7 +1630,7 @@ struct Model
         RcvState &r = x.Q;
         const bool echoing = r.ecn_r == E_CE_RCVD || r.ecn_r == E_SENDING_ECE;
         const bool ece = force_ece || (!no_ece && echoing);
-        if (U(!force_ece && ece))
+        if (TW_RARE(!force_ece && ece))
             r.ecn_r = E_SENDING_ECE;
         r.delack_at = -1;
         r.delack_count = 0;
@@ -1649,7 +1661,7 @@ struct Model
     {
         RcvState &r = x.Q;
         const bool flips = (bool)r.ce_state != ce;
-        if (U(flips && r.reserved && r.prior_flag))
+        if (TW_RARE(flips && r.reserved && r.prior_flag))
             rcv_ack(x, f, r.prior_rcv_nxt, !ce, ce, now);
         r.ce_state = ce ? 1 : 0;
         if (U(ce))
@@ -1664,7 +1676,7 @@ struct Model
         if (U(!x.dctcp))
             return;
         RcvState &r = x.Q;
-        if (U((p.flags & F_CE) && r.ecn_ce_seq < (int64_t)p.sa))
+        if (TW_RARE((p.flags & F_CE) && r.ecn_ce_seq < (int64_t)p.sa))
         {
             r.ecn_ce_seq = p.sa;
             r.ecn_r = E_CE_RCVD;
@@ -1678,7 +1690,7 @@ struct Model
     {
         if (U(!x.dctcp))
             return;
-        if (U((p.flags & F_CE) && !(s.s_ce & 1)))
+        if (TW_RARE((p.flags & F_CE) && !(s.s_ce & 1)))
         {
             s.s_ce = 3;
             s.ecn_s = E_CE_RCVD;
@@ -1698,17 +1710,17 @@ struct Model
         Batch &B = *x.B;
         RcvState &r = x.Q;
         const uint32_t from = seq > r.rcv_nxt ? seq : r.rcv_nxt;
-        if (U(from >= end))
+        if (TW_RARE(from >= end))
             return false;
         uint32_t *lo = B.oo_s + x.cr.oo_off, *hi = B.oo_e + x.cr.oo_off;
         const uint32_t cap = x.cr.oo_cap, h0 = r.ooo_h;
         uint32_t n = r.ooo_n;
-        if (U(n == 0 && from == r.rcv_nxt))
+        if (TW_USUAL(n == 0 && from == r.rcv_nxt))
         {
             // in order, nothing held: delivered without a place in the ring
             r.rcv_nxt = end;
             r.ooo_h = 0;
-            if (U(r.r_fin >= 0 && r.rcv_nxt == (uint32_t)r.r_fin))
+            if (TW_RARE(r.r_fin >= 0 && r.rcv_nxt == (uint32_t)r.r_fin))
                 r.rcv_nxt++; // (the FIN's sequence number)
             return true;
         }
@@ -1775,7 +1787,7 @@ struct Model
         }
         r.ooo_n = n;
         r.ooo_h = n ? head : 0;
-        if (U(r.r_fin >= 0 && r.rcv_nxt == (uint32_t)r.r_fin))
+        if (TW_RARE(r.r_fin >= 0 && r.rcv_nxt == (uint32_t)r.r_fin))
             r.rcv_nxt++; // (the FIN's sequence number)
         return true;
     }
@@ -1820,12 +1832,12 @@ struct Model
     {
         RcvState &r = x.Q;
         const uint32_t before = r.rcv_nxt;
-        if (U(!reasm_add(x, f, seq, seq + len)))
+        if (TW_RARE(!reasm_add(x, f, seq, seq + len)))
         {
             rcv_ack(x, f, r.rcv_nxt, false, false, now);
             return;
         }
-        if (U(!fin && before < r.rcv_nxt && rcv_fin_in(r)))
+        if (TW_RARE(!fin && before < r.rcv_nxt && rcv_fin_in(r)))
         {
             rcv_peer_closed(x, f, now);
             return;
@@ -1852,35 +1864,35 @@ struct Model
     static __device__ void rcv_segment(Host &x, int f, const Frame &p, int64_t now)
     {
         RcvState &r = x.Q;
-        if (U(!r.r_up || r.r_st == R_CLOSED))
+        if (TW_RARE(!r.r_up || r.r_st == R_CLOSED))
             return;
         const bool fin = p.flags & F_FIN;
         const uint32_t seq = p.sa, len = (p.flags & F_DATA) ? p.len - 42u : 0u, end = seq + len;
         if (U(len && r.r_est))
         {
             const bool stale = r.r_st == R_LAST_ACK ? seq != r.rcv_nxt : end < r.rcv_nxt;
-            if (U(stale))
+            if (TW_RARE(stale))
             {
                 rcv_ack(x, f, r.rcv_nxt, false, true, now);
                 return;
             }
         }
         rcv_ecn_in(x, f, p, now);
-        if (U((p.flags & F_CWR) && r.r_est && r.r_st == R_OPEN && r.ecn_r != E_CE_RCVD))
+        if (TW_RARE((p.flags & F_CWR) && r.r_est && r.r_st == R_OPEN && r.ecn_r != E_CE_RCVD))
             r.ecn_r = E_IDLE;
-        if (U(!r.r_est))
+        if (TW_RARE(!r.r_est))
         {
             if (U(fin && seq != r.rcv_nxt))
                 return;
             rcv_established(r);
         }
-        if (U(r.r_st == R_LAST_ACK))
+        if (TW_RARE(r.r_st == R_LAST_ACK))
         {
             if (U(fin || seq == r.rcv_nxt))
                 rcv_closed(r);
             return;
         }
-        if (U(!fin))
+        if (TW_USUAL(!fin))
         {
             rcv_data(x, f, seq, len, false, now);
             return;
@@ -1939,7 +1951,7 @@ struct Model
     static __device__ void on_frame_snd(Host &x, int f, const Frame &p, int64_t now)
     {
         SndState &s = x.S;
-        if (U(p.flags & F_SYN))
+        if (TW_RARE(p.flags & F_SYN))
         {
             if (U(s.st != S_SYN_SENT))
                 return;
@@ -1952,11 +1964,11 @@ struct Model
             app_write(x, f, now, w);
             return;
         }
-        if (U(s.fin & FIN_TW))
+        if (TW_RARE(s.fin & FIN_TW))
             return;
         snd_ecn_in(x, s, p);
         ack_in(x, f, p.sa, p.flags & F_ECE, now);
-        if (U(!(p.flags & F_FIN)))
+        if (TW_USUAL(!(p.flags & F_FIN)))
             return;
         s.fin |= FIN_TW;
         emit(x, f, F_ACK, 0, 1, CTRL_FRAME, false, now);
@@ -1967,13 +1979,13 @@ struct Model
     {
         RcvState &r = x.Q;
         const bool syn = p.flags & F_SYN;
-        if (U(!syn && r.r_up && r.r_srtt < 0 && r.r_synack_t >= 0))
+        if (TW_RARE(!syn && r.r_up && r.r_srtt < 0 && r.r_synack_t >= 0))
         {
             const int64_t m = now - r.r_synack_t;
             r.r_srtt = m;
             r.r_rttvar = m / 2;
         }
-        if (U(syn))
+        if (TW_RARE(syn))
         {
             if (U(!r.r_up))
             {
@@ -1988,16 +2000,16 @@ struct Model
             rcv_synack(x, f, now);
             return;
         }
-        if (U(p.flags & (F_DATA | F_FIN)))
+        if (TW_USUAL(p.flags & (F_DATA | F_FIN)))
         {
             rcv_segment(x, f, p, now);
             return;
         }
-        if (U(!r.r_up || r.r_st == R_CLOSED))
+        if (TW_RARE(!r.r_up || r.r_st == R_CLOSED))
             return;
         rcv_ecn_in(x, f, p, now);
         rcv_established(r);
-        if (U(r.r_st == R_LAST_ACK))
+        if (TW_RARE(r.r_st == R_LAST_ACK))
             rcv_closed(r);
     }
     // one event per frame: the side's record in LDS for its duration
@@ -2036,6 +2048,13 @@ struct Model
         return r <= 0;
     }
 
+    // the slot of time `at`, from slot t's end E0 on without a 64-bit division
+    static __device__ __forceinline__ int64_t slot_of(int64_t at, int64_t E0, int64_t t)
+    {
+        const uint64_t d = (uint64_t)(at - E0); // (huge before E0)
+        return d < 0x100000000ull ? t + 1 + (uint32_t)d / (uint32_t)SLOT_PS : at / SLOT_PS;
+    }
+
     // -------------------------------------------------------------- one slot of a host
     // its arrivals: the later part of slot t-2's message of its in-link, the earlier of t-1's
     struct HostIn
@@ -2052,13 +2071,13 @@ struct Model
         const int queued = B.q_size[lid];
         if (t >= 2)
         {
-            const long long v = coh_load(B.msg_cnt + (size_t)((t - 2) % NRING) * B.nlinks + in.in);
+            const long long v = coh_load(msg_cnt_of(B, t - 2, in.in));
             if (msg_slot(v) == t - 2)
                 in.i2 = msg_early(v), in.n2 = msg_sent(v);
         }
         if (t >= 1)
         {
-            const long long v = coh_load(B.msg_cnt + (size_t)((t - 1) % NRING) * B.nlinks + in.in);
+            const long long v = coh_load(msg_cnt_of(B, t - 1, in.in));
             in.n1 = msg_slot(v) == t - 1 ? msg_early(v) : 0;
         }
         if (in.i2 < in.n2 || in.n1 > 0 || t >= w || queued != 0)
@@ -2085,11 +2104,11 @@ struct Model
         const unsigned long long pr0 = wall_clock64();
         unsigned long long pr_ev = 0, pr_n = 0;
 #endif
-        const Frame *m2 = B.msg + ((size_t)((t + NRING - 2) % NRING) * B.nlinks + hi.in) * MAX_TX;
-        const Frame *m1 = B.msg + ((size_t)((t + NRING - 1) % NRING) * B.nlinks + hi.in) * MAX_TX;
+        const Frame *m2 = msg_of(B, t + NRING - 2, hi.in);
+        const Frame *m1 = msg_of(B, t + NRING - 1, hi.in);
         const int n2 = hi.n2, n1 = hi.n1;
         int i2 = hi.i2, i1 = 0;
-        const int rt = (int)(t % NRING);
+        const int rt = (int)ring_of(t);
         Host x;
         x.nic.load(B, W, R, lid, t, rt, st, st_cap);
         x.B = &B;
@@ -2200,7 +2219,7 @@ struct Model
             const unsigned long long pq = wall_clock64();
             pr_n++;
 #endif
-            if (U(now == tp && B.cs[B.mg_conn[pm]].m_first != pm))
+            if (TW_RARE(now == tp && B.cs[B.mg_conn[pm]].m_first != pm))
             {
                 // a later message of a connection (FlowSender::SendMessage)
                 const int m = pm;
@@ -2213,7 +2232,7 @@ struct Model
                 if (U(s.st == S_EST))
                     app_write(x, f, now, x.echain);
             }
-            else if (U(now == tp))
+            else if (TW_RARE(now == tp))
             {
                 // a connection's application starts: SYN
                 const int m = pm;
@@ -2233,7 +2252,7 @@ struct Model
                 s.timing_time = now;
                 emit(x, f, F_SYN, 0, 0, SYN_FRAME, false, now);
             }
-            else if (U(now == td && (now != tr || timer_before_arrival(x, due[x.id], i2 < n2 ? m2 + i2 : m1 + i1))))
+            else if (TW_RARE(now == td && (now != tr || timer_before_arrival(x, due[x.id], i2 < n2 ? m2 + i2 : m1 + i1))))
             {
                 Due d = due[x.id++];
                 x.due_head = x.id < x.nd ? due[x.id].at : INT64_MAX;
@@ -2274,7 +2293,7 @@ struct Model
                         r.reserved = 1;
                         rcv_ack(x, f, r.rcv_nxt, false, false, now);
                     }
-                    else if (U(d.kind == 4 && r.r_last_at == d.at && r.r_st == R_LAST_ACK))
+                    else if (TW_RARE(d.kind == 4 && r.r_last_at == d.at && r.r_st == R_LAST_ACK))
                     {
                         if (U(r.r_last_n == 0))
                             rcv_closed(r);
@@ -2287,12 +2306,12 @@ struct Model
                             timer_chain(x, B.dchain, f, lr);
                         }
                     }
-                    else if (U(d.kind == 5 && r.r_frx_at == d.at && r.r_st == R_LAST_ACK))
+                    else if (TW_RARE(d.kind == 5 && r.r_frx_at == d.at && r.r_st == R_LAST_ACK))
                     {
                         r.r_frx_at = -1;
                         rcv_fin_ack(x, f, now);
                     }
-                    else if (U(d.kind == 3 && r.srv_syn_at == d.at && !r.r_est))
+                    else if (TW_RARE(d.kind == 3 && r.srv_syn_at == d.at && !r.r_est))
                     {
                         r.srv_syn_at = -1;
                         rcv_synack(x, f, now);
@@ -2344,7 +2363,7 @@ struct Model
         int64_t next = nb_s < nb_r ? nb_s : nb_r;
         if (U(pn < pe && B.mg_start[B.pend_msg[pn]] < next))
             next = B.mg_start[B.pend_msg[pn]];
-        int64_t wk = x.nic.size > 0 ? t + 1 : (next == INT64_MAX ? INT64_MAX : next / SLOT_PS);
+        int64_t wk = x.nic.size > 0 ? t + 1 : (next == INT64_MAX ? INT64_MAX : slot_of(next, E0, t));
         B.wake[h] = wk;
         *wake = wk;
 #ifdef TW_PROF
@@ -2382,16 +2401,17 @@ struct Model
         }
         if (W.kind == TOPO_LEAFSPINE)
         {
+            const int leaf = (int)div_small(dst, W.hpl_m);
             if (sw < W.leaves)
-                return dst / W.hpl == sw ? dst % W.hpl : W.hpl + up;
-            return dst / W.hpl;
+                return leaf == sw ? dst - leaf * W.hpl : W.hpl + up;
+            return leaf;
         }
         const int hk = W.hk, E = W.k * hk;
-        int dst_pod = dst / (hk * hk), dst_edge = (dst / hk) % hk;
+        const int rack = (int)div_small(dst, W.hk_m), dst_pod = (int)div_small(dst, W.hk2_m);
         if (sw < E)
-            return (dst_pod == sw / hk && dst_edge == sw % hk) ? dst % hk : hk + up;
+            return rack == sw ? dst - rack * hk : hk + up; // (edge switches in the racks' order)
         if (sw < 2 * E)
-            return dst_pod == (sw - E) / hk ? dst_edge : hk + up;
+            return dst_pod == (int)div_small(sw - E, W.hk_m) ? rack - dst_pod * hk : hk + up;
         return dst_pod;
     }
     static __device__ int route(Batch &B, World &W, int sw, const FrameHead &p, int ep)
@@ -2419,13 +2439,12 @@ struct Model
             return e == sw ? 0 : B.g_rt_n[rt_index(W, ep, sw, e)];
         }
         if (W.kind == TOPO_LEAFSPINE)
-            return sw < W.leaves ? (dst / W.hpl == sw ? 0 : W.ecmp_n) : 1;
-        const int hk = W.hk, E = W.k * hk;
-        int dst_pod = dst / (hk * hk), dst_edge = (dst / hk) % hk;
+            return sw < W.leaves ? ((int)div_small(dst, W.hpl_m) == sw ? 0 : W.ecmp_n) : 1;
+        const int E = W.k * W.hk;
         if (sw < E)
-            return dst_pod == sw / hk && dst_edge == sw % hk ? 0 : W.ecmp_n;
+            return (int)div_small(dst, W.hk_m) == sw ? 0 : W.ecmp_n; // (edge switches in the racks' order)
         if (sw < 2 * E)
-            return dst_pod == (sw - E) / hk ? 1 : W.ecmp_n;
+            return div_small(dst, W.hk2_m) == div_small(sw - E, W.hk_m) ? 1 : W.ecmp_n;
         return 1;
     }
     // simultaneous arrivals: the longer frame first, then the upstream starts' chains, then
@@ -2455,6 +2474,9 @@ struct Model
     static constexpr int SW_LDS_INLINK = SW_LDS_EGRESS + 64 * EGRESS_LDS;
     static constexpr int SW_LDS_TOTAL = SW_LDS_INLINK + 64;
     static constexpr uint32_t NO_EGRESS = 0xFF;
+    // an arrival in the sort lists: its frame's place among the messages of the world's links (MAX_TX
+    // each), in those of slot t - 2 or, with REF_EARLY, t - 1
+    static constexpr uint32_t REF_EARLY = 0x80000000u;
     static_assert(SLOT_PS < 1 << 20, "an arrival's time in its slot: 20 bits");
     static constexpr int COUNT_RUN = 4; // arrivals' heads read together
     struct SwLds
@@ -2479,8 +2501,8 @@ struct Model
         in.n1 = win[2];
         if (link < 0)
             link = 0; // (an unused port has an empty window)
-        in.m2 = B.msg + ((size_t)((t + NRING - 2) % NRING) * B.nlinks + link) * MAX_TX;
-        in.m1 = B.msg + ((size_t)((t + NRING - 1) % NRING) * B.nlinks + link) * MAX_TX;
+        in.m2 = msg_of(B, t + NRING - 2, link);
+        in.m1 = msg_of(B, t + NRING - 1, link);
         return in;
     }
     // One lane of a switch's slot: port q of world-local switch swl (inactive lanes idle).
@@ -2529,13 +2551,13 @@ struct Model
         {
             if (t >= 2)
             {
-                const long long v = coh_load(B.msg_cnt + (size_t)((t - 2) % NRING) * B.nlinks + in_link);
+                const long long v = coh_load(msg_cnt_of(B, t - 2, in_link));
                 if (msg_slot(v) == t - 2)
                     w0 = msg_early(v), w1 = msg_sent(v);
             }
             if (t >= 1)
             {
-                const long long v = coh_load(B.msg_cnt + (size_t)((t - 1) % NRING) * B.nlinks + in_link);
+                const long long v = coh_load(msg_cnt_of(B, t - 1, in_link));
                 w2 = msg_slot(v) == t - 1 ? msg_early(v) : 0;
             }
         }
@@ -2627,6 +2649,7 @@ struct Model
         int *row = L.rows + x.q * (W.k + 1);
         const uint32_t *eg = lane_egress_lds(L, x);
         const int n = in.count();
+        const uint32_t first = (uint32_t)(L.wave[SW_LDS_INLINK + sw_lane_of(L, x)] - W.link0) * MAX_TX; // (of the in-link's message)
         auto scatter = [&](auto *ts, auto *ref) {
             for (int j = 0; j < n; j++)
             {
@@ -2648,7 +2671,8 @@ struct Model
                     continue;
                 int at = L.base[e] + row[e]++;
                 ts[at] = at_ts;
-                ref[at] = (uint32_t)(x.q << 16 | j);
+                const int late = in.n2 - in.i2; // (the arrivals of slot t - 2's message come first)
+                ref[at] = first + (j < late ? (uint32_t)(in.i2 + j) : REF_EARLY | (uint32_t)(j - late));
             }
         };
         if (sw_lists_in_lds(W, L))
@@ -2680,9 +2704,10 @@ struct Model
         const int n = L.cnt[x.q], b0 = L.base[x.q];
         if (n == 0 && B.q_size[x.lid] == 0)
             return 0; // (nothing to send: the port's message of an older slot stands for an empty one)
-        auto frame_at = [&](uint32_t r) -> const Frame * { return lane_input(B, W, x, t, L, (int)(r >> 16)).at((int)(r & 0xFFFF)); };
+        const Frame *const m2 = msg_of(B, t + NRING - 2, W.link0), *const m1 = msg_of(B, t + NRING - 1, W.link0);
+        auto frame_at = [&](uint32_t r) -> const Frame * { return (r & REF_EARLY ? m1 : m2) + (r & ~REF_EARLY); };
         Fifo eg;
-        const int rt = (int)(t % NRING);
+        const int rt = (int)ring_of(t);
         eg.load(B, W, R, x.lid, t, rt);
         // an insertion sort by (time, frame_before): chain comparison is no strict weak order
         // when chains are truncated, and this gives the reference's order in every case. (Inlined at

@@ -80,6 +80,12 @@ constexpr uint32_t MSS = 1460;
 constexpr int CTRL_FRAME = 42, SYN_FRAME = 46;
 constexpr int MAX_TX = 300;    // frames one link can start in a slot (the model's cap)
 constexpr int NRING = 3;       // link message ring: slots t-2, t-1 (read) and t (written)
+TW_HD inline uint32_t ring_of(int64_t t) { return (uint32_t)t % NRING; } // (0 <= t < 2^31)
+// The kernel's quotients by numbers fixed for a world: n / d from the high half of n * ceil(2^32 / d),
+// exact while n * d < 2^32 (d == 1: m = 0). A division by a value unknown to the compiler is some 40
+// instructions, and a 64-bit one, by a constant too, ten quarter-rate multiplications.
+TW_HD inline uint32_t div_small_m(uint32_t d) { return d > 1 ? (uint32_t)((0x100000000ull + d - 1) / d) : 0; }
+TW_HD inline uint32_t div_small(uint32_t n, uint32_t m) { return m ? (uint32_t)((uint64_t)n * m >> 32) : n; }
 // A link's message count word for slot t: the slot in the high 32 bits, then how many of its
 // frames arrive before the end of slot t + 1, then how many it holds. The receiver takes the
 // first ones in slot t + 1 and the rest in slot t + 2; frames start in order, one after another,
@@ -261,7 +267,8 @@ struct WorldDesc
     int32_t kind, k, hk, H, S, ecmp_n, leaves, spines, hpl, n_fail;
     int32_t host0, sw0, link0, L, conn0, nconn, msg0, M;
     int32_t rng0;  // first switch's MRG32k3a state (-1: per-flow ECMP)
-    int32_t pad;
+    uint32_t hk_m, hk2_m, hpl_m; // hk, hk * hk and hpl for div_small
+    uint32_t pad;
     int64_t max_slots;
     // topology files: offsets of the world's rows in the batch tables: host switch/port
     // [H], route offsets and counts [epoch][S][S] (offsets relative to the world's port

@@ -986,6 +986,7 @@ static int pack(tw_batch &b, const tw_pack_cfg &cfg)
         memset(&d, 0, sizeof d);
         d.kind = w.kind, d.k = w.k, d.hk = w.hk, d.H = w.H, d.S = w.S, d.ecmp_n = w.ecmp_n;
         d.leaves = w.leaves, d.spines = w.spines, d.hpl = w.hpl, d.n_fail = w.n_fail;
+        d.hk_m = div_small_m(w.hk), d.hk2_m = div_small_m(w.hk * w.hk), d.hpl_m = div_small_m(w.hpl);
         d.host0 = (int32_t)H, d.sw0 = (int32_t)S, d.link0 = (int32_t)L, d.L = w.L, d.conn0 = (int32_t)NC, d.nconn = w.NC;
         d.msg0 = (int32_t)M, d.M = w.M;
         d.rng0 = w.rng.empty() ? -1 : (int32_t)RNG;
