@@ -85,3 +85,24 @@ def test_gpu_launch_shapes(team, hosts, runs):
         if not b.counters(0)[25]:  # (no tie left undecided by chains of 9)
             assert [(str(e), str(d)) for e, d in zip(est, done)] == exp, name
         b.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("team,budget", [(1, 997), (16, 61), (52, 61), (0, 997)])
+def test_gpu_resumed_launches(team, budget):
+    """A run cut into launches of `budget` slots (idle skips, a world's end inside a launch) goes on
+    where it stood: ns-3's times, and the slots and packet-events of one launch."""
+    import twins_amd
+    name, fl, ref, args = [c for c in CASES if c[0] == "k8_incast16-cubic-fin"][0]
+    print(f"case {name}", flush=True)
+    w = twins_amd.World(args + [f"--flows={util.GOLDEN}/{fl}"])
+    whole = twins_amd.Batch([w])
+    one = whole.run()
+    whole.close()
+    b = twins_amd.Batch([w], team_blocks=team, slot_budget=budget)
+    st = b.run()
+    assert (st.worlds_done, st.slots_max, st.packet_events) == (1, one.slots_max, one.packet_events)
+    assert st.launches == -(-st.slots_max // budget)
+    est, done = b.fct(0)
+    assert [(str(e), str(d)) for e, d in zip(est, done)] == util.read_cols(os.path.join(util.GOLDEN, ref), (4, 5))
+    b.close()

@@ -1,7 +1,7 @@
 // The RDMA slot kernel for gfx950. A world runs on a team of T workgroups (256 threads, 4 waves
 // each) for all of its slots; teams take worlds from a queue, longest first. In a slot the world's
 // work items are dealt over the team's waves: a host item is up to hpw hosts side by side (a lane
-// runs one host's events, src/rdma/rstep.cuh:1649-2112), a switch item is one switch on one wave
+// runs one host's events, src/rdma/rstep.cuh:1649-2112), a switch item is one switch on one wave or workgroup
 // (its ports in LDS; a safe slot runs each egress port's events on a lane of its own, otherwise lane
 // 0 runs them all; rdma_model.h switch_slot). Entities only read what earlier slots filed
 // (src/rdma/rdma.h:12-16), so a slot needs one team barrier; the last workgroup to arrive decides the

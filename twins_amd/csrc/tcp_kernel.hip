@@ -12,7 +12,7 @@
 // The launch plan gives each team its size T, its workgroups and the queue of worlds it takes
 // from, so one launch can run small worlds a workgroup each and large ones over many CUs.
 // T = 1 needs only the workgroup barrier, so a world's state stays within one CU. T > 1
-// synchronises through an agent-scope arrive counter and generation word per team; the grid is
+// synchronises through agent-scope words per team, one round trip a slot (TeamState, SlotGo); the grid is
 // at most what the GPU holds at once, so all of a team's workgroups are resident, and every wait
 // is bounded (a timeout ends the world with an error flag instead of hanging the queue). Each world's team
 // accounts the device clock time it spent on it (WorldRun::ticks), the input of the autotuner.

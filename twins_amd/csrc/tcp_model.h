@@ -1275,7 +1275,7 @@ struct Model
     // A connection's sending side (TcpSocketBase with its TxBuffer, as the model restates it):
     // segments leave through the host's queue, the retransmission timer follows the oldest
     // unacknowledged byte, and ACKs drive ns-3's congestion states (open, disorder, CWR,
-    // recovery, loss). Every function works on the record of the event's connection in LDS.
+    // recovery, loss). Every function works on the record of the event's connection (Host::S).
     // one segment of up to max_size bytes at seq (SendDataPacket): CWR on the first new segment
     // after an echo, FIN on the last byte once the application closed; the timer is armed if
     // idle; *o: the frame; returns its bytes
@@ -2012,7 +2012,7 @@ struct Model
         if (TW_RARE(r.r_st == R_LAST_ACK))
             rcv_closed(r);
     }
-    // one event per frame: the side's record in LDS for its duration
+    // one event per frame, on the side's record
     static __device__ void on_frame(Host &x, const Frame &p, int64_t now)
     {
         const int f = (int)p.flow;
@@ -2531,12 +2531,17 @@ struct Model
     {
         return reinterpret_cast<uint32_t *>(L.wave + SW_LDS_EGRESS) + sw_lane_of(L, x) * EGRESS_LDS;
     }
-    static __device__ int lane_egress(Batch &B, World &W, const SwLane &x, int j, const FrameHead &p)
+    // (its equal-cost index in a sprayed world: the draw of arrival j)
+    static __device__ __forceinline__ int lane_draw(World &W, const SwLane &x, int j)
+    {
+        return W.rng0 >= 0 ? x.scr_up[x.q * 2 * MAX_TX + j] : 0;
+    }
+    static __device__ int lane_egress(Batch &B, World &W, const SwLane &x, int draw, const FrameHead &p)
     {
         int ep = W.n_fail ? epoch_of(B, W, p.ts) : 0;
         if (port_down(B, W, x.swl, x.q, ep))
             return -1; // dropped on arrival at a down interface
-        return W.rng0 >= 0 ? route_up(B, W, x.swl, p.dst, x.scr_up[x.q * 2 * MAX_TX + j], ep) : route(B, W, x.swl, p, ep);
+        return W.rng0 >= 0 ? route_up(B, W, x.swl, p.dst, draw, ep) : route(B, W, x.swl, p, ep);
     }
     // 1: the ingress window of port q (tail of slot t-2's message from S0 on, head of t-1's
     // before E0) into LDS; the port's row of egress counts cleared
@@ -2581,16 +2586,20 @@ struct Model
         for (int j0 = 0; j0 < n; j0 += COUNT_RUN)
         {
             FrameHead h[COUNT_RUN];
+            int draw[COUNT_RUN];
 #pragma unroll
             for (int u = 0; u < COUNT_RUN; u++)
+            {
                 h[u] = in.head(j0 + u < n ? j0 + u : n - 1);
+                draw[u] = lane_draw(W, x, j0 + u < n ? j0 + u : n - 1);
+            }
 #pragma unroll
             for (int u = 0; u < COUNT_RUN; u++)
             {
                 const int j = j0 + u;
                 if (j >= n)
                     break;
-                const int e = lane_egress(B, W, x, j, h[u]);
+                const int e = lane_egress(B, W, x, draw[u], h[u]);
                 if (j < EGRESS_LDS)
                     eg[j] = (uint32_t)(h[u].ts - t * SLOT_PS) | (e >= 0 ? (uint32_t)e : NO_EGRESS) << 20;
                 if (e >= 0)
@@ -2665,7 +2674,7 @@ struct Model
                 {
                     const FrameHead p = in.head(j);
                     at_ts = p.ts;
-                    e = lane_egress(B, W, x, j, p);
+                    e = lane_egress(B, W, x, lane_draw(W, x, j), p);
                 }
                 if (e < 0)
                     continue;
@@ -2799,15 +2808,9 @@ struct Model
             Spray sp;
             spray_init(B, W, x, t, L, sp);
             wave_sync();
-            for (;;)
-            {
-                spray_put(x, L, sp);
-                wave_sync();
-                const bool done = spray_pick(B, W, R, x, t, L, sp);
-                wave_sync();
-                if (done)
-                    break;
-            }
+            while (!spray_pick(B, W, R, x, t, L, sp))
+                ;
+            wave_sync();
             spray_end(B, W, x, L, sp);
         }
         wave_sync();
@@ -2832,11 +2835,12 @@ struct Model
     // of the ports' arrival lists, equal times decided in port order by frame_before. Packets
     // arriving at a down port draw nothing; a packet with no route draws nothing and gets 0.
     // The k lanes of the switch run the merge in lockstep, each holding its own port's list: a
-    // step exchanges the heads through LDS, every lane finds the same winner and makes the same
-    // draw (each lane carries the stream), the winner records it. Heads and route counts of the
+    // step finds the earliest head over the lanes, every lane the same one, and every lane makes the
+    // same draw (each carries the stream); the winner records it. Heads and route counts of the
     // first 32 arrivals of a port sit in LDS (computed by the port's lane beforehand); frames are
-    // read only to break equal times. The phases (init, then put / pick until done, then end) run
-    // with wave_sync() between them; a CPU check may run each phase over the lanes in turn.
+    // read only to break equal times. The phases (init, then pick until done, then end) run with
+    // wave_sync() between them; a CPU check runs each phase over the lanes in turn, and exchanges the
+    // heads by a phase of its own (spray_put) before every pick.
     static constexpr int SPRAY_CACHE = 32;
     static constexpr uint32_t SPRAY_NONE = 0xFFFFFFFFu;
     struct Spray
@@ -2898,6 +2902,41 @@ struct Model
             return true;
         const int k = W.k;
         const int64_t S0 = t * SLOT_PS;
+#if defined(__HIP_DEVICE_COMPILE__)
+        // the earliest head (the first port holding it): a minimum over the switch's lanes by shuffles
+        // (a step reading every port's head from LDS in a loop, twice, was most of a sprayed slot)
+        const int lane0 = sw_lane_of(L, x) - x.q;
+        uint32_t m = sp.head == SPRAY_NONE ? SPRAY_NONE : (sp.head & 0xFFFFFu) << 6 | (uint32_t)x.q;
+        for (int d = 1; d < k; d <<= 1)
+        {
+            const uint32_t u = __shfl_down(m, d);
+            m = x.q + d < k && u < m ? u : m;
+        }
+        m = __shfl(m, lane0);
+        if (m == SPRAY_NONE)
+        {
+            sp.done = true;
+            return true;
+        }
+        int best = (int)(m & 63);
+        uint64_t same = __ballot(sp.head != SPRAY_NONE && (sp.head & 0xFFFFFu) == m >> 6) >> lane0;
+        same &= (k < 64 ? 1ull << k : 0ull) - 1;
+        same &= same - 1; // (but the first)
+        if (same)
+        {
+            // equal times: port order, frame_before decides (the reference's scan over the ports)
+            L.base[x.q] = sp.p;
+            wave_sync();
+            for (; same; same &= same - 1)
+            {
+                const int q = __builtin_ctzll(same);
+                if (frame_before(R, lane_input(B, W, x, t, L, q).at(L.base[q]), lane_input(B, W, x, t, L, best).at(L.base[best])))
+                    best = q;
+            }
+            wave_sync();
+        }
+        const uint32_t nr = __shfl(sp.head, lane0 + best) >> 20;
+#else
         // the earliest head (the first port holding it)
         int best = -1;
         uint32_t bt = SPRAY_NONE;
@@ -2926,6 +2965,7 @@ struct Model
                 best = q;
         }
         const uint32_t nr = (uint32_t)L.cnt[best] >> 20;
+#endif
         uint8_t draw = 0;
         if (nr != 255u && nr)
             draw = (uint8_t)tw_mrg_integer(sp.g, nr);
