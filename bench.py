@@ -509,7 +509,7 @@ def rdma_leg(a):
                    "reference": "src/rdma (the reference's model) compiled for the CPU: oracle/_ref/twins-rdma-cpu"},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 3), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 6), "traffic": rdma_traffic_bytes(),
-                     "traffic_source": "HBM bytes per step (2 launches: a launch ends after 1 s) of this kernel on this workload: "
+                     "traffic_source": "HBM bytes per step (a launch) of this kernel on this workload: "
                                        "rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE runs scaled by a 1 GiB copy's readings "
                                        "(profiles/rdma_team_kernel_config3.md)",
                      "kernel": "rdma_team_kernel",
