@@ -50,6 +50,20 @@ def test_cpu_build_batch_equals_single_runs(cpu_bin, tmp_path):
     assert rdma_util.sum_counters(got) == rdma_util.sum_counters([j[5] for j in sel])
 
 
+def run_units(*args):
+    d = os.path.dirname(rdma_util.CPU_BIN)
+    subprocess.run(["make", "-C", d, "units"], check=True, capture_output=True)
+    r = subprocess.run([os.path.join(d, "units"), *args], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-3000:]
+
+
+def test_out_buckets_of_unlike_delays():
+    """Frames over links of one slot's delay to 4,000: filed by arrival slot, found in a step or two; a
+    world of 20 us links beside one of 1 us (the slot of both) has the flows it has alone."""
+    run_units("out_buckets")
+    run_units("unlike_delays", rdma_util.CONFIG, f"{rdma_util.INPUTS}/ft4.topo", f"{rdma_util.INPUTS}/inc1.csv")
+
+
 def test_serving_loop_on_cpu(tmp_path):
     """The serving loop (trd_server_*) with the kernel's steps on the CPU: four reference jobs in an
     arena that holds the two k=8 worlds only one at a time (admission waits for memory), every

@@ -691,6 +691,7 @@ static int pack(trd_batch &b, trd_world *const *worlds, int W, const trd_pack_cf
             if (nb > 4096)
                 return fail(TW_EINVAL, "a link's delay (%lld ns) is too long for the slot (%lld ns)", (long long)x.delay, (long long)D);
             x.nb = (uint32_t)nb;
+            x.skip = (uint32_t)(x.delay / D);
             x.cap = (uint32_t)cap;
             x.moff = nframes;
             x.coff = (uint32_t)ncnt;

@@ -376,13 +376,14 @@ struct Link
     uint64_t bps;
     uint64_t moff;
     uint32_t coff, nb, cap, rc;
+    uint32_t skip; // whole slots of its delay: no frame of a slot arrives before the skip-th after it
 };
 
 // a sender's place in its out link's ring (src/rdma/rstep.cuh:45-66)
 struct OutBucket
 {
     int64_t hi;     // the open bucket's end (0: none open)
-    int64_t a, end; // the arrival slot reached (the open bucket's, or before any the running slot) and its end
+    int64_t a, end; // the arrival slot reached (the open bucket's, or before any the first a frame can have) and its end
     uint32_t b, pb; // its places in the link's ring and in the world's pending-slot ring
     uint64_t base;
     uint32_t cnt, n;
@@ -633,10 +634,10 @@ RD_HD void ob_open(SimRef s, OutBucket &o, int link, int64_t last, int64_t slot,
 {
     const Link l = s.li[link];
     o.hi = 0;
-    o.a = slot;
-    o.end = (slot + 1) * s.D;
-    o.b = ring_place(slot, l.nb);
-    o.pb = ring_place(slot, (uint32_t)pend_n);
+    o.a = slot + l.skip;
+    o.end = (o.a + 1) * s.D;
+    o.b = ring_place(o.a, l.nb);
+    o.pb = ring_place(o.a, (uint32_t)pend_n);
     o.link = link;
     o.last = last;
     o.txs[0] = o.txs[1] = 0;
@@ -666,9 +667,11 @@ RD_HD void ob_flush(SimRef s, OutBucket &o)
     o.hi = 0;
 }
 // a place in the bucket of the frame's arrival slot (null: full, counted). A link's frames arrive one
-// after another, so the arrival slot is found by stepping on from the last one's: one or two steps,
-// where the quotient and the ring places took three 64-bit divisions (some 500 instructions that
-// every lane of the wave waited for)
+// after another, so the arrival slot is found by stepping on from the last one's, or from the first
+// a frame of the running slot can arrive in (ob_open: the link's delay may be thousands of slots of
+// the batch's shortest one): a step or two, and over a slot one for each slot of tx time, where the
+// quotient and the ring places took three 64-bit divisions (some 500 instructions that every lane of
+// the wave waited for)
 RD_HD LFrame RD_G *ob_push(SimRef s, uint32_t *pend, int pend_n, int64_t ts, OutBucket &o)
 {
     if (ts >= o.hi)
