@@ -6,9 +6,12 @@
 #include <cstring>
 #include <hip/hip_runtime_api.h>
 
+size_t shim_bytes = 0; // of all device allocations so far
+
 extern "C" {
 hipError_t hipMalloc(void **p, size_t n)
 {
+    shim_bytes += n;
     *p = calloc(1, n ? n : 1);
     return *p ? hipSuccess : hipErrorOutOfMemory;
 }

@@ -1,0 +1,90 @@
+// TEST INFRASTRUCTURE: checks of single functions of libtwins_core's TCP side on the CPU (the kernel's
+// launch replaced by the harness, kernel_cpu.cpp); "units CHECK" exits non-zero and says what differs.
+#include <cstdio>
+#include <cstring>
+#include <fstream>
+#include <string>
+#include <vector>
+#include "../../../include/twins.h"
+
+extern size_t shim_bytes;
+static int bad = 0;
+#define CHECK(c, ...)                                                                                                                     \
+    do                                                                                                                                    \
+    {                                                                                                                                     \
+        if (!(c))                                                                                                                         \
+        {                                                                                                                                 \
+            bad++;                                                                                                                        \
+            printf(__VA_ARGS__);                                                                                                          \
+            printf(" (%s)\n", #c);                                                                                                        \
+        }                                                                                                                                 \
+    } while (0)
+
+static tw_world *world(const char *dir, const char *flows, std::vector<std::string> more = {})
+{
+    const std::string path = std::string(dir) + "/units.csv";
+    std::ofstream(path) << flows;
+    more.insert(more.begin(), {"--k=4", "--flows=" + path});
+    std::vector<const char *> a;
+    for (auto &x : more)
+        a.push_back(x.c_str());
+    tw_world *w = nullptr;
+    CHECK(tw_world_create_args((int)a.size(), a.data(), &w) == 0, "%s", tw_last_error());
+    return w;
+}
+// the device memory of a batch of this world
+static size_t packed(tw_world *w, int runs)
+{
+    tw_pack_cfg c = {};
+    c.chain_runs = runs;
+    c.blocks = c.team_blocks = 1; // (the same launch scratch for every world)
+    tw_batch *b = nullptr;
+    const size_t before = shim_bytes;
+    CHECK(tw_batch_create(&w, 1, &c, &b) == 0, "%s", tw_last_error());
+    tw_batch_destroy(b);
+    return shim_bytes - before;
+}
+
+// The footprint that admission to the serving loop and tw_world_info give counts what a world's records
+// take: between two worlds alike but for one quantity it grows by no less than the memory does (the
+// rest of a batch, its launch's scratch, is the same for both).
+static void footprint(const char *dir)
+{
+    const char *head = "src,dst,flow_size,start_ns\n";
+    std::string many = head;
+    for (int i = 0; i < 4000; i++)
+        many += std::to_string(i % 16) + "," + std::to_string((i + 5) % 16) + ",1000," + std::to_string(i * 100) + "\n";
+    struct
+    {
+        const char *what;
+        std::string flows;
+        std::vector<std::string> more;
+    } const cases[] = {{"ledger places", std::string(head) + "0,5,900000000,0\n", {"--rtt_ring=600000"}},
+                       {"flows", many, {}},
+                       {"queue", std::string(head) + "0,5,1000,0\n", {"--queue=5000"}},
+                       {"larger network", std::string(head) + "0,5,1000,0\n", {"--k=16"}},
+                       {"spray streams", std::string(head) + "0,5,1000,0\n", {"--spray=1"}}};
+    for (auto &c : cases)
+    {
+        tw_world *a = world(dir, (std::string(head) + "0,5,1000,0\n").c_str()), *b = world(dir, c.flows.c_str(), c.more);
+        tw_world_info ia, ib;
+        tw_world_info_get(a, &ia);
+        tw_world_info_get(b, &ib);
+        const long long info = (long long)(ib.device_bytes - ia.device_bytes), mem = (long long)(packed(b, 9) - packed(a, 9));
+        printf("%s: footprint +%lld, memory +%lld\n", c.what, info, mem);
+        CHECK(info >= mem && info <= mem + mem / 100 + 4096, "%s", c.what);
+        tw_world_destroy(a);
+        tw_world_destroy(b);
+    }
+}
+
+int main(int argc, char **argv)
+{
+    const char *what = argc > 1 ? argv[1] : "";
+    if (!strcmp(what, "footprint") && argc > 2)
+        footprint(argv[2]);
+    else
+        return 2;
+    printf("%s: %d differences\n", what, bad);
+    return bad != 0;
+}

@@ -20,6 +20,18 @@ def harness():
     return BIN
 
 
+def run_units(harness, *args):
+    r = subprocess.run([os.path.join(HARNESS, "units"), *args], capture_output=True, text=True, timeout=300,
+                       env={**os.environ, "ASAN_OPTIONS": "detect_leaks=0"})
+    assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-3000:]
+
+
+def test_footprint_counts_what_is_packed(harness, tmp_path):
+    """tw_world_info's device_bytes (the serving loop's admission) grows with a world's flows, ledger
+    places, queues, network and spray streams as the memory packing allocates does."""
+    run_units(harness, "footprint", str(tmp_path))
+
+
 @pytest.mark.parametrize("name", CASES)
 def test_kernel_code_on_cpu_matches_ns3(harness, name, tmp_path):
     by_name = {c[0]: c for c in util.cases()}

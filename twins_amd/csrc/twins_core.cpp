@@ -577,18 +577,25 @@ extern "C" int tw_world_destroy(tw_world *w)
     return TW_OK;
 }
 
-static uint64_t world_bytes(const tw_world &w, int runs)
+// the device memory of a world's part of a batch: the arrays of pack(), by what they are counted in
+template <int RUNS>
+static uint64_t world_bytes_of(const tw_world &w)
 {
-    const uint64_t F = runs == 25 ? 128 : 64, CHB = (runs + 1) * 4;
-    uint64_t b = 0;
-    b += (uint64_t)NRING * w.L * MAX_TX * F + (uint64_t)NRING * w.L * 8;          // link messages
-    b += (uint64_t)w.L * (std::max(w.queue, 1) + 2) * F + (uint64_t)w.L * (40 + CHB); // queues
+    typedef BatchT<RUNS> B;
+    const uint64_t F = sizeof(typename B::Frame), CHB = B::CW * 4;
+    uint64_t b = sizeof(WorldDesc) + sizeof(WorldRun);
     b += (uint64_t)w.NC * (sizeof(ConnStatic) + sizeof(SndRec) + sizeof(RcvRec) + 4 * CHB);
-    b += w.it_total * 21 + w.oo_total * 8;
-    b += (uint64_t)w.M * 40 + (uint64_t)w.H * (2 * MAX_ACTIVE * 4 + MAX_DUE * 16 + 40);
-    b += w.rt_off.size() * 5 + w.rt_ports.size() + w.port_dn.size() + w.rng.size() * 48;
+    b += w.it_total * (sizeof(SentEntry) + sizeof(SentNote)) + w.oo_total * 8;
+    b += (uint64_t)w.M * (3 * 4 + 3 * 8);               // messages: connection, end, place in their host's order; start, times
+    b += (uint64_t)w.H * (5 * 4 + 1 + 3 * 8);           // hosts: counters, congestion control, wake-up and timers
+    b += (uint64_t)w.H * (2 * MAX_ACTIVE * 4 + MAX_DUE * sizeof(Due));
+    b += (uint64_t)w.L * (4 + 8 + 5 * 4 + 2 * 8 + CHB); // links: in-link and queue
+    b += (uint64_t)w.L * ((std::max(w.queue, 1) + 2) * F + NRING * (MAX_TX * F + 8)); // queued frames, link messages
+    b += (uint64_t)w.S * 4 + w.rng.size() * sizeof(TwMrgState);
+    b += (w.host_sw.size() + w.host_port.size()) * 4 + w.rt_off.size() * 5 + w.rt_ports.size() + w.port_dn.size() + w.fail_t.size() * 8;
     return b;
 }
+static uint64_t world_bytes(const tw_world &w, int runs) { return runs == 25 ? world_bytes_of<25>(w) : world_bytes_of<9>(w); }
 
 extern "C" int tw_world_info_get(const tw_world *w, tw_world_info *info)
 {
