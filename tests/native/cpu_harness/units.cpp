@@ -8,6 +8,10 @@
 #include "../../../include/twins.h"
 
 extern size_t shim_bytes;
+namespace tw
+{
+extern bool cpu_time_out;
+}
 static int bad = 0;
 #define CHECK(c, ...)                                                                                                                     \
     do                                                                                                                                    \
@@ -78,11 +82,36 @@ static void footprint(const char *dir)
     }
 }
 
+// A barrier that times out in a world's first slot is reported as such, by both ways to run a batch.
+static void timeout_error(const char *dir)
+{
+    tw_world *w[2] = {world(dir, "src,dst,flow_size,start_ns\n0,5,1000,0\n"), nullptr};
+    w[1] = w[0];
+    for (int n = 1; n <= 2; n++)
+        for (int noalloc = 0; noalloc < 2; noalloc++)
+        {
+            tw_pack_cfg c = {};
+            c.blocks = c.team_blocks = 1;
+            tw_batch *b = nullptr;
+            CHECK(tw_batch_create(w, n, &c, &b) == 0, "%s", tw_last_error());
+            tw::cpu_time_out = true;
+            tw_run_stats st;
+            const int rc = noalloc ? tw_batch_run_noalloc(b, &st) : tw_batch_run(b, &st);
+            tw::cpu_time_out = false;
+            CHECK(rc == TW_EDEVICE && strstr(tw_last_error(), "a team barrier timed out"), "%d worlds, noalloc %d: error %d, %s", n, noalloc, rc,
+                  tw_last_error());
+            tw_batch_destroy(b);
+        }
+    tw_world_destroy(w[0]);
+}
+
 int main(int argc, char **argv)
 {
     const char *what = argc > 1 ? argv[1] : "";
     if (!strcmp(what, "footprint") && argc > 2)
         footprint(argv[2]);
+    else if (!strcmp(what, "timeout_error") && argc > 2)
+        timeout_error(argv[2]);
     else
         return 2;
     printf("%s: %d differences\n", what, bad);

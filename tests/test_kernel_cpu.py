@@ -26,6 +26,11 @@ def run_units(harness, *args):
     assert r.returncode == 0, r.stdout[-3000:] + r.stderr[-3000:]
 
 
+def test_barrier_timeout_is_reported_as_one(harness, tmp_path):
+    """A team barrier that times out before any slot ended: TW_EDEVICE, as after one that ran some."""
+    run_units(harness, "timeout_error", str(tmp_path))
+
+
 def test_footprint_counts_what_is_packed(harness, tmp_path):
     """tw_world_info's device_bytes (the serving loop's admission) grows with a world's flows, ledger
     places, queues, network and spray streams as the memory packing allocates does."""

@@ -1408,6 +1408,21 @@ static void capture(tw_batch &b)
     (void)hipGetLastError();
 }
 
+// Every launch runs at least one slot of every unfinished world it reaches, or ends it with an error
+// (a team whose barrier timed out writes no slots: its world's error is reported once all have ended).
+static bool launch_advanced(const std::vector<WorldRun> &run, std::vector<int64_t> &slots_before, int unfinished_before)
+{
+    int64_t ran = 0;
+    int unfinished = 0;
+    for (size_t i = 0; i < run.size(); i++)
+    {
+        ran += run[i].slots_run - slots_before[i];
+        slots_before[i] = run[i].slots_run;
+        unfinished += !run[i].finished;
+    }
+    return ran > 0 || unfinished < unfinished_before;
+}
+
 extern "C" int tw_batch_run(tw_batch *b, tw_run_stats *stats)
 {
     if (!b)
@@ -1444,14 +1459,8 @@ extern "C" int tw_batch_run(tw_batch *b, tw_run_stats *stats)
         HIPCHK(hipEventElapsedTime(&ms, b->ev0, b->ev1));
         st.kernel_s += ms / 1000.0;
         st.launches++;
-        // every launch runs at least one slot of every unfinished world it reaches
-        int64_t ran = 0;
-        for (int i = 0; i < W; i++)
-            ran += b->run_host[i].slots_run - slots_before[i];
-        if (ran == 0)
+        if (!launch_advanced(b->run_host, slots_before, unfinished))
             return fail(TW_ESTATE, "a launch ran no slot of the %d unfinished worlds", unfinished);
-        for (int i = 0; i < W; i++)
-            slots_before[i] = b->run_host[i].slots_run;
     }
     st.wall_s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     for (auto &r : b->run_host)
@@ -1536,13 +1545,7 @@ extern "C" int tw_batch_run_noalloc(tw_batch *b, tw_run_stats *stats)
         HIPCHK(hipEventElapsedTime(&ms, b->ev0, b->ev1));
         st.kernel_s += ms / 1000.0;
         st.launches++;
-        int64_t ran = 0;
-        for (int i = 0; i < W; i++)
-        {
-            ran += b->run_host[i].slots_run - b->slots_before[i];
-            b->slots_before[i] = b->run_host[i].slots_run;
-        }
-        if (ran == 0)
+        if (!launch_advanced(b->run_host, b->slots_before, unfinished))
             return fail(TW_ESTATE, "a launch ran no slot of the %d unfinished worlds", unfinished);
     }
     st.wall_s = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
