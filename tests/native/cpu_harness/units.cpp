@@ -6,6 +6,7 @@
 #include <string>
 #include <vector>
 #include "../../../include/twins.h"
+#include "../../../twins_amd/csrc/tcp_state.h"
 
 extern size_t shim_bytes;
 namespace tw
@@ -105,11 +106,29 @@ static void timeout_error(const char *dir)
     tw_world_destroy(w[0]);
 }
 
+// The word that hands a team its next slot holds every slot whose time a 64-bit picosecond count can
+// state, beside the flags and the count.
+static void slot_word()
+{
+    using tw::SlotGo;
+    const int64_t last = INT64_MAX / tw::SLOT_PS;
+    for (int64_t t : {(int64_t)0, (int64_t)1, (int64_t)0x7FFFFFFF, (int64_t)0xFFFFFFFF, (int64_t)0x100000000, (int64_t)0x100000007, last})
+        for (unsigned flags = 0; flags < 8; flags++)
+            for (unsigned count : {0u, 1u, 0xFFFFu, 0x12345u})
+            {
+                const unsigned long long g = SlotGo::pack(t, flags, count);
+                CHECK(SlotGo::next(g) == t && SlotGo::flags(g) == flags && SlotGo::count(g) == (count & 0xFFFFu), "slot %lld flags %u count %u: %lld %u %u",
+                      (long long)t, flags, count, (long long)SlotGo::next(g), SlotGo::flags(g), SlotGo::count(g));
+            }
+}
+
 int main(int argc, char **argv)
 {
     const char *what = argc > 1 ? argv[1] : "";
     if (!strcmp(what, "footprint") && argc > 2)
         footprint(argv[2]);
+    else if (!strcmp(what, "slot_word"))
+        slot_word();
     else if (!strcmp(what, "timeout_error") && argc > 2)
         timeout_error(argv[2]);
     else

@@ -106,3 +106,21 @@ def test_gpu_resumed_launches(team, budget):
     est, done = b.fct(0)
     assert [(str(e), str(d)) for e, d in zip(est, done)] == util.read_cols(os.path.join(util.GOLDEN, ref), (4, 5))
     b.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("team", [1, 3, 0])
+def test_gpu_skip_past_32_bit_slots(team, tmp_path):
+    """An idle world skips to a flow that starts after slot 2^32 and ends at its last slot (a link's
+    messages are of slots below 2^31, so that flow's SYNs are lost there, on the CPU alike)."""
+    import twins_amd
+    flows = tmp_path / "late.csv"
+    flows.write_text("src,dst,flow_size,start_ns\n0,5,100000,0\n1,9,100000,4300000000000\n")
+    w = twins_amd.World(["--k=4", f"--flows={flows}", "--max_slots=4300100000"])
+    b = twins_amd.Batch([w], team_blocks=team)
+    print(f"team {team}", flush=True)
+    st = b.run()
+    est, done = b.fct(0)
+    assert (st.worlds_done, st.launches, b.counters(0)[26]) == (1, 1, 652)
+    assert (list(est), list(done)) == ([12044, -1], [71653, -1])
+    b.close()

@@ -31,6 +31,12 @@ def test_barrier_timeout_is_reported_as_one(harness, tmp_path):
     run_units(harness, "timeout_error", str(tmp_path))
 
 
+def test_slot_word_holds_any_slot(harness):
+    """The next slot a team is told, past 2^32 too (--max_slots is not bounded, and an idle world skips
+    to its next event)."""
+    run_units(harness, "slot_word")
+
+
 def test_footprint_counts_what_is_packed(harness, tmp_path):
     """tw_world_info's device_bytes (the serving loop's admission) grows with a world's flows, ledger
     places, queues, network and spray streams as the memory packing allocates does."""

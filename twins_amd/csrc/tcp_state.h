@@ -80,7 +80,7 @@ constexpr uint32_t MSS = 1460;
 constexpr int CTRL_FRAME = 42, SYN_FRAME = 46;
 constexpr int MAX_TX = 300;    // frames one link can start in a slot (the model's cap)
 constexpr int NRING = 3;       // link message ring: slots t-2, t-1 (read) and t (written)
-TW_HD inline uint32_t ring_of(int64_t t) { return (uint32_t)t % NRING; } // (0 <= t < 2^31)
+TW_HD inline uint32_t ring_of(int64_t t) { return (uint32_t)t % NRING; } // (messages are of slots below 2^31: msg_word)
 // The kernel's quotients by numbers fixed for a world: n / d from the high half of n * ceil(2^32 / d),
 // exact while n * d < 2^32 (d == 1: m = 0). A division by a value unknown to the compiler is some 40
 // instructions, and a 64-bit one, by a constant too, ten quarter-rate multiplications.
@@ -316,19 +316,22 @@ struct alignas(128) TeamState
     unsigned long long prof[4]; // TW_PROF: this slot's maxima (hosts, switches, work); last ticket time
 };
 
-// What the last workgroup of a slot tells the others, in one word: the next slot, how the world
-// goes on, and the count of slots run in this launch (its low bits), which they wait for.
+// What the last workgroup of a slot tells the others, in one word: the next slot (44 bits: any slot
+// whose time is a 64-bit count of picoseconds), how the world goes on, and above them the count of
+// slots run in this launch (its low 16 bits), which they wait for.
 struct SlotGo
 {
     static constexpr unsigned FIN = 1, IDLE = 2, ERR = 4;
+    static constexpr int BITS = 44;
     TW_HD static unsigned long long pack(int64_t next, unsigned flags, unsigned count)
     {
-        return (unsigned long long)(count & 0xFFFFu) << 48 | (unsigned long long)flags << 32 | (uint32_t)next;
+        return (unsigned long long)(count & 0xFFFFu) << 48 | (unsigned long long)flags << BITS | (unsigned long long)next;
     }
     TW_HD static unsigned count(unsigned long long g) { return (unsigned)(g >> 48); }
-    TW_HD static unsigned flags(unsigned long long g) { return (unsigned)(g >> 32) & 0xFFFFu; }
-    TW_HD static int64_t next(unsigned long long g) { return (int64_t)(uint32_t)g; }
+    TW_HD static unsigned flags(unsigned long long g) { return (unsigned)(g >> BITS) & 0xFu; }
+    TW_HD static int64_t next(unsigned long long g) { return (int64_t)(g & ((1ull << BITS) - 1)); }
 };
+static_assert(INT64_MAX / SLOT_PS < (int64_t)1 << SlotGo::BITS, "a slot fits its place");
 
 // The serving loop (tcp_server_kernel): requests are single-world batches resident in device
 // memory. Queue q's requests are req[q * cap + i] in order; the host publishes tail[q] and the
