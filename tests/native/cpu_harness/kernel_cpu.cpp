@@ -39,6 +39,8 @@ static inline T atomicMin(T *p, U v)
 
 namespace tw
 {
+// frames of a host's slot that go through a workspace: few, so that slots take both ways
+constexpr int STAGED = 3;
 template <int RUNS>
 static void run_cpu(BatchT<RUNS> &B, int64_t budget)
 {
@@ -59,10 +61,15 @@ static void run_cpu(BatchT<RUNS> &B, int64_t budget)
             for (int hl = 0; hl < W.H; hl++)
             {
                 int64_t x = INT64_MAX;
-                SndState ls;
-                RcvState lr;
-                ConnStatic lc;
-                act += Md::host_step(B, W, R, hl, t, &x, &ls, &lr, &lc);
+                // (the frames out: the first STAGED through a workspace of its own, as the kernel's through LDS)
+                typename Md::HostIn in;
+                if (Md::host_open(B, W, hl, t, in, &x))
+                {
+                    std::vector<typename Md::Frame> st(STAGED);
+                    int staged = 0;
+                    act += Md::host_run(B, W, R, hl, t, &x, in, st.data(), STAGED, &staged);
+                    std::copy_n(st.data(), staged, Md::msg_of(B, t, W.link0 + hl));
+                }
                 wk = std::min(wk, (unsigned long long)x);
             }
             for (int sw = 0; sw < W.S; sw++)

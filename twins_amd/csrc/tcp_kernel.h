@@ -10,8 +10,8 @@ namespace tw
 constexpr double SERVER_WAIT_S = 600.0;
 // a launch of the persistent world-queue kernel: `blocks` workgroups of `threads` (their teams,
 // sizes and queues are the batch's TeamPlan); `teams` when a team has several workgroups (the
-// grid must then fit the GPU at once); `one` when every world has a wave for each of its work items
-// at one host per item (the kernel built for that); each world runs at most slot_budget slots per launch
+// grid must then fit the GPU at once); `one` when every world's host items are of one host on every
+// team that may take it (the kernel built for that); each world runs at most slot_budget slots per launch
 struct LaunchShape
 {
     int blocks, threads, teams, one;

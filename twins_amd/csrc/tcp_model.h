@@ -420,7 +420,7 @@ struct Model
         int sf, rf;
         uint32_t max_it; // the longest sent ledger of the slot
         // What the running event sends, queued after its handler by the one place that builds frames
-        // (host_step's loop): the frames asked for (at most 4: an ACK at a CE edge, one for the data,
+        // (host_run's loop): the frames asked for (at most 4: an ACK at a CE edge, one for the data,
         // the close's; or one segment sent again), then, if fill, segments while the window has room,
         // then one more asked for after that.
         Out ask[4], post;
@@ -2085,16 +2085,9 @@ struct Model
         *wake = w;
         return false;
     }
-    // (src/step.cuh:2263-2528): returns 1 if it sent or holds frames; *wake: its next slot
-    // (three arguments of callers that keep record slots are taken and not used)
-    static __device__ int host_step(Batch &B, World &W, WorldRun *R, int hl, int64_t t, int64_t *wake, SndState *, RcvState *, ConnStatic *)
-    {
-        HostIn in;
-        int staged;
-        return host_open(B, W, hl, t, in, wake) ? host_run(B, W, R, hl, t, wake, in, nullptr, 0, &staged) : 0;
-    }
-    // the slot of a host that has events; st: the lane's workspace for the first st_cap frames out,
-    // which the caller moves to the link's message (*staged of them)
+    // the slot of a host that has events (src/step.cuh:2263-2528): returns 1 if it sent or holds frames;
+    // *wake: its next slot; st: the lane's workspace for the first st_cap frames out, which the caller
+    // moves to the link's message (*staged of them)
     static __device__ int host_run(Batch &B, World &W, WorldRun *R, int hl, int64_t t, int64_t *wake, const HostIn &hi, Frame *st, int st_cap,
                                    int *staged)
     {
