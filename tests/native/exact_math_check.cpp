@@ -1,6 +1,7 @@
 // Host-side check of the device math replicas (twins_amd/csrc/exact_math.h) against what ns-3 itself
 // computes on x86-64: libm's pow (glibc's FMA variant on an FMA host) and GetSeconds summed in x87
 // long double. Built with g++ -ffp-contract=off; exits non-zero on any bit difference.
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <random>
@@ -72,6 +73,30 @@ int main(int argc, char **argv)
             sbad++;
         }
     }
-    printf("pow: %ld of %ld differ; seconds: %ld of %ld differ\n", bad, tot, sbad, n);
-    return bad || sbad;
+    // MRG32k3a (exact_math.h) against the recurrence in 64-bit integers: the remainder over all values its
+    // products can take, half of them next to a multiple of the modulus, then a stream's states
+    long mbad = 0;
+    const int64_t m[2] = {4294967087ll, 4294944443ll}, pos[2] = {1403580, 527612}, neg[2] = {810728, 1370589};
+    auto mod = [](int64_t v, int64_t q) { return (v % q + q) % q; };
+    for (long i = 0; i < n; i++)
+        for (int g = 0; g < 2; g++)
+        {
+            const int64_t lo = -neg[g] * (m[g] - 1), hi = pos[g] * (m[g] - 1);
+            int64_t v = lo + (int64_t)(rng() % (uint64_t)(hi - lo + 1));
+            if (i & 1)
+                v = std::min(hi, std::max(lo, v - mod(v, m[g]) + (int64_t)(rng() % 5) - 2));
+            mbad += tw_mrg_mod((double)v, (double)m[g], 1.0 / (double)m[g]) != (double)mod(v, m[g]);
+        }
+    TwMrg st = {{12345, 12345, 12345, 12345, 12345, 12345}};
+    int64_t s[6] = {12345, 12345, 12345, 12345, 12345, 12345};
+    for (long i = 0; i < n; i++)
+    {
+        const int64_t p = mod(pos[0] * s[1] - neg[0] * s[0], m[0]), q = mod(pos[1] * s[5] - neg[1] * s[3], m[1]);
+        s[0] = s[1], s[1] = s[2], s[2] = p, s[3] = s[4], s[4] = s[5], s[5] = q;
+        (void)tw_mrg_u01(st);
+        for (int k = 0; k < 6; k++)
+            mbad += st.s[k] != (double)s[k];
+    }
+    printf("pow: %ld of %ld differ; seconds: %ld of %ld differ; mrg: %ld differ\n", bad, tot, sbad, n, mbad);
+    return bad || sbad || mbad;
 }

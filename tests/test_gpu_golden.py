@@ -69,9 +69,11 @@ def test_gpu_batch_equals_standalone(tmp_path):
 @pytest.mark.parametrize("runs", [9, 25])
 @pytest.mark.parametrize("team,hosts", [(0, 0), (52, 1), (1, 1), (3, 5), (1, 64), (16, 33)])
 def test_gpu_launch_shapes(team, hosts, runs):
-    """One host to a wave (the kernel whose hosts' branches are wave-uniform) and 5 to 64 (a lane
-    each, 100 staged frames a host down to none), on teams of few and many waves: loss and its
-    repair, sprayed reordering, FIN and a torus give ns-3's stored times."""
+    """One host to a wave (the kernel whose hosts' branches are wave-uniform, every frame of a slot
+    staged) and 5 to 64 (a lane each, down to 9 staged frames a host, 4 with chains of 25, the others
+    stored as they are sent), on teams of few and many waves: loss and its repair, sprayed reordering
+    (the draws' merge by shuffles), FIN and a torus give ns-3's stored times. None of these runs leaves
+    a tie undecided, with chains of 9 or 25."""
     import twins_amd
     pick = [c for c in CASES if c[0] in ("k8_incast16-cubic-fin", "k8_a2a30-newreno-spray", "torus6_a2a30-dctcp-base")]
     assert len(pick) == 3
@@ -82,8 +84,8 @@ def test_gpu_launch_shapes(team, hosts, runs):
         assert b.run().worlds_done == 1
         est, done = b.fct(0)
         exp = util.read_cols(os.path.join(util.GOLDEN, ref), (4, 5))
-        if not b.counters(0)[25]:  # (no tie left undecided by chains of 9)
-            assert [(str(e), str(d)) for e, d in zip(est, done)] == exp, name
+        assert b.counters(0)[25] == 0, name
+        assert [(str(e), str(d)) for e, d in zip(est, done)] == exp, name
         b.close()
 
 
