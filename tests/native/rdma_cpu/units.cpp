@@ -110,11 +110,33 @@ static void unlike_delays(const char *config, const char *topo, const char *flow
         trd_world_destroy(x);
 }
 
+// The launch shapes of FatTree worlds on a GPU of 256 workgroups: what is resident, and what runs by workgroup.
+static void fattrees(int k, int W, std::vector<int> &hosts, std::vector<int> &switches)
+{
+    hosts.assign(W, k * k * k / 4);
+    switches.assign(W, 5 * k * k / 4);
+}
+static void lone_world()
+{
+    // two callers' worlds, each alone in its batch, are resident together
+    for (int k : {4, 8, 16, 32})
+        for (int cap : {1, 64, 256})
+        {
+            std::vector<int> h, s;
+            fattrees(k, 1, h, s);
+            const rd::LaunchShape x = rd::launch_shape(h.data(), s.data(), 1, cap, true, 0, 0);
+            CHECK(x.T >= 1 && x.T <= cap && x.T <= 128, "k=%d alone on %d: %d workgroups", k, cap, x.T);
+            CHECK(x.hpw >= 1 && x.hpw <= 64, "k=%d alone on %d: %d hosts an item", k, cap, x.hpw);
+        }
+}
+
 int main(int argc, char **argv)
 {
     const char *what = argc > 1 ? argv[1] : "";
     if (!strcmp(what, "out_buckets"))
         out_buckets();
+    else if (!strcmp(what, "lone_world"))
+        lone_world();
     else if (!strcmp(what, "unlike_delays") && argc > 4)
         unlike_delays(argv[2], argv[3], argv[4]);
     else

@@ -64,6 +64,12 @@ def test_out_buckets_of_unlike_delays():
     run_units("unlike_delays", rdma_util.CONFIG, f"{rdma_util.INPUTS}/ft4.topo", f"{rdma_util.INPUTS}/inc1.csv")
 
 
+def test_lone_world_leaves_room_for_another():
+    """A world alone takes at most half the GPU's workgroups: two launched at once are both resident
+    (each waiting for workgroups the other holds, they would end only by their barriers' time limit)."""
+    run_units("lone_world")
+
+
 def test_serving_loop_on_cpu(tmp_path):
     """The serving loop (trd_server_*) with the kernel's steps on the CPU: four reference jobs in an
     arena that holds the two k=8 worlds only one at a time (admission waits for memory), every

@@ -926,41 +926,13 @@ extern "C" int trd_batch_run(trd_batch *b, trd_run_stats *st)
     int launches = 0;
     double kernel_s = 0;
     int64_t prev = -1;
-    // The launch shape: one team size and hosts per host item. Every world that fits runs at once, each
-    // on its share of the GPU (worlds queued behind others leave it idle when few are left). A slot
-    // lasts as long as its longest item, and a wave runs unlike hosts one after another, so the fewest
-    // hosts per item (a power of two) of these: a switch a workgroup and four host items a workgroup,
-    // all side by side; else every item on a wave of its own; else every host item. Measured (kernel
-    // time): 24 FatTree k=8 worlds of 128 hosts (DCQCN, HPCC and DCTCP) 145 ms on teams of 16 at 64
-    // hosts per item (16 worlds at once), 88, 84 and 90 ms on teams of 10 at 2, 4 and 8 hosts; FatTree
-    // k=8 (HPCC) alone 104, 85 and 85 ms on 128 workgroups at 2 and 112 and 208 at 1; two 512-host
-    // leaf-spines 124, 107 and 121 ms on 128 workgroups each at 1, 2 and 4.
     const int cap = b->max_teams;
-    const int share = std::max(1, cap / b->W);
-    auto by_group = [&](int i, int h) { return b->ss[i] + ((b->hs[i] + h - 1) / h + 3) / 4; };
-    auto by_wave = [&](int i, int h) { return (b->hs[i] + h - 1) / h + b->ss[i]; };
     const bool grouped = b->kmax <= rd::KS;
-    int T = b->team_blocks > 0 ? std::min(b->team_blocks, cap) : share, hpw = b->hpw;
-    for (int rule = grouped ? 0 : 1; hpw <= 0 && rule < 3; rule++)
-        for (int h = 1; hpw <= 0 && h <= 64; h *= 2)
-        {
-            bool fits = true;
-            for (int i = 0; i < b->W; i++)
-                fits = fits && (rule == 0 ? by_group(i, h) <= T : rule == 1 ? by_wave(i, h) <= 4 * T : (b->hs[i] + h - 1) / h <= 4 * T);
-            if (fits)
-                hpw = h;
-        }
-    hpw = hpw > 0 ? hpw : 64;
+    const rd::LaunchShape shape = rd::launch_shape(b->hs.data(), b->ss.data(), b->W, cap, grouped, b->team_blocks, b->hpw);
+    const int T = shape.T, hpw = shape.hpw;
     vector<int> items(b->W);
-    int most = 1;
     for (int i = 0; i < b->W; i++)
-    {
-        items[i] = by_wave(i, hpw);
-        most = std::max(most, grouped ? by_group(i, hpw) : items[i]);
-    }
-    if (b->team_blocks <= 0)
-        T = std::min(T, most);
-    T = std::max(1, std::min(T, cap));
+        items[i] = rd::wave_items(b->hs[i], b->ss[i], hpw);
     // worlds by work items, largest first
     vector<int> order(b->W);
     for (int i = 0; i < b->W; i++)
@@ -976,7 +948,7 @@ extern "C" int trd_batch_run(trd_batch *b, trd_run_stats *st)
         rd::LaunchCfg L = {};
         L.T = T;
         L.hpw = hpw;
-        L.by_group = grouped ? 3 : 0;
+        L.by_group = grouped ? 1 : 0;
         L.nq = (int)queue.size();
         L.queue = b->queue_d;
         L.qnext = b->qnext_d;

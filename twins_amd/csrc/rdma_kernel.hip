@@ -146,16 +146,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
         const World wd = s.wd[w];
         WorldRun &r = s.run[w];
         uint32_t *pend = s.pend + wd.pend_off;
-        const int hpw = L.hpw, nhw = (wd.nh + hpw - 1) / hpw;
+        const int hpw = L.hpw, nhw = host_items(wd.nh, hpw);
         // Work items: a wave each, or, where the team has about a workgroup per switch, a switch for a
         // whole workgroup (its ports over four waves: a wave's lanes run unlike events one after
         // another, so fewer ports a wave is a shorter slot: FatTree k=8 a2a, HPCC, the longest switch of
         // a slot 191 us on a wave, 134 us on four) and a host item for each of its waves. With more
         // switches than that, a wave each runs more of them side by side.
-        const bool by_group = L.by_group && wd.ns + (nhw + WAVES - 1) / WAVES <= L.by_group * T;
+        const bool by_group = L.by_group && runs_by_group(wd.nh, wd.ns, hpw, T);
         const int ngh = (nhw + WAVES - 1) / WAVES;
         const int first = by_group ? rank : rank * WAVES + wv, step = by_group ? T : T * WAVES;
-        const int host_items = by_group ? ngh : nhw, items = host_items + wd.ns;
+        const int hosts = by_group ? ngh : nhw, items = hosts + wd.ns;
         const long long t_world = wall_clock64();
         for (;;)
         {
@@ -181,7 +181,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
 #ifdef RD_PROF
                 const long long q0 = wall_clock64();
 #endif
-                if (it < host_items)
+                if (it < hosts)
                 {
                     const int hi = by_group ? it * WAVES + wv : it;
                     const int e0 = hi * hpw, n = wd.nh - e0 < hpw ? wd.nh - e0 : hpw;
@@ -193,7 +193,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
                 }
                 else
                 {
-                    const int x = wd.s0 + (it - host_items);
+                    const int x = wd.s0 + (it - hosts);
                     const int deg = s.si[x].deg;
                     bool busy = false;
                     const bool run = s.sw_busy[x] || __any(switch_has_input(s, x, sl, lane, 64));
@@ -226,7 +226,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
                     }
                 }
 #ifdef RD_PROF
-                (it < host_items ? ph : psw) += wall_clock64() - q0;
+                (it < hosts ? ph : psw) += wall_clock64() - q0;
 #endif
             }
 #ifdef RD_PROF
