@@ -129,6 +129,23 @@ static void lone_world()
             CHECK(x.hpw >= 1 && x.hpw <= 64, "k=%d alone on %d: %d hosts an item", k, cap, x.hpw);
         }
 }
+static void one_rule()
+{
+    // what runs by workgroup has a workgroup for each of its items, and what does not was given hosts per
+    // item for a wave each (where any number of them fits)
+    for (int k : {4, 8, 16})
+        for (int W : {1, 2, 3, 4, 12, 24, 40, 130, 256})
+        {
+            std::vector<int> h, s;
+            fattrees(k, W, h, s);
+            const rd::LaunchShape x = rd::launch_shape(h.data(), s.data(), W, 256, true, 0, 0);
+            const bool by_group = rd::runs_by_group(h[0], s[0], x.hpw, x.T);
+            const int group = rd::group_items(h[0], s[0], x.hpw), wave = rd::wave_items(h[0], s[0], x.hpw);
+            CHECK(!by_group || group <= x.T, "%d of k=%d: %d workgroup items on %d", W, k, group, x.T);
+            CHECK(by_group || wave <= 4 * x.T || s[0] + 1 > 4 * x.T, "%d of k=%d: %d wave items on %d workgroups", W, k, wave, x.T);
+            CHECK(x.T * W <= 256, "%d of k=%d: teams of %d", W, k, x.T);
+        }
+}
 
 int main(int argc, char **argv)
 {
@@ -137,6 +154,8 @@ int main(int argc, char **argv)
         out_buckets();
     else if (!strcmp(what, "lone_world"))
         lone_world();
+    else if (!strcmp(what, "one_rule"))
+        one_rule();
     else if (!strcmp(what, "unlike_delays") && argc > 4)
         unlike_delays(argv[2], argv[3], argv[4]);
     else

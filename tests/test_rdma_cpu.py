@@ -70,6 +70,11 @@ def test_lone_world_leaves_room_for_another():
     run_units("lone_world")
 
 
+def test_switches_by_workgroup_only_side_by_side():
+    """The kernel runs a world's switches on workgroups by the rule its launch shape was chosen by."""
+    run_units("one_rule")
+
+
 def test_serving_loop_on_cpu(tmp_path):
     """The serving loop (trd_server_*) with the kernel's steps on the CPU: four reference jobs in an
     arena that holds the two k=8 worlds only one at a time (admission waits for memory), every

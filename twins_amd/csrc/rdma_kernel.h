@@ -36,8 +36,12 @@ struct LaunchCfg
 RD_HD int host_items(int hosts, int hpw) { return (hosts + hpw - 1) / hpw; }
 RD_HD int wave_items(int hosts, int switches, int hpw) { return host_items(hosts, hpw) + switches; }
 RD_HD int group_items(int hosts, int switches, int hpw) { return switches + (host_items(hosts, hpw) + LAUNCH_WAVES - 1) / LAUNCH_WAVES; }
-// does a team of T workgroups run the world by workgroup?
-RD_HD bool runs_by_group(int hosts, int switches, int hpw, int T) { return group_items(hosts, switches, hpw) <= 3 * T; }
+// Does a team of T workgroups run the world by workgroup? Where all of it fits side by side: with a second
+// round of workgroups a slot takes longer than with a wave each (kernel time by workgroup up to three
+// rounds, and side by side only: FatTree k=16 (DCQCN) alone on 128 workgroups 62 and 38.5 ms, two k=16
+// worlds 73 and 54, four k=8 worlds 39 and 30, 101 uneven ones on teams of 8 217 and 155; nothing of
+// 17 batches was slower).
+RD_HD bool runs_by_group(int hosts, int switches, int hpw, int T) { return group_items(hosts, switches, hpw) <= T; }
 
 // The launch shape: one team size and hosts per host item. Every world that fits runs at once, each
 // on its share of the GPU (worlds queued behind others leave it idle when few are left). A slot
@@ -49,7 +53,7 @@ RD_HD bool runs_by_group(int hosts, int switches, int hpw, int T) { return group
 // k=8 (HPCC) alone 104, 85 and 85 ms on 128 workgroups at 2 and 112 and 208 at 1; two 512-host
 // leaf-spines 124, 107 and 121 ms on 128 workgroups each at 1, 2 and 4.
 // A world alone takes at most half of the GPU (as one of the TCP model does), so that two callers'
-// are resident together: a team is resident as a whole or waits at its barrier for ever.
+// are resident together: a team of which a part waits for a place waits at its barrier meanwhile.
 constexpr int ALONE = 128;
 struct LaunchShape
 {

@@ -147,11 +147,10 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
         WorldRun &r = s.run[w];
         uint32_t *pend = s.pend + wd.pend_off;
         const int hpw = L.hpw, nhw = host_items(wd.nh, hpw);
-        // Work items: a wave each, or, where the team has about a workgroup per switch, a switch for a
+        // Work items: a wave each, or, where the team has the workgroups (runs_by_group), a switch for a
         // whole workgroup (its ports over four waves: a wave's lanes run unlike events one after
         // another, so fewer ports a wave is a shorter slot: FatTree k=8 a2a, HPCC, the longest switch of
-        // a slot 191 us on a wave, 134 us on four) and a host item for each of its waves. With more
-        // switches than that, a wave each runs more of them side by side.
+        // a slot 191 us on a wave, 134 us on four) and a host item for each of its waves.
         const bool by_group = L.by_group && runs_by_group(wd.nh, wd.ns, hpw, T);
         const int ngh = (nhw + WAVES - 1) / WAVES;
         const int first = by_group ? rank : rank * WAVES + wv, step = by_group ? T : T * WAVES;
