@@ -4,6 +4,7 @@
 #include <cstring>
 #include <fstream>
 #include <string>
+#include <type_traits>
 #include <vector>
 #include "../../../include/twins.h"
 #include "../../../twins_amd/csrc/tcp_state.h"
@@ -122,11 +123,20 @@ static void slot_word()
             }
 }
 
+// What a team's workgroups are told at a world's start takes no plain store: that would stay in the L2
+// of the writer's XCD until a fence writes it back, and the others read it as soon as they are released.
+static void team_words()
+{
+    CHECK((!std::is_assignable<decltype(tw::TeamState::world) &, int>::value), "TCP: world");
+}
+
 int main(int argc, char **argv)
 {
     const char *what = argc > 1 ? argv[1] : "";
     if (!strcmp(what, "footprint") && argc > 2)
         footprint(argv[2]);
+    else if (!strcmp(what, "team_words"))
+        team_words();
     else if (!strcmp(what, "slot_word"))
         slot_word();
     else if (!strcmp(what, "timeout_error") && argc > 2)

@@ -3,6 +3,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 #include "../../../twins_amd/csrc/rdma_model.h"
 #include "../../../twins_amd/csrc/rdma_kernel.h"
@@ -146,6 +147,14 @@ static void one_rule()
             CHECK(x.T * W <= 256, "%d of k=%d: teams of %d", W, k, x.T);
         }
 }
+// What a team's workgroups are told at a world's start takes no plain store (see the TCP check of it)
+static void team_words()
+{
+    CHECK((!std::is_assignable<decltype(rd::TeamState::world) &, int>::value), "world");
+    CHECK((!std::is_assignable<decltype(rd::TeamState::act) &, unsigned>::value), "act");
+    CHECK((!std::is_assignable<decltype(rd::TeamState::stop) &, int>::value), "stop");
+    CHECK((!std::is_assignable<decltype(rd::TeamState::wake) &, unsigned long long>::value), "wake");
+}
 
 int main(int argc, char **argv)
 {
@@ -154,6 +163,8 @@ int main(int argc, char **argv)
         out_buckets();
     else if (!strcmp(what, "lone_world"))
         lone_world();
+    else if (!strcmp(what, "team_words"))
+        team_words();
     else if (!strcmp(what, "one_rule"))
         one_rule();
     else if (!strcmp(what, "unlike_delays") && argc > 4)

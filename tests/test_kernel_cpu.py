@@ -37,6 +37,12 @@ def test_slot_word_holds_any_slot(harness):
     run_units(harness, "slot_word")
 
 
+def test_team_words_are_handed_over_coherently(harness):
+    """The world a team claims (and what goes with it) is stored device-coherently: the words' type takes
+    no other store."""
+    run_units(harness, "team_words")
+
+
 def test_footprint_counts_what_is_packed(harness, tmp_path):
     """tw_world_info's device_bytes (the serving loop's admission) grows with a world's flows, ledger
     places, queues, network and spray streams as the memory packing allocates does."""

@@ -64,6 +64,11 @@ def test_out_buckets_of_unlike_delays():
     run_units("unlike_delays", rdma_util.CONFIG, f"{rdma_util.INPUTS}/ft4.topo", f"{rdma_util.INPUTS}/inc1.csv")
 
 
+def test_team_words_are_handed_over_coherently():
+    """As for the TCP kernel: the world a team claims, its activity, wake-up and stop words."""
+    run_units("team_words")
+
+
 def test_lone_world_leaves_room_for_another():
     """A world alone takes at most half the GPU's workgroups: two launched at once are both resident
     (each waiting for workgroups the other holds, they would end only by their barriers' time limit)."""

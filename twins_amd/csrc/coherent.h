@@ -52,6 +52,31 @@ inline __device__ void coh_store(__attribute__((address_space(1))) T *p, T v)
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 #endif
+// A word that a team's workgroups hand each other and that has no plain access: a plain store stays in the
+// L2 of the writer's XCD until a fence writes it back, and the others, released without one, would read
+// the word as it was before. `at()` is for atomics.
+template <typename T>
+class CohWord
+{
+    T v;
+
+  public:
+    CohWord() = default;
+    CohWord(const CohWord &) = default;
+    CohWord &operator=(const CohWord &) = default; // (host copies of the records that hold one)
+#if defined(__HIPCC__)
+    __host__ __device__
+#endif
+    T get() const { return coh_load(&v); }
+#if defined(__HIPCC__)
+    __host__ __device__
+#endif
+    void set(T x) { coh_store(&v, x); }
+#if defined(__HIPCC__)
+    __host__ __device__
+#endif
+    T *at() { return &v; }
+};
 // a record of whole 8-byte words, word by word (the words' loads or stores issued together)
 template <typename R>
 #if defined(__HIPCC__)

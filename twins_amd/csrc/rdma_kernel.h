@@ -10,10 +10,11 @@ namespace rd
 struct TeamState
 {
     unsigned arrive, gen;
-    int world, err;
-    unsigned act;
-    int stop;
-    unsigned long long wake;
+    twc::CohWord<int> world;
+    int err;
+    twc::CohWord<unsigned> act;
+    twc::CohWord<int> stop;
+    twc::CohWord<unsigned long long> wake;
     unsigned long long prof[2]; // (profiling builds: the slot's longest host and switch items)
 };
 // one launch: teams of T workgroups take worlds queue[0 .. nq) in order (qnext: the next index);

@@ -74,7 +74,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     const long long t_launch = wall_clock64();
     unsigned gen = 0;
 
-    // the team barrier; the last workgroup to arrive runs `last` first. Within a world (fenced
+    // the team barrier; the last workgroup to arrive runs `last` first, whose stores are device-coherent
+    // (a fenced barrier's release is ahead of it). Within a world (fenced
     // false) it has no cache fences: what the workgroups hand each other goes through coherent
     // accesses (rdma_model.h), so each wave only waits for its own stores to complete, and the
     // entities' own records stay in the caches from slot to slot (an agent-scope fence on the
@@ -125,14 +126,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
     {
         // the team's next world (none once the launch's time is up: the host launches again)
         if (barrier([&] {
-                ts->world = wall_clock64() - t_launch > LAUNCH_TICKS ? L.nq : (int)atomicAdd(L.qnext, 1u);
-                ts->act = 0;
-                ts->wake = ~0ull;
-                ts->stop = 0;
+                ts->world.set(wall_clock64() - t_launch > LAUNCH_TICKS ? L.nq : (int)atomicAdd(L.qnext, 1u));
+                ts->act.set(0);
+                ts->wake.set(~0ull);
+                ts->stop.set(0);
             }, true))
             return;
         if (tid == 0)
-            s_w = __hip_atomic_load(&ts->world, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            s_w = ts->world.get();
         __syncthreads();
         if (s_w >= L.nq)
             return;
@@ -162,7 +163,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
             {
                 s_slot = __hip_atomic_load(&r.slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 s_stop = __hip_atomic_load(&r.finished, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ||
-                         __hip_atomic_load(&ts->stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                         ts->stop.get();
                 s_act = 0;
                 s_wake = ~0ull;
             }
@@ -251,20 +252,20 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))
             if (tid == 0)
             {
                 if (s_act)
-                    atomicOr(&ts->act, s_act);
+                    atomicOr(ts->act.at(), s_act);
                 if (s_wake != ~0ull)
-                    atomicMin(&ts->wake, s_wake);
+                    atomicMin(ts->wake.at(), s_wake);
             }
             if (barrier([&] {
 #ifdef RD_PROF
                     atomicAdd(&s.ev[22], atomicExch(&ts->prof[0], 0ull));
                     atomicAdd(&s.ev[23], atomicExch(&ts->prof[1], 0ull));
 #endif
-                    slot_end(s, wd, r, pend, atomicOr(&ts->act, 0u), atomicMin(&ts->wake, ~0ull));
-                    coh_store(&ts->act, 0u);
-                    coh_store(&ts->wake, ~0ull);
+                    slot_end(s, wd, r, pend, atomicOr(ts->act.at(), 0u), atomicMin(ts->wake.at(), ~0ull));
+                    ts->act.set(0);
+                    ts->wake.set(~0ull);
                     if (wall_clock64() - t_launch > LAUNCH_TICKS)
-                        coh_store(&ts->stop, 1);
+                        ts->stop.set(1);
                 }, false))
                 return;
 #ifdef RD_PROF

@@ -79,9 +79,10 @@ __device__ __forceinline__ void world_loop(const BatchT<RUNS> *__restrict__ Bp, 
     // a barrier wait's limit; the server's claim waits as long as a request may take to come
     unsigned long long wait_limit = WAIT_TICKS;
 
-    // The barrier at a world's start and end; the last workgroup to arrive runs `last` first.
-    // Agent-scope release and acquire, so that the world's records, written with plain stores, are
-    // in memory when it ends and no stale copy is read when it starts. The barrier between slots
+    // The barrier at a world's start and end; the last workgroup to arrive runs `last` first, whose
+    // stores are device-coherent (the release is ahead of it). Agent-scope release and acquire, so that
+    // the world's records, written with plain stores, are in memory when it ends and no stale copy is
+    // read when it starts. The barrier between slots
     // (the end of the slot loop) has no cache fence: what workgroups hand each other from slot to
     // slot goes through device-coherent accesses only (coh_load / coh_store, tcp_state.h), so it is
     // enough that every wave's stores have completed (s_waitcnt) before its workgroup arrives; the
@@ -132,10 +133,10 @@ __device__ __forceinline__ void world_loop(const BatchT<RUNS> *__restrict__ Bp, 
         if constexpr (!SRV)
         {
             // the team's next world, from its queue
-            if (team_barrier([&] { ts->world = atomicAdd(Bp->queue_next + P.queue, 1); }))
+            if (team_barrier([&] { ts->world.set(atomicAdd(Bp->queue_next + P.queue, 1)); }))
                 return;
             if (tid == 0)
-                s_w = __hip_atomic_load(&ts->world, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                s_w = ts->world.get();
             __syncthreads();
             const int qi = s_w;
             if (qi >= Bp->wq_len[P.queue])
@@ -167,14 +168,14 @@ __device__ __forceinline__ void world_loop(const BatchT<RUNS> *__restrict__ Bp, 
                         break;
                     __builtin_amdgcn_s_sleep(8);
                 }
-                ts->world = got;
+                ts->world.set(got);
             });
             wait_limit = WAIT_TICKS;
             if (err)
                 return;
             if (tid == 0)
             {
-                s_w = __hip_atomic_load(&ts->world, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                s_w = ts->world.get();
                 if (s_w >= 0)
                     s_b = reinterpret_cast<const BatchT<RUNS> *>(S.req[(size_t)q * S.cap + s_w].batch);
             }

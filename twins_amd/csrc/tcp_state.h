@@ -310,7 +310,8 @@ struct alignas(128) TeamState
     unsigned pad1;
     unsigned long long go; // (nobody waits for gen and go at the same time)
     unsigned pad2[28];
-    int32_t world, err;
+    twc::CohWord<int32_t> world; // what the last workgroup to arrive at a world's start claimed
+    int32_t err;
     unsigned slot_arrive[2];    // workgroups that have arrived, and << 16 those with activity
     unsigned long long wake[2]; // ~ of the earliest wake-up of those without
     unsigned long long prof[4]; // TW_PROF: this slot's maxima (hosts, switches, work); last ticket time
