@@ -102,13 +102,24 @@ static void run_cpu(BatchT<RUNS> &B, int64_t budget)
                         Md::spray_init(B, W, lanes[q], t, L, sp[q]);
                     for (;;)
                     {
+                        // (spray_pick, its minimum, ballot and shuffles over the lanes by loops)
+                        uint32_t m = Md::SPRAY_NONE;
                         for (int q = 0; q < k; q++)
-                            Md::spray_put(lanes[q], L, sp[q]);
-                        bool done = true;
-                        for (int q = 0; q < k; q++)
-                            done &= Md::spray_pick(B, W, R, lanes[q], t, L, sp[q]);
-                        if (done)
+                            m = std::min(m, Md::spray_key(lanes[q], sp[q]));
+                        if (m == Md::SPRAY_NONE)
                             break;
+                        uint64_t same = 0;
+                        for (int q = 0; q < k; q++)
+                        {
+                            same |= (uint64_t)(Md::spray_key(lanes[q], sp[q]) != Md::SPRAY_NONE && Md::spray_key(lanes[q], sp[q]) >> 6 == m >> 6) << q;
+                            L.base[q] = sp[q].p;
+                        }
+                        int best = m & 63;
+                        for (int q = 0; q < k; q++) // (every lane decides, and counts what it cannot, as on the GPU)
+                            best = Md::spray_tie(B, W, R, lanes[q], t, L, m & 63, same & (same - 1));
+                        const uint32_t nr = sp[best].head >> 20;
+                        for (int q = 0; q < k; q++)
+                            Md::spray_take(B, W, lanes[q], t, L, sp[q], best, nr);
                     }
                     for (int q = 0; q < k; q++)
                         Md::spray_end(B, W, lanes[q], L, sp[q]);

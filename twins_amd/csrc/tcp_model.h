@@ -2832,8 +2832,8 @@ struct Model
     // same draw (each carries the stream); the winner records it. Heads and route counts of the
     // first 32 arrivals of a port sit in LDS (computed by the port's lane beforehand); frames are
     // read only to break equal times. The phases (init, then pick until done, then end) run with
-    // wave_sync() between them; a CPU check runs each phase over the lanes in turn, and exchanges the
-    // heads by a phase of its own (spray_put) before every pick.
+    // wave_sync() between them; a CPU check runs each phase over the lanes in turn, with a loop over them
+    // for spray_pick's minimum, ballot and shuffles.
     static constexpr int SPRAY_CACHE = 32;
     static constexpr uint32_t SPRAY_NONE = 0xFFFFFFFFu;
     struct Spray
@@ -2881,25 +2881,48 @@ struct Model
         for (int i = 0; i < 6; i++)
             sp.g.s[i] = gs.s[i];
     }
-    static __device__ void spray_put(const SwLane &x, const SwLds &L, Spray &sp)
+    // a lane's head as the lanes' minimum takes it: its time, then its port
+    static __device__ uint32_t spray_key(const SwLane &x, const Spray &sp)
     {
-        if (!x.active)
-            return;
-        L.cnt[x.q] = (int)sp.head;
-        L.base[x.q] = sp.p;
+        return sp.head == SPRAY_NONE ? SPRAY_NONE : (sp.head & 0xFFFFFu) << 6 | (uint32_t)x.q;
     }
+    // Equal times, of port `best` (the first) and the ports `same` after it: in port order, frame_before
+    // decides (the reference's scan over the ports). L.base: each port's place in its list.
+    static __device__ int spray_tie(Batch &B, World &W, WorldRun *R, const SwLane &x, int64_t t, const SwLds &L, int best, uint64_t same)
+    {
+        for (; same; same &= same - 1)
+        {
+            const int q = __builtin_ctzll(same);
+            if (frame_before(R, lane_input(B, W, x, t, L, q).at(L.base[q]), lane_input(B, W, x, t, L, best).at(L.base[best])))
+                best = q;
+        }
+        return best;
+    }
+    // port `best`'s head, with nr routes (255: a down port), has its draw; its lane goes on to the next
+    static __device__ void spray_take(Batch &B, World &W, const SwLane &x, int64_t t, const SwLds &L, Spray &sp, int best, uint32_t nr)
+    {
+        uint8_t draw = 0;
+        if (nr != 255u && nr)
+            draw = (uint8_t)tw_mrg_integer(sp.g, nr);
+        if (best == x.q)
+        {
+            if (nr != 255u)
+                x.scr_up[x.q * 2 * MAX_TX + sp.p] = draw;
+            sp.p++;
+            sp.head = sp.p < sp.c ? spray_entry(B, W, x, L, sp, t * SLOT_PS, sp.p) : SPRAY_NONE;
+        }
+    }
+#if defined(__HIPCC__)
     // one step of the merge; true when the switch has no arrivals left
     static __device__ bool spray_pick(Batch &B, World &W, WorldRun *R, const SwLane &x, int64_t t, const SwLds &L, Spray &sp)
     {
         if (!x.active || sp.done)
             return true;
         const int k = W.k;
-        const int64_t S0 = t * SLOT_PS;
-#if defined(__HIP_DEVICE_COMPILE__)
         // the earliest head (the first port holding it): a minimum over the switch's lanes by shuffles
         // (a step reading every port's head from LDS in a loop, twice, was most of a sprayed slot)
         const int lane0 = sw_lane_of(L, x) - x.q;
-        uint32_t m = sp.head == SPRAY_NONE ? SPRAY_NONE : (sp.head & 0xFFFFFu) << 6 | (uint32_t)x.q;
+        uint32_t m = spray_key(x, sp);
         for (int d = 1; d < k; d <<= 1)
         {
             const uint32_t u = __shfl_down(m, d);
@@ -2917,60 +2940,15 @@ struct Model
         same &= same - 1; // (but the first)
         if (same)
         {
-            // equal times: port order, frame_before decides (the reference's scan over the ports)
             L.base[x.q] = sp.p;
             wave_sync();
-            for (; same; same &= same - 1)
-            {
-                const int q = __builtin_ctzll(same);
-                if (frame_before(R, lane_input(B, W, x, t, L, q).at(L.base[q]), lane_input(B, W, x, t, L, best).at(L.base[best])))
-                    best = q;
-            }
+            best = spray_tie(B, W, R, x, t, L, best, same);
             wave_sync();
         }
-        const uint32_t nr = __shfl(sp.head, lane0 + best) >> 20;
-#else
-        // the earliest head (the first port holding it)
-        int best = -1;
-        uint32_t bt = SPRAY_NONE;
-        for (int q = 0; q < k; q++)
-        {
-            const uint32_t h = (uint32_t)L.cnt[q] & 0xFFFFFu;
-            if (L.cnt[q] != (int)SPRAY_NONE && (best < 0 || h < bt))
-            {
-                best = q;
-                bt = h;
-            }
-        }
-        if (best < 0)
-        {
-            sp.done = true;
-            return true;
-        }
-        // equal times: port order, frame_before decides (the reference's scan over the ports)
-        for (int q = best + 1; q < k; q++)
-        {
-            if (L.cnt[q] == (int)SPRAY_NONE || ((uint32_t)L.cnt[q] & 0xFFFFFu) != bt)
-                continue;
-            const Frame *f = lane_input(B, W, x, t, L, q).at(L.base[q]);
-            const Frame *b = lane_input(B, W, x, t, L, best).at(L.base[best]);
-            if (frame_before(R, f, b))
-                best = q;
-        }
-        const uint32_t nr = (uint32_t)L.cnt[best] >> 20;
-#endif
-        uint8_t draw = 0;
-        if (nr != 255u && nr)
-            draw = (uint8_t)tw_mrg_integer(sp.g, nr);
-        if (best == x.q)
-        {
-            if (nr != 255u)
-                x.scr_up[x.q * 2 * MAX_TX + sp.p] = draw;
-            sp.p++;
-            sp.head = sp.p < sp.c ? spray_entry(B, W, x, L, sp, S0, sp.p) : SPRAY_NONE;
-        }
+        spray_take(B, W, x, t, L, sp, best, __shfl(sp.head, lane0 + best) >> 20);
         return false;
     }
+#endif
     static __device__ void spray_end(Batch &B, World &W, const SwLane &x, const SwLds &L, Spray &sp)
     {
         if (!x.active)
