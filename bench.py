@@ -224,7 +224,9 @@ def serve_leg(a):
                            small_teams=resident - cus // 8 - rblocks - zl * nl - zm * nm)
     rsrv = rdma.Server(max_blocks=rblocks) if n_rdma else None
     # every serve_check-th request against the oracle (TCP) or the reference's RDMA build, on the
-    # host's cores, each as soon as its result is in (the checks overlap the serving)
+    # host's cores once all results are in: during the serving the checks took the serving thread's
+    # processor (and interpreter lock), and the latencies were theirs (1,000 requests: p50 4.2 s with
+    # the checks beside it, 1.6 s without)
     ref = os.path.join(ROOT, "oracle", "_ref", "twins-rdma-cpu")
 
     def check(i, got):
@@ -237,12 +239,13 @@ def serve_leg(a):
                            capture_output=True, timeout=1800)
             rows = open(out).read().splitlines()
             os.remove(out)
-            return i, rows, got.splitlines()
+            start, fct = got
+            return i, rows, [f"{j} {start[j]} {fct[j]}" for j in range(len(fct)) if fct[j] >= 0]
         out = os.path.join(a.sweep_dir, f"s{i:04d}.csv")
         _, ev, rows = oracle_world(reqs[i][1], out)
-        return i, rows, got
+        return i, rows, list(zip(*got))
     pool = cf.ThreadPoolExecutor(max(1, a.cpu_cores - 2))
-    checks = []
+    results = []
     sid = {}
     arrival, finish = {}, {}
     events = 0
@@ -281,7 +284,7 @@ def serve_leg(a):
                     events += ev[38]
                     inexact += any(ev[j] for j in rdma.INEXACT)
                     if i % a.serve_check == 0:
-                        checks.append(pool.submit(check, i, "".join(f"{j} {start[j]} {fct[j]}\n" for j in range(len(fct)) if fct[j] >= 0)))
+                        results.append((i, (start, fct)))
             else:
                 s_ = srv.state(sid[i])
                 if s_ in (twins_amd.REQ_DONE, twins_amd.REQ_FAILED):
@@ -289,7 +292,7 @@ def serve_leg(a):
                     finish[i] = time.perf_counter() - t_start
                     events += ev[26]
                     if i % a.serve_check == 0:
-                        checks.append(pool.submit(check, i, list(zip(est, done))))
+                        results.append((i, (est, done)))
         if time.perf_counter() - last_log > 10:
             last_log = time.perf_counter()
             # (the TCP requests admitted and not yet taken, by their worlds' device footprint)
@@ -323,6 +326,7 @@ def serve_leg(a):
             kind_lat["rdma" if kind else "tcp"] = {"requests": len(xs), "p50_s": round(pct(xs, 0.5), 4), "p99_s": round(pct(xs, 0.99), 4)}
     t_chk = time.time()
     same = total = checked = 0
+    checks = [pool.submit(check, i, got) for i, got in results]
     for f in checks:
         i, rows, got = f.result()
         if rows is None:
