@@ -61,6 +61,7 @@ __device__ __forceinline__ void world_loop(const BatchT<RUNS> *__restrict__ Bp, 
     __shared__ unsigned s_act, s_flags;
     __shared__ unsigned long long s_wake;
     __shared__ const BatchT<RUNS> *s_b;
+    __shared__ int s_id; // (serving: the request's id)
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), nwaves = blockDim.x >> 6;
     const int32_t *team_of = SRV ? Sp->team_of : Bp->team_of;
     const TeamPlan *plans = SRV ? Sp->plan : Bp->plan;
@@ -177,7 +178,15 @@ __device__ __forceinline__ void world_loop(const BatchT<RUNS> *__restrict__ Bp, 
             {
                 s_w = ts->world.get();
                 if (s_w >= 0)
-                    s_b = reinterpret_cast<const BatchT<RUNS> *>(S.req[(size_t)q * S.cap + s_w].batch);
+                {
+                    // (system-scope loads, as the tail's: the host writes a line's entries one after another
+                    // while workgroups read the ones before, and only the workgroup that saw the tail has
+                    // acquired at system scope)
+                    ServerReq *r = S.req + (size_t)q * S.cap + s_w;
+                    s_b = reinterpret_cast<const BatchT<RUNS> *>(
+                        __hip_atomic_load(reinterpret_cast<uint64_t *>(&r->batch), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM));
+                    s_id = __hip_atomic_load(&r->id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                }
             }
             __syncthreads();
             if (s_w < 0)
@@ -227,8 +236,7 @@ __device__ __forceinline__ void world_loop(const BatchT<RUNS> *__restrict__ Bp, 
                     if constexpr (SRV)
                     {
                         __threadfence_system();
-                        __hip_atomic_store(Sp->done + Sp->req[(size_t)P.queue * Sp->cap + s_w].id, 1, __ATOMIC_RELEASE,
-                                           __HIP_MEMORY_SCOPE_SYSTEM);
+                        __hip_atomic_store(Sp->done + s_id, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
                     }
                 }
                 break;
@@ -403,8 +411,7 @@ __device__ __forceinline__ void world_loop(const BatchT<RUNS> *__restrict__ Bp, 
                         if (rank == 0)
                         {
                             __threadfence_system();
-                            __hip_atomic_store(Sp->done + Sp->req[(size_t)P.queue * Sp->cap + s_w].id, 2, __ATOMIC_RELEASE,
-                                               __HIP_MEMORY_SCOPE_SYSTEM);
+                            __hip_atomic_store(Sp->done + s_id, 2, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
                         }
                 }
                 return;
