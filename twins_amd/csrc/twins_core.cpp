@@ -1022,6 +1022,18 @@ static int pack(tw_batch &b, const tw_pack_cfg &cfg)
     std::vector<int32_t> q_cap(L), q_red_k(L), q_limit(L);
     std::vector<TwMrgState> rng(RNG);
     std::vector<WorldRun> run(W);
+    const std::vector<int64_t> none(H, INT64_MAX);
+    const std::vector<long long> no_msg((size_t)NRING * L, msg_word(-1, 0, 0)); // of no slot
+    // (a serving request's uploads are asynchronous copies of these: they outlive them on every way out)
+    struct UploadsEnd
+    {
+        hipStream_t s;
+        ~UploadsEnd()
+        {
+            if (s)
+                (void)hipStreamSynchronize(s);
+        }
+    } uploads_end{b.up};
     SndRec s0;
     memset((void *)&s0, 0, sizeof s0);
     s0.cwnd = INIT_CWND, s0.ssthresh = 0xFFFFFFFFu, s0.first_partial = 1;
@@ -1133,11 +1145,8 @@ static int pack(tw_batch &b, const tw_pack_cfg &cfg)
     ZERO(act_rcv, H * MAX_ACTIVE);
     UP(host_cc, host_cc);
     UP(wake, wake);
-    {
-        std::vector<int64_t> none(H, INT64_MAX);
-        UP(tmin_s, none);
-        UP(tmin_r, none);
-    }
+    UP(tmin_s, none);
+    UP(tmin_r, none);
     ZERO(due, H * MAX_DUE);
     UP(in_link, in_link);
     UP(sw_world, sw_world);
@@ -1153,10 +1162,7 @@ static int pack(tw_batch &b, const tw_pack_cfg &cfg)
     ZERO(q_last_chain, L * CW);
     if ((rc = dev_alloc(b, &B.msg, (size_t)NRING * L * MAX_TX)))
         return rc;
-    {
-        std::vector<long long> init((size_t)NRING * L, msg_word(-1, 0, 0)); // of no slot
-        UP(msg_cnt, init);
-    }
+    UP(msg_cnt, no_msg);
     UP(g_host_sw, g_host_sw);
     UP(g_host_port, g_host_port);
     UP(g_rt_off, g_rt_off);
