@@ -57,6 +57,36 @@ def test_server_results_equal_reference(tmp_path):
 
 
 @pytest.mark.gpu
+def test_teams_of_several_workgroups_claim_side_by_side(tmp_path):
+    """Ten FatTree k=16 requests for eight teams of four workgroups, which all claim at once and some
+    twice: each request's flows and packet-events are those of its world in a batch of its own."""
+    import twins_amd
+    from twins_amd import workloads
+    worlds = []
+    for i in range(10):
+        f = tmp_path / f"f{i}.csv"
+        f.write_text(workloads.pareto_flows(100 + i, 150 + 20 * i, 1024))
+        worlds.append(twins_amd.World(["--k=16", f"--flows={f}", "--tcp=" + ("dctcp", "cubic", "newreno")[i % 3]]))
+    want = []
+    for w in worlds:
+        b = twins_amd.Batch([w])
+        b.run()
+        want.append((*map(list, b.fct(0)), b.counters(0)[26]))
+        b.close()
+    for turn in range(2):
+        print(f"server {turn}", flush=True)
+        srv = twins_amd.Server(arena_bytes=10 << 30, mid_teams=8, mid_size=4, idle_s=1.0)
+        ids = [srv.submit(w) for w in worlds]
+        t0 = time.time()
+        while srv.poll().done < len(ids) and time.time() - t0 < 60:
+            time.sleep(0.002)
+        for i, exp in zip(ids, want):
+            est, done, ev = srv.result(i)
+            assert (list(est), list(done), ev[26]) == exp, f"request {i}"
+        srv.close()
+
+
+@pytest.mark.gpu
 def test_serving_mix_every_request(tmp_path):
     """Config 5 in small: 48 requests (FatTree k 4/8/16, up to 6,000 flows, a quarter with a link
     failure; 30% of them RDMA worlds under DCQCN, HPCC or DCTCP) arriving Poisson at 100/s, served
